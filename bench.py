@@ -59,12 +59,12 @@ def stage_bytes(stats, name):
                 stats["bitmap_reset_bytes"])
     if name == "levels":
         return (kb + 4) * stats["level_elems"]
-    if name == "neighbor_fill":
-        return 108 * N
-    if name == "nodes":
-        # records written (code, is_leaf, origin, width, parent, childs), the
-        # level keys read, and the voxel codes copied out
-        return (2 * kb + 53) * N + 2 * kb * U
+    if name == "emit":
+        # node arrays and neighbor slots written, the parent groups' keys,
+        # groups, first children and child masks read once (per eight nodes),
+        # and the voxel codes copied out; the reference's records are added by
+        # the caller when the same launch writes them
+        return (kb + 161) * N + (kb + 9) * N // 8 + 2 * kb * U
     if name == "attr_write":
         # vertex / edge / face records written, node origin and width read
         return 16 * stats["n_vertices"] + 28 * stats["n_edges"] + 28 * stats["n_faces"] + 16 * N
@@ -78,8 +78,7 @@ def stage_bytes(stats, name):
 # scaled by the same counters on a device-to-device copy of 1 GiB: FETCH_SIZE
 # x 2, WRITE_SIZE x 1; profiles/batch256_hbm_traffic.md).  Used to fill
 # roofline.traffic for this run's launch.
-TRAFFIC_PER_ALG_BYTE = {"attr_write": 1.000, "neighbor_fill": 1.000, "nodes": 1.00,
-                        "unique_level1": 1.00, "voxelize": 4.2}
+TRAFFIC_PER_ALG_BYTE = {"attr_write": 1.000, "unique_level1": 1.00, "voxelize": 4.2}
 
 
 def dedup_gbs(stats, stages):
@@ -377,8 +376,9 @@ def _roofline(stats, stages):
     dev = {k: v for k, v in stages.items() if not k.startswith("setup") and k != "start"}
     dom = max(dev, key=dev.get)
     b = stage_bytes(stats, dom)
-    if dom == "nodes" and "neighbor_fill" not in stages:
-        b += stage_bytes(stats, "neighbor_fill")  # concurrent passes: the node kernels fill
+    if dom == "emit" and "attr_write" not in stages:
+        # the emission writes the records too, where they stand at fixed offsets
+        b += 16 * stats["n_vertices"] + 28 * stats["n_edges"]
     ach = b / (stages[dom] * 1e-3) / 1e9 if stages[dom] > 0 else 0.0
     ratio = TRAFFIC_PER_ALG_BYTE.get(dom)
     return {"bound": "hbm", "kernel": dom, "achieved": round(ach, 1), "peak": HBM_PEAK_GBS,

@@ -1,14 +1,14 @@
 // k_attrs.hip -- node records, neighbors and vertex / edge / face records.
 //
 // Node records (createNode_1 / createNode_2 / createRemainNode,
-// SVO.cu:237-339) are written one thread per node, eight threads per parent
-// group, after the level phase has fixed every node count:
+// SVO.cu:237-339) are written after the level phase has fixed every node
+// count, in output order, from the level arrays:
 //   code    = (group parent << 3) | k
 //   origin  = gridOrigin + width * (float)decode(code)   per axis
 //   isLeaf  = false only for occupied nodes above level 1
 //   childs  = child level offset + 8 * (rank of the node's code in its level) + c
 //   parent  = the parent group's node in the level above
-// The root (the single-code level) is written separately.  Node arrays are
+// The root is its level's single code.  Node arrays are
 // structure-of-arrays; the reference's 168-byte records are produced on copy.
 //
 // Neighbors (SVO.cu:522-565).  REFERENCE: the stored table holds UINT_MAX
@@ -34,38 +34,7 @@ namespace {
 
 constexpr int BLOCK = 256;
 
-struct LevelPtrs {
-  const void* elem[24];
-};
-
-template <typename K>
-__device__ inline void decode_origin(const MeshParams& P, float w, K code, float o[3]) {
-  uint32_t x, y, z;
-  demorton3<K>(code, x, y, z);
-  o[0] = P.origin[0] + w * (float)x;
-  o[1] = P.origin[1] + w * (float)y;
-  o[2] = P.origin[2] + w * (float)z;
-}
-
-__device__ inline void store_code(const NodeArrays& out, uint64_t t, uint64_t c) {
-  if (out.code_bytes == 8) ((uint64_t*)out.code)[t] = c;
-  else ((uint32_t*)out.code)[t] = (uint32_t)c;
-}
-
-__device__ inline void store_childs(uint32_t* ch, uint32_t base, bool valid) {
-  uint4 a, b;
-  if (valid) {
-    a = make_uint4(base, base + 1, base + 2, base + 3);
-    b = make_uint4(base + 4, base + 5, base + 6, base + 7);
-  } else {
-    a = make_uint4(NONE, NONE, NONE, NONE);
-    b = a;
-  }
-  reinterpret_cast<uint4*>(ch)[0] = a;
-  reinterpret_cast<uint4*>(ch)[1] = b;
-}
-
-// Node (group g at `level`, child key k): shared by the node and neighbor kernels.
+// Node (group g at `level`, child key k) of the neighbor kernel.
 template <typename K>
 struct GroupNode {
   bool live;
@@ -105,196 +74,6 @@ __device__ inline GroupNode<K> group_node(int level, KeyLayout<K> kl, const K* e
                           (uint32_t)(r.P & 7));
   }
   return r;
-}
-
-// Everything a node record needs, gathered in two rounds of loads that do not
-// depend on each other within a round: the group arrays, then what is keyed
-// by the mesh and by the first child.
-template <typename K>
-struct NodeIn {
-  K P, e;
-  uint32_t fc, gnext, depth, spn_first;
-  uint64_t g, nn, nbase, off_l, off_p, off_c;
-  LevelSpan sp;
-  float w, ox, oy, oz;
-  bool in;
-};
-
-constexpr int NODES_PT = 4;  // nodes per thread, their loads in flight together
-
-// One thread per node, eight per parent group, NODES_PT nodes per thread
-// BLOCK apart (so stores stay contiguous across a wave).  All loads of the
-// thread's nodes are issued before the first is used.
-template <typename K>
-__global__ __launch_bounds__(BLOCK) void k_emit_nodes(
-    int level, KeyLayout<K> kl, const K* elem_l, uint64_t n_elem_l, const K* elem_next,
-    const uint32_t* group_next, const uint32_t* first_child_next, uint64_t n_groups,
-    const LevelSpan* spans, uint32_t n_levels, const MeshTreeState* state,
-    const MeshNodeLayout* layout, const MeshParams* params, NodeArrays out) {
-  if (out.skip && *out.skip) return;  // graph replay over changed sizes
-  const uint64_t base = (uint64_t)blockIdx.x * BLOCK * NODES_PT + threadIdx.x;
-  const uint32_t k = (uint32_t)(threadIdx.x & 7);
-  NodeIn<K> a[NODES_PT];
-#pragma unroll
-  for (int u = 0; u < NODES_PT; ++u) {  // first loads: the parent group
-    const uint64_t g0 = (base + (uint64_t)u * BLOCK) >> 3;
-    a[u].in = g0 < n_groups;
-    a[u].g = a[u].in ? g0 : 0;
-    a[u].P = elem_next[a[u].g];
-    a[u].fc = first_child_next[a[u].g];
-    a[u].gnext = group_next[a[u].g];
-  }
-  auto mesh_fields = [&](NodeIn<K>& q, uint32_t m) {
-    q.depth = state[m].depth;
-    const MeshNodeLayout* L = layout + m;
-    q.nn = L->n_nodes;
-    q.nbase = L->node_base;
-    q.off_l = L->level_off[level - 1];
-    q.off_p = L->level_off[level];
-    q.off_c = level >= 2 ? L->level_off[level - 2] : 0;
-    q.w = L->width[level - 1];
-    q.sp = spans[(uint64_t)m * n_levels + (level - 1)];
-    q.spn_first = spans[(uint64_t)m * n_levels + level].group_first;
-    q.ox = params[m].origin[0];
-    q.oy = params[m].origin[1];
-    q.oz = params[m].origin[2];
-  };
-#pragma unroll
-  for (int u = 0; u < NODES_PT; ++u) {  // second loads: mesh records, child key
-    const uint32_t m = kl.mesh(a[u].P);
-    // a wave's nodes nearly always share one mesh: its per-mesh records are
-    // then read once for the wave (scalar loads) instead of once per lane
-    const uint32_t m0 = __builtin_amdgcn_readfirstlane(m);
-    if (__all(m == m0)) mesh_fields(a[u], m0);
-    else mesh_fields(a[u], m);
-    const uint64_t j = (uint64_t)a[u].fc + k;
-    a[u].e = j < n_elem_l ? elem_l[j] : (K)0;
-  }
-  if (out.fill_neighbors) {
-    // the nodes' 27 neighbor slots, all NONE (the roots' slots and the
-    // intended semantics' neighbors are written by later kernels), issued
-    // while the child keys are still loading: they need the mesh records
-    // only.  When the wave's 64 nodes are live and consecutive, their 1728
-    // slots are one contiguous run, written by the wave with 16-byte stores.
-#pragma unroll
-    for (int u = 0; u < NODES_PT; ++u) {
-      const NodeIn<K>& q = a[u];
-      const bool live = q.in && q.depth > (uint32_t)level && q.nn != 0;
-      const uint64_t tn = q.nbase + q.off_l + 8ull * (q.g - q.sp.group_first) + k;
-      const uint64_t tb = tn - __lane_id();
-      const uint64_t tb0 =
-          ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(tb >> 32)) << 32) |
-          (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)tb);
-      if (__all(live && tb == tb0)) {
-        // 1728 slots from a 4-byte boundary: up to 3 single slots to reach
-        // a 16-byte boundary, 16-byte stores, then the remaining slots
-        uint32_t* nb = out.neighbors + 27 * tb0;
-        const uint32_t head = (uint32_t)((4 - (((uintptr_t)nb >> 2) & 3)) & 3);
-        const uint32_t lane = __lane_id();
-        if (lane < head) nb[lane] = NONE;
-        uint4* body = (uint4*)(nb + head);
-        const uint32_t n4 = (1728 - head) >> 2;
-        const uint4 none4 = make_uint4(NONE, NONE, NONE, NONE);
-#pragma unroll
-        for (uint32_t i = 0; i < 7; ++i)
-          if (lane + 64 * i < n4) body[lane + 64 * i] = none4;
-        const uint32_t tail = (1728 - head) & 3;
-        if (lane < tail) nb[head + 4 * n4 + lane] = NONE;
-      } else if (live) {
-        uint32_t* nb = out.neighbors + 27 * tn;
-#pragma unroll
-        for (int i = 0; i < 27; ++i) nb[i] = NONE;
-      }
-    }
-  }
-#pragma unroll
-  for (int u = 0; u < NODES_PT; ++u) {
-    const NodeIn<K>& q = a[u];
-    const uint64_t j = (uint64_t)q.fc + k;
-    // a depth-1 tree's level-1 group is no node group; a mesh rejected after
-    // the level phase has no nodes
-    const bool live = q.in && q.depth > (uint32_t)level && q.nn != 0;
-    uint32_t bit =
-        (live && j < n_elem_l && kl.parent(q.e) == q.P) ? 1u << (uint32_t)(q.e & 7) : 0u;
-    bit |= __shfl_xor(bit, 1);
-    bit |= __shfl_xor(bit, 2);
-    bit |= __shfl_xor(bit, 4);
-    if (!live) continue;
-    const uint32_t mask = bit;
-    const bool real = (mask >> k) & 1u;
-    const uint64_t local = q.off_l + 8ull * (q.g - q.sp.group_first) + k;
-    const uint64_t t = q.nbase + local;
-    const uint32_t parent = q.depth == (uint32_t)level + 1
-                                ? (uint32_t)q.off_p  // the root
-                                : (uint32_t)(q.off_p + 8ull * (q.gnext - q.spn_first) +
-                                             (uint32_t)(q.P & 7));
-    const K code = (kl.code(q.P) << 3) | (K)k;
-    uint32_t x, y, z;
-    demorton3<K>(code, x, y, z);
-    store_code(out, t, (uint64_t)code);
-    out.is_leaf[t] = (level == 1 || !real) ? 1 : 0;
-    // gridOrigin + width * Vector3f(x, y, z), per axis (SVO.cu:262)
-    out.origin[3 * t + 0] = q.ox + q.w * (float)x;
-    out.origin[3 * t + 1] = q.oy + q.w * (float)y;
-    out.origin[3 * t + 2] = q.oz + q.w * (float)z;
-    out.width[t] = q.w;
-    out.parent[t] = parent;
-    uint32_t cbase = 0;
-    const bool has_childs = real && level >= 2;
-    if (has_childs) {
-      const uint64_t i = (uint64_t)q.fc + __popc(mask & ((1u << k) - 1u));
-      cbase = (uint32_t)(q.off_c + 8ull * (i - q.sp.elem_first));
-    }
-    store_childs(out.childs + 8 * t, cbase, has_childs);
-  }
-}
-
-template <typename K>
-__global__ void k_emit_roots(KeyLayout<K> kl, LevelPtrs lp, uint32_t n_meshes,
-                             const LevelSpan* spans, uint32_t n_levels,
-                             const MeshTreeState* state, const MeshNodeLayout* layout,
-                             const MeshParams* params, NodeArrays out) {
-  if (out.skip && *out.skip) return;  // graph replay over changed sizes
-  const uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= n_meshes) return;
-  const uint32_t d = state[m].depth;
-  const MeshNodeLayout& L = layout[m];
-  if (d == 0 || L.n_nodes == 0) return;
-  const uint64_t local = L.level_off[d - 1];
-  const uint64_t t = L.node_base + local;
-  const K key = ((const K*)lp.elem[d - 1])[state[m].root_elem];
-  const K code = kl.code(key);
-  const float w = L.width[d - 1];
-  float o[3];
-  decode_origin<K>(params[m], w, code, o);
-  store_code(out, t, (uint64_t)code);
-  out.is_leaf[t] = d == 1 ? 1 : 0;
-  out.origin[3 * t + 0] = o[0];
-  out.origin[3 * t + 1] = o[1];
-  out.origin[3 * t + 2] = o[2];
-  out.width[t] = w;
-  out.parent[t] = NONE;
-  store_childs(out.childs + 8 * t, d >= 2 ? (uint32_t)L.level_off[d - 2] : 0u, d >= 2);
-  // findNeighbors<true> (SVO.cu:528-529): root.neighbors[13] = root index,
-  // every other slot NONE (written here when no fill kernel ran)
-  if (out.fill_neighbors) {
-    for (int i = 0; i < 27; ++i)
-      out.neighbors[27 * t + i] = (i == 13 && d >= 2) ? (uint32_t)local : NONE;
-  } else if (d >= 2) {
-    out.neighbors[27 * t + 13] = (uint32_t)local;
-  }
-  (void)spans;
-  (void)n_levels;
-}
-
-template <typename K>
-__global__ void k_copy_voxels(KeyLayout<K> kl, const K* elem1, uint64_t n, void* out,
-                              int out_bytes) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const K c = kl.code(elem1[i]);
-  if (out_bytes == 8) ((uint64_t*)out)[i] = (uint64_t)c;
-  else ((uint32_t*)out)[i] = (uint32_t)c;
 }
 
 // Grid-stride (n may exceed what one launch can index: 108 bytes of
@@ -353,10 +132,14 @@ __global__ __launch_bounds__(BLOCK) void k_neighbors_level(
 
 // ---------------------------------------------------------------- vertex / edge / face
 // Edge endpoints in units of the node width, in the order of SVO.cu:638-663.
-__constant__ uint8_t EDGE_OFS[12][2][3] = {
-    {{0, 0, 0}, {0, 1, 0}}, {{0, 1, 0}, {1, 1, 0}}, {{1, 1, 0}, {1, 0, 0}}, {{1, 0, 0}, {0, 0, 0}},
-    {{0, 0, 1}, {0, 1, 1}}, {{0, 1, 1}, {1, 1, 1}}, {{1, 1, 1}, {1, 0, 1}}, {{1, 0, 1}, {0, 0, 1}},
-    {{0, 0, 0}, {0, 0, 1}}, {{0, 1, 0}, {0, 1, 1}}, {{1, 1, 0}, {1, 1, 1}}, {{1, 0, 0}, {1, 0, 1}}};
+#define SVO_EDGE_ENDS                                                                           \
+  {{{0, 0, 0}, {0, 1, 0}}, {{0, 1, 0}, {1, 1, 0}}, {{1, 1, 0}, {1, 0, 0}},                      \
+   {{1, 0, 0}, {0, 0, 0}}, {{0, 0, 1}, {0, 1, 1}}, {{0, 1, 1}, {1, 1, 1}},                      \
+   {{1, 1, 1}, {1, 0, 1}}, {{1, 0, 1}, {0, 0, 1}}, {{0, 0, 0}, {0, 0, 1}},                      \
+   {{0, 1, 0}, {0, 1, 1}}, {{1, 1, 0}, {1, 1, 1}}, {{1, 0, 0}, {1, 0, 1}}}
+constexpr uint8_t EDGE_ENDS[12][2][3] = SVO_EDGE_ENDS;  // for tables built when compiling
+__constant__ uint8_t EDGE_OFS[12][2][3] = SVO_EDGE_ENDS;
+#undef SVO_EDGE_ENDS
 // Faces: -x, +x, -y, +y, -z, +z as (lo corner, hi corner) and the cell across.
 __constant__ uint8_t FACE_OFS[6][2][3] = {{{0, 0, 0}, {0, 1, 1}}, {{1, 0, 0}, {1, 1, 1}},
                                           {{0, 0, 0}, {1, 0, 1}}, {{0, 1, 0}, {1, 1, 1}},
@@ -643,87 +426,356 @@ __global__ __launch_bounds__(BLOCK) void k_attr_write(int semantics, NodeArrays 
   }
 }
 
-// Reference records when no record can equal its predecessor (the host has
-// checked that every width is positive, finite and not absorbed by the
-// coordinates, so all corners of a node are distinct and thrust::unique keeps
-// everything): node t's records sit at the identity offsets 8t and 12t.
-// A block handles 64 consecutive nodes: four lanes per node build two
-// vertices and three edges each into LDS, then the block streams its
-// contiguous 8 KiB of vertex records and 21 KiB of edge records out as
-// aligned 16-byte stores (64 * 336 bytes and 64 * 128 bytes are multiples
-// of 16).  The mesh of the first node is found once per block.
-constexpr int REF_NODES = 64;
+// ---------------------------------------------------------------- emission
+// Everything a pass outputs, in one launch.  The outputs are bound by their
+// stores (169 bytes a node and 464 of reference records against about 2 read),
+// and what the memory reaches depends on
+//  * how close together the stores in flight lie: one 16-byte store per thread
+//    with workgroups in address order runs at the rate of a plain fill
+//    (6.7 TB/s), 4 / 8 stores per thread reach 5.9 / 5.6, a grid-stride loop
+//    4.7;
+//  * what a store waits for: origins and widths (16 bytes a node) read back
+//    from memory that the writes keep busy held the edge records at 3.8 TB/s.
+// So the arrays are written by consecutive workgroups in output order: the
+// node arrays of rows of ROW nodes (a thread computes a node into LDS, then
+// the workgroup writes 16-byte pieces), then edge records (two pieces a
+// thread), vertex records, neighbor slots and voxel codes (one piece a
+// thread).  Each part recomputes what it needs of its nodes from the level
+// arrays, a few bytes per group of eight nodes that the caches hold.
+// Measured on 16.1 M nodes with records (10.2 GB): 1,510 us, 6.7 TB/s; a node
+// kernel per level beside a fill, then records from origins and widths, took
+// 2,070 us.
+constexpr int ROW = 512;  // nodes per row = threads per workgroup
+constexpr int EDGE_BLOCKS = 21;  // workgroups per 2 * ROW nodes
+constexpr int VERT_BLOCKS = 8;   // workgroups per row
+constexpr uint32_t BLOCKS_PER_LAUNCH = 1u << 22;  // below 2^32 threads per launch
+constexpr int REC_NODES = 2 * ROW / 21 + 2;  // nodes that a workgroup's edge pieces touch
+constexpr int REC_VALS = 12;  // words per node in LDS: origin (bare, + 0, + w) x 3, owner, padding
 
-__device__ inline void stream_out(const uint32_t* src, uint32_t n_dw, uint32_t* dst) {
-  const uint32_t nq = n_dw >> 2;
-  for (uint32_t q = threadIdx.x; q < nq; q += BLOCK)
-    store_stream(reinterpret_cast<uint4*>(dst) + q, reinterpret_cast<const uint4*>(src)[q]);
-  for (uint32_t d = (nq << 2) + threadIdx.x; d < n_dw; d += BLOCK) dst[d] = src[d];
+// Read-only data through the scalar cache: uniform addresses become scalar loads.
+template <typename T>
+__device__ inline const __attribute__((address_space(4))) T* scalar_ptr(const T* p) {
+  return (const __attribute__((address_space(4))) T*)p;
 }
 
-__global__ __launch_bounds__(BLOCK) void k_ref_records(const float* origin, const float* width,
-                                                       uint64_t n_nodes, const uint64_t* mbase,
-                                                       uint32_t n_meshes, uint32_t* verts,
-                                                       uint32_t* edges) {
-  __shared__ __align__(16) uint32_t sv[REF_NODES * 32];
-  __shared__ __align__(16) uint32_t se[REF_NODES * 84];
-  __shared__ uint32_t s_mesh;
-  const uint64_t first = (uint64_t)blockIdx.x * REF_NODES;
-  if (first >= n_nodes) return;
-  const uint32_t nn = (uint32_t)((n_nodes - first) < REF_NODES ? (n_nodes - first) : REF_NODES);
-  if (threadIdx.x == 0) s_mesh = find_mesh64(mbase, n_meshes, first);
-  __syncthreads();
-  const uint32_t ln = threadIdx.x >> 2, part = threadIdx.x & 3;
-  if (ln < nn) {
-    const uint64_t t = first + ln;
-    uint32_t m = s_mesh;
-    while (m + 1 < n_meshes && mbase[m + 1] <= t) ++m;
-    const uint32_t self = (uint32_t)(t - mbase[m]);
-    NodeGeom g;
-    g.o[0] = origin[3 * t];
-    g.o[1] = origin[3 * t + 1];
-    g.o[2] = origin[3 * t + 2];
-    g.w = width[t];
-    for (int j = 2 * part; j < 2 * part + 2; ++j) {
-      float p[3];
-      ref_corner(g.w, j, p);
-      uint32_t* d = sv + 32 * ln + 4 * j;
-      d[0] = __float_as_uint(p[0]);
-      d[1] = __float_as_uint(p[1]);
-      d[2] = __float_as_uint(p[2]);
-      d[3] = self;
-    }
-    for (int i = 3 * part; i < 3 * part + 3; ++i) {
-      float a[3], b[3];
-      ref_edge(g, i, a, b);
-      uint32_t* d = se + 84 * ln + 7 * i;
-      d[0] = __float_as_uint(a[0]);
-      d[1] = __float_as_uint(a[1]);
-      d[2] = __float_as_uint(a[2]);
-      d[3] = __float_as_uint(b[0]);
-      d[4] = __float_as_uint(b[1]);
-      d[5] = __float_as_uint(b[2]);
-      d[6] = self;
-    }
+// Index of the segment that holds node t (the same t in every lane): the wave
+// compares 64 segment starts at a time.
+__device__ inline uint32_t find_seg(const uint32_t* seg_first, uint32_t n_segs, uint32_t t) {
+  uint32_t lo = 0, n = n_segs;
+  const uint32_t lane = __lane_id();
+  while (true) {
+    const uint32_t step = (n + 63) / 64, i = lane * step;
+    const bool at = i < n && seg_first[lo + i] <= t;
+    const uint32_t last = 63u - (uint32_t)__builtin_clzll(__ballot(at));  // seg_first[lo] <= t
+    lo += last * step;
+    if (step == 1) return __builtin_amdgcn_readfirstlane(lo);
+    n = n - last * step < step ? n - last * step : step;
   }
-  __syncthreads();
-  stream_out(sv, 32 * nn, verts + 32 * first);
-  stream_out(se, 84 * nn, edges + 84 * first);
 }
 
-__global__ void k_ref_totals(uint64_t n_nodes, const uint64_t* mbase, uint32_t n_meshes,
-                             unsigned long long* totals) {
-  const uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m == 0) {
-    totals[0] = 8 * n_nodes;
-    totals[1] = 12 * n_nodes;
-    totals[2] = 0;
+// Runs body(seg, d) for the lanes' nodes t (in ascending lane order; at least
+// t_first), d the node's place in its segment, one segment at a time with the
+// segment uniform over the wave.
+template <typename F>
+__device__ inline void for_segments(const NodeSeg* segs, const uint32_t* seg_first,
+                                    uint32_t n_segs, uint32_t t_first, uint32_t t, bool active,
+                                    F body) {
+  const auto* sg = scalar_ptr(segs) + find_seg(seg_first, n_segs, t_first);
+  while (__any(active)) {
+    if (active && t < sg->t1) {
+      body(sg, t - sg->t0);
+      active = false;
+    }
+    ++sg;
   }
-  if (m < n_meshes) {
-    totals[4 + 3 * m] = 8 * mbase[m];
-    totals[4 + 3 * m + 1] = 12 * mbase[m];
-    totals[4 + 3 * m + 2] = 0;
+}
+
+template <typename K>
+__device__ inline uint32_t axis_of(K code, uint32_t a) {
+  return sizeof(K) == 4 ? compact3_32((uint32_t)code >> a)
+                        : (uint32_t)compact3_64((uint64_t)code >> a);
+}
+
+// Edge piece p (words 4p .. 4p + 3 of a node's 84): the four words' LDS slots,
+// four bits each.  Slot a is the bare origin of axis a (the zero offset,
+// SVO.cu:640-662), 3 + a origin + 0, 6 + a origin + width, 9 the owner.
+struct PieceTable {
+  uint16_t slots[21];
+};
+constexpr PieceTable make_piece_table() {
+  PieceTable t{};
+  for (int p = 0; p < 21; ++p) {
+    uint32_t v = 0;
+    for (int k = 0; k < 4; ++k) {
+      const int word = 4 * p + k, edge = word / 7, c = word % 7;
+      uint32_t slot = 9;
+      if (c < 6) {
+        const uint8_t(&e)[3] = EDGE_ENDS[edge][c / 3];
+        const int a = c % 3;
+        slot = !e[0] && !e[1] && !e[2] ? a : e[a] ? 6 + a : 3 + a;
+      }
+      v |= slot << (4 * k);
+    }
+    t.slots[p] = (uint16_t)v;
   }
+  return t;
+}
+__constant__ PieceTable PIECES = make_piece_table();
+
+// LDS values of one axis of a node's records
+__device__ inline void stage_axis(uint32_t* v, uint32_t a, float o, float w) {
+  v[a] = __float_as_uint(o);
+  v[3 + a] = __float_as_uint(o + 0.0f);
+  v[6 + a] = __float_as_uint(o + w);
+}
+
+// Piece p of a row's edge records from the staged values of its nodes, the
+// first of them node `f` of the row; s_piece holds PIECES.
+__device__ inline uint4 edge_piece(const uint32_t* s_val, const uint32_t* s_piece, uint32_t f,
+                                   uint32_t p) {
+  const uint32_t n = p / 21, slots = s_piece[p - 21 * n];
+  const uint32_t* v = s_val + REC_VALS * (n - f);
+  return make_uint4(v[slots & 15], v[(slots >> 4) & 15], v[(slots >> 8) & 15], v[slots >> 12]);
+}
+
+__device__ inline uint4 vert_piece(float w, uint32_t j, uint32_t owner) {
+  float p[3];
+  ref_corner(w, (int)j, p);
+  return make_uint4(__float_as_uint(p[0]), __float_as_uint(p[1]), __float_as_uint(p[2]), owner);
+}
+
+// Node arrays of one row.
+template <typename K>
+__device__ inline void emit_nodes(const EmitArgs<K>& A, uint64_t row, uint32_t* lds) {
+  // LDS: children base, parent, width, origin, code (two words), leaf bytes
+  uint32_t *s_ch = lds, *s_par = lds + ROW, *s_w = lds + 2 * ROW, *s_org = lds + 3 * ROW,
+           *s_code = lds + 6 * ROW;
+  uint8_t* s_leaf = (uint8_t*)(lds + 8 * ROW);
+  const uint64_t t0 = row * ROW;
+  const uint32_t i = threadIdx.x, t = (uint32_t)t0 + i;
+  const bool wide = A.out.code_bytes == 8;
+  for_segments(A.segs, A.seg_first, A.n_segs, t & ~63u, t, t < A.n_nodes,
+               [&](auto* sg, uint32_t d) {
+    const uint32_t kind = sg->level_kind, level = kind & 255u;
+    const float w = sg->width;
+    uint32_t parent = NONE, child = NONE;
+    bool leaf = level == 1;
+    const K* elem = (const K*)sg->elem;
+    K code;
+    if (kind & SEG_ROOT) {
+      code = A.kl.code(elem[0]);
+      if (level >= 2) child = sg->child0;
+    } else {
+      const uint32_t g = d >> 3, k = d & 7;
+      const K P = elem[g];
+      const uint32_t fc = sg->first_child[g], kids = sg->kids[g];
+      parent = sg->parent0;
+      if (!(kind & SEG_ROOT_CHILD)) parent += 8 * sg->group[g] + (uint32_t)(P & 7);
+      code = (A.kl.code(P) << 3) | (K)k;
+      const bool real = (kids >> k) & 1u;
+      leaf = leaf || !real;
+      if (real && level >= 2) child = sg->child0 + 8 * (fc + __popc(kids & ((1u << k) - 1u)));
+    }
+    s_ch[i] = child;
+    s_par[i] = parent;
+    s_w[i] = __float_as_uint(w);
+    // gridOrigin + width * Vector3f(x, y, z), per axis (SVO.cu:262)
+#pragma unroll
+    for (uint32_t a = 0; a < 3; ++a)
+      s_org[3 * i + a] = __float_as_uint(sg->origin[a] + w * (float)axis_of(code, a));
+    if (wide) {
+      s_code[2 * i] = (uint32_t)code;
+      s_code[2 * i + 1] = (uint32_t)((uint64_t)code >> 32);
+    } else {
+      s_code[i] = (uint32_t)code;
+    }
+    s_leaf[i] = leaf ? 1 : 0;
+  });
+  __syncthreads();
+  const uint64_t n = A.n_nodes - t0 < ROW ? A.n_nodes - t0 : ROW;  // nodes of the row
+  // children: two pieces per node
+#pragma unroll
+  for (uint32_t u = 0; u < 2; ++u) {
+    const uint32_t q = u * ROW + i, ln = q >> 1;
+    if (ln < n) {
+      const uint32_t b = s_ch[ln], c = b + 4 * (q & 1);
+      store_stream((uint4*)(A.out.childs + 8 * t0) + q,
+                   b == NONE ? make_uint4(NONE, NONE, NONE, NONE)
+                             : make_uint4(c, c + 1, c + 2, c + 3));
+    }
+  }
+  // the other arrays: pieces of ROW / 4 words each (origin 3, parent, width,
+  // code 1 or 2), then the leaf bytes
+  auto put = [&](const uint32_t* src, void* dst, uint32_t words, uint32_t q) {
+    if (4 * q < n * words)
+      store_stream((uint4*)((uint32_t*)dst + words * t0) + q, ((const uint4*)src)[q]);
+  };
+  constexpr uint32_t Q = ROW / 4;
+  if (i < 3 * Q) put(s_org, A.out.origin, 3, i);
+  else put(s_par, A.out.parent, 1, i - 3 * Q);
+  if (i < Q) put(s_w, A.out.width, 1, i);
+  else if (i < 3 * Q) {
+    if (wide) put(s_code, A.out.code, 2, i - Q);
+    else if (i < 2 * Q) put(s_code, A.out.code, 1, i - Q);
+  } else if (16 * (i - 3 * Q) < n && i < 3 * Q + ROW / 16) {
+    store_stream((uint4*)(A.out.is_leaf + t0) + (i - 3 * Q), ((const uint4*)s_leaf)[i - 3 * Q]);
+  }
+}
+
+// Piece q of the neighbor slots, the reference's: NONE but for the root's own
+// slot 13 (findNeighbors<true>, SVO.cu:528-529).  The root of a pass of one
+// mesh is its last node; with more roots k_root_slots writes their slots
+// afterwards, so that no fill waits for a lookup.
+template <typename K>
+__device__ inline void emit_neighbors(const EmitArgs<K>& A, uint64_t q) {
+  if (4 * q >= 27 * A.n_nodes) return;
+  uint4 v = make_uint4(NONE, NONE, NONE, NONE);
+  if (A.n_roots == 1 && A.n_nodes > 1) {
+    const uint32_t root = (uint32_t)A.n_nodes - 1;
+    const uint64_t c = 27 * (A.n_nodes - 1) + 13 - 4 * q;  // wraps far up past the slot
+    if (c == 0) v.x = root;
+    else if (c == 1) v.y = root;
+    else if (c == 2) v.z = root;
+    else if (c == 3) v.w = root;
+  }
+  store_stream((uint4*)A.out.neighbors + q, v);
+}
+
+__global__ void k_root_slots(const NodeSeg* segs, uint32_t n_segs, NodeArrays out) {
+  const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= n_segs || (out.skip && *out.skip)) return;
+  const uint32_t kind = segs[s].level_kind;
+  if ((kind & SEG_ROOT) && (kind & 255u) >= 2)
+    out.neighbors[27 * (uint64_t)segs[s].t0 + 13] = segs[s].local0;
+}
+
+// The workgroup stages the 10 values that a node's edge words are made of
+// (three per axis and the owner) and builds its pieces from them: 21 of them
+// per node, EDGE_BLOCKS workgroups of two pieces a thread per 2 * ROW nodes.
+template <typename K>
+__device__ inline void emit_edges(const EmitArgs<K>& A, uint32_t row, uint32_t block,
+                                  uint32_t* lds) {
+  uint32_t *s_val = lds, *s_piece = lds + REC_NODES * REC_VALS;
+  const uint32_t t0 = row * 2 * ROW;
+  const uint32_t f = block * 2 * ROW / 21;  // the workgroup's first node, in its row
+  const uint32_t ln = threadIdx.x / 3, a = threadIdx.x - 3 * ln;
+  const uint32_t t = t0 + f + ln;
+  if (threadIdx.x < 192) {  // three waves hold the 3 * REC_NODES threads
+    const uint32_t wave_t = t0 + f + (threadIdx.x & ~63u) / 3;
+    if (wave_t < A.n_nodes)
+      for_segments(A.segs, A.seg_first, A.n_segs, wave_t, t, ln < REC_NODES && t < A.n_nodes,
+                   [&](auto* sg, uint32_t d) {
+        const bool root = sg->level_kind & SEG_ROOT;
+        const K key = A.kl.code(((const K*)sg->elem)[root ? 0u : d >> 3]);
+        const K code = root ? key : (key << 3) | (K)(d & 7);
+        const float w = sg->width;
+        uint32_t* v = s_val + REC_VALS * ln;
+        stage_axis(v, a, sg->origin[a] + w * (float)axis_of(code, a), w);
+        if (a == 0) v[9] = sg->local0 + d;
+      });
+  } else if (threadIdx.x - 192 < 21) {
+    s_piece[threadIdx.x - 192] = PIECES.slots[threadIdx.x - 192];
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t u = 0; u < 2; ++u) {
+    const uint32_t p = (2 * block + u) * ROW + threadIdx.x;
+    if (t0 + p / 21 < A.n_nodes)
+      store_stream((uint4*)A.edges + 21 * (uint64_t)t0 + p, edge_piece(s_val, s_piece, f, p));
+  }
+}
+
+template <typename K>
+__device__ inline void emit_verts(const EmitArgs<K>& A, uint64_t row, uint32_t block) {
+  const uint32_t p = block * ROW + threadIdx.x;
+  const uint64_t t0 = row * ROW;
+  const uint32_t t = (uint32_t)t0 + (p >> 3), wave_t = (uint32_t)t0 + ((p & ~63u) >> 3);
+  if (wave_t >= A.n_nodes) return;
+  for_segments(A.segs, A.seg_first, A.n_segs, wave_t, t, t < A.n_nodes,
+               [&](auto* sg, uint32_t d) {
+    store_stream((uint4*)A.verts + 8 * t0 + p, vert_piece(sg->width, p & 7, sg->local0 + d));
+  });
+}
+
+// Piece q of the voxel codes: the level-1 keys without their mesh bits.
+template <typename K>
+__device__ inline void emit_voxels(const EmitArgs<K>& A, uint64_t q) {
+  if (A.out.code_bytes == 8) {
+    const uint64_t i = 2 * q;
+    if (i >= A.n_voxels) return;
+    const uint64_t c0 = A.kl.code(A.voxels_in[i]);
+    const uint64_t c1 = i + 1 < A.n_voxels ? A.kl.code(A.voxels_in[i + 1]) : (K)0;
+    store_stream((uint4*)A.voxels + q, make_uint4((uint32_t)c0, (uint32_t)(c0 >> 32),
+                                                  (uint32_t)c1, (uint32_t)(c1 >> 32)));
+  } else {
+    const uint64_t i = 4 * q;
+    if (i >= A.n_voxels) return;
+    const uint32_t cnt = A.n_voxels - i < 4 ? (uint32_t)(A.n_voxels - i) : 4u;
+    K k[4];
+    load_consecutive(A.voxels_in + i, ((uintptr_t)A.voxels_in & 15) == 0, cnt, k);
+    store_stream((uint4*)A.voxels + q,
+                 make_uint4((uint32_t)A.kl.code(k[0]), (uint32_t)A.kl.code(k[1]),
+                            (uint32_t)A.kl.code(k[2]), (uint32_t)A.kl.code(k[3])));
+  }
+}
+
+// Workgroups go round the 8 XCDs in turn.  Of each 128 workgroups of a part
+// (of n), XCD x takes 16 consecutive ones, so that the keys that neighboring
+// workgroups share are found in its L2 (edge records of 16.1 M nodes: 905 us
+// without it, 792 with; the node arrays, whose workgroups share no keys, are
+// faster without it).
+__device__ inline uint32_t xcd_run(uint32_t b, uint32_t n) {
+  return (b | 127u) < n ? (b & ~127u) | ((b & 7u) << 4) | ((b >> 3) & 15u) : b;
+}
+
+// Workgroups of each part, in the order they run.
+struct EmitBlocks {
+  uint32_t nodes, edges, verts, neighbors, voxels;
+};
+
+template <typename K>
+__global__ __launch_bounds__(ROW) void k_emit(EmitArgs<K> A, EmitBlocks B, uint32_t block0) {
+  __shared__ __align__(16) uint32_t lds[8 * ROW + ROW / 4];
+  if (A.out.skip && *A.out.skip) return;  // graph replay over changed sizes
+  uint32_t b = block0 + blockIdx.x;
+  if (b < B.nodes) return emit_nodes(A, b, lds);
+  b -= B.nodes;
+  if (b < B.edges) b = xcd_run(b, B.edges);
+  if (b < B.edges) return emit_edges(A, b / EDGE_BLOCKS, b % EDGE_BLOCKS, lds);
+  b -= B.edges;
+  if (b < B.verts) return emit_verts(A, b / VERT_BLOCKS, b % VERT_BLOCKS);
+  b -= B.verts;
+  if (b < B.neighbors) return emit_neighbors(A, (uint64_t)b * ROW + threadIdx.x);
+  emit_voxels(A, (uint64_t)(b - B.neighbors) * ROW + threadIdx.x);
+}
+
+// The records of nodes that the caller gives: the same pieces from origins
+// and widths in memory, one piece a thread.
+__global__ __launch_bounds__(ROW) void k_ref_records(const float* origin, const float* width,
+                                                     uint64_t n_nodes, uint32_t block0,
+                                                     uint32_t edge_blocks, uint32_t* verts,
+                                                     uint32_t* edges) {
+  __shared__ uint32_t s_val[REC_NODES * REC_VALS], s_piece[21];
+  const uint32_t block = block0 + blockIdx.x;
+  if (block >= edge_blocks) {
+    const uint64_t p = (uint64_t)(block - edge_blocks) * ROW + threadIdx.x, t = p >> 3;
+    if (t < n_nodes)
+      store_stream((uint4*)verts + p, vert_piece(width[t], p & 7, (uint32_t)t));
+    return;
+  }
+  const uint64_t t0 = (uint64_t)(block / EDGE_BLOCKS) * ROW;
+  const uint32_t b = block % EDGE_BLOCKS;
+  const uint32_t f = b * ROW / 21, ln = threadIdx.x / 3, a = threadIdx.x - 3 * ln;
+  const uint64_t t = t0 + f + ln;
+  if (ln < ROW / 21 + 2 && t < n_nodes) {
+    stage_axis(s_val + REC_VALS * ln, a, origin[3 * t + a], width[t]);
+    if (a == 0) s_val[REC_VALS * ln + 9] = (uint32_t)t;
+  }
+  if (threadIdx.x < 21) s_piece[threadIdx.x] = PIECES.slots[threadIdx.x];
+  __syncthreads();
+  const uint32_t p = b * ROW + threadIdx.x;
+  if (t0 + p / 21 < n_nodes)
+    store_stream((uint4*)edges + 21 * t0 + p, edge_piece(s_val, s_piece, f, p));
 }
 
 // 168-byte SVONode records (SVO.h:20-35), one thread per 32-bit word.
@@ -759,37 +811,20 @@ inline uint32_t grid_for(uint64_t threads) { return (uint32_t)((threads + BLOCK 
 }  // namespace
 
 template <typename K>
-void launch_emit_level_nodes(int level, KeyLayout<K> kl, const void* elem_l, uint64_t n_elem_l,
-                             const void* elem_next, const uint32_t* elem_group_next,
-                             const uint32_t* first_child_next, uint64_t n_groups,
-                             const LevelSpan* spans, uint32_t n_levels,
-                             const MeshTreeState* state, const MeshNodeLayout* layout,
-                             const MeshParams* params, NodeArrays out, hipStream_t s) {
-  if (n_groups == 0) return;
-  hipLaunchKernelGGL(k_emit_nodes<K>, dim3(grid_for((8 * n_groups + NODES_PT - 1) / NODES_PT)),
-                     dim3(BLOCK), 0, s, level, kl,
-                     (const K*)elem_l, n_elem_l, (const K*)elem_next, elem_group_next,
-                     first_child_next, n_groups, spans, n_levels, state, layout, params, out);
-}
-
-template <typename K>
-void launch_emit_roots(KeyLayout<K> kl, void* const* level_elems, uint32_t n_meshes,
-                       const LevelSpan* spans, uint32_t n_levels, const MeshTreeState* state,
-                       const MeshNodeLayout* layout, const MeshParams* params, int semantics,
-                       NodeArrays out, hipStream_t s) {
-  (void)semantics;
-  LevelPtrs lp;
-  for (uint32_t l = 0; l < 24; ++l) lp.elem[l] = l < n_levels ? level_elems[l] : nullptr;
-  hipLaunchKernelGGL(k_emit_roots<K>, dim3((n_meshes + 63) / 64), dim3(64), 0, s, kl, lp,
-                     n_meshes, spans, n_levels, state, layout, params, out);
-}
-
-template <typename K>
-void launch_copy_voxels(KeyLayout<K> kl, const void* elem1, uint64_t n, void* out,
-                        int out_bytes, hipStream_t s) {
-  if (n == 0) return;
-  hipLaunchKernelGGL(k_copy_voxels<K>, dim3(grid_for(n)), dim3(BLOCK), 0, s, kl,
-                     (const K*)elem1, n, out, out_bytes);
+void launch_emit(const EmitArgs<K>& a, hipStream_t s) {
+  const uint32_t rows = (uint32_t)((a.n_nodes + ROW - 1) / ROW);
+  auto blocks = [](uint64_t words) { return (uint32_t)(((words + 3) / 4 + ROW - 1) / ROW); };
+  const EmitBlocks b{rows, a.records ? EDGE_BLOCKS * ((rows + 1) / 2) : 0,
+                     a.records ? VERT_BLOCKS * rows : 0,
+                     a.neighbors ? blocks(27 * a.n_nodes) : 0,
+                     blocks(a.n_voxels * (uint64_t)(a.out.code_bytes / 4))};
+  const uint32_t n = b.nodes + b.edges + b.verts + b.neighbors + b.voxels;
+  for (uint32_t b0 = 0; b0 < n; b0 += BLOCKS_PER_LAUNCH)
+    hipLaunchKernelGGL(k_emit<K>, dim3(std::min(n - b0, BLOCKS_PER_LAUNCH)),
+                       dim3(ROW), 0, s, a, b, b0);
+  if (a.neighbors && a.n_roots > 1)
+    hipLaunchKernelGGL(k_root_slots, dim3((a.n_segs + 63) / 64), dim3(64), 0, s, a.segs, a.n_segs,
+                       a.out);
 }
 
 // Sets *flag when any of the n words differs from its expected value.
@@ -849,15 +884,14 @@ void launch_attrs_write(int semantics, const NodeArrays& nodes, uint64_t n_nodes
                      mesh_node_base, n_meshes, blocks, (const uint64_t*)partial, out, mesh_first);
 }
 
-void launch_ref_attrs(const NodeArrays& nodes, uint64_t n_nodes, const uint64_t* mesh_node_base,
-                      uint32_t n_meshes, AttrOut out, hipStream_t s) {
-  hipLaunchKernelGGL(k_ref_totals, dim3((n_meshes + 255) / 256), dim3(BLOCK), 0, s, n_nodes,
-                     mesh_node_base, n_meshes, out.totals);
-  if (n_nodes == 0) return;
-  hipLaunchKernelGGL(k_ref_records, dim3((uint32_t)((n_nodes + REF_NODES - 1) / REF_NODES)),
-                     dim3(BLOCK), 0, s, (const float*)nodes.origin, (const float*)nodes.width,
-                     n_nodes, mesh_node_base, n_meshes, (uint32_t*)out.verts,
-                     (uint32_t*)out.edges);
+void launch_ref_records(const float* origin, const float* width, uint64_t n_nodes,
+                        svo_vertex_t* verts, svo_edge_t* edges, hipStream_t s) {
+  const uint32_t rows = (uint32_t)((n_nodes + ROW - 1) / ROW);
+  const uint32_t n = rows * (EDGE_BLOCKS + VERT_BLOCKS);
+  for (uint32_t b0 = 0; b0 < n; b0 += BLOCKS_PER_LAUNCH)
+    hipLaunchKernelGGL(k_ref_records, dim3(std::min(n - b0, BLOCKS_PER_LAUNCH)), dim3(ROW), 0, s,
+                       origin, width, n_nodes, b0, rows * EDGE_BLOCKS, (uint32_t*)verts,
+                       (uint32_t*)edges);
 }
 
 void launch_pack_aos(const NodeArrays& nodes, uint64_t first, uint64_t n, void* dst,
@@ -875,16 +909,7 @@ void launch_query_neighbors(const uint32_t* neighbors, uint64_t n_nodes, const u
 }
 
 #define SVO_INST(K)                                                                              \
-  template void launch_emit_level_nodes<K>(int, KeyLayout<K>, const void*, uint64_t,             \
-                                           const void*, const uint32_t*, const uint32_t*,        \
-                                           uint64_t, const LevelSpan*, uint32_t,                 \
-                                           const MeshTreeState*, const MeshNodeLayout*,          \
-                                           const MeshParams*, NodeArrays, hipStream_t);          \
-  template void launch_emit_roots<K>(KeyLayout<K>, void* const*, uint32_t, const LevelSpan*,     \
-                                     uint32_t, const MeshTreeState*, const MeshNodeLayout*,      \
-                                     const MeshParams*, int, NodeArrays, hipStream_t);           \
-  template void launch_copy_voxels<K>(KeyLayout<K>, const void*, uint64_t, void*, int,           \
-                                      hipStream_t);                                              \
+  template void launch_emit<K>(const EmitArgs<K>&, hipStream_t);                                 \
   template void launch_neighbors_level<K>(int, KeyLayout<K>, const void*, const uint32_t*,       \
                                           uint64_t, const LevelSpan*, uint32_t,                  \
                                           const MeshTreeState*, const MeshNodeLayout*,           \

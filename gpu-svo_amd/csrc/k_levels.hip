@@ -12,7 +12,8 @@
 //   root        = the only key of its mesh at this level (the reference's
 //                 single-code level), which ends that mesh's tree,
 //   output      = next level's keys (the group parents, already sorted and
-//                 unique) and, per group, the index of its first child.
+//                 unique) and, per group, the index of its first child and the
+//                 mask of the children it has.
 // Level 1 is fused with the de-duplication of the sorted hit keys.  Node
 // records are written later from these arrays (k_attrs.hip), once the node
 // counts are known.
@@ -387,13 +388,15 @@ __device__ inline uint32_t mesh_of_word(const uint64_t* bm_off, uint32_t n_meshe
 // bit would leave about four in five idle at surface densities), and staging
 // turns the lanes' strided stores into whole cache lines.  A key is staged
 // as its 16-bit bit index in the tile (the tile's first key is added at
-// copy-out) and a group as the index of its first key only (its parent is
-// read back from that key), so the workgroup's LDS stays near 26 KB for
-// either key width and six workgroups fit a CU.  A round with more than
+// copy-out) and a group as its word in the round and byte in the word (its
+// parent, first key and child mask are read back from the word), so the
+// workgroup's LDS stays near 26 KB for either key width and six workgroups
+// fit a CU.  A round with more than
 // EMIT_CAP keys (dense tiles) stores its keys and groups directly.  The
 // tile's words are zeroed after they are read.
 constexpr uint32_t EMIT_CAP = 2048;
 static_assert((EMIT_CAP & (EMIT_CAP - 1)) == 0, "the copy-out masks slot indices");
+static_assert(BM_TILE % BLOCK == 0, "a round's words lie inside the tile's LDS arrays");
 static_assert(BM_TILE == BITMAP_TILE_WORDS, "mesh regions start on tile boundaries");
 
 template <typename K>
@@ -401,14 +404,14 @@ __global__ __launch_bounds__(BLOCK) void k_bm_emit(uint32_t* bits, uint64_t n_wo
                                                    const uint64_t* bm_off, uint32_t n_meshes,
                                                    KeyLayout<K> kl, const uint32_t* tile_u,
                                                    const uint32_t* tile_g, K* elem1, K* elem2,
-                                                   uint32_t* first_child2,
+                                                   uint32_t* first_child2, uint8_t* kids2,
                                                    const unsigned long long* counts,
                                                    LevelSpan* spans, uint32_t n_levels,
                                                    MeshTreeState* state, uint64_t* status,
                                                    uint32_t* tickets) {
   __shared__ uint32_t tmp[8];
   __shared__ uint32_t s_word[BM_TILE], s_pre[BM_TILE];
-  __shared__ uint16_t s_idx[BM_TILE], s_key[EMIT_CAP], s_fc[BLOCK * 4];
+  __shared__ uint16_t s_idx[BM_TILE], s_key[EMIT_CAP], s_grp[BLOCK * 4];
   __shared__ K s_kbase;  // key of the tile's bit 0
   const uint64_t tw0 = (uint64_t)blockIdx.x * BM_TILE;
   const uint32_t l0 = threadIdx.x * BM_WPT;
@@ -501,26 +504,24 @@ __global__ __launch_bounds__(BLOCK) void k_bm_emit(uint32_t* bits, uint64_t n_wo
       // nonzero bytes runs as often as the wave's fullest word has them,
       // nearly always four).  A group's first child is the unique key of
       // the byte's lowest set bit (the set bits below it are those of the
-      // lower bytes); its parent is parent(word's key 0) + byte index.
+      // lower bytes); its parent is parent(word's key 0) + byte index, its
+      // child mask the byte itself.
       uint32_t lg = (pre >> 17) - g0;
-      const uint32_t pu_w = pre & 0x1FFFFu;
       if (stage) {
 #pragma unroll
         for (uint32_t b = 0; b < 4; ++b) {
-          if ((word >> (8 * b)) & 0xFFu) {
-            s_fc[lg] = (uint16_t)(pu_w + (b ? __popc(word & ((1u << (8 * b)) - 1u)) : 0u));
-            ++lg;
-          }
+          if ((word >> (8 * b)) & 0xFFu) s_grp[lg++] = (uint16_t)((threadIdx.x << 2) | b);
         }
       } else {
+        const uint32_t pu_w = pre & 0x1FFFFu;
         const K phi = kl.parent(kbase + (K)wb);
-        K* dp = elem2 + (uint64_t)bg + g0;
-        uint32_t* df = first_child2 + (uint64_t)bg + g0;
+        const uint64_t d0 = (uint64_t)bg + g0;
 #pragma unroll
         for (uint32_t b = 0; b < 4; ++b) {
           if ((word >> (8 * b)) & 0xFFu) {
-            dp[lg] = phi | (K)b;
-            df[lg] = bu + pu_w + (b ? __popc(word & ((1u << (8 * b)) - 1u)) : 0u);
+            elem2[d0 + lg] = phi | (K)b;
+            first_child2[d0 + lg] = bu + pu_w + (b ? __popc(word & ((1u << (8 * b)) - 1u)) : 0u);
+            kids2[d0 + lg] = (uint8_t)(word >> (8 * b));
             ++lg;
           }
         }
@@ -542,21 +543,50 @@ __global__ __launch_bounds__(BLOCK) void k_bm_emit(uint32_t* bits, uint64_t n_wo
       }
       // groups, ng <= 4 * BLOCK: one step
       const uint32_t i0 = threadIdx.x;
-      uint32_t f[4], v[4];
+      uint32_t c[4], word[4], pre[4], idx[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) f[j] = s_fc[i0 + j * BLOCK];
+      for (int j = 0; j < 4; ++j) c[j] = s_grp[i0 + j * BLOCK] & (4 * BLOCK - 1);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = s_key[(f[j] - u0) & (EMIT_CAP - 1)];
-      K* dp = elem2 + (uint64_t)bg + g0;
-      uint32_t* df = first_child2 + (uint64_t)bg + g0;
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t wi = r0 + (c[j] >> 2);  // r0 <= BM_TILE - BLOCK
+        word[j] = s_word[wi];
+        pre[j] = s_pre[wi];
+        idx[j] = s_idx[wi];
+      }
+      const uint64_t d0 = (uint64_t)bg + g0;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (i0 + j * BLOCK < ng) {
-          dp[i0 + j * BLOCK] = kl.parent(kbase + (K)v[j]);
-          df[i0 + j * BLOCK] = bu + f[j];
+          const uint32_t sh = 8 * (c[j] & 3u);
+          const uint64_t d = d0 + i0 + j * BLOCK;
+          elem2[d] = kl.parent(kbase + (K)((idx[j] << 5) | sh));
+          first_child2[d] = bu + (pre[j] & 0x1FFFFu) + __popc(word[j] & ((1u << sh) - 1u));
+          kids2[d] = (uint8_t)(word[j] >> sh);
         }
     }
     __syncthreads();
+  }
+}
+
+// Child masks of the level-2 elements from the unique keys of level 1 (the
+// sort path; the bitmap path reads them off its bytes): one thread per group,
+// whose members are at most eight consecutive keys.
+template <typename K>
+__global__ __launch_bounds__(BLOCK) void k_first_kids(const K* elem1, const K* elem2,
+                                                      const uint32_t* first_child2,
+                                                      const unsigned long long* counts,
+                                                      KeyLayout<K> kl, uint8_t* kids2) {
+  const uint64_t n1 = counts[0], n2 = counts[1], stride = (uint64_t)gridDim.x * BLOCK;
+  for (uint64_t g = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; g < n2; g += stride) {
+    const K P = elem2[g];
+    const uint64_t f = first_child2[g];
+    uint32_t mask = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const K e = f + j < n1 ? elem1[f + j] : (K)~(K)P;
+      if (f + j < n1 && kl.parent(e) == P) mask |= 1u << (uint32_t)(e & 7);
+    }
+    kids2[g] = (uint8_t)mask;
   }
 }
 
@@ -579,11 +609,12 @@ template <typename K>
 __global__ __launch_bounds__(BLOCK) void k_level_pass(
     int level, const K* elem, const unsigned long long* n_ptr, KeyLayout<K> kl,
     MeshTreeState* state, uint32_t* group_l, K* elem_next, uint32_t* first_child_next,
-    LevelSpan* spans, uint32_t n_levels, uint64_t* status, uint32_t* ticket, uint32_t epoch,
-    unsigned long long* count_next) {
+    uint8_t* kids_next, LevelSpan* spans, uint32_t n_levels, uint64_t* status, uint32_t* ticket,
+    uint32_t epoch, unsigned long long* count_next) {
   __shared__ K s_edge[2][BLOCK];
   __shared__ K s_key[TILE];
   __shared__ uint32_t s_val[TILE];
+  __shared__ uint8_t s_kid[TILE];
   __shared__ uint32_t tmp[4];
   __shared__ uint32_t s_tile;
   __shared__ uint32_t s_base;
@@ -638,6 +669,7 @@ __global__ __launch_bounds__(BLOCK) void k_level_pass(
       uint32_t rg = exg;
       K pk = r.prev;
       bool hp = r.has_prev;
+      uint32_t mask = 0;  // children of the thread's current group so far
 #pragma unroll
       for (int e = 0; e < EPT; ++e) {
         gv[e] = NONE;
@@ -655,10 +687,13 @@ __global__ __launch_bounds__(BLOCK) void k_level_pass(
             sp.group_first = sp.group_end = 0;
           } else if (fl & 1u) {
             if (fl & 2u) {
+              if (rg > exg) s_kid[rg - 1] = (uint8_t)mask;
               s_key[rg] = kl.parent(key);
               s_val[rg] = (uint32_t)i;
               ++rg;
+              mask = 0;
             }
+            mask |= 1u << (uint32_t)(key & 7);
             gv[e] = bg + rg - 1;
             const bool more = e + 1 < EPT && (uint32_t)(e + 1) < r.cnt;
             const bool hn = more || r.has_next;
@@ -677,6 +712,17 @@ __global__ __launch_bounds__(BLOCK) void k_level_pass(
           hp = true;
         }
       }
+      if (rg > exg) {
+        // the thread's last group may go on past its run: at most seven more
+        // keys, which the next thread or tile holds too
+        const K P = s_key[rg - 1];
+        for (uint64_t i = r.i0 + r.cnt; i < n; ++i) {
+          const K key = elem[i];
+          if (kl.parent(key) != P) break;
+          mask |= 1u << (uint32_t)(key & 7);
+        }
+        s_kid[rg - 1] = (uint8_t)mask;
+      }
     }
     if (vec_out && r.cnt == EPT) {
       uint4* q = (uint4*)(group_l + r.i0);
@@ -692,6 +738,7 @@ __global__ __launch_bounds__(BLOCK) void k_level_pass(
     for (uint32_t i = threadIdx.x; i < tg; i += BLOCK) {
       elem_next[(uint64_t)bg + i] = s_key[i];
       first_child_next[(uint64_t)bg + i] = s_val[i];
+      kids_next[(uint64_t)bg + i] = s_kid[i];
     }
     __syncthreads();
   }
@@ -723,6 +770,13 @@ void launch_level_first(const K* sorted, const unsigned long long* n_sorted, uin
   hipLaunchKernelGGL(k_first_pass<K>, dim3(grid_tiles(cap, blocks)), dim3(BLOCK), 0, s, sorted,
                      n_sorted, kl, (K*)l1.elem, (K*)l2.elem, l2.first_child,
                      spans1, n_levels, status, tickets, 1u, counts);
+  if (l2.kids) {
+    const uint64_t kb = std::min<uint64_t>((cap + BLOCK - 1) / BLOCK, 8192);
+    hipLaunchKernelGGL(k_first_kids<K>, dim3((uint32_t)std::max<uint64_t>(1, kb)), dim3(BLOCK), 0,
+                       s, (const K*)l1.elem, (const K*)l2.elem,
+                       (const uint32_t*)l2.first_child, (const unsigned long long*)counts, kl,
+                       l2.kids);
+  }
 }
 
 size_t bitmap_level_tmp_bytes(uint64_t n_words) {
@@ -755,7 +809,7 @@ void launch_level_first_bitmap(uint32_t* bits, uint64_t n_words, const uint64_t*
   uint64_t* status = (uint64_t*)((char*)lvl_tmp + 256);
   hipLaunchKernelGGL(k_bm_emit<K>, dim3((uint32_t)tiles), dim3(BLOCK), 0, s, bits, n_words,
                      bm_off, n_meshes, kl, (const uint32_t*)tile_u, (const uint32_t*)tile_g,
-                     (K*)l1.elem, (K*)l2.elem, l2.first_child,
+                     (K*)l1.elem, (K*)l2.elem, l2.first_child, l2.kids,
                      (const unsigned long long*)counts, spans1, n_levels, state, status,
                      tickets);
 }
@@ -775,8 +829,8 @@ void launch_level(int level, KeyLayout<K> kl, LevelArrays cur, LevelArrays next,
   // counts[level-1] = elements of this level; counts[level] = elements of the next
   hipLaunchKernelGGL(k_level_pass<K>, dim3(grid_tiles(cur.cap, blocks)), dim3(BLOCK), 0, s,
                      level, (const K*)cur.elem, counts + (level - 1), kl, state,
-                     cur.elem_group, (K*)next.elem, next.first_child, spans, n_levels, status,
-                     tickets + (level - 1), (uint32_t)level, counts + level);
+                     cur.elem_group, (K*)next.elem, next.first_child, next.kids, spans, n_levels,
+                     status, tickets + (level - 1), (uint32_t)level, counts + level);
 }
 
 template void launch_level_first<uint32_t>(const uint32_t*, const unsigned long long*, uint64_t,

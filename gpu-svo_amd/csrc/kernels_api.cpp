@@ -89,7 +89,7 @@ int octree_level(const K* sorted, uint64_t n, int code_bits, K* unique, uint64_t
   if (hipMemcpyAsync(in, sorted, sizeof(K) * n, hipMemcpyHostToDevice, s) == hipSuccess &&
       hipMemcpyAsync(cnt, hn, sizeof hn, hipMemcpyHostToDevice, s) == hipSuccess) {
     const KeyLayout<K> kl{code_bits, (K)(lim - 1)};
-    const LevelArrays l1{e1, nullptr, nullptr, n}, l2{e2, nullptr, fc, n};
+    const LevelArrays l1{e1, nullptr, nullptr, nullptr, n}, l2{e2, nullptr, fc, nullptr, n};
     launch_level_first<K>(in, cnt, n, kl, l1, l2, cnt + 1, spans, 1, Tuning{}.scan_blocks, tmp, s);
     if (hipMemcpyAsync(hc, cnt, sizeof hc, hipMemcpyDeviceToHost, s) == hipSuccess &&
         hipStreamSynchronize(s) == hipSuccess && hipGetLastError() == hipSuccess &&
@@ -177,21 +177,13 @@ int svo_k_ref_vertex_edge(int device, const float* origin, const float* width, u
   float* d_w = (float*)B.get(4 * n_nodes);
   void* d_v = B.get(sizeof(svo_vertex) * 8 * n_nodes);
   void* d_e = B.get(sizeof(svo_edge) * 12 * n_nodes);
-  uint64_t* d_base = (uint64_t*)B.get(16);
-  unsigned long long* d_tot = (unsigned long long*)B.get(64);
-  if (!d_o || !d_w || !d_v || !d_e || !d_base || !d_tot) return SVO_E_OOM;
+  if (!d_o || !d_w || !d_v || !d_e) return SVO_E_OOM;
   hipStream_t s;
   if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) return SVO_E_HIP;
   int st = SVO_E_HIP;
-  const uint64_t base[2] = {0, n_nodes};  // one mesh: owners are node indices
   if (hipMemcpyAsync(d_o, origin, 12 * n_nodes, hipMemcpyHostToDevice, s) == hipSuccess &&
-      hipMemcpyAsync(d_w, width, 4 * n_nodes, hipMemcpyHostToDevice, s) == hipSuccess &&
-      hipMemcpyAsync(d_base, base, 16, hipMemcpyHostToDevice, s) == hipSuccess) {
-    NodeArrays na{};
-    na.origin = d_o;
-    na.width = d_w;
-    AttrOut out{(svo_vertex*)d_v, (svo_edge*)d_e, nullptr, d_tot};
-    launch_ref_attrs(na, n_nodes, d_base, 1, out, s);
+      hipMemcpyAsync(d_w, width, 4 * n_nodes, hipMemcpyHostToDevice, s) == hipSuccess) {
+    launch_ref_records(d_o, d_w, n_nodes, (svo_vertex*)d_v, (svo_edge*)d_e, s);
     if (hipGetLastError() == hipSuccess &&
         hipMemcpyAsync(vertices, d_v, sizeof(svo_vertex) * 8 * n_nodes, hipMemcpyDeviceToHost,
                        s) == hipSuccess &&

@@ -62,25 +62,25 @@ static void trim_peer_caches(const Context* self) {
 // a process makes but not for streams made after others were destroyed (a
 // second context's four lanes were measured on two queues, pairwise
 // serialized).  So lane streams are made once per process and device, the
-// first request making a burst of LANE_BURST main streams and then their
-// side streams, before any other stream of the library (the first context
-// on the device makes the burst before its own copy stream), and contexts
-// borrow them: a context gives its lanes' streams back when it releases its
-// lanes, and the next context reuses them with their queues.
+// first request making a burst of LANE_BURST of them before any other stream
+// of the library (the first context on the device makes the burst before its
+// own copy stream), and contexts borrow them: a context gives its lanes'
+// streams back when it releases its lanes, and the next context reuses them
+// with their queues.
 namespace {
 constexpr int LANE_BURST = 4;
-struct PooledStreams {
-  hipStream_t stream, side;
+struct PooledStream {
+  hipStream_t stream;
   bool busy;
 };
 std::mutex g_stream_pool_mu;
-std::map<int, std::vector<PooledStreams>> g_stream_pool;
+std::map<int, std::vector<PooledStream>> g_stream_pool;
 
-// Appends n (stream, side) pairs to the pool of the current device: the n
-// main streams first, then the side streams.  Caller holds g_stream_pool_mu.
-int grow_pool(std::vector<PooledStreams>& pool, int n) {
+// Appends n streams to the pool of the current device.  Caller holds
+// g_stream_pool_mu.
+int grow_pool(std::vector<PooledStream>& pool, int n) {
   std::vector<hipStream_t> made;
-  for (int i = 0; i < 2 * n; ++i) {
+  for (int i = 0; i < n; ++i) {
     hipStream_t q = nullptr;
     if (hipStreamCreateWithFlags(&q, hipStreamNonBlocking) != hipSuccess) {
       for (hipStream_t m : made) hipStreamDestroy(m);
@@ -88,21 +88,21 @@ int grow_pool(std::vector<PooledStreams>& pool, int n) {
     }
     made.push_back(q);
   }
-  for (int i = 0; i < n; ++i) pool.push_back({made[i], made[n + i], false});
+  for (hipStream_t q : made) pool.push_back({q, false});
   return SVO_OK;
 }
 
 // Makes the first burst of `dev` (the current device) if it has none yet.
 int prepare_streams(int dev) {
   std::lock_guard<std::mutex> lk(g_stream_pool_mu);
-  std::vector<PooledStreams>& pool = g_stream_pool[dev];
+  std::vector<PooledStream>& pool = g_stream_pool[dev];
   return pool.empty() ? grow_pool(pool, LANE_BURST) : SVO_OK;
 }
 
-// Lends a (stream, side) pair of `dev` (the current device) to a lane.
-int take_streams(int dev, hipStream_t& stream, hipStream_t& side) {
+// Lends a stream of `dev` (the current device) to a lane.
+int take_stream(int dev, hipStream_t& stream) {
   std::lock_guard<std::mutex> lk(g_stream_pool_mu);
-  std::vector<PooledStreams>& pool = g_stream_pool[dev];
+  std::vector<PooledStream>& pool = g_stream_pool[dev];
   size_t i = 0;
   while (i < pool.size() && pool[i].busy) ++i;
   if (i == pool.size()) {
@@ -111,13 +111,12 @@ int take_streams(int dev, hipStream_t& stream, hipStream_t& side) {
   }
   pool[i].busy = true;
   stream = pool[i].stream;
-  side = pool[i].side;
   return SVO_OK;
 }
 
-void give_streams(int dev, hipStream_t stream) {
+void give_stream(int dev, hipStream_t stream) {
   std::lock_guard<std::mutex> lk(g_stream_pool_mu);
-  for (PooledStreams& p : g_stream_pool[dev])
+  for (PooledStream& p : g_stream_pool[dev])
     if (p.stream == stream) p.busy = false;
 }
 }  // namespace
@@ -144,13 +143,10 @@ void Context::release_lanes() {
   hipSetDevice(device);
   for (auto& l : lanes) {
     if (l->stream) hipStreamSynchronize(l->stream);
-    if (l->side) hipStreamSynchronize(l->side);
     l->ws.release_all();
     for (auto e : l->events) hipEventDestroy(e);
-    if (l->fork) hipEventDestroy(l->fork);
-    if (l->join) hipEventDestroy(l->join);
     if (l->pinned) hipHostFree(l->pinned);
-    if (l->stream) give_streams(device, l->stream);
+    if (l->stream) give_stream(device, l->stream);
   }
   lanes.clear();
   free_lanes.clear();
@@ -178,14 +174,7 @@ Lane* Context::acquire_lane(int prefer) {
   auto make_lane = [&]() -> bool {
     auto l = std::make_unique<Lane>();
     hipSetDevice(device);
-    if (take_streams(device, l->stream, l->side) != SVO_OK) return false;
-    if (hipEventCreateWithFlags(&l->fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&l->join, hipEventDisableTiming) != hipSuccess) {
-      give_streams(device, l->stream);
-      if (l->fork) hipEventDestroy(l->fork);
-      if (l->join) hipEventDestroy(l->join);
-      return false;
-    }
+    if (take_stream(device, l->stream) != SVO_OK) return false;
     l->ws.ctx = this;
     free_lanes.push_back(l.get());
     lanes.push_back(std::move(l));
@@ -447,7 +436,7 @@ double pass_bytes_bound(const svo_params* p, int kb, uint64_t P, uint64_t T, int
   double lv = 0.0, cap = key_cap;
   for (int l = 1; l <= levels + 1; ++l) {
     if (l >= 2) cap = std::min(cap, cells_at(l));
-    lv += K * cap + (l >= 2 ? 8.0 * cap : 0.0) + 3 * 256.0;
+    lv += K * cap + (l >= 2 ? 9.0 * cap : 0.0) + 4 * 256.0;
   }
   const double n_big = (double)T + rows / 512.0;
   const double ws_common = 12.0 * P + 12.0 * T + (double)order_bytes(T) + 2 * 256.0 + lv +
@@ -801,14 +790,6 @@ struct StageTimer {
   Lane& L;
   std::vector<std::string> names;
   size_t used = 0;
-  // stages timed on the side stream: name, start event, end event (indices
-  // into L.events past the main-stream marks)
-  struct Range {
-    std::string name;
-    size_t a, b;
-  };
-  std::vector<Range> ranges;
-  std::vector<hipEvent_t> side_ev;
   bool off = false;  // no events (a pass under graph capture)
   StageTimer(Context& c, Lane& l, bool disabled = false) : C(c), L(l), off(disabled) {}
   // Timing-only events: no system-scope fence when they complete (a fence
@@ -829,24 +810,6 @@ struct StageTimer {
     names.push_back(name);
     ++used;
   }
-  // Records a timing event on `st` (the side stream); returns its index.
-  size_t side_mark(hipStream_t st) {
-    if (!C.timing || off) return 0;
-    const size_t i = side_ev.size();
-    // side events live in L.events after a fixed block of 64 main marks
-    const size_t slot = 64 + i;
-    while (L.events.size() <= slot) {
-      hipEvent_t e;
-      if (create_event(&e) != hipSuccess) return 0;
-      L.events.push_back(e);
-    }
-    hipEventRecord(L.events[slot], st);
-    side_ev.push_back(L.events[slot]);
-    return i;
-  }
-  void side_range(const char* name, size_t a, size_t b) {
-    if (C.timing) ranges.push_back({name, a, b});
-  }
   // Hands the pass's stage windows and sizes to the call's figures.
   void publish(CallTiming& ct, const svo_pass_stats& ps) {
     std::vector<double> a, b;
@@ -859,15 +822,6 @@ struct StageTimer {
         a.push_back(x);
         b.push_back(y);
         nm.push_back(names[i]);
-      }
-    if (C.timing && ct.ref)
-      for (const Range& r : ranges) {
-        float x = 0, y = 0;
-        hipEventElapsedTime(&x, ct.ref, side_ev[r.a]);
-        hipEventElapsedTime(&y, ct.ref, side_ev[r.b]);
-        a.push_back(x);
-        b.push_back(y);
-        nm.push_back(r.name);
       }
     ct.add(nm, a, b, ps);
   }
@@ -1105,7 +1059,8 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     size_t total = 0;
     // level 1 keeps only its keys: its group index per key is never read
     for (uint32_t l = 1; l <= NL + 1; ++l)
-      total += align256(sizeof(K) * cap[l]) + (l >= 2 ? 2 * align256(4 * cap[l]) : 0);
+      total += align256(sizeof(K) * cap[l]) +
+               (l >= 2 ? 2 * align256(4 * cap[l]) + align256(cap[l]) : 0);
     char* base = nullptr;
     SVO_TRY(W.get("levels", total, (void**)&base));
     for (uint32_t l = 1; l <= NL + 1; ++l) {
@@ -1117,9 +1072,12 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
         base += align256(4 * cap[l]);
         lv[l].first_child = (uint32_t*)base;
         base += align256(4 * cap[l]);
+        lv[l].kids = (uint8_t*)base;
+        base += align256(cap[l]);
       } else {
         lv[l].elem_group = nullptr;
         lv[l].first_child = nullptr;
+        lv[l].kids = nullptr;
       }
     }
   }
@@ -1286,7 +1244,7 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     if (rec) rec->out = out;
   }
   // From here on kernels of this pass write the output block.  On an error
-  // return, wait for both streams before `out` (declared above, so destroyed
+  // return, wait for the stream before `out` (declared above, so destroyed
   // after this guard) gives the block back to the context's cache, where
   // another lane could take it while this pass's kernels still write it.
   struct DrainOnError {
@@ -1295,7 +1253,6 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     ~DrainOnError() {
       if (!armed) return;
       hipStreamSynchronize(L.stream);
-      hipStreamSynchronize(L.side);
       hipGetLastError();
     }
   } drain{L};
@@ -1309,7 +1266,6 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
   na.childs = (uint32_t*)(ob + o_ch);
   na.neighbors = (uint32_t*)(ob + o_nb);
   na.code_bytes = cbytes;
-  na.fill_neighbors = 0;
   na.skip = capture ? rec->d_flag : nullptr;
   out->voxels = ob + o_vx;
   out->verts = (svo_vertex*)(ob + o_v);
@@ -1318,94 +1274,127 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
   out->code_bytes = cbytes;
 
   // ---- B: node records, neighbors, vertex/edge/face records
+  // runs of nodes of one mesh and level, in node order, for the emission
+  if (N >= (1ull << 32)) return SVO_E_OOM;  // 169 bytes a node: beyond the device
+  std::vector<NodeSeg> segs;
+  std::vector<uint32_t> seg_first;
+  uint32_t n_roots = 0;
+  for (uint32_t i = 0; i < n; ++i) {
+    const MeshNodeLayout& Lm = lay[i];
+    if (Lm.n_nodes == 0) continue;
+    ++n_roots;
+    const LevelSpan* sp = h_spans + (uint64_t)i * NL;
+    for (uint32_t l = 1; l <= Lm.depth; ++l) {
+      NodeSeg g{};
+      g.local0 = (uint32_t)Lm.level_off[l - 1];
+      g.t0 = (uint32_t)Lm.node_base + g.local0;
+      g.t1 = (uint32_t)(Lm.node_base + (l < Lm.depth ? Lm.level_off[l] : Lm.n_nodes));
+      g.level_kind = l;
+      g.width = Lm.width[l - 1];
+      for (int a = 0; a < 3; ++a) g.origin[a] = h_par[i].origin[a];
+      g.child0 = l >= 2 ? (uint32_t)Lm.level_off[l - 2] : 0u;
+      if (l == Lm.depth) {
+        g.level_kind |= SEG_ROOT;
+        g.elem = (const K*)lv[l].elem + h_state[i].root_elem;
+      } else {
+        const LevelArrays& up = lv[l + 1];
+        const uint32_t g0 = sp[l - 1].group_first;
+        g.elem = (const K*)up.elem + g0;
+        g.group = up.elem_group + g0;
+        g.first_child = up.first_child + g0;
+        g.kids = up.kids + g0;
+        // mod 2^32: the sums they start are node indices
+        if (l >= 2) g.child0 -= 8u * sp[l - 1].elem_first;
+        g.parent0 = (uint32_t)Lm.level_off[l];
+        if (l + 1 == Lm.depth) g.level_kind |= SEG_ROOT_CHILD;
+        else g.parent0 -= 8u * sp[l].group_first;
+      }
+      seg_first.push_back(g.t0);
+      segs.push_back(g);
+    }
+  }
+  const uint32_t n_segs = (uint32_t)segs.size();
   char* bctl = nullptr;
   const size_t sz_lay = align256(sizeof(MeshNodeLayout) * n), sz_nb = align256(8 * (n + 1)),
-               sz_tot = align256(8 * (4 + 3 * n));
-  SVO_TRY(W.get("bctl", sz_lay + sz_nb + sz_tot, (void**)&bctl));
+               sz_segs = align256(sizeof(NodeSeg) * n * NL), sz_sf = align256(4 * n * NL),
+               sz_up = sz_lay + sz_nb + sz_segs + sz_sf, sz_tot = align256(8 * (4 + 3 * n));
+  SVO_TRY(W.get("bctl", sz_up + sz_tot, (void**)&bctl));
   MeshNodeLayout* d_lay = (MeshNodeLayout*)bctl;
   uint64_t* d_nbase = (uint64_t*)(bctl + sz_lay);
-  unsigned long long* d_tot = (unsigned long long*)(bctl + sz_lay + sz_nb);
+  NodeSeg* d_segs = (NodeSeg*)(bctl + sz_lay + sz_nb);
+  uint32_t* d_seg_first = (uint32_t*)(bctl + sz_lay + sz_nb + sz_segs);
+  unsigned long long* d_tot = (unsigned long long*)(bctl + sz_up);
   if (!capture) {
-    SVO_TRY(L.ensure_pinned(sz_lay + sz_nb + sz_tot));
-    std::memcpy(L.pinned, lay.data(), sizeof(MeshNodeLayout) * n);
-    std::memcpy((char*)L.pinned + sz_lay, node_base.data(), 8 * (n + 1));
-    HIP_TRY(hipMemcpyAsync(bctl, L.pinned, sz_lay + sz_nb, hipMemcpyHostToDevice, s));
+    SVO_TRY(L.ensure_pinned(sz_up + sz_tot));
+    char* up = (char*)L.pinned;
+    std::memcpy(up, lay.data(), sizeof(MeshNodeLayout) * n);
+    std::memcpy(up + sz_lay, node_base.data(), 8 * (n + 1));
+    std::memcpy(up + sz_lay + sz_nb, segs.data(), sizeof(NodeSeg) * n_segs);
+    std::memcpy(up + sz_lay + sz_nb + sz_segs, seg_first.data(), 4 * n_segs);
+    HIP_TRY(hipMemcpyAsync(bctl, up, sz_up, hipMemcpyHostToDevice, s));
   }
-  launch_fill_u32((uint32_t*)d_tot, 0u, sz_tot / 4, s);
   timer.mark("setup_b");
-  // When this pass runs alone on the context, the neighbor fill (a pure
-  // write stream) runs on the side stream beside the node records (bound by
-  // their loads' latency); the roots' neighbor slot is written after the
-  // join.  Concurrent passes already overlap each other, and their extra
-  // streams would outnumber the hardware queues: there the node and root
-  // kernels write the neighbor slots themselves (wave-coalesced stores
-  // beside their record writes).
-  bool side_fill = C.active_passes.load() == 1 && !capture;
-  if (side_fill && (hipEventRecord(L.fork, s) != hipSuccess ||
-                    hipStreamWaitEvent(L.side, L.fork, 0) != hipSuccess)) {
-    hipGetLastError();
-    side_fill = false;  // fill in order instead
-  }
-  if (side_fill) {
-    const size_t e0 = timer.side_mark(L.side);
-    launch_fill_u32(na.neighbors, NONE, 27 * N, L.side);
-    const size_t e1 = timer.side_mark(L.side);
-    timer.side_range("neighbor_fill", e0, e1);
-    if (hipEventRecord(L.join, L.side) != hipSuccess) {
-      hipGetLastError();
-      hipStreamSynchronize(L.side);  // no join event: wait for the fill here
-      side_fill = false;
-    }
-  } else {
-    na.fill_neighbors = 1;
-  }
-  for (uint32_t l = 1; l < NL; ++l)
-    launch_emit_level_nodes<K>((int)l, kl, lv[l].elem, h_counts[l - 1], lv[l + 1].elem,
-                               lv[l + 1].elem_group, lv[l + 1].first_child, h_counts[l], d_spans,
-                               NL, d_state, d_lay, d_par, na, s);
-  if (side_fill && hipStreamWaitEvent(s, L.join, 0) != hipSuccess) {
-    hipStreamSynchronize(L.side);  // the fill writes the output block: let it end first
-    return SVO_E_HIP;
-  }
-  {
-    std::vector<void*> lp(NL + 1, nullptr);
-    for (uint32_t l = 1; l <= NL; ++l) lp[l - 1] = lv[l].elem;
-    launch_emit_roots<K>(kl, lp.data(), n, d_spans, NL, d_state, d_lay, d_par, sem, na, s);
-  }
-  launch_copy_voxels<K>(kl, lv[1].elem, U1, out->voxels, cbytes, s);
-  timer.mark("nodes");
-  if (sem == SVO_SEM_INTENDED)
+  // Reference records stand at the identity offsets when no record can equal
+  // its predecessor: then their totals follow from the layout, and one launch
+  // writes all that the pass outputs.  Else they are counted and written after it.
+  const bool identity =
+      want_attrs && sem == SVO_SEM_REFERENCE && no_adjacent_duplicates(lay, h_par, mstat);
+  EmitArgs<K> ea{};
+  ea.kl = kl;
+  ea.segs = d_segs;
+  ea.seg_first = d_seg_first;
+  ea.n_segs = n_segs;
+  ea.n_roots = n_roots;
+  ea.n_nodes = N;
+  ea.out = na;
+  ea.voxels_in = (const K*)lv[1].elem;
+  ea.n_voxels = U1;
+  ea.voxels = out->voxels;
+  ea.verts = out->verts;
+  ea.edges = out->edges;
+  ea.neighbors = true;
+  ea.records = identity;
+  launch_emit<K>(ea, s);
+  timer.mark("emit");
+  if (sem == SVO_SEM_INTENDED) {
     for (uint32_t l = NL - 1; l >= 1; --l)
       launch_neighbors_level<K>((int)l, kl, lv[l + 1].elem, lv[l + 1].elem_group, h_counts[l],
                                 d_spans, NL, d_state, d_lay, na, s);
-  timer.mark("neighbors");
+    timer.mark("neighbors");
+  }
   void* attr_tmp = nullptr;
-  if (want_attrs && N) {
+  const bool counted = want_attrs && !identity && N;
+  std::vector<uint64_t> tot(4 + 3 * (size_t)n, 0);
+  if (counted) {
+    launch_fill_u32((uint32_t*)d_tot, 0u, sz_tot / 4, s);
     AttrOut ao{out->verts, out->edges, out->faces, d_tot};
-    if (sem == SVO_SEM_REFERENCE && no_adjacent_duplicates(lay, h_par, mstat)) {
-      timer.mark("attr_count");
-      launch_ref_attrs(na, N, d_nbase, n, ao, s);
-    } else {
-      SVO_TRY(W.get("attr_tmp", attr_tmp_bytes(plan.tuning.scan_blocks), &attr_tmp));
-      const uint32_t ab = grid_for(N, 2048, plan.tuning.scan_blocks);
-      launch_attrs_count(sem, na, N, d_nbase, n, ab, attr_tmp, ao, s);
-      timer.mark("attr_count");
-      launch_attrs_write(sem, na, N, d_nbase, n, ab, attr_tmp, ao, s);
+    SVO_TRY(W.get("attr_tmp", attr_tmp_bytes(plan.tuning.scan_blocks), &attr_tmp));
+    const uint32_t ab = grid_for(N, 2048, plan.tuning.scan_blocks);
+    launch_attrs_count(sem, na, N, d_nbase, n, ab, attr_tmp, ao, s);
+    timer.mark("attr_count");
+    launch_attrs_write(sem, na, N, d_nbase, n, ab, attr_tmp, ao, s);
+    timer.mark("attr_write");
+  } else if (identity) {
+    tot[0] = 8 * N;
+    tot[1] = 12 * N;
+    for (uint32_t i = 0; i < n; ++i) {
+      tot[4 + 3 * i] = 8 * node_base[i];
+      tot[4 + 3 * i + 1] = 12 * node_base[i];
     }
   }
-  timer.mark("attr_write");
-  std::vector<uint64_t> tot;
   if (capture) {
-    if (rec->tot.size() != 4 + 3 * (size_t)n) return SVO_E_INVALID;
-    tot = rec->tot;
-    launch_check_equal(d_tot, rec->d_expect + 16 + rec->a1.size(), 8 * (4 + 3 * n), rec->d_flag,
-                       s);
+    if (rec->tot.size() != tot.size()) return SVO_E_INVALID;
+    if (counted) {
+      tot = rec->tot;
+      launch_check_equal(d_tot, rec->d_expect + 16 + rec->a1.size(), 8 * tot.size(), rec->d_flag,
+                         s);
+    }
   } else {
     uint64_t* h_tot = (uint64_t*)L.pinned;
-    HIP_TRY(hipMemcpyAsync(h_tot, d_tot, 8 * (4 + 3 * n), hipMemcpyDeviceToHost, s));
+    if (counted) HIP_TRY(hipMemcpyAsync(h_tot, d_tot, 8 * tot.size(), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     HIP_TRY(hipGetLastError());
-    tot.assign(h_tot, h_tot + 4 + 3 * n);
+    if (counted) tot.assign(h_tot, h_tot + tot.size());
     if (rec) rec->tot = tot;
   }
 
@@ -1491,7 +1480,7 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     drain.armed = false;  // nothing ran: the graph is being recorded
     return SVO_OK;
   }
-  drain.armed = false;  // both streams were synchronized above
+  drain.armed = false;  // the stream was synchronized above
   return SVO_OK;
 }
 
@@ -1532,11 +1521,6 @@ int run_plan_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const 
 int run_pass(Context& C, const std::vector<MeshInput>& in, const std::vector<uint32_t>& sel,
              std::vector<svo_tree*>& trees, std::vector<int>& statuses, CallTiming& ct,
              int lane_pref = -1) {
-  struct ActivePass {
-    Context& c;
-    explicit ActivePass(Context& x) : c(x) { c.active_passes.fetch_add(1); }
-    ~ActivePass() { c.active_passes.fetch_sub(1); }
-  } active(C);
   if (sel.empty()) return SVO_OK;
   Plan plan;
   plan.timing = &ct;
@@ -1551,7 +1535,6 @@ int run_pass(Context& C, const std::vector<MeshInput>& in, const std::vector<uin
   if (st != SVO_OK) {
     // the lane's workspaces are reused by its next pass: let this one end
     hipStreamSynchronize(L->stream);
-    hipStreamSynchronize(L->side);
     hipGetLastError();
     for (uint32_t i : plan.idx) {
       delete trees[i];
@@ -1646,11 +1629,8 @@ BatchPlan::~BatchPlan() {
   for (auto& l : lanes) {
     l->ws.release_all();
     for (auto ev : l->events) hipEventDestroy(ev);
-    if (l->fork) hipEventDestroy(l->fork);
-    if (l->join) hipEventDestroy(l->join);
     if (l->pinned) hipHostFree(l->pinned);
     if (l->stream) hipStreamDestroy(l->stream);
-    if (l->side) hipStreamDestroy(l->side);
   }
   for (auto& o : owned) C.dev_free(o.first, o.second);
 }
@@ -1677,11 +1657,7 @@ int plan_create(Context& C, const std::vector<MeshInput>& user, std::unique_ptr<
   if (sel.size() > 64) return SVO_E_INVALID;
   for (size_t g = 0; g < sel.size(); ++g) {
     auto l = std::make_unique<Lane>();
-    if (hipStreamCreateWithFlags(&l->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipStreamCreateWithFlags(&l->side, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&l->fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&l->join, hipEventDisableTiming) != hipSuccess)
-      return SVO_E_HIP;
+    if (hipStreamCreateWithFlags(&l->stream, hipStreamNonBlocking) != hipSuccess) return SVO_E_HIP;
     l->ws.ctx = &C;
     bp->lanes.push_back(std::move(l));
   }

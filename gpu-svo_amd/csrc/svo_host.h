@@ -38,13 +38,9 @@ struct Workspace {
   size_t total() const;
 };
 
-// One stream and its workspace; one build runs on a lane at a time.  `side`
-// runs work of the pass that overlaps the main stream (forked and joined
-// with `fork` / `join`).
+// One stream and its workspace; one build runs on a lane at a time.
 struct Lane {
   hipStream_t stream = nullptr;
-  hipStream_t side = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr;
   Workspace ws;
   void* pinned = nullptr;  // host readback area
   size_t pinned_bytes = 0;
@@ -80,7 +76,6 @@ struct Context : std::enable_shared_from_this<Context> {
   uint64_t budget = 0;  // 0 = unbounded
   std::atomic<uint64_t> in_use{0};
   std::atomic<uint64_t> ws_bytes{0};  // part of in_use held by lane workspaces (reused)
-  std::atomic<int> active_passes{0};  // pipeline passes running on the context
   std::atomic<int> servers{0};        // live svo_server objects on the context
   Tuning tuning;                      // guarded by mu; a pass works on a snapshot
   std::mutex mu;

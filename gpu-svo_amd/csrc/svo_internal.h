@@ -87,13 +87,15 @@ struct LevelArrays {
   void* elem;            // K[cap]: sorted unique keys of this level (S_l)
   uint32_t* elem_group;  // [cap]: group index (at this level) of each element (l >= 2)
   uint32_t* first_child; // [cap]: for groups of the level below: first member index
+  uint8_t* kids;         // [cap]: for groups of the level below: bit k set if child 8p + k exists
   uint64_t cap;
 };
 // Level 1 from the sorted hit keys: unique codes, their groups, and the
 // level-2 element array (parents).  Counts go to counts[0] (level 1 elements)
 // and counts[1] (level 2 elements).  n_sorted <= cap; `blocks` bounds the
 // persistent grid; `tmp` needs level_tmp_bytes(cap) bytes and is shared with
-// the later levels of the same pass (launch_level_first prepares it).
+// the later levels of the same pass (launch_level_first prepares it).  l2.kids
+// may be null (no child masks).
 template <typename K>
 void launch_level_first(const K* sorted, const unsigned long long* n_sorted, uint64_t cap,
                         KeyLayout<K> kl, LevelArrays l1, LevelArrays l2,
@@ -142,6 +144,32 @@ struct MeshNodeLayout {
   float width[24];       // node width per level
 };
 
+// A run of consecutive nodes of one mesh and level, or one root, in node
+// order; computed on the host beside the layout.  Node t of a level's run is
+// child (t - t0) & 7 of the level's parent group (t - t0) / 8.  One aligned
+// record holds all that the emission needs of a run, so that a workgroup
+// fetches it with one round of scalar loads.
+struct alignas(64) NodeSeg {
+  uint32_t t0, t1;   // nodes [t0, t1) of the pass
+  uint32_t local0;   // index of node t0 within its mesh
+  uint32_t level_kind;  // level in bits 0-7, SEG_* above
+  uint32_t child0;   // children of the node whose first child is element i start at child0 + 8i
+  uint32_t parent0;  // parent of group g: parent0 + 8 * elem_group[g] + (key & 7)
+  float width;
+  float origin[3];   // gridOrigin
+  uint32_t pad[2];
+  // the run's parent groups (level + 1's arrays, from its first group on):
+  // keys, their own groups, first children and child masks; a root's own key
+  const void* elem;
+  const uint32_t* group;
+  const uint32_t* first_child;
+  const uint8_t* kids;
+};
+enum : uint32_t {
+  SEG_ROOT = 1u << 8,       // the root: child0 is its first child (level >= 2)
+  SEG_ROOT_CHILD = 1u << 9, // children of the root: parent0 is the root
+};
+
 struct NodeArrays {
   void* code;            // uint32 or uint64 per node (code_bytes)
   uint8_t* is_leaf;
@@ -151,30 +179,34 @@ struct NodeArrays {
   uint32_t* childs;      // 8 per node
   uint32_t* neighbors;   // 27 per node
   int code_bytes;
-  // Nonzero: the node and root kernels also set each node's 27 neighbor
-  // slots to NONE; zero: a fill kernel does that before them.
-  int fill_neighbors;
   // Graph-captured passes: when *skip is nonzero (a size differs from the
   // recorded run) the node, neighbor and record kernels return at once, so
   // that nothing is written past the recorded layout.  Null otherwise.
   const uint32_t* skip;
 };
 
+// Everything of a pass's output in one launch, in output order: node arrays,
+// voxel codes and, as `neighbors` / `records` ask, the reference's neighbor
+// slots and its vertex and edge records at the identity offsets (8 and 12
+// per node, valid when no record can equal its predecessor).  Every output
+// array starts on a 16-byte boundary and may be written up to the next one.
 template <typename K>
-void launch_emit_level_nodes(int level, KeyLayout<K> kl, const void* elem_l, uint64_t n_elem_l,
-                             const void* elem_next, const uint32_t* elem_group_next,
-                             const uint32_t* first_child_next, uint64_t n_groups,
-                             const LevelSpan* spans, uint32_t n_levels,
-                             const MeshTreeState* state, const MeshNodeLayout* layout,
-                             const MeshParams* params, NodeArrays out, hipStream_t s);
+struct EmitArgs {
+  KeyLayout<K> kl;
+  const NodeSeg* segs;        // in node order
+  const uint32_t* seg_first;  // first node of each
+  uint32_t n_segs, n_roots;
+  uint64_t n_nodes;           // below 2^32 (more would not fit the device)
+  NodeArrays out;
+  const K* voxels_in;  // level-1 keys
+  uint64_t n_voxels;
+  void* voxels;
+  svo_vertex_t* verts;
+  svo_edge_t* edges;
+  bool neighbors, records;
+};
 template <typename K>
-void launch_emit_roots(KeyLayout<K> kl, void* const* level_elems, uint32_t n_meshes,
-                       const LevelSpan* spans, uint32_t n_levels, const MeshTreeState* state,
-                       const MeshNodeLayout* layout, const MeshParams* params, int semantics,
-                       NodeArrays out, hipStream_t s);
-template <typename K>
-void launch_copy_voxels(KeyLayout<K> kl, const void* elem1, uint64_t n, void* out,
-                        int out_bytes, hipStream_t s);
+void launch_emit(const EmitArgs<K>& a, hipStream_t s);
 void launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s);
 // Sets *flag (atomic OR of 1) when the `bytes` bytes (a multiple of 4, both
 // 4-byte aligned) at `got` differ from those at `want`.
@@ -200,10 +232,10 @@ void launch_attrs_count(int semantics, const NodeArrays& nodes, uint64_t n_nodes
 void launch_attrs_write(int semantics, const NodeArrays& nodes, uint64_t n_nodes,
                         const uint64_t* mesh_node_base, uint32_t n_meshes, uint32_t blocks,
                         void* tmp, AttrOut out, hipStream_t s);
-// Reference-semantics records at identity offsets (8 and 12 per node), valid
-// when no record can equal its predecessor; also writes the totals.
-void launch_ref_attrs(const NodeArrays& nodes, uint64_t n_nodes, const uint64_t* mesh_node_base,
-                      uint32_t n_meshes, AttrOut out, hipStream_t s);
+// The reference's vertex and edge records of given nodes (origin 3 floats and
+// width 1 float each) at the identity offsets, owner = the node's index.
+void launch_ref_records(const float* origin, const float* width, uint64_t n_nodes,
+                        svo_vertex_t* verts, svo_edge_t* edges, hipStream_t s);
 // 168-byte SVONode records for nodes [first, first + n) (32-bit codes).
 void launch_pack_aos(const NodeArrays& nodes, uint64_t first, uint64_t n, void* dst,
                      hipStream_t s);
