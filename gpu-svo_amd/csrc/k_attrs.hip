@@ -23,7 +23,8 @@
 // stored table has no other entries (root[13] is the root); a record equal to
 // its predecessor is dropped (uniqueVert / uniqueEdge).  INTENDED: a vertex,
 // edge or face is kept by the same-level sharing node with the smallest
-// index.  Count -> scan -> write, node-major.
+// index.  A word per node says which it keeps; count -> scan -> write,
+// node-major.
 #include <algorithm>
 
 #include "svo_internal.h"
@@ -33,48 +34,6 @@ namespace svo {
 namespace {
 
 constexpr int BLOCK = 256;
-
-// Node (group g at `level`, child key k) of the neighbor kernel.
-template <typename K>
-struct GroupNode {
-  bool live;
-  uint32_t m;
-  K P;            // parent key (element g of the next level)
-  uint64_t local; // node index within its mesh
-  uint32_t parent;
-};
-
-template <typename K>
-__device__ inline GroupNode<K> group_node(int level, KeyLayout<K> kl, const K* elem_next,
-                                          const uint32_t* group_next, uint64_t n_groups,
-                                          const LevelSpan* spans, uint32_t n_levels,
-                                          const MeshTreeState* state,
-                                          const MeshNodeLayout* layout, uint64_t g, uint32_t k) {
-  GroupNode<K> r;
-  r.live = false;
-  r.m = 0;
-  r.P = 0;
-  r.local = 0;
-  r.parent = NONE;
-  if (g >= n_groups) return r;
-  r.P = elem_next[g];
-  r.m = kl.mesh(r.P);
-  const uint32_t depth = state[r.m].depth;
-  if (depth <= (uint32_t)level) return r;  // depth-1 tree: its level-1 group is not a node group
-  const MeshNodeLayout& L = layout[r.m];
-  if (L.n_nodes == 0) return r;  // mesh rejected after the level phase
-  r.live = true;
-  const LevelSpan sp = spans[(uint64_t)r.m * n_levels + (level - 1)];
-  r.local = L.level_off[level - 1] + 8ull * (g - sp.group_first) + k;
-  if (depth == (uint32_t)level + 1) {
-    r.parent = (uint32_t)L.level_off[level];  // the root
-  } else {
-    const LevelSpan spn = spans[(uint64_t)r.m * n_levels + level];
-    r.parent = (uint32_t)(L.level_off[level] + 8ull * (group_next[g] - spn.group_first) +
-                          (uint32_t)(r.P & 7));
-  }
-  return r;
-}
 
 // Grid-stride (n may exceed what one launch can index: 108 bytes of
 // neighbors per node are 2^32 words at 160M nodes).  p is 16-byte aligned.
@@ -89,47 +48,6 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t v, uint64_t n) {
   }
 }
 
-// Neighbor LUTs (MortonLUT.h:531-597) in closed form: slot s = (dx+1) +
-// 3(dy+1) + 9(dz+1); child k's neighbor in direction d is child
-// ((k+d) mod 2 per axis) of the parent-level neighbor floor((k+d)/2).
-__device__ inline void nb_lut(uint32_t k, uint32_t s, uint32_t& pslot, uint32_t& child) {
-  const int d[3] = {(int)(s % 3) - 1, (int)((s / 3) % 3) - 1, (int)(s / 9) - 1};
-  const int mul[3] = {1, 3, 9};
-  int ps = 0, ch = 0;
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    const int c = (int)((k >> a) & 1u) + d[a];
-    const int p = c < 0 ? -1 : (c >> 1);
-    ps += (p + 1) * mul[a];
-    ch |= (c & 1) << a;
-  }
-  pslot = (uint32_t)ps;
-  child = (uint32_t)ch;
-}
-
-template <typename K>
-__global__ __launch_bounds__(BLOCK) void k_neighbors_level(
-    int level, KeyLayout<K> kl, const K* elem_next, const uint32_t* group_next,
-    uint64_t n_groups, const LevelSpan* spans, uint32_t n_levels, const MeshTreeState* state,
-    const MeshNodeLayout* layout, NodeArrays nodes) {
-  if (nodes.skip && *nodes.skip) return;  // graph replay over changed sizes
-  const uint64_t gid = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
-  const uint64_t g = gid >> 3;
-  const uint32_t k = (uint32_t)(gid & 7);
-  const GroupNode<K> gn = group_node(level, kl, elem_next, group_next, n_groups, spans, n_levels,
-                                     state, layout, g, k);
-  if (!gn.live) return;
-  const uint64_t base = layout[gn.m].node_base;
-  const uint32_t* pn_row = nodes.neighbors + 27 * (base + gn.parent);
-  uint32_t* row = nodes.neighbors + 27 * (base + gn.local);
-  for (uint32_t s = 0; s < 27; ++s) {
-    uint32_t ps, ch;
-    nb_lut(k, s, ps, ch);
-    const uint32_t pn = pn_row[ps];
-    row[s] = pn != NONE ? nodes.childs[8 * (base + pn) + ch] : NONE;
-  }
-}
-
 // ---------------------------------------------------------------- vertex / edge / face
 // Edge endpoints in units of the node width, in the order of SVO.cu:638-663.
 #define SVO_EDGE_ENDS                                                                           \
@@ -141,10 +59,10 @@ constexpr uint8_t EDGE_ENDS[12][2][3] = SVO_EDGE_ENDS;  // for tables built when
 __constant__ uint8_t EDGE_OFS[12][2][3] = SVO_EDGE_ENDS;
 #undef SVO_EDGE_ENDS
 // Faces: -x, +x, -y, +y, -z, +z as (lo corner, hi corner) and the cell across.
-__constant__ uint8_t FACE_OFS[6][2][3] = {{{0, 0, 0}, {0, 1, 1}}, {{1, 0, 0}, {1, 1, 1}},
-                                          {{0, 0, 0}, {1, 0, 1}}, {{0, 1, 0}, {1, 1, 1}},
-                                          {{0, 0, 0}, {1, 1, 0}}, {{0, 0, 1}, {1, 1, 1}}};
-__constant__ uint8_t FACE_SLOT[6] = {12, 14, 10, 16, 4, 22};
+constexpr uint8_t FACE_ENDS[6][2][3] = {{{0, 0, 0}, {0, 1, 1}}, {{1, 0, 0}, {1, 1, 1}},
+                                        {{0, 0, 0}, {1, 0, 1}}, {{0, 1, 0}, {1, 1, 1}},
+                                        {{0, 0, 0}, {1, 1, 0}}, {{0, 0, 1}, {1, 1, 1}}};
+constexpr int FACE_SLOT[6] = {12, 14, 10, 16, 4, 22};
 
 // origin + Vector3f(0|w, 0|w, 0|w), with the bare origin for the zero offset
 // (SVO.cu:640-662).
@@ -184,245 +102,21 @@ __device__ inline bool edge_eq(const float* a0, const float* b0, const float* a1
   return (eq3(a0, a1) && eq3(b0, b1)) || (eq3(a0, b1) && eq3(b0, a1));
 }
 
-// Cells sharing corner j: d in {b-1, b} per axis, x fastest (SVO.cu:567-584).
-__device__ inline uint32_t vert_slot(int j, int q) {
-  const int dx = ((j >> 0) & 1) - 1 + ((q >> 0) & 1);
-  const int dy = ((j >> 1) & 1) - 1 + ((q >> 1) & 1);
-  const int dz = ((j >> 2) & 1) - 1 + ((q >> 2) & 1);
-  return (uint32_t)((dx + 1) + 3 * (dy + 1) + 9 * (dz + 1));
-}
-// Cells sharing edge i: the two axes the edge does not run along take
-// {o-1, o}; the running axis takes 0 (SVO.cu:610-627).
-__device__ inline uint32_t edge_slot(int i, int q) {
-  const uint8_t* a = EDGE_OFS[i][0];
-  const uint8_t* b = EDGE_OFS[i][1];
-  int d[3];
-  int bitpos = 0;
-  for (int ax = 0; ax < 3; ++ax) {
-    if (a[ax] != b[ax]) {
-      d[ax] = 0;
+// Writes words [w0, w0 + n) of dst, value(i) the word w0 + i: 16-byte pieces,
+// single words where a piece lies across either end.  dst is 16-byte aligned.
+template <typename F>
+__device__ inline void write_words(uint32_t* dst, uint64_t w0, uint32_t n, uint32_t tid,
+                                   uint32_t threads, F value) {
+  const uint32_t head = (uint32_t)w0 & 3u;  // words of the first piece before w0
+  uint32_t* p = dst + (w0 - head);
+  for (uint32_t q = tid; 4 * q < head + n; q += threads) {
+    const uint32_t i = 4 * q - head;  // wraps for words before w0
+    if (4 * q >= head && i + 4 <= n) {
+      store_stream((uint4*)p + q, make_uint4(value(i), value(i + 1), value(i + 2), value(i + 3)));
     } else {
-      d[ax] = (int)a[ax] - 1 + ((q >> bitpos) & 1);
-      ++bitpos;
+      for (uint32_t j = 0; j < 4; ++j)
+        if (i + j < n) p[4 * (uint64_t)q + j] = value(i + j);
     }
-  }
-  return (uint32_t)((d[0] + 1) + 3 * (d[1] + 1) + 9 * (d[2] + 1));
-}
-
-__device__ inline uint32_t find_mesh64(const uint64_t* base, uint32_t n_meshes, uint64_t t) {
-  uint32_t lo = 0, hi = n_meshes;
-  while (hi - lo > 1) {
-    const uint32_t mid = (lo + hi) >> 1;
-    if (base[mid] <= t) lo = mid; else hi = mid;
-  }
-  return lo;
-}
-
-struct AttrCounts {
-  uint32_t v, e, f;
-};
-
-// Counts (and optionally writes) the records of node t.
-template <bool WRITE>
-__device__ inline AttrCounts node_attrs(int semantics, const NodeArrays& n, uint64_t t,
-                                        uint64_t local, uint64_t vpos, uint64_t epos,
-                                        uint64_t fpos, AttrOut out) {
-  AttrCounts c = {0, 0, 0};
-  const NodeGeom g = load_geom(n, t);
-  const uint32_t self = (uint32_t)local;
-  if (semantics == SVO_SEM_REFERENCE) {
-    float prev[3];
-    if (local > 0) ref_corner(n.width[t - 1], 7, prev);
-    for (int j = 0; j < 8; ++j) {
-      float p[3];
-      ref_corner(g.w, j, p);
-      const bool keep = (j == 0 && local == 0) || !eq3(p, prev);
-      if (keep) {
-        if (WRITE) {
-          svo_vertex_t r;
-          r.p[0] = p[0];
-          r.p[1] = p[1];
-          r.p[2] = p[2];
-          r.owner = self;
-          out.verts[vpos + c.v] = r;
-        }
-        ++c.v;
-      }
-      prev[0] = p[0];
-      prev[1] = p[1];
-      prev[2] = p[2];
-    }
-    float pa[3], pb[3];
-    if (local > 0) {
-      const NodeGeom gp = load_geom(n, t - 1);
-      ref_edge(gp, 11, pa, pb);
-    }
-    for (int i = 0; i < 12; ++i) {
-      float a[3], b[3];
-      ref_edge(g, i, a, b);
-      const bool keep = (i == 0 && local == 0) || !edge_eq(a, b, pa, pb);
-      if (keep) {
-        if (WRITE) {
-          svo_edge_t r;
-          for (int q = 0; q < 3; ++q) {
-            r.a[q] = a[q];
-            r.b[q] = b[q];
-          }
-          r.owner = self;
-          out.edges[epos + c.e] = r;
-        }
-        ++c.e;
-      }
-      for (int q = 0; q < 3; ++q) {
-        pa[q] = a[q];
-        pb[q] = b[q];
-      }
-    }
-    return c;
-  }
-  const uint32_t* nb = n.neighbors + 27 * t;
-  for (int j = 0; j < 8; ++j) {
-    uint32_t owner = self;
-    for (int q = 0; q < 8; ++q) {
-      const uint32_t v = nb[vert_slot(j, q)];
-      owner = v < owner ? v : owner;
-    }
-    if (owner != self) continue;
-    if (WRITE) {
-      const uint8_t ofs[3] = {(uint8_t)(j & 1), (uint8_t)((j >> 1) & 1), (uint8_t)((j >> 2) & 1)};
-      svo_vertex_t r;
-      offset_point(g.o, g.w, ofs, r.p);
-      r.owner = self;
-      out.verts[vpos + c.v] = r;
-    }
-    ++c.v;
-  }
-  for (int i = 0; i < 12; ++i) {
-    uint32_t owner = self;
-    for (int q = 0; q < 4; ++q) {
-      const uint32_t v = nb[edge_slot(i, q)];
-      owner = v < owner ? v : owner;
-    }
-    if (owner != self) continue;
-    if (WRITE) {
-      svo_edge_t r;
-      ref_edge(g, i, r.a, r.b);
-      r.owner = self;
-      out.edges[epos + c.e] = r;
-    }
-    ++c.e;
-  }
-  for (int f = 0; f < 6; ++f) {
-    const uint32_t v = nb[FACE_SLOT[f]];
-    if (v < self) continue;
-    if (WRITE) {
-      svo_edge_t r;
-      offset_point(g.o, g.w, FACE_OFS[f][0], r.a);
-      offset_point(g.o, g.w, FACE_OFS[f][1], r.b);
-      r.owner = self;
-      out.faces[fpos + c.f] = r;
-    }
-    ++c.f;
-  }
-  return c;
-}
-
-__device__ inline void block_range(uint64_t n, uint32_t G, uint32_t b, uint64_t& beg,
-                                   uint64_t& end) {
-  const uint64_t chunk = (n + G - 1) / G;
-  beg = (uint64_t)b * chunk;
-  if (beg > n) beg = n;
-  end = beg + chunk;
-  if (end > n) end = n;
-}
-
-__global__ __launch_bounds__(BLOCK) void k_attr_count(int semantics, NodeArrays nodes,
-                                                      uint64_t n_nodes, const uint64_t* mbase,
-                                                      uint32_t n_meshes, uint32_t G,
-                                                      uint64_t* partial) {
-  if (nodes.skip && *nodes.skip) return;  // graph replay over changed sizes
-  __shared__ uint64_t tmp[4];
-  uint64_t beg, end;
-  block_range(n_nodes, G, blockIdx.x, beg, end);
-  uint64_t sv = 0, se = 0, sf = 0;
-  AttrOut none = {nullptr, nullptr, nullptr, nullptr};
-  uint32_t m = beg < end ? find_mesh64(mbase, n_meshes, beg) : 0;
-  for (uint64_t t = beg + threadIdx.x; t < end; t += BLOCK) {
-    while (m + 1 < n_meshes && mbase[m + 1] <= t) ++m;
-    const AttrCounts c = node_attrs<false>(semantics, nodes, t, t - mbase[m], 0, 0, 0, none);
-    sv += c.v;
-    se += c.e;
-    sf += c.f;
-  }
-  uint64_t tv, te, tf;
-  block_excl_scan256(sv, tmp, tv);
-  block_excl_scan256(se, tmp, te);
-  block_excl_scan256(sf, tmp, tf);
-  if (threadIdx.x == 0) {
-    partial[3 * blockIdx.x] = tv;
-    partial[3 * blockIdx.x + 1] = te;
-    partial[3 * blockIdx.x + 2] = tf;
-  }
-}
-
-__global__ __launch_bounds__(BLOCK) void k_triple_scan(uint64_t* partial, uint32_t G,
-                                                       unsigned long long* totals) {
-  __shared__ uint64_t tmp[4];
-  const uint32_t per = (G + BLOCK - 1) / BLOCK;
-  const uint32_t b0 = threadIdx.x * per;
-  for (int c = 0; c < 3; ++c) {
-    uint64_t s = 0;
-    for (uint32_t k = 0; k < per; ++k)
-      if (b0 + k < G) s += partial[3 * (b0 + k) + c];
-    uint64_t tot;
-    uint64_t run = block_excl_scan256(s, tmp, tot);
-    for (uint32_t k = 0; k < per; ++k)
-      if (b0 + k < G) {
-        const uint64_t v = partial[3 * (b0 + k) + c];
-        partial[3 * (b0 + k) + c] = run;
-        run += v;
-      }
-    if (threadIdx.x == 0) totals[c] = tot;
-  }
-}
-
-__global__ __launch_bounds__(BLOCK) void k_attr_write(int semantics, NodeArrays nodes,
-                                                      uint64_t n_nodes, const uint64_t* mbase,
-                                                      uint32_t n_meshes, uint32_t G,
-                                                      const uint64_t* partial, AttrOut out,
-                                                      uint64_t* mesh_first) {
-  if (nodes.skip && *nodes.skip) return;  // graph replay over changed sizes
-  __shared__ uint64_t tmp[4];
-  uint64_t beg, end;
-  block_range(n_nodes, G, blockIdx.x, beg, end);
-  uint64_t bv = partial[3 * blockIdx.x], be = partial[3 * blockIdx.x + 1],
-           bf = partial[3 * blockIdx.x + 2];
-  AttrOut none = {nullptr, nullptr, nullptr, nullptr};
-  uint32_t m = beg < end ? find_mesh64(mbase, n_meshes, beg) : 0;
-  for (uint64_t tb = beg; tb < end; tb += BLOCK) {
-    const uint64_t t = tb + threadIdx.x;
-    AttrCounts c = {0, 0, 0};
-    uint64_t local = 0;
-    if (t < end) {
-      while (m + 1 < n_meshes && mbase[m + 1] <= t) ++m;
-      local = t - mbase[m];
-      c = node_attrs<false>(semantics, nodes, t, local, 0, 0, 0, none);
-    }
-    uint64_t tv, te, tf;
-    const uint64_t ov = block_excl_scan256((uint64_t)c.v, tmp, tv) + bv;
-    const uint64_t oe = block_excl_scan256((uint64_t)c.e, tmp, te) + be;
-    const uint64_t of = block_excl_scan256((uint64_t)c.f, tmp, tf) + bf;
-    if (t < end) {
-      node_attrs<true>(semantics, nodes, t, local, ov, oe, of, out);
-      if (local == 0) {
-        mesh_first[3 * m] = ov;
-        mesh_first[3 * m + 1] = oe;
-        mesh_first[3 * m + 2] = of;
-      }
-    }
-    bv += tv;
-    be += te;
-    bf += tf;
   }
 }
 
@@ -778,6 +472,329 @@ __global__ __launch_bounds__(ROW) void k_ref_records(const float* origin, const 
     store_stream((uint4*)edges + 21 * t0 + p, edge_piece(s_val, s_piece, f, p));
 }
 
+// ---------------------------------------------------------------- intended neighbors
+// Which records a node keeps: bits 0-7 its vertices, 8-19 its edges, 20-25
+// its faces (intended semantics).
+constexpr uint32_t KEEP_FACES = 20, KEEP_EDGES = 8, KEEP_ALL = (1u << 26) - 1u;
+
+// Neighbor slots of the cells that share corner j (d in {b - 1, b} per axis,
+// SVO.cu:567-584), edge i (the two axes that it does not run along take
+// {o - 1, o}, SVO.cu:610-627) and face f, without the node's own slot 13.
+struct ShareTable {
+  uint32_t cells[26];
+};
+constexpr ShareTable make_share_table() {
+  ShareTable t{};
+  for (int j = 0; j < 8; ++j)
+    for (int q = 0; q < 8; ++q) {
+      int slot = 13;
+      for (int a = 0, mul = 1; a < 3; ++a, mul *= 3) slot += (((j >> a) & 1) - 1 + ((q >> a) & 1)) * mul;
+      t.cells[j] |= 1u << slot;
+    }
+  for (int i = 0; i < 12; ++i)
+    for (int q = 0; q < 4; ++q) {
+      int slot = 13, bit = 0;
+      for (int a = 0, mul = 1; a < 3; ++a, mul *= 3)
+        if (EDGE_ENDS[i][0][a] == EDGE_ENDS[i][1][a])
+          slot += ((int)EDGE_ENDS[i][0][a] - 1 + ((q >> bit++) & 1)) * mul;
+      t.cells[KEEP_EDGES + i] |= 1u << slot;
+    }
+  for (int f = 0; f < 6; ++f) t.cells[KEEP_FACES + f] = 1u << FACE_SLOT[f];
+  for (int r = 0; r < 26; ++r) t.cells[r] &= ~(1u << 13);
+  return t;
+}
+constexpr ShareTable SHARED = make_share_table();
+
+// Neighbor rows of one level (SVO.cu:522-565 as intended): slot s of child k
+// of a group is a child of the parent's neighbor floor((k + d) / 2), child
+// (k + d) mod 2 per axis (the closed form of the LUTs, MortonLUT.h:531-597).
+// All eight children draw on the parent's 27 neighbors only, and a node's
+// children are consecutive, so a workgroup looks up 27 first children per
+// group (a thread per node looked up 27 per node: 216 per group, and wrote its
+// row with a stride of 108 bytes), builds the rows of 32 groups in LDS and
+// writes them, one contiguous run, in 16-byte pieces.  On the way each node's
+// records are decided: one is kept by the sharing node of the smallest index
+// (`keep`, one word per node, when set), so that the records never read the
+// rows again.  2.4 M nodes of the finest level: 940 us before, 95 now.
+constexpr uint32_t NB_GROUPS = 32;
+__global__ __launch_bounds__(8 * NB_GROUPS) void k_neighbors_level(
+    const NodeSeg* segs, const uint32_t* level_segs, const uint32_t* level_blocks,
+    uint32_t n_level_segs, int key_bytes, NodeArrays nodes, uint32_t* keep) {
+  constexpr uint32_t THREADS = 8 * NB_GROUPS;
+  __shared__ uint32_t s_first[NB_GROUPS * 27];
+  __shared__ __align__(16) uint32_t s_row[THREADS * 27];
+  if (nodes.skip && *nodes.skip) return;  // graph replay over changed sizes
+  const uint32_t i = find_seg(level_blocks, n_level_segs, blockIdx.x);
+  const auto* sg = scalar_ptr(segs) + scalar_ptr(level_segs)[i];
+  const uint32_t kind = sg->level_kind, tid = threadIdx.x;
+  if (kind & SEG_ROOT) {  // findNeighbors<true>: the root's own slot alone
+    if (tid < 27)
+      nodes.neighbors[27 * (uint64_t)sg->t0 + tid] =
+          tid == 13 && (kind & 255u) >= 2 ? sg->local0 : NONE;
+    if (tid == 0 && keep) keep[sg->t0] = KEEP_ALL;
+    return;
+  }
+  const uint32_t g0 = (blockIdx.x - scalar_ptr(level_blocks)[i]) * NB_GROUPS;
+  const uint32_t left = (sg->t1 - sg->t0) / 8 - g0, ng = left < NB_GROUPS ? left : NB_GROUPS;
+  const uint64_t base = sg->t0 - sg->local0;  // the mesh's first node
+  for (uint32_t x = tid; x < 27 * ng; x += THREADS) {
+    const uint32_t gl = x / 27, s = x - 27 * gl, g = g0 + gl;
+    uint32_t pn;
+    if (kind & SEG_ROOT_CHILD) {
+      pn = s == 13 ? sg->parent0 : NONE;
+    } else {
+      const uint32_t oct = (key_bytes == 8 ? ((const uint32_t*)sg->elem)[2 * (uint64_t)g]
+                                           : ((const uint32_t*)sg->elem)[g]) & 7u;
+      pn = nodes.neighbors[27 * (base + (sg->parent0 + 8 * sg->group[g] + oct)) + s];
+    }
+    s_first[x] = pn != NONE ? nodes.childs[8 * (base + pn)] : NONE;
+  }
+  __syncthreads();
+  if (tid < 8 * ng) {
+    const uint32_t self = sg->local0 + 8 * g0 + tid;
+    // per axis and d = -1, 0, 1: the parent's neighbor and the child in it
+    uint32_t off[3][3], ch[3][3];
+#pragma unroll
+    for (uint32_t a = 0, mul = 1; a < 3; ++a, mul *= 3) {
+      const uint32_t bit = (tid >> a) & 1u;
+      off[a][0] = (bit - 1) * mul;
+      off[a][1] = 0;
+      off[a][2] = bit * mul;
+      ch[a][0] = ch[a][2] = (bit ^ 1u) << a;
+      ch[a][1] = bit << a;
+    }
+    const uint32_t* first = s_first + 27 * (tid >> 3) + 13;
+    uint32_t lower = 0;
+#pragma unroll
+    for (uint32_t s = 0; s < 27; ++s) {
+      const uint32_t x = s % 3, y = s / 3 % 3, z = s / 9;
+      const uint32_t f = first[(int32_t)(off[0][x] + off[1][y] + off[2][z])];
+      const uint32_t v = f != NONE ? f + (ch[0][x] | ch[1][y] | ch[2][z]) : NONE;
+      s_row[27 * tid + s] = v;
+      if (v < self) lower |= 1u << s;
+    }
+    if (keep) {
+      uint32_t k = 0;
+#pragma unroll
+      for (uint32_t r = 0; r < 26; ++r) k |= (lower & SHARED.cells[r]) == 0 ? 1u << r : 0u;
+      keep[sg->t0 + 8 * g0 + tid] = k;
+    }
+  }
+  __syncthreads();
+  // the rows, 216 * ng words from a 4-byte boundary
+  const uint64_t w0 = 27 * ((uint64_t)sg->t0 + 8 * g0);
+  write_words(nodes.neighbors, w0, 216 * ng, tid, THREADS, [&](uint32_t i) { return s_row[i]; });
+}
+
+// ---------------------------------------------------------------- kept records
+// Records by keep masks: count per block of KEEP_BLOCK nodes, scan, write.
+
+// Reference semantics when a record may equal its predecessor, which drops it
+// (uniqueVert / uniqueEdge, SVO.cu:679-720): a node's vertices and edges
+// against their predecessors, the last of them the previous node's.
+__global__ __launch_bounds__(ROW) void k_ref_keep(NodeArrays nodes, uint64_t n_nodes,
+                                                  const NodeSeg* segs, const uint32_t* seg_first,
+                                                  uint32_t n_segs, uint32_t* keep) {
+  if (nodes.skip && *nodes.skip) return;  // graph replay over changed sizes
+  const uint32_t t = blockIdx.x * ROW + threadIdx.x;
+  if ((t & ~63u) >= n_nodes) return;
+  for_segments(segs, seg_first, n_segs, t & ~63u, t, t < n_nodes, [&](auto* sg, uint32_t d) {
+    const bool first = sg->local0 + d == 0;
+    const NodeGeom g = load_geom(nodes, t), gp = first ? g : load_geom(nodes, t - 1);
+    uint32_t k = 0;
+    float prev[3], p[3], pa[3], pb[3], a[3], b[3];
+    ref_corner(gp.w, 7, prev);
+    for (int j = 0; j < 8; ++j) {
+      ref_corner(g.w, j, p);
+      if ((j == 0 && first) || !eq3(p, prev)) k |= 1u << j;
+      for (int q = 0; q < 3; ++q) prev[q] = p[q];
+    }
+    ref_edge(gp, 11, pa, pb);
+    for (int i = 0; i < 12; ++i) {
+      ref_edge(g, i, a, b);
+      if ((i == 0 && first) || !edge_eq(a, b, pa, pb)) k |= 1u << (KEEP_EDGES + i);
+      for (int q = 0; q < 3; ++q) {
+        pa[q] = a[q];
+        pb[q] = b[q];
+      }
+    }
+    keep[t] = k;
+  });
+}
+
+__device__ inline void keep_counts(uint32_t k, uint32_t& v, uint32_t& e, uint32_t& f) {
+  v = __popc(k & 0xFFu);
+  e = __popc((k >> KEEP_EDGES) & 0xFFFu);
+  f = __popc(k >> KEEP_FACES);
+}
+
+// One wave per block of KEEP_BLOCK nodes: counts[3 * block + {v, e, f}].
+constexpr uint32_t KEEP_BLOCK = 512;
+__global__ __launch_bounds__(BLOCK) void k_keep_count(const uint32_t* keep, uint64_t n_nodes,
+                                                      uint32_t* counts, const uint32_t* skip) {
+  if (skip && *skip) return;  // graph replay over changed sizes
+  const uint64_t block = (uint64_t)blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6);
+  if (block * KEEP_BLOCK >= n_nodes) return;
+  uint32_t sv = 0, se = 0, sf = 0;
+#pragma unroll
+  for (uint32_t u = 0; u < KEEP_BLOCK / 64; ++u) {
+    const uint64_t t = block * KEEP_BLOCK + u * 64 + __lane_id();
+    uint32_t v, e, f;
+    keep_counts(t < n_nodes ? keep[t] : 0u, v, e, f);
+    sv += v;
+    se += e;
+    sf += f;
+  }
+  sv = wave_sum_u32(sv);
+  se = wave_sum_u32(se);
+  sf = wave_sum_u32(sf);
+  if (__lane_id() == 0) {
+    counts[3 * block] = sv;
+    counts[3 * block + 1] = se;
+    counts[3 * block + 2] = sf;
+  }
+}
+
+// Exclusive sums of the block counts (one workgroup) and the totals.
+constexpr uint32_t KEEP_SCAN = 1024;
+__global__ __launch_bounds__(KEEP_SCAN) void k_keep_scan(const uint32_t* counts, uint32_t n_blocks,
+                                                         uint64_t* offsets,
+                                                         unsigned long long* totals,
+                                                         const uint32_t* skip) {
+  if (skip && *skip) return;  // graph replay over changed sizes
+  __shared__ uint32_t s_wave[3][KEEP_SCAN / 64];
+  uint64_t carry[3] = {0, 0, 0};
+  const uint32_t wave = threadIdx.x >> 6;
+  for (uint32_t b0 = 0; b0 < n_blocks; b0 += KEEP_SCAN) {
+    const uint32_t b = b0 + threadIdx.x;
+    uint32_t c[3], inc[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      c[k] = b < n_blocks ? counts[3 * (uint64_t)b + k] : 0u;
+      inc[k] = wave_incl_scan_dpp(c[k]);  // at most 1024 * 6144 over the workgroup
+      if ((threadIdx.x & 63) == 63) s_wave[k][wave] = inc[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      uint32_t pre = 0, all = 0;
+      for (uint32_t w = 0; w < KEEP_SCAN / 64; ++w) {
+        const uint32_t x = s_wave[k][w];
+        if (w < wave) pre += x;
+        all += x;
+      }
+      if (b < n_blocks) offsets[3 * (uint64_t)b + k] = carry[k] + pre + inc[k] - c[k];
+      carry[k] += all;
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x < 3) totals[threadIdx.x] = carry[threadIdx.x];
+}
+
+// Words of the records in the LDS slots of a node's values (REC_VALS per node;
+// slots 10 and 11 hold width and width * 0).
+struct WordTable {
+  uint8_t edge[84], face[42], vert[32], ref_vert[32];
+};
+constexpr WordTable make_word_table() {
+  WordTable t{};
+  auto slot = [](const uint8_t(&e)[3], int a) {
+    return (uint8_t)(!e[0] && !e[1] && !e[2] ? a : e[a] ? 6 + a : 3 + a);
+  };
+  for (int w = 0; w < 84; ++w)
+    t.edge[w] = w % 7 == 6 ? 9 : slot(EDGE_ENDS[w / 7][w % 7 / 3], w % 7 % 3);
+  for (int w = 0; w < 42; ++w)
+    t.face[w] = w % 7 == 6 ? 9 : slot(FACE_ENDS[w / 7][w % 7 / 3], w % 7 % 3);
+  for (int j = 0; j < 8; ++j) {
+    const uint8_t corner[3] = {(uint8_t)(j & 1), (uint8_t)(j >> 1 & 1), (uint8_t)(j >> 2 & 1)};
+    for (int a = 0; a < 3; ++a) {
+      t.vert[4 * j + a] = slot(corner, a);
+      t.ref_vert[4 * j + a] = corner[a] ? 10 : 11;
+    }
+    t.vert[4 * j + 3] = t.ref_vert[4 * j + 3] = 9;
+  }
+  return t;
+}
+__constant__ WordTable WORDS = make_word_table();
+
+// Writes the kept records of a block of nodes: the nodes' values and the list
+// of kept records (node and record, in order) are staged in LDS, then every
+// record array's run of words is written in 16-byte pieces, each word looked
+// up from its record.  (A thread per node that wrote its own records scattered
+// 16- and 28-byte stores, after deciding twice from its neighbor row which they
+// are: 1,240 us on 3.3 M nodes and 300 for the count; 188 and 5 now.)
+__global__ __launch_bounds__(KEEP_BLOCK) void k_keep_write(
+    bool reference, NodeArrays nodes, uint64_t n_nodes, const NodeSeg* segs,
+    const uint32_t* seg_first, uint32_t n_segs, const uint32_t* keep, const uint64_t* offsets,
+    AttrOut out) {
+  if (nodes.skip && *nodes.skip) return;  // graph replay over changed sizes
+  __shared__ uint32_t s_val[KEEP_BLOCK * REC_VALS];
+  __shared__ uint16_t s_list[KEEP_BLOCK * 12];
+  __shared__ uint8_t s_word[84 + 42 + 32];
+  __shared__ uint32_t s_sum[2][KEEP_BLOCK / 64];
+  const uint32_t tid = threadIdx.x, t = blockIdx.x * KEEP_BLOCK + tid;
+  if (tid < 84) s_word[tid] = WORDS.edge[tid];
+  else if (tid < 84 + 42) s_word[tid] = WORDS.face[tid - 84];
+  else if (tid < 84 + 42 + 32)
+    s_word[tid] = reference ? WORDS.ref_vert[tid - 126] : WORDS.vert[tid - 126];
+  const uint32_t k = t < n_nodes ? keep[t] : 0u;
+  uint32_t nv, ne, nf;
+  keep_counts(k, nv, ne, nf);
+  // exclusive sums over the block: vertices (low half) and edges, faces
+  uint32_t a = nv | (ne << 16), b = nf;
+  const uint32_t ia = wave_incl_scan_dpp(a), ib = wave_incl_scan_dpp(b);
+  if ((tid & 63) == 63) {
+    s_sum[0][tid >> 6] = ia;
+    s_sum[1][tid >> 6] = ib;
+  }
+  __syncthreads();
+  uint32_t ta = 0, tb = 0, pa = 0, pb = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < KEEP_BLOCK / 64; ++w) {
+    if (w < tid >> 6) {
+      pa += s_sum[0][w];
+      pb += s_sum[1][w];
+    }
+    ta += s_sum[0][w];
+    tb += s_sum[1][w];
+  }
+  a = pa + ia - a;
+  b = pb + ib - b;
+  const uint64_t ov = offsets[3 * (uint64_t)blockIdx.x], oe = offsets[3 * (uint64_t)blockIdx.x + 1],
+                 of = offsets[3 * (uint64_t)blockIdx.x + 2];
+  if ((t & ~63u) < n_nodes)
+    for_segments(segs, seg_first, n_segs, t & ~63u, t, t < n_nodes, [&](auto* sg, uint32_t d) {
+      const uint32_t local = sg->local0 + d;
+      const NodeGeom g = load_geom(nodes, t);
+      uint32_t* v = s_val + REC_VALS * tid;
+#pragma unroll
+      for (uint32_t x = 0; x < 3; ++x) stage_axis(v, x, g.o[x], g.w);
+      v[9] = local;
+      v[10] = __float_as_uint(g.w * 1.0f);
+      v[11] = __float_as_uint(g.w * 0.0f);
+      if (local == 0) {
+        unsigned long long* first = out.totals + 4 + 3 * sg->mesh;
+        first[0] = ov + (a & 0xFFFFu);
+        first[1] = oe + (a >> 16);
+        first[2] = of + b;
+      }
+    });
+  // kind by kind through one list: `bits` the node's records, `at` its place
+  auto records = [&](uint32_t bits, uint32_t at, uint32_t count, uint32_t words,
+                     const uint8_t* word, uint32_t* dst, uint64_t first) {
+    for (; bits; bits &= bits - 1u) s_list[at++] = (uint16_t)((tid << 4) | __builtin_ctz(bits));
+    __syncthreads();
+    write_words(dst, first * words, count * words, tid, KEEP_BLOCK, [&](uint32_t i) {
+      const uint32_t r = i / words, e = s_list[r];
+      return s_val[REC_VALS * (e >> 4) + word[words * (e & 15u) + (i - r * words)]];
+    });
+    __syncthreads();
+  };
+  records(k & 0xFFu, a & 0xFFFFu, ta & 0xFFFFu, 4u, s_word + 126, (uint32_t*)out.verts, ov);
+  records((k >> KEEP_EDGES) & 0xFFFu, a >> 16, ta >> 16, 7u, s_word, (uint32_t*)out.edges, oe);
+  if (!reference) records(k >> KEEP_FACES, b, tb, 7u, s_word + 84, (uint32_t*)out.faces, of);
+}
+
 // 168-byte SVONode records (SVO.h:20-35), one thread per 32-bit word.
 __global__ void k_pack_aos(NodeArrays n, uint64_t first, uint64_t count, uint32_t* dst) {
   const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -852,36 +869,42 @@ void launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s) {
   hipLaunchKernelGGL(k_fill_u32, dim3((uint32_t)blocks), dim3(BLOCK), 0, s, p, value, n);
 }
 
-template <typename K>
-void launch_neighbors_level(int level, KeyLayout<K> kl, const void* elem_next,
-                            const uint32_t* elem_group_next, uint64_t n_groups,
-                            const LevelSpan* spans, uint32_t n_levels,
-                            const MeshTreeState* state, const MeshNodeLayout* layout,
-                            NodeArrays nodes, hipStream_t s) {
-  if (n_groups == 0) return;
-  hipLaunchKernelGGL(k_neighbors_level<K>, dim3(grid_for(8 * n_groups)), dim3(BLOCK), 0, s,
-                     level, kl, (const K*)elem_next, elem_group_next, n_groups, spans, n_levels,
-                     state, layout, nodes);
+void launch_neighbors_level(const NodeSeg* segs, const uint32_t* level_segs,
+                            const uint32_t* level_blocks, uint32_t n_level_segs, uint32_t blocks,
+                            int key_bytes, NodeArrays nodes, uint32_t* keep, hipStream_t s) {
+  if (blocks == 0) return;
+  hipLaunchKernelGGL(k_neighbors_level, dim3(blocks), dim3(8 * NB_GROUPS), 0, s, segs, level_segs,
+                     level_blocks, n_level_segs, key_bytes, nodes, keep);
 }
 
-size_t attr_tmp_bytes(uint32_t blocks) { return (size_t)3 * blocks * sizeof(uint64_t); }
-
-void launch_attrs_count(int semantics, const NodeArrays& nodes, uint64_t n_nodes,
-                        const uint64_t* mesh_node_base, uint32_t n_meshes, uint32_t blocks,
-                        void* tmp, AttrOut out, hipStream_t s) {
-  uint64_t* partial = (uint64_t*)tmp;
-  hipLaunchKernelGGL(k_attr_count, dim3(blocks), dim3(BLOCK), 0, s, semantics, nodes, n_nodes,
-                     mesh_node_base, n_meshes, blocks, partial);
-  hipLaunchKernelGGL(k_triple_scan, dim3(1), dim3(BLOCK), 0, s, partial, blocks, out.totals);
+uint32_t neighbor_blocks(const NodeSeg& seg) {
+  return seg.level_kind & SEG_ROOT ? 1u : ((seg.t1 - seg.t0) / 8 + NB_GROUPS - 1) / NB_GROUPS;
 }
 
-void launch_attrs_write(int semantics, const NodeArrays& nodes, uint64_t n_nodes,
-                        const uint64_t* mesh_node_base, uint32_t n_meshes, uint32_t blocks,
-                        void* tmp, AttrOut out, hipStream_t s) {
-  uint64_t* partial = (uint64_t*)tmp;
-  uint64_t* mesh_first = (uint64_t*)out.totals + 4;  // [3 * n_meshes] after the totals
-  hipLaunchKernelGGL(k_attr_write, dim3(blocks), dim3(BLOCK), 0, s, semantics, nodes, n_nodes,
-                     mesh_node_base, n_meshes, blocks, (const uint64_t*)partial, out, mesh_first);
+// keep masks, then per block of nodes the counts (padded to 8 bytes) and offsets
+static uint64_t keep_blocks(uint64_t n_nodes) { return (n_nodes + KEEP_BLOCK - 1) / KEEP_BLOCK; }
+size_t keep_bytes(uint64_t n_nodes) {
+  return (size_t)(4 * KEEP_BLOCK + 16 + 24) * keep_blocks(n_nodes);
+}
+
+void launch_kept_records(int semantics, const NodeArrays& nodes, uint64_t n_nodes,
+                         const NodeSeg* segs, const uint32_t* seg_first, uint32_t n_segs,
+                         void* tmp, AttrOut out, hipStream_t s) {
+  const uint32_t nb = (uint32_t)keep_blocks(n_nodes);
+  uint32_t* keep = (uint32_t*)tmp;
+  uint64_t* offsets = (uint64_t*)(keep + (uint64_t)KEEP_BLOCK * nb);
+  uint32_t* counts = (uint32_t*)(offsets + 3 * (uint64_t)nb);
+  const bool reference = semantics == SVO_SEM_REFERENCE;
+  if (reference)
+    hipLaunchKernelGGL(k_ref_keep, dim3((uint32_t)((n_nodes + ROW - 1) / ROW)), dim3(ROW), 0, s,
+                       nodes, n_nodes, segs, seg_first, n_segs, keep);
+  hipLaunchKernelGGL(k_keep_count, dim3((nb + 3) / 4), dim3(BLOCK), 0, s, (const uint32_t*)keep,
+                     n_nodes, counts, nodes.skip);
+  hipLaunchKernelGGL(k_keep_scan, dim3(1), dim3(KEEP_SCAN), 0, s, (const uint32_t*)counts, nb,
+                     offsets, out.totals, nodes.skip);
+  hipLaunchKernelGGL(k_keep_write, dim3(nb), dim3(KEEP_BLOCK), 0, s, reference, nodes, n_nodes,
+                     segs, seg_first, n_segs, (const uint32_t*)keep, (const uint64_t*)offsets,
+                     out);
 }
 
 void launch_ref_records(const float* origin, const float* width, uint64_t n_nodes,
@@ -908,14 +931,7 @@ void launch_query_neighbors(const uint32_t* neighbors, uint64_t n_nodes, const u
                      slot, n, out);
 }
 
-#define SVO_INST(K)                                                                              \
-  template void launch_emit<K>(const EmitArgs<K>&, hipStream_t);                                 \
-  template void launch_neighbors_level<K>(int, KeyLayout<K>, const void*, const uint32_t*,       \
-                                          uint64_t, const LevelSpan*, uint32_t,                  \
-                                          const MeshTreeState*, const MeshNodeLayout*,           \
-                                          NodeArrays, hipStream_t);
-SVO_INST(uint32_t)
-SVO_INST(uint64_t)
-#undef SVO_INST
+template void launch_emit<uint32_t>(const EmitArgs<uint32_t>&, hipStream_t);
+template void launch_emit<uint64_t>(const EmitArgs<uint64_t>&, hipStream_t);
 
 }  // namespace svo

@@ -441,8 +441,8 @@ double pass_bytes_bound(const svo_params* p, int kb, uint64_t P, uint64_t T, int
   const double n_big = (double)T + rows / 512.0;
   const double ws_common = 12.0 * P + 12.0 * T + (double)order_bytes(T) + 2 * 256.0 + lv +
                            (double)level_tmp_bytes(kc) +
-                           sizeof(BigItem) * std::max(n_big, 1.0) + (double)attr_tmp_bytes(4096) +
-                           (1 << 20);  // control buffers of one mesh
+                           sizeof(BigItem) * std::max(n_big, 1.0) + 4.1 * N + 4096.0 +
+                           (1 << 20);  // keep masks; control buffers of one mesh
   const double ws_bitmap = 4.0 * bm_words + (double)bitmap_level_tmp_bytes(bm_words);
   const double ws_sort = 2.0 * K * key_cap + (double)radix_sort_tmp_bytes(kc);
   const double ws = ws_common + std::max(ws_bitmap, ws_sort);
@@ -1030,11 +1030,6 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     SVO_TRY(W.get("keys_b", sizeof(K) * key_cap, (void**)&keys_b));
   }
   SVO_TRY(W.get("big", sizeof(BigItem) * std::max<uint64_t>(n_big, 1), (void**)&big));
-  // fixed grids sized from host-known capacities (small inputs get small grids)
-  auto grid_for = [](uint64_t cap_elems, uint64_t per_block, uint32_t max_blocks) {
-    const uint64_t b = (cap_elems + per_block - 1) / per_block;
-    return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(b, max_blocks));
-  };
   if (!use_bm) SVO_TRY(W.get("sort_tmp", radix_sort_tmp_bytes(key_cap), &sort_tmp));
   SVO_TRY(W.get("lvl_tmp", level_tmp_bytes(use_bm ? u_cap : key_cap), &lvl_tmp));
   // level capacities: cap_1 = unique voxels bound (box cells >= hits >=
@@ -1290,6 +1285,7 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
       g.t0 = (uint32_t)Lm.node_base + g.local0;
       g.t1 = (uint32_t)(Lm.node_base + (l < Lm.depth ? Lm.level_off[l] : Lm.n_nodes));
       g.level_kind = l;
+      g.mesh = i;
       g.width = Lm.width[l - 1];
       for (int a = 0; a < 3; ++a) g.origin[a] = h_par[i].origin[a];
       g.child0 = l >= 2 ? (uint32_t)Lm.level_off[l - 2] : 0u;
@@ -1314,23 +1310,36 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     }
   }
   const uint32_t n_segs = (uint32_t)segs.size();
+  // intended neighbors: the segments of each level (the roots with level 1's)
+  // and their workgroups
+  std::vector<uint32_t> level_segs, level_blocks, level_at(NL + 2, 0), level_grid(NL + 2, 0);
+  if (sem == SVO_SEM_INTENDED)
+    for (uint32_t l = 1; l <= NL; ++l) {
+      for (uint32_t k = 0; k < n_segs; ++k) {
+        const bool root = segs[k].level_kind & SEG_ROOT;
+        if (root ? l != 1 : (segs[k].level_kind & 255u) != l) continue;
+        level_segs.push_back(k);
+        level_blocks.push_back(level_grid[l]);
+        level_grid[l] += neighbor_blocks(segs[k]);
+      }
+      level_at[l + 1] = (uint32_t)level_segs.size();
+    }
   char* bctl = nullptr;
-  const size_t sz_lay = align256(sizeof(MeshNodeLayout) * n), sz_nb = align256(8 * (n + 1)),
-               sz_segs = align256(sizeof(NodeSeg) * n * NL), sz_sf = align256(4 * n * NL),
-               sz_up = sz_lay + sz_nb + sz_segs + sz_sf, sz_tot = align256(8 * (4 + 3 * n));
+  const size_t sz_segs = align256(sizeof(NodeSeg) * n * NL), sz_sf = align256(4 * n * NL),
+               sz_up = sz_segs + 3 * sz_sf, sz_tot = align256(8 * (4 + 3 * n));
   SVO_TRY(W.get("bctl", sz_up + sz_tot, (void**)&bctl));
-  MeshNodeLayout* d_lay = (MeshNodeLayout*)bctl;
-  uint64_t* d_nbase = (uint64_t*)(bctl + sz_lay);
-  NodeSeg* d_segs = (NodeSeg*)(bctl + sz_lay + sz_nb);
-  uint32_t* d_seg_first = (uint32_t*)(bctl + sz_lay + sz_nb + sz_segs);
+  NodeSeg* d_segs = (NodeSeg*)bctl;
+  uint32_t* d_seg_first = (uint32_t*)(bctl + sz_segs);
+  uint32_t* d_level_segs = (uint32_t*)(bctl + sz_segs + sz_sf);
+  uint32_t* d_level_blocks = (uint32_t*)(bctl + sz_segs + 2 * sz_sf);
   unsigned long long* d_tot = (unsigned long long*)(bctl + sz_up);
   if (!capture) {
     SVO_TRY(L.ensure_pinned(sz_up + sz_tot));
     char* up = (char*)L.pinned;
-    std::memcpy(up, lay.data(), sizeof(MeshNodeLayout) * n);
-    std::memcpy(up + sz_lay, node_base.data(), 8 * (n + 1));
-    std::memcpy(up + sz_lay + sz_nb, segs.data(), sizeof(NodeSeg) * n_segs);
-    std::memcpy(up + sz_lay + sz_nb + sz_segs, seg_first.data(), 4 * n_segs);
+    std::memcpy(up, segs.data(), sizeof(NodeSeg) * n_segs);
+    std::memcpy(up + sz_segs, seg_first.data(), 4 * n_segs);
+    std::memcpy(up + sz_segs + sz_sf, level_segs.data(), 4 * level_segs.size());
+    std::memcpy(up + sz_segs + 2 * sz_sf, level_blocks.data(), 4 * level_blocks.size());
     HIP_TRY(hipMemcpyAsync(bctl, up, sz_up, hipMemcpyHostToDevice, s));
   }
   timer.mark("setup_b");
@@ -1352,27 +1361,25 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
   ea.voxels = out->voxels;
   ea.verts = out->verts;
   ea.edges = out->edges;
-  ea.neighbors = true;
+  ea.neighbors = sem == SVO_SEM_REFERENCE;
   ea.records = identity;
   launch_emit<K>(ea, s);
   timer.mark("emit");
+  const bool counted = want_attrs && !identity && N;
+  uint32_t* keep = nullptr;
+  if (counted) SVO_TRY(W.get("keep", keep_bytes(N), (void**)&keep));
   if (sem == SVO_SEM_INTENDED) {
-    for (uint32_t l = NL - 1; l >= 1; --l)
-      launch_neighbors_level<K>((int)l, kl, lv[l + 1].elem, lv[l + 1].elem_group, h_counts[l],
-                                d_spans, NL, d_state, d_lay, na, s);
+    for (uint32_t l = NL; l >= 1; --l)
+      launch_neighbors_level(d_segs, d_level_segs + level_at[l], d_level_blocks + level_at[l],
+                             level_at[l + 1] - level_at[l], level_grid[l], (int)sizeof(K), na,
+                             keep, s);
     timer.mark("neighbors");
   }
-  void* attr_tmp = nullptr;
-  const bool counted = want_attrs && !identity && N;
   std::vector<uint64_t> tot(4 + 3 * (size_t)n, 0);
   if (counted) {
     launch_fill_u32((uint32_t*)d_tot, 0u, sz_tot / 4, s);
     AttrOut ao{out->verts, out->edges, out->faces, d_tot};
-    SVO_TRY(W.get("attr_tmp", attr_tmp_bytes(plan.tuning.scan_blocks), &attr_tmp));
-    const uint32_t ab = grid_for(N, 2048, plan.tuning.scan_blocks);
-    launch_attrs_count(sem, na, N, d_nbase, n, ab, attr_tmp, ao, s);
-    timer.mark("attr_count");
-    launch_attrs_write(sem, na, N, d_nbase, n, ab, attr_tmp, ao, s);
+    launch_kept_records(sem, na, N, d_segs, d_seg_first, n_segs, keep, ao, s);
     timer.mark("attr_write");
   } else if (identity) {
     tot[0] = 8 * N;

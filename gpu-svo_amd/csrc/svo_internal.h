@@ -157,7 +157,8 @@ struct alignas(64) NodeSeg {
   uint32_t parent0;  // parent of group g: parent0 + 8 * elem_group[g] + (key & 7)
   float width;
   float origin[3];   // gridOrigin
-  uint32_t pad[2];
+  uint32_t mesh;
+  uint32_t pad;
   // the run's parent groups (level + 1's arrays, from its first group on):
   // keys, their own groups, first children and child masks; a root's own key
   const void* elem;
@@ -212,26 +213,28 @@ void launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s);
 // 4-byte aligned) at `got` differ from those at `want`.
 void launch_check_equal(const void* got, const void* want, uint64_t bytes, uint32_t* flag,
                         hipStream_t s);
-template <typename K>
-void launch_neighbors_level(int level, KeyLayout<K> kl, const void* elem_next,
-                            const uint32_t* elem_group_next, uint64_t n_groups,
-                            const LevelSpan* spans, uint32_t n_levels,
-                            const MeshTreeState* state, const MeshNodeLayout* layout,
-                            NodeArrays nodes, hipStream_t s);
-// Vertex / edge / face records: count, scan, write.
+// Neighbor rows of one level, intended semantics, from the rows of the level
+// above, and (when `keep` is set) which records each node keeps.  The level's
+// segments segs[level_segs[i]] own workgroups from level_blocks[i] on,
+// neighbor_blocks(segment) each; the roots, whose rows need no level above,
+// may stand among them.
+uint32_t neighbor_blocks(const NodeSeg& seg);
+void launch_neighbors_level(const NodeSeg* segs, const uint32_t* level_segs,
+                            const uint32_t* level_blocks, uint32_t n_level_segs, uint32_t blocks,
+                            int key_bytes, NodeArrays nodes, uint32_t* keep, hipStream_t s);
+// Vertex, edge and face records by keep masks.
 struct AttrOut {
   svo_vertex_t* verts;
   svo_edge_t* edges;
   svo_edge_t* faces;
-  unsigned long long* totals;  // [3] totals after the write
+  unsigned long long* totals;  // [3] totals, then from [4] on 3 first records per mesh
 };
-size_t attr_tmp_bytes(uint32_t blocks);
-void launch_attrs_count(int semantics, const NodeArrays& nodes, uint64_t n_nodes,
-                        const uint64_t* mesh_node_base, uint32_t n_meshes, uint32_t blocks,
-                        void* tmp, AttrOut out, hipStream_t s);
-void launch_attrs_write(int semantics, const NodeArrays& nodes, uint64_t n_nodes,
-                        const uint64_t* mesh_node_base, uint32_t n_meshes, uint32_t blocks,
-                        void* tmp, AttrOut out, hipStream_t s);
+// `tmp` holds keep_bytes(n_nodes) bytes and begins with the nodes' keep masks
+// (written by launch_neighbors_level; by this call, reference semantics).
+size_t keep_bytes(uint64_t n_nodes);
+void launch_kept_records(int semantics, const NodeArrays& nodes, uint64_t n_nodes,
+                         const NodeSeg* segs, const uint32_t* seg_first, uint32_t n_segs,
+                         void* tmp, AttrOut out, hipStream_t s);
 // The reference's vertex and edge records of given nodes (origin 3 floats and
 // width 1 float each) at the identity offsets, owner = the node's index.
 void launch_ref_records(const float* origin, const float* width, uint64_t n_nodes,
