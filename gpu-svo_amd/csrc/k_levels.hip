@@ -316,9 +316,16 @@ __global__ __launch_bounds__(BLOCK) void k_bm_scan(uint32_t* tile_u, uint32_t* t
                                                    const uint32_t* tile_r, uint32_t tiles,
                                                    uint64_t* scan_status,
                                                    unsigned long long* counts,
-                                                   unsigned long long* reset_bytes) {
+                                                   unsigned long long* reset_bytes,
+                                                   const unsigned long long* hits,
+                                                   unsigned long long* n_hits) {
   __shared__ uint64_t tmp[4];
   __shared__ uint32_t s_chunk, s_base[2], s_reset[BLOCK / 64];
+  static_assert(HIT_SLOTS == 64, "a wave adds up the hit counters");
+  if (blockIdx.x == 0 && threadIdx.x < 64) {
+    const uint64_t h = wave_sum((uint64_t)hits[threadIdx.x * HIT_STRIDE]);
+    if (threadIdx.x == 0) *n_hits = h;
+  }
   uint32_t* ticket = (uint32_t*)scan_status;  // word 0; chunk c uses words 2 + 2c, 3 + 2c
   if (threadIdx.x == 0) s_chunk = atomicAdd(ticket, 1u);
   __syncthreads();
@@ -790,7 +797,9 @@ void launch_level_first_bitmap(uint32_t* bits, uint64_t n_words, const uint64_t*
                                uint32_t n_meshes, KeyLayout<K> kl, LevelArrays l1,
                                LevelArrays l2, unsigned long long* counts, LevelSpan* spans1,
                                uint32_t n_levels, MeshTreeState* state, void* tmp,
-                               void* lvl_tmp, unsigned long long* reset_bytes, hipStream_t s) {
+                               void* lvl_tmp, unsigned long long* reset_bytes,
+                               const unsigned long long* hits, unsigned long long* n_hits,
+                               hipStream_t s) {
   const uint64_t tiles = (std::max<uint64_t>(n_words, 1) + BM_TILE - 1) / BM_TILE;
   const uint64_t chunks = (tiles + SC_CHUNK - 1) / SC_CHUNK;
   uint32_t* tile_u = (uint32_t*)tmp;
@@ -802,7 +811,8 @@ void launch_level_first_bitmap(uint32_t* bits, uint64_t n_words, const uint64_t*
   hipLaunchKernelGGL(k_bm_count, dim3((uint32_t)tiles), dim3(BLOCK), 0, s, bits, n_words, tile_u,
                      tile_g, tile_r, scan_status, n_status);
   hipLaunchKernelGGL(k_bm_scan, dim3((uint32_t)chunks), dim3(BLOCK), 0, s, tile_u, tile_g,
-                     (const uint32_t*)tile_r, (uint32_t)tiles, scan_status, counts, reset_bytes);
+                     (const uint32_t*)tile_r, (uint32_t)tiles, scan_status, counts, reset_bytes, hits,
+                     n_hits);
   // the emission also writes the level-1 spans and depth-1 roots, and clears
   // the later levels' look-back words and tickets (launch_level)
   uint32_t* tickets = (uint32_t*)lvl_tmp;
@@ -845,11 +855,13 @@ template void launch_level_first_bitmap<uint32_t>(uint32_t*, uint64_t, const uin
                                                   uint32_t, KeyLayout<uint32_t>, LevelArrays,
                                                   LevelArrays, unsigned long long*, LevelSpan*,
                                                   uint32_t, MeshTreeState*, void*, void*,
+                                                  unsigned long long*, const unsigned long long*,
                                                   unsigned long long*, hipStream_t);
 template void launch_level_first_bitmap<uint64_t>(uint32_t*, uint64_t, const uint64_t*,
                                                   uint32_t, KeyLayout<uint64_t>, LevelArrays,
                                                   LevelArrays, unsigned long long*, LevelSpan*,
                                                   uint32_t, MeshTreeState*, void*, void*,
+                                                  unsigned long long*, const unsigned long long*,
                                                   unsigned long long*, hipStream_t);
 template void launch_level<uint32_t>(int, KeyLayout<uint32_t>, LevelArrays, LevelArrays,
                                      unsigned long long*, LevelSpan*, uint32_t, MeshTreeState*,

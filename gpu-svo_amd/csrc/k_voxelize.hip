@@ -8,18 +8,17 @@
 // Work distribution (the reference gives one thread per triangle):
 //  * k_classify   one lane per triangle: box cells -> key capacity and the
 //                 number of big-triangle chunks (exact, read back once).
-//  * k_vox_small  one lane per triangle whose box has <= small_max cells,
-//                 the workgroup's triangles handed out in order of box size;
-//                 lanes walk their box row by row, and the yz-projection
-//                 test, which does not depend on x, is evaluated once per
-//                 row (an exact hoist: the same operands, the same rounding).
-//                 Larger triangles are cut into chunks of 512 rows and queued.
-//  * k_vox_big    one wave64 per queued item of 512 rows: each lane takes
-//                 eight rows, prunes each to the x-range outside of which a
-//                 test provably fails (row_range) and tests the cells left
-//                 in it.
-// Hits are staged per wave in LDS and flushed with one atomic per ~1K keys.
+//  * k_vox_rows   one wave per run of triangles: a lane sets up a triangle,
+//                 then the wave's lanes take the box rows (y, z) of all of
+//                 them in turn.  Triangles over the size limit are queued in
+//                 items of 512 rows, each a wave's work in a second launch.
+// A row's cells are found from the x-interval that the tests leave, in place
+// of testing each cell (below); the cells that rounding could decide either
+// way are tested with the reference's float operations.
+#include <algorithm>
+
 #include "svo_internal.h"
+#include "svo_scan.h"
 
 namespace svo {
 namespace {
@@ -47,6 +46,23 @@ __device__ inline uint32_t find_mesh(const uint64_t* base, uint32_t n_meshes, ui
     const uint32_t mid = (lo + hi) >> 1;
     if (base[mid] <= gid) lo = mid; else hi = mid;
   }
+  return lo;
+}
+
+// The mesh of triangle gid >= first, `first` the same in every lane of the
+// wave: one step of 64 comparisons per factor 64 of meshes finds the mesh of
+// `first`, which nearly always is that of the whole wave.
+__device__ inline uint32_t find_mesh_wave(const uint64_t* base, uint32_t n_meshes, uint64_t first,
+                                          uint64_t gid) {
+  uint32_t lo = 0, n = n_meshes;
+  while (n > 1) {
+    const uint32_t step = (n + 63) / 64, i = __lane_id() * step;
+    const uint64_t at = __ballot(i < n && base[lo + i] <= first);
+    const uint32_t last = 63u - (uint32_t)__builtin_clzll(at);  // base[lo] <= first
+    lo += last * step;
+    n = n - last * step < step ? n - last * step : step;
+  }
+  while (lo + 1 < n_meshes && base[lo + 1] <= gid) ++lo;
   return lo;
 }
 
@@ -244,164 +260,162 @@ __device__ inline void tri_setup(const float v[3][3], const MeshParams& P, TriSe
   }
 }
 
-// Row terms of cell row (y, z): everything of the 13 tests that does not
-// depend on x.  Returns false when a yz-projection test fails (the whole row
-// is empty).
+// Rows by interval.  In row (y, z) each of the seven tests left (plane, three
+// xy edges, three zx edges) is affine in x, so that the cells that pass are
+// those between the tests' roots.  A root is found in float as
+// -(row terms) * (1 / slope) and is wrong, together with the rounding of the
+// test itself, by less than
+//   9 u M / |slope|,  M = |slope| * (largest x + 1) + |row terms|,  u = 2^-24,
+// slope per cell and M over the triangle's box: the test (two products, two
+// sums) rounds within 4 u M; the sum of the row terms, the slope, its
+// reciprocal and the root within 4 u M / |slope|; the root +- e within
+// u M / |slope|.  e = 12 u M / |slope| leaves a third for the rounding of M
+// and e themselves.  So a cell beyond root +- e fails for certain, one inside
+// root -+ e passes for certain, and the few between are tested as the
+// reference does (cell_hit).  A test of slope zero bounds nothing (error
+// ROW_FREE: no cell is certain).  Where a test's M is so small or large that
+// its products could underflow or overflow, or is no number, every cell of the
+// triangle's box goes to cell_hit.
+constexpr float ROW_ERR = 12.0f * 0x1p-24f, ROW_FREE = 1e30f;
+
+// What a row needs of its triangle, in 15 16-byte pieces of LDS.
+struct alignas(16) RowTri {
+  float yz[3][4];                // ne.y, ne.z, de of the yz edges; n.y, n.z, u.y
+  float uz, inv_ny; int32_t y0, z0;
+  float xy_y[3], nx;             // y slopes of the xy edges
+  float zx_z[3], d1;             // z slopes of the zx edges
+  float xy_d[3], d2;
+  float zx_d[3], ux;
+  float inv[7]; int32_t ny;      // 1 / slope: plane, xy edges, zx edges
+  float err[7]; int32_t x0;      // e of the same
+  float xy_x[3]; int32_t x1;     // x slopes (cell_hit only)
+  float zx_x[3]; uint32_t row0;  // item index - row
+  uint32_t key_lo, key_hi;       // mesh key or first 64-bit bitmap word
+  uint32_t exact, pad;           // nonzero: no interval holds
+};
+static_assert(sizeof(RowTri) == 15 * 16, "fifteen pieces");
+
+// False when M lies outside (lo, hi) (also for NaN).
+__device__ inline bool row_bound(float slope, float rest, float xmax, float lo, float hi,
+                                 float& inv, float& err) {
+  const float b = fabsf(slope), M = b * xmax + rest;
+  inv = 1.0f / slope;
+  err = M * fabsf(inv) * ROW_ERR;
+  if (!(b > 0.0f && err < ROW_FREE)) {
+    inv = 0.0f;
+    err = ROW_FREE;
+  }
+  return M > lo && M < hi;
+}
+
+__device__ inline void row_setup(const TriSetup& S, RowTri& T) {
+  bool ok = true;
+  const float xmax = (float)S.g1[0] + 1.0f, ymax = ((float)S.g1[1] + 1.0f) * S.u[1],
+              zmax = ((float)S.g1[2] + 1.0f) * S.u[2];
+  for (int i = 0; i < 3; ++i) {
+    T.yz[i][0] = S.ne[1][i][0];
+    T.yz[i][1] = S.ne[1][i][1];
+    T.yz[i][2] = S.de[1][i];
+    T.xy_x[i] = S.ne[0][i][0];
+    T.xy_y[i] = S.ne[0][i][1];
+    T.zx_z[i] = S.ne[2][i][0];
+    T.zx_x[i] = S.ne[2][i][1];
+    T.xy_d[i] = S.de[0][i];
+    T.zx_d[i] = S.de[2][i];
+    ok &= row_bound(S.ne[0][i][0] * S.u[0], fabsf(S.ne[0][i][1]) * ymax + fabsf(S.de[0][i]),
+                    xmax, 0x1p-90f, 0x1p100f, T.inv[1 + i], T.err[1 + i]);
+    ok &= row_bound(S.ne[2][i][1] * S.u[0], fabsf(S.ne[2][i][0]) * zmax + fabsf(S.de[2][i]),
+                    xmax, 0x1p-90f, 0x1p100f, T.inv[4 + i], T.err[4 + i]);
+  }
+  // the plane test multiplies two such values
+  ok &= row_bound(S.n[0] * S.u[0],
+                  fabsf(S.n[1]) * ymax + fabsf(S.n[2]) * zmax + fabsf(S.d1) + fabsf(S.d2), xmax,
+                  0x1p-50f, 0x1p60f, T.inv[0], T.err[0]);
+  T.exact = ok ? 0u : 1u;
+  T.yz[0][3] = S.n[1];
+  T.yz[1][3] = S.n[2];
+  T.yz[2][3] = S.u[1];
+  T.uz = S.u[2];
+  T.nx = S.n[0];
+  T.d1 = S.d1;
+  T.d2 = S.d2;
+  T.ux = S.u[0];
+  T.x0 = S.g0[0];
+  T.x1 = S.g1[0];
+  T.y0 = S.g0[1];
+  T.z0 = S.g0[2];
+  T.ny = S.g1[1] - S.g0[1] + 1;
+  T.inv_ny = 1.0f / (float)T.ny;
+}
+
+// The reference's terms of row (y, z): everything of the 13 tests that does
+// not depend on x.  False when a yz-projection test fails (the row is empty).
 struct RowTerms {
   float A;       // n.y*p.y + n.z*p.z  (inner sum of n.dot(p))
   float rxy[3];  // ne_xy[i].y * p.y
   float rzx[3];  // ne_zx[i].x * p.z
 };
-// The tests are combined without short-circuit: every lane evaluates all of
-// them (the same operations and roundings), so the wave runs no branches.
-__device__ inline bool row_terms(const TriSetup& S, int y, int z, RowTerms& R) {
-  const float py = (float)y * S.u[1];
-  const float pz = (float)z * S.u[2];
+__device__ inline bool row_terms(const RowTri& T, int y, int z, RowTerms& R) {
+  const float py = (float)y * T.yz[2][3];
+  const float pz = (float)z * T.uz;
   bool ok = true;
-  for (int i = 0; i < 3; ++i)
-    ok &= !((S.ne[1][i][0] * py + S.ne[1][i][1] * pz) + S.de[1][i] < 0.0f);
-  R.A = S.n[1] * py + S.n[2] * pz;
+  for (int i = 0; i < 3; ++i) ok &= !((T.yz[i][0] * py + T.yz[i][1] * pz) + T.yz[i][2] < 0.0f);
+  R.A = T.yz[0][3] * py + T.yz[1][3] * pz;
   for (int i = 0; i < 3; ++i) {
-    R.rxy[i] = S.ne[0][i][1] * py;
-    R.rzx[i] = S.ne[2][i][0] * pz;
+    R.rxy[i] = T.xy_y[i] * py;
+    R.rzx[i] = T.zx_z[i] * pz;
   }
   return ok;
 }
-__device__ inline bool cell_hit(const TriSetup& S, const RowTerms& R, int x) {
-  const float px = (float)x * S.u[0];
-  const float t = S.n[0] * px + R.A;
-  bool ok = !((t + S.d1) * (t + S.d2) > 0.0f);
+// The reference's tests of cell x of the row.
+__device__ inline bool cell_hit(const RowTri& T, const RowTerms& R, int x) {
+  const float px = (float)x * T.ux;
+  const float t = T.nx * px + R.A;
+  bool ok = !((t + T.d1) * (t + T.d2) > 0.0f);
   for (int i = 0; i < 3; ++i) {
-    ok &= !((S.ne[0][i][0] * px + R.rxy[i]) + S.de[0][i] < 0.0f);
-    ok &= !((R.rzx[i] + S.ne[2][i][1] * px) + S.de[2][i] < 0.0f);
+    ok &= !((T.xy_x[i] * px + R.rxy[i]) + T.xy_d[i] < 0.0f);
+    ok &= !((R.rzx[i] + T.zx_x[i] * px) + T.zx_d[i] < 0.0f);
   }
   return ok;
 }
 
-// Conservative x-range [xa, xb] of row (y, z): outside it the plane test or
-// one of the xy / zx edge tests fails for certain.  Each test is affine in x;
-// its root is computed in double and widened by two cells plus a bound on
-// the float rounding of the test (2^-20 of the magnitudes involved, several
-// times the few half-ulp roundings of the float evaluation).  Tests whose
-// x-slope is tiny are not used.  Skipping cells outside the range therefore
-// never changes the set of hits.  The x-slopes and their reciprocals depend
-// on the triangle only (RangeConst, once per triangle); a root is the row
-// term times the reciprocal, within a few double ulps of the quotient, far
-// inside the margin.
-struct RangeConst {
-  double a, ia;        // plane test: slope n.x * u.x and its reciprocal
-  double b[6], ib[6];  // xy edges 0-2, zx edges 0-2
-};
-
-__device__ inline void range_const(const TriSetup& S, RangeConst& C) {
-  const double ux = S.u[0];
-  C.a = (double)S.n[0] * ux;
-  C.ia = C.a != 0.0 ? 1.0 / C.a : 0.0;
-  for (int i = 0; i < 6; ++i) {
-    C.b[i] = (double)(i < 3 ? S.ne[0][i][0] : S.ne[2][i - 3][1]) * ux;
-    C.ib[i] = C.b[i] != 0.0 ? 1.0 / C.b[i] : 0.0;
-  }
-}
-
-__device__ inline void row_range(const TriSetup& S, const RangeConst& C, const RowTerms& R,
-                                 int& xa, int& xb) {
-  double lo = S.g0[0], hi = S.g1[0];
-  const double xmax = (double)S.g1[0] + 1.0;
+// Cells [xa, xb] of the row may hit, [ia, ib] hit for certain (either may be
+// empty).
+__device__ inline void row_range(const RowTri& T, const RowTerms& R, int& xa, int& xb, int& ia,
+                                 int& ib) {
+  float lo = (float)T.x0, hi = (float)T.x1, ilo = lo, ihi = hi;
   {
-    const double a = C.a;
-    const double d1 = S.d1, d2 = S.d2, A = R.A;
-    const double mag = fabs(a) * xmax + fabs(A) + fabs(d1) + fabs(d2);
-    if (fabs(a) > 1e-12 * (mag + 1e-30) && fabs(a) > 1e-15) {
-      const double err = mag * 0x1p-20 * fabs(C.ia) + 2.0;
-      double x1 = (-fmax(d1, d2) - A) * C.ia, x2 = (-fmin(d1, d2) - A) * C.ia;
-      if (x1 > x2) {
-        const double t = x1;
-        x1 = x2;
-        x2 = t;
-      }
-      lo = fmax(lo, floor(x1 - err));
-      hi = fmin(hi, ceil(x2 + err));
-    }
+    const float r1 = (-T.d1 - R.A) * T.inv[0], r2 = (-T.d2 - R.A) * T.inv[0];
+    const float a = fminf(r1, r2), b = fmaxf(r1, r2), e = T.err[0];
+    lo = fmaxf(lo, a - e);
+    hi = fminf(hi, b + e);
+    ilo = fmaxf(ilo, a + e);
+    ihi = fminf(ihi, b - e);
   }
-  for (int i = 0; i < 6; ++i) {
-    // xy: ne.x * px + rxy + de >= 0;  zx: rzx + ne.y * px + de >= 0
-    const double b = C.b[i];
-    const double c = i < 3 ? (double)R.rxy[i] + (double)S.de[0][i]
-                           : (double)R.rzx[i - 3] + (double)S.de[2][i - 3];
-    const double mag = fabs(b) * xmax + fabs(c) + fabs(i < 3 ? R.rxy[i] : R.rzx[i - 3]);
-    if (!(fabs(b) > 1e-12 * (mag + 1e-30) && fabs(b) > 1e-30)) continue;
-    const double err = mag * 0x1p-20 * fabs(C.ib[i]) + 2.0;
-    const double root = -c * C.ib[i];
-    if (b > 0) lo = fmax(lo, floor(root - err));
-    else hi = fmin(hi, ceil(root + err));
+#pragma unroll
+  for (int i = 1; i < 7; ++i) {
+    const float c = i < 4 ? R.rxy[i - 1] + T.xy_d[i - 1] : R.rzx[i - 4] + T.zx_d[i - 4];
+    const float inv = T.inv[i], e = T.err[i], root = -c * inv;
+    // rising tests pass above their root, falling ones below; an unused test
+    // (inv 0) counts as falling with root 0
+    const bool up = inv > 0.0f;
+    lo = fmaxf(lo, up ? root - e : -ROW_FREE);
+    ilo = fmaxf(ilo, up ? root + e : -ROW_FREE);
+    hi = fminf(hi, up ? ROW_FREE : root + e);
+    ihi = fminf(ihi, up ? ROW_FREE : root - e);
   }
-  xa = lo > (double)S.g1[0] ? S.g1[0] + 1 : (int)lo;
-  xb = hi < (double)S.g0[0] ? S.g0[0] - 1 : (int)hi;
+  const float below = (float)T.x0 - 1.0f, above = (float)T.x1 + 1.0f;
+  xa = (int)ceilf(fminf(lo, above));
+  xb = (int)floorf(fmaxf(hi, below));
+  ia = (int)ceilf(fminf(ilo, above));
+  ib = (int)floorf(fmaxf(ihi, below));
+  if (T.exact) {
+    xa = T.x0;
+    xb = T.x1;
+    ia = 0;
+    ib = -1;
+  }
 }
-
-template <typename K>
-struct Stager {
-  K* buf;            // this wave's LDS stage
-  uint32_t n = 0;    // wave-uniform count
-  K* keys;
-  unsigned long long* count;
-  __device__ inline void flush() {
-    wave_sync();
-    uint64_t base = 0;
-    if (__lane_id() == 0) base = atomicAdd(count, (unsigned long long)n);
-    base = bcast_first(base);
-    for (uint32_t i = __lane_id(); i < n; i += 64) keys[base + i] = buf[i];
-    wave_sync();
-    n = 0;
-  }
-  __device__ inline void push(bool hit, K key) {
-    const uint64_t mask = __ballot(hit);
-    if (mask == 0) return;
-    if (hit) buf[n + lanes_below(mask)] = key;
-    n += (uint32_t)__popcll(mask);
-    if (n > STAGE - 64) flush();
-  }
-  __device__ inline void finish() {
-    if (n) flush();
-  }
-};
-
-// Occupancy-bitmap output: bit (code & 31) of word bm_off[mesh] + code / 32
-// is set for every hit (the dense flag array of SVO.cu:180-182 at one bit per
-// cell).  Each lane keeps the word of its last hit and ORs it into memory
-// only when a hit falls in another word (consecutive cells of a row share a
-// word up to four at a time), so the atomics issued are fewer than the hits.
-// Raw hits are counted per wave and added once at the end.
-struct BitSink {
-  uint32_t* bits;
-  unsigned long long* count;
-  uint64_t n = 0;          // wave-uniform
-  uint64_t pend_word = 0;  // per lane
-  uint32_t pend_bits = 0;
-  __device__ inline void flush_lane() {
-    if (pend_bits)
-      __hip_atomic_fetch_or(bits + pend_word, pend_bits, __ATOMIC_RELAXED,
-                            __HIP_MEMORY_SCOPE_AGENT);
-  }
-  __device__ inline void push(bool hit, uint64_t word, uint32_t bit) {
-    const uint64_t mask = __ballot(hit);
-    if (mask == 0) return;
-    n += (uint64_t)__popcll(mask);
-    if (hit) {
-      if (word != pend_word) {
-        flush_lane();
-        pend_word = word;
-        pend_bits = 0;
-      }
-      pend_bits |= 1u << bit;
-    }
-  }
-  __device__ inline void finish() {
-    flush_lane();
-    pend_bits = 0;
-    if (n && __lane_id() == 0) atomicAdd(count, (unsigned long long)n);
-  }
-};
 
 // Where a voxelization kernel puts its hits: keys (staged, for the sort) or
 // the occupancy bitmap.
@@ -410,61 +424,25 @@ struct VoxOut {
   K* keys;                // key path
   uint32_t* bits;         // bitmap path
   const uint64_t* bm_off; // bitmap words before each mesh
-  unsigned long long* count;
+  unsigned long long* count;  // key path: keys stored
+  unsigned long long* hits;   // bitmap path: HIT_SLOTS counters HIT_STRIDE apart
 };
 
-// Big-triangle work item: 512 rows (y, z) of the box, eight per lane (256
-// and 128 rows measured slower: more items, each paying the triangle set-up).
+// Big-triangle work item: 512 rows (y, z) of the box.
 constexpr uint64_t BIG_ROWS = 512;
 
-// Voxelization order.  One lane walks each small triangle's box, so a wave
-// runs as long as the largest box among its 64 triangles.  k_classify gives
-// every triangle a size class (one byte: triangles past the one-lane limit,
-// which k_vox_small only queues, first, then eighth-octave classes of the box
-// cells, exact below 32 cells, largest first), and k_order sorts each run of
-// ORDER_GROUP consecutive triangles by class into `order`: the waves of a run
-// see boxes of about one size.  Triangles of one class keep roughly their
-// input order, which keeps the neighbouring triangles of a mesh together.  k_vox_small deals the runs' workgroup slots
-// out slot-major (the first slot of every run, then the second, ...), so the
-// workgroups of the largest boxes start first and the launch ends on the
-// smallest.  The order does not change the hits.
-constexpr uint32_t ORDER_THREADS = 1024;
-constexpr uint32_t ORDER_PER = 8;  // triangles per thread of k_order
-constexpr uint32_t ORDER_GROUP = ORDER_THREADS * ORDER_PER;
-constexpr uint32_t ORDER_BINS = 256;
-static_assert(ORDER_GROUP % BLOCK == 0, "a run fills whole workgroups of k_vox_small");
-
-// Size class, largest boxes first: 0 past the one-lane limit, then
-// 254 - (eighth-octave class of the cells); 255 for triangles that walk
-// nothing (failed mesh, bad index).
-__device__ inline uint32_t size_bin(uint64_t cells, uint64_t small_max) {
-  if (cells > small_max) return 0;
-  if (cells < 32) return ORDER_BINS - 2 - (uint32_t)cells;
-  const uint32_t e = 63u - (uint32_t)__builtin_clzll(cells);  // >= 5
-  const uint32_t b = 32u + 8u * (e - 5u) + (uint32_t)((cells >> (e - 3u)) & 7u);
-  return ORDER_BINS - 2 - (b < ORDER_BINS - 3 ? b : ORDER_BINS - 3);
-}
-
-// A pass of at most 8 runs (65,536 triangles) keeps the triangles' own
-// order: there the run sort's kernel (7-9 us, on the pass's critical path)
-// costs more than the voxelizer saves (256 single-mesh passes of 320-81,920
-// triangles took 80 ms sorted against 71-79 ms unsorted).
-inline bool sorted_order(uint64_t n_tris) { return n_tris > 8ull * ORDER_GROUP; }
-
 // Candidate cells and big-triangle chunk counts (added to totals[0],
-// totals[1]) and each triangle's size class (bins[gid], when bins is set).
-// A grid-stride loop over a bounded grid: the two totals take one atomic per
+// totals[1]).  A grid-stride loop over a bounded grid: the two totals take one atomic per
 // workgroup, and atomics on one address serialize.
 constexpr uint32_t CLASSIFY_BLOCKS = 1024;
 __global__ __launch_bounds__(BLOCK) void k_classify(const MeshDev* meshes,
                                                     const MeshParams* params,
                                                     const uint64_t* tri_base, uint32_t n_meshes,
                                                     uint64_t n_tris, uint32_t small_max,
-                                                    unsigned long long* totals, uint8_t* bins) {
+                                                    unsigned long long* totals) {
   uint64_t cells = 0, chunks = 0;
   for (uint64_t gid = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; gid < n_tris;
        gid += (uint64_t)gridDim.x * BLOCK) {
-    uint32_t bin = ORDER_BINS - 1;
     const uint32_t m = find_mesh(tri_base, n_meshes, gid);
     const MeshDev& md = meshes[m];
     const MeshParams& P = params[m];
@@ -477,9 +455,7 @@ __global__ __launch_bounds__(BLOCK) void k_classify(const MeshDev* meshes,
       const uint64_t sm = md.small_max ? md.small_max : small_max;
       cells += c;
       if (c > sm) chunks += (ny * nz + BIG_ROWS - 1) / BIG_ROWS;
-      bin = size_bin(c, sm);
     }
-    if (bins) bins[gid] = (uint8_t)bin;
   }
   for (int off = 32; off > 0; off >>= 1) {
     cells += __shfl_xor(cells, off);
@@ -498,77 +474,6 @@ __global__ __launch_bounds__(BLOCK) void k_classify(const MeshDev* meshes,
   }
 }
 
-// One workgroup per run of ORDER_GROUP triangles: a counting sort of the
-// run's size classes into `order`.  Each wave counts its triangles in a
-// histogram of its own (a run's triangles fall into few classes, and LDS
-// atomics on one address serialize across the whole workgroup), the
-// (class, wave) counts are scanned class-major, and every triangle lands at
-// its class's and wave's offset plus its rank in the wave's count.  Thread t
-// takes triangles t, t + 1024, ... of the run, so the lanes of a wave hold
-// consecutive triangles and a class's triangles from one wave land near each
-// other (the order of ranks within one atomic instruction is the hardware's).
-constexpr uint32_t ORDER_WAVES = ORDER_THREADS / 64;
-__global__ __launch_bounds__(ORDER_THREADS) void k_order(const uint8_t* bins, uint64_t n_tris,
-                                                         uint32_t* order) {
-  __shared__ uint32_t s_cnt[ORDER_BINS][ORDER_WAVES];  // then (class, wave) offsets
-  __shared__ uint32_t s_tot[ORDER_BINS];
-  const uint32_t wave = threadIdx.x >> 6;
-  for (uint32_t i = threadIdx.x; i < ORDER_BINS * ORDER_WAVES; i += ORDER_THREADS)
-    (&s_cnt[0][0])[i] = 0;
-  __syncthreads();
-  const uint64_t g0 = (uint64_t)blockIdx.x * ORDER_GROUP;
-  uint32_t bin[ORDER_PER], rank[ORDER_PER];
-#pragma unroll
-  for (uint32_t k = 0; k < ORDER_PER; ++k) {
-    const uint64_t gid = g0 + k * ORDER_THREADS + threadIdx.x;
-    bin[k] = gid < n_tris ? bins[gid] : 0u;
-  }
-#pragma unroll
-  for (uint32_t k = 0; k < ORDER_PER; ++k)
-    rank[k] = g0 + k * ORDER_THREADS + threadIdx.x < n_tris
-                  ? atomicAdd(&s_cnt[bin[k]][wave], 1u) : 0u;
-  __syncthreads();
-  // per class: exclusive prefix over the waves, total to s_tot
-  if (threadIdx.x < ORDER_BINS) {
-    uint32_t t = 0;
-#pragma unroll
-    for (uint32_t w = 0; w < ORDER_WAVES; ++w) {
-      const uint32_t c = s_cnt[threadIdx.x][w];
-      s_cnt[threadIdx.x][w] = t;
-      t += c;
-    }
-    s_tot[threadIdx.x] = t;
-  }
-  __syncthreads();
-  if (threadIdx.x < 64) {
-    // exclusive scan of the class totals, four classes per lane
-    const uint32_t l = threadIdx.x;
-    uint32_t c[4], t = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      c[j] = s_tot[4 * l + j];
-      t += c[j];
-    }
-    uint32_t inc = t;
-    for (int d = 1; d < 64; d <<= 1) {
-      const uint32_t o = __shfl_up(inc, d);
-      if (l >= (uint32_t)d) inc += o;
-    }
-    uint32_t ex = inc - t;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      s_tot[4 * l + j] = ex;
-      ex += c[j];
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (uint32_t k = 0; k < ORDER_PER; ++k) {
-    const uint64_t gid = g0 + k * ORDER_THREADS + threadIdx.x;
-    if (gid < n_tris) order[g0 + s_tot[bin[k]] + s_cnt[bin[k]][wave] + rank[k]] = (uint32_t)gid;
-  }
-}
-
 __global__ void k_flag_bad_index(const MeshDev* meshes, MeshParams* params,
                                  const uint64_t* tri_base, uint32_t n_meshes, uint64_t n_tris) {
   const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -580,157 +485,231 @@ __global__ void k_flag_bad_index(const MeshDev* meshes, MeshParams* params,
     if (t[k] < 0 || (uint64_t)t[k] >= md.n_points) atomicOr(&params[m].status, ERR_INDEX);
 }
 
-template <typename K, bool BITMAP>
-__global__ __launch_bounds__(BLOCK) void k_vox_small(
-    const MeshDev* meshes, const MeshParams* params, const uint64_t* tri_base, uint32_t n_meshes,
-    uint64_t n_tris, int cb, uint32_t small_max, const uint32_t* order, VoxOut<K> out,
-    BigItem* big, unsigned long long* big_count, uint64_t big_cap) {
-  __shared__ K stage[BITMAP ? 1 : WAVES][BITMAP ? 1 : STAGE];
-  Stager<K> st;
-  st.buf = stage[BITMAP ? 0 : threadIdx.x >> 6];
-  st.keys = out.keys;
-  st.count = out.count;
-  BitSink bs;
-  bs.bits = out.bits;
-  bs.count = out.count;
-  // triangles in the order k_classify wrote (boxes of about one size per
-  // wave), workgroup slots of the runs dealt out slot-major
-  const uint32_t runs = (uint32_t)((n_tris + ORDER_GROUP - 1) / ORDER_GROUP);
-  const uint64_t pos = (uint64_t)(blockIdx.x % runs) * ORDER_GROUP +
-                       (uint64_t)(blockIdx.x / runs) * BLOCK + threadIdx.x;
-  const uint64_t gid = pos >= n_tris ? n_tris : order ? order[pos] : pos;
-  TriSetup S;
-  uint64_t count = 0;
-  K mesh_key = 0;
-  uint64_t wbase = 0;
-  if (gid < n_tris) {
-    const uint32_t m = find_mesh(tri_base, n_meshes, gid);
-    const MeshDev& md = meshes[m];
-    const MeshParams P = params[m];
-    float v[3][3];
-    if (P.status == 0 && load_tri(md, P, gid - md.tri_base, v)) {
-      tri_setup(v, P, S);
-      const uint64_t nx = S.g1[0] - S.g0[0] + 1, ny = S.g1[1] - S.g0[1] + 1,
-                     nz = S.g1[2] - S.g0[2] + 1;
-      const uint64_t cells = nx * ny * nz;
-      if (cells <= (md.small_max ? md.small_max : small_max)) {
-        count = cells;
-      } else {
-        const uint64_t nch = (ny * nz + BIG_ROWS - 1) / BIG_ROWS;
-        const uint64_t at = atomicAdd(big_count, (unsigned long long)nch);
-        for (uint64_t j = 0; j < nch; ++j)
-          if (at + j < big_cap) big[at + j] = BigItem{(uint32_t)gid, (uint32_t)(j * BIG_ROWS)};
-      }
-      mesh_key = (K)m << cb;
-      if (BITMAP) wbase = out.bm_off[m];
+// Voxelizes runs of `per_wave` triangles, a wave each (ITEMS: the queued items
+// of big triangles, one each).  A triangle's box rows go to the lanes of its
+// wave, so that a wave's time follows the rows of all its triangles and not
+// the largest of them, and a row costs its 15 LDS pieces and about 290
+// instructions however many cells it crosses, and about 85 per four cells it
+// hits.  Bound by those instructions on soups (100,000 triangles at res 1024:
+// 58 us, and 24 for the queued items; a lane per triangle that tested every
+// cell of its box took 216 and 75), by the atomics on small triangles
+// (327,680 at res 512: 75 us, 39 without them; 110 before).
+//
+// Bitmap bits go through a table in LDS before they reach memory, 64 cells
+// (4 x 4 x 4) an entry: an atomic on memory that all XCDs share is carried out
+// beyond their L2s, about 30 G of them a second whatever their width, and
+// neighboring rows and triangles set bits of the same words.  A word whose
+// slot holds another goes to memory at once.
+constexpr uint32_t MAX_PER_WAVE = 32;
+constexpr int WORD_SLOT_BITS = 9;
+constexpr uint32_t WORD_SLOTS = 1u << WORD_SLOT_BITS, NO_WORD = 0xFFFFFFFFu;
+struct WordTable {
+  unsigned long long bits[WORD_SLOTS];
+  uint32_t word[WORD_SLOTS];
+};
+__device__ inline void or_memory(uint32_t* bitmap, uint64_t word, unsigned long long bits) {
+  __hip_atomic_fetch_or((unsigned long long*)bitmap + word, bits, __ATOMIC_RELAXED,
+                        __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void set_bits(WordTable& t, uint32_t* bitmap, uint64_t word,
+                                unsigned long long bits) {
+  if (word < NO_WORD) {
+    const uint32_t slot = ((uint32_t)word * 0x9E3779B1u) >> (32 - WORD_SLOT_BITS);
+    const uint32_t old = atomicCAS(&t.word[slot], NO_WORD, (uint32_t)word);
+    if (old == NO_WORD || old == (uint32_t)word) {
+      atomicOr(&t.bits[slot], bits);
+      return;
     }
   }
-  uint64_t c = 0;
-  int x = S.g0[0], y = S.g0[1], z = S.g0[2];
-  bool row_ok = false;
-  RowTerms R;
-  // the Morton code of (x, y, z) as an x part (back to mx0 at each row start)
-  // and a y|z part stepped row by row
-  const K MX = morton_x_mask<K>(), MY = MX << 1, MZ = MX << 2;
-  K mx0 = 0, my0 = 0, cyz = 0;
-  if (count) {
-    mx0 = morton3<K>((uint32_t)S.g0[0], 0u, 0u);
-    my0 = morton3<K>(0u, (uint32_t)S.g0[1], 0u);
-    cyz = my0 | morton3<K>(0u, 0u, (uint32_t)S.g0[2]);
+  or_memory(bitmap, word, bits);
+}
+
+template <typename K, bool BITMAP, bool ITEMS>
+__global__ __launch_bounds__(BLOCK) void k_vox_rows(
+    const MeshDev* meshes, const MeshParams* params, const uint64_t* tri_base, uint32_t n_meshes,
+    uint64_t n_tris, int cb, uint32_t small_max, uint32_t per_wave, VoxOut<K> out, BigItem* big,
+    unsigned long long* big_count, uint64_t big_cap) {
+  __shared__ RowTri s_tri[WAVES][ITEMS ? 1 : MAX_PER_WAVE];
+  __shared__ uint32_t s_mark[WAVES][64];
+  __shared__ K s_key[BITMAP ? 1 : WAVES][BITMAP ? 1 : STAGE];
+  __shared__ WordTable s_words[1];  // (bitmap path only: the key path leaves it out)
+  const uint32_t w = threadIdx.x >> 6, lane = __lane_id();
+  const uint64_t wave = (uint64_t)blockIdx.x * WAVES + w;
+  if (BITMAP) {
+    for (uint32_t i = threadIdx.x; i < WORD_SLOTS; i += BLOCK) {
+      s_words[0].word[i] = NO_WORD;
+      s_words[0].bits[i] = 0;
+    }
+    __syncthreads();
   }
-  K cx = mx0;
-  while (__any(c < count)) {
-    bool hit = false;
-    K code = 0;
-    if (c < count) {
-      if (x == S.g0[0]) row_ok = row_terms(S, y, z, R);
-      if (row_ok) {
-        hit = cell_hit(S, R, x);
-        code = cx | cyz;
-      }
-      if (row_ok && x < S.g1[0]) {
-        ++x;
-        ++c;
-        cx = dilated_inc(cx, MX);
-      } else {  // end of row, or an empty row skipped as a whole
-        c += (uint64_t)(S.g1[0] - x + 1);
-        x = S.g0[0];
-        cx = mx0;
-        if (++y > S.g1[1]) {
-          y = S.g0[1];
-          ++z;
-          cyz = dilated_inc((cyz & ~MY) | my0, MZ);
+  // ---- set-up: a lane per triangle
+  uint64_t gid = n_tris, first = 0;
+  uint32_t row0 = 0;
+  bool mine;
+  if (ITEMS) {
+    const uint64_t queued = *big_count, n_items = queued < big_cap ? queued : big_cap;
+    mine = lane == 0 && wave < n_items;
+    if (mine) {
+      gid = big[wave].tri;
+      row0 = big[wave].row0;
+    }
+    mine = mine && gid < n_tris;
+    first = bcast_first(gid);
+  } else {
+    first = wave * per_wave;
+    gid = first + lane;
+    mine = lane < per_wave && gid < n_tris;
+  }
+  uint32_t rows = 0;
+  const uint32_t m =
+      first < n_tris ? find_mesh_wave(tri_base, n_meshes, first, mine ? gid : first) : 0u;
+  {
+    uint32_t chunks = 0;
+    TriSetup S;
+    if (mine) {
+      const MeshDev& md = meshes[m];
+      const MeshParams P = params[m];
+      float v[3][3];
+      if (P.status == 0 && load_tri(md, P, gid - md.tri_base, v)) {
+        tri_setup(v, P, S);
+        const uint64_t nx = S.g1[0] - S.g0[0] + 1, ny = S.g1[1] - S.g0[1] + 1,
+                       nz = S.g1[2] - S.g0[2] + 1;
+        if (ITEMS) {
+          rows = (uint32_t)std::min<uint64_t>(BIG_ROWS, ny * nz - row0);
+        } else if (nx * ny * nz <= (md.small_max ? md.small_max : small_max)) {
+          rows = (uint32_t)(ny * nz);
         } else {
-          cyz = dilated_inc(cyz, MY);
+          chunks = (uint32_t)((ny * nz + BIG_ROWS - 1) / BIG_ROWS);
         }
       }
     }
-    if (BITMAP) bs.push(hit, wbase + (uint64_t)(code >> 5), (uint32_t)(code & 31));
-    else st.push(hit, mesh_key | code);
-  }
-  if (BITMAP) bs.finish();
-  else st.finish();
-}
-
-// One wave per work item of 512 rows: each lane prunes eight rows of the item
-// to their x-ranges and walks them; each inner loop runs as long as the
-// longest pruned row of the 64.
-template <typename K, bool BITMAP>
-__global__ __launch_bounds__(BLOCK) void k_vox_big(const MeshDev* meshes,
-                                                   const MeshParams* params,
-                                                   const uint64_t* tri_base, uint32_t n_meshes,
-                                                   int cb, const BigItem* big, uint64_t big_cap,
-                                                   const unsigned long long* big_count,
-                                                   uint64_t n_tris, VoxOut<K> out) {
-  __shared__ K stage[BITMAP ? 1 : WAVES][BITMAP ? 1 : STAGE];
-  const uint32_t w = threadIdx.x >> 6;
-  const uint32_t lane = __lane_id();
-  Stager<K> st;
-  st.buf = stage[BITMAP ? 0 : w];
-  st.keys = out.keys;
-  st.count = out.count;
-  BitSink bs;
-  bs.bits = out.bits;
-  bs.count = out.count;
-  const uint64_t item_id = (uint64_t)blockIdx.x * WAVES + w;
-  const uint64_t queued = *big_count;
-  const uint64_t n_items = queued < big_cap ? queued : big_cap;
-  if (item_id < n_items && big[item_id].tri < n_tris) {
-    const BigItem it = big[item_id];
-    const uint32_t m = find_mesh(tri_base, n_meshes, it.tri);
-    const MeshDev& md = meshes[m];
-    const MeshParams P = params[m];
-    float v[3][3];
-    load_tri(md, P, it.tri - md.tri_base, v);  // indices were checked when queued
-    TriSetup S;
-    tri_setup(v, P, S);
-    RangeConst RC;
-    range_const(S, RC);
-    const uint64_t ny = S.g1[1] - S.g0[1] + 1, nz = S.g1[2] - S.g0[2] + 1;
-    const K mesh_key = (K)m << cb;
-    const uint64_t wbase = BITMAP ? out.bm_off[m] : 0;
-    for (uint64_t k = 0; k < BIG_ROWS; k += 64) {
-      const uint64_t r = (uint64_t)it.row0 + k + lane;
-      int y = 0, z = 0, xa = 0, xb = -1;
-      RowTerms R;
-      if (r < ny * nz) {
-        y = S.g0[1] + (int)(r % ny);
-        z = S.g0[2] + (int)(r / ny);
-        if (row_terms(S, y, z, R)) row_range(S, RC, R, xa, xb);
-      }
-      // the code steps with x; past xb it is not used
-      K code = morton3<K>((uint32_t)xa, (uint32_t)y, (uint32_t)z);
-      const K MX = morton_x_mask<K>();
-      for (int x = xa; __any(x <= xb); ++x) {
-        const bool hit = (x <= xb) & cell_hit(S, R, x);
-        if (BITMAP) bs.push(hit, wbase + (uint64_t)(code >> 5), (uint32_t)(code & 31));
-        else st.push(hit, mesh_key | code);
-        code = dilated_inc(code, MX);
-      }
+    if (!ITEMS && __any(chunks != 0)) {
+      // one atomic per wave for its triangles' items
+      const uint32_t inc = wave_incl_scan_dpp(chunks);
+      uint64_t at = 0;
+      if (lane == 63) at = atomicAdd(big_count, (unsigned long long)inc);
+      at = (uint64_t)__shfl((uint32_t)at, 63) | ((uint64_t)__shfl((uint32_t)(at >> 32), 63) << 32);
+      at += inc - chunks;
+      for (uint32_t j = 0; j < chunks; ++j)
+        if (at + j < big_cap) big[at + j] = BigItem{(uint32_t)gid, j * (uint32_t)BIG_ROWS};
+    }
+    if (rows) {
+      RowTri& T = s_tri[w][ITEMS ? 0 : lane];
+      row_setup(S, T);
+      const uint64_t k = BITMAP ? out.bm_off[m] / 2 : (uint64_t)m << cb;  // (whole tiles)
+      T.key_lo = (uint32_t)k;
+      T.key_hi = (uint32_t)(k >> 32);
     }
   }
-  if (BITMAP) bs.finish();
-  else st.finish();
+  const uint32_t inc_rows = wave_incl_scan_dpp(rows), start = inc_rows - rows;
+  const uint32_t total = __builtin_amdgcn_readlane(inc_rows, 63);
+  if (rows) s_tri[w][ITEMS ? 0 : lane].row0 = start - row0;
+  wave_sync();
+  // ---- rows: a lane each
+  uint64_t n_hits = 0;      // bitmap path: this lane's
+  uint32_t staged = 0;      // key path: keys in s_key (the same in every lane)
+  uint32_t owner = 0;       // 1 + the triangle of the last item taken
+  constexpr K MX = (K)(sizeof(K) == 4 ? 0x09249249u : 0x1249249249249249ull);
+  auto flush = [&]() {
+    wave_sync();
+    uint64_t base = 0;
+    if (lane == 0) base = atomicAdd(out.count, (unsigned long long)staged);
+    base = bcast_first(base);
+    for (uint32_t i = lane; i < staged; i += 64) out.keys[base + i] = s_key[BITMAP ? 0 : w][i];
+    wave_sync();
+    staged = 0;
+  };
+  for (uint32_t base = 0; base < total; base += 64) {
+    const uint32_t item = base + lane;
+    // the triangle of an item: triangles mark where their rows begin, and the
+    // last mark at or before the item counts
+    uint32_t tr = 0;
+    if (!ITEMS) {
+      s_mark[w][lane] = 0;
+      wave_sync();
+      if (rows && start >= base && start - base < 64) s_mark[w][start - base] = lane + 1;
+      wave_sync();
+      const uint32_t mark = s_mark[w][lane];
+      owner = wave_incl_max_dpp(lane == 0 && mark == 0 ? owner : mark);
+      tr = owner - 1;
+      owner = __builtin_amdgcn_readlane(owner, 63);
+    }
+    const RowTri& T = s_tri[w][tr];
+    const uint32_t r = item - T.row0;
+    int y, z;
+    if (ITEMS) {
+      z = (int)(r / (uint32_t)T.ny);
+      y = (int)(r - (uint32_t)z * (uint32_t)T.ny);
+    } else {
+      // r < 2^20 (the limit on box cells), so that the quotient of
+      // r + 1/2 lies at least 2^-21 of itself from a whole number: exact
+      z = (int)(((float)r + 0.5f) * T.inv_ny);
+      y = (int)r - z * T.ny;
+    }
+    y += T.y0;
+    z += T.z0;
+    int xa = 0, xb = -1, ia = 0, ib = -1;
+    RowTerms R;
+    if (item < total && row_terms(T, y, z, R)) row_range(T, R, xa, xb, ia, ib);
+    // four cells at a time: they share a bitmap word
+    const uint64_t kbase = (uint64_t)T.key_lo | ((uint64_t)T.key_hi << 32);
+    int x = xa & ~3;
+    K code = morton3<K>((uint32_t)x, (uint32_t)y, (uint32_t)z);
+    while (__any(x <= xb)) {
+      uint32_t hit = 0, test = 0;
+      if (x <= xb) {
+        // bits [a, b] of four
+        auto span = [&](int a, int b) -> uint32_t {
+          a = a > x ? a - x : 0;
+          b = b < x + 3 ? b - x : 3;
+          return a <= b ? (2u << b) - (1u << a) : 0u;
+        };
+        test = span(xa, xb);
+        hit = span(ia, ib) & test;
+        test &= ~hit;
+      }
+      while (__any(test != 0)) {  // cells that rounding could decide either way
+        if (test) {
+          const uint32_t j = __builtin_ctz(test);
+          if (cell_hit(T, R, x + (int)j)) hit |= 1u << j;
+          test &= test - 1u;
+        }
+      }
+      if (BITMAP) {
+        if (hit) {
+          n_hits += __popc(hit);
+          // cells 0-3 of the group are bits 0, 1, 8, 9 from its place
+          set_bits(s_words[0], out.bits, kbase + (uint64_t)(code >> 6),
+                   (unsigned long long)((hit & 3u) | ((hit & 12u) << 6)) << (code & 63));
+        }
+      } else {
+        const uint32_t cnt = __popc(hit), inc = wave_incl_scan_dpp(cnt);
+        uint32_t at = staged + inc - cnt;
+        for (uint32_t h = hit; h; h &= h - 1u) {
+          const uint32_t j = __builtin_ctz(h);
+          s_key[BITMAP ? 0 : w][at++] = (K)kbase | code | (K)((j & 1u) | ((j & 2u) << 2));
+        }
+        staged += __builtin_amdgcn_readlane(inc, 63);
+        if (staged > STAGE - 256) flush();
+      }
+      x += 4;
+      // x + 4 in the code: the bits of x from bit 2 on (bits 0 and 1 are zero)
+      constexpr K M4 = MX & ~(K)9;
+      code = (((code | ~M4) + 1) & M4) | (code & ~M4);
+    }
+  }
+  if (BITMAP) {
+    uint32_t h = (uint32_t)n_hits;  // a lane's rows hold fewer than 2^32 cells
+    h = wave_sum_u32(h);
+    if (h && lane == 0)
+      atomicAdd(out.hits + (wave % HIT_SLOTS) * HIT_STRIDE, (unsigned long long)h);
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < WORD_SLOTS; i += BLOCK)
+      if (s_words[0].word[i] != NO_WORD)
+        or_memory(out.bits, s_words[0].word[i], s_words[0].bits[i]);
+  } else if (staged) {
+    flush();
+  }
 }
 
 }  // namespace
@@ -752,67 +731,63 @@ void launch_params(const MeshDev* meshes, uint32_t n_meshes, const uint32_t* acc
 
 void launch_classify(const MeshDev* meshes, const MeshParams* params, const uint64_t* tri_base,
                      uint32_t n_meshes, uint64_t n_tris, const Tuning& tn,
-                     unsigned long long* totals, uint32_t* order, uint8_t* bins, hipStream_t s) {
+                     unsigned long long* totals, hipStream_t s) {
   if (n_tris == 0) return;
   const uint32_t blocks = (uint32_t)((n_tris + BLOCK - 1) / BLOCK);
   hipLaunchKernelGGL(k_flag_bad_index, dim3(blocks), dim3(BLOCK), 0, s, meshes,
                      const_cast<MeshParams*>(params), tri_base, n_meshes, n_tris);
   hipLaunchKernelGGL(k_classify, dim3(std::min<uint32_t>(blocks, CLASSIFY_BLOCKS)), dim3(BLOCK), 0,
-                     s, meshes, params, tri_base, n_meshes, n_tris, tn.small_max_cells, totals,
-                     sorted_order(n_tris) ? bins : nullptr);
-  if (!sorted_order(n_tris)) return;
-  const uint32_t runs = (uint32_t)((n_tris + ORDER_GROUP - 1) / ORDER_GROUP);
-  hipLaunchKernelGGL(k_order, dim3(runs), dim3(ORDER_THREADS), 0, s, (const uint8_t*)bins, n_tris,
-                     order);
+                     s, meshes, params, tri_base, n_meshes, n_tris, tn.small_max_cells, totals);
 }
 
-size_t order_bytes(uint64_t n_tris) {
-  // order (uint32 per triangle), then the size classes (one byte each)
-  const uint64_t n = std::max<uint64_t>(n_tris, 1);
-  return ((4 * n + 255) & ~(uint64_t)255) + ((n + 255) & ~(uint64_t)255);
+template <typename K, bool BITMAP>
+static void launch_rows(const MeshDev* meshes, const MeshParams* params, const uint64_t* tri_base,
+                        uint32_t n_meshes, uint64_t n_tris, int cb, const Tuning& tn,
+                        const VoxOut<K>& out, BigItem* big, unsigned long long* big_count,
+                        uint64_t big_cap, hipStream_t s) {
+  // triangles per wave: 32 while that leaves 8 waves to each of the 1024
+  // SIMDs, fewer in smaller passes (at least 4: a wave sets up as many
+  // triangles at a time as it has).  Waves that stage keys take as many as
+  // leaves 2 to a SIMD: each reserves its keys' places at least once, and
+  // atomics on the one key count follow each other at about 6 ns.
+  uint32_t per = MAX_PER_WAVE;
+  while (per > 4 && n_tris / per < (BITMAP ? 8192 : 2048)) per /= 2;
+  const uint64_t waves = (n_tris + per - 1) / per;
+  hipLaunchKernelGGL((k_vox_rows<K, BITMAP, false>), dim3((uint32_t)((waves + WAVES - 1) / WAVES)),
+                     dim3(BLOCK), 0, s, meshes, params, tri_base, n_meshes, n_tris, cb,
+                     tn.small_max_cells, per, out, big, big_count, big_cap);
+  if (big_cap)
+    hipLaunchKernelGGL((k_vox_rows<K, BITMAP, true>),
+                       dim3((uint32_t)((big_cap + WAVES - 1) / WAVES)), dim3(BLOCK), 0, s, meshes,
+                       params, tri_base, n_meshes, n_tris, cb, tn.small_max_cells, 1u, out, big,
+                       big_count, big_cap);
 }
 
 template <typename K>
 void launch_voxelize(const MeshDev* meshes, const MeshParams* params, const uint64_t* tri_base,
                      uint32_t n_meshes, uint64_t n_tris, int cb, const Tuning& tn, K* keys,
                      uint32_t* bitmap, const uint64_t* bm_off, unsigned long long* key_count,
-                     const uint32_t* order, BigItem* big, unsigned long long* big_count,
+                     unsigned long long* hits, BigItem* big, unsigned long long* big_count,
                      uint64_t big_cap, hipStream_t s) {
   if (n_tris == 0) return;
-  const VoxOut<K> out{keys, bitmap, bm_off, key_count};
-  if (!sorted_order(n_tris)) order = nullptr;  // the triangles' own order
-  // every run of ORDER_GROUP triangles has ORDER_GROUP / BLOCK workgroup slots
-  const uint32_t blocks = (uint32_t)((n_tris + ORDER_GROUP - 1) / ORDER_GROUP) *
-                          (ORDER_GROUP / BLOCK);
-  const uint32_t bblocks = (uint32_t)((big_cap + WAVES - 1) / WAVES);
-  if (bitmap) {
-    hipLaunchKernelGGL((k_vox_small<K, true>), dim3(blocks), dim3(BLOCK), 0, s, meshes, params,
-                       tri_base, n_meshes, n_tris, cb, tn.small_max_cells, order, out,
-                       big, big_count, big_cap);
-    if (big_cap)
-      hipLaunchKernelGGL((k_vox_big<K, true>), dim3(bblocks), dim3(BLOCK), 0, s, meshes, params,
-                         tri_base, n_meshes, cb, (const BigItem*)big, big_cap,
-                         (const unsigned long long*)big_count, n_tris, out);
-  } else {
-    hipLaunchKernelGGL((k_vox_small<K, false>), dim3(blocks), dim3(BLOCK), 0, s, meshes, params,
-                       tri_base, n_meshes, n_tris, cb, tn.small_max_cells, order, out,
-                       big, big_count, big_cap);
-    if (big_cap)
-      hipLaunchKernelGGL((k_vox_big<K, false>), dim3(bblocks), dim3(BLOCK), 0, s, meshes, params,
-                         tri_base, n_meshes, cb, (const BigItem*)big, big_cap,
-                         (const unsigned long long*)big_count, n_tris, out);
-  }
+  const VoxOut<K> out{keys, bitmap, bm_off, key_count, hits};
+  if (bitmap)
+    launch_rows<K, true>(meshes, params, tri_base, n_meshes, n_tris, cb, tn, out, big, big_count,
+                         big_cap, s);
+  else
+    launch_rows<K, false>(meshes, params, tri_base, n_meshes, n_tris, cb, tn, out, big, big_count,
+                          big_cap, s);
 }
 
 template void launch_voxelize<uint32_t>(const MeshDev*, const MeshParams*, const uint64_t*,
                                         uint32_t, uint64_t, int, const Tuning&, uint32_t*,
                                         uint32_t*, const uint64_t*, unsigned long long*,
-                                        const uint32_t*, BigItem*, unsigned long long*, uint64_t,
-                                        hipStream_t);
+                                        unsigned long long*, BigItem*, unsigned long long*,
+                                        uint64_t, hipStream_t);
 template void launch_voxelize<uint64_t>(const MeshDev*, const MeshParams*, const uint64_t*,
                                         uint32_t, uint64_t, int, const Tuning&, uint64_t*,
                                         uint32_t*, const uint64_t*, unsigned long long*,
-                                        const uint32_t*, BigItem*, unsigned long long*, uint64_t,
-                                        hipStream_t);
+                                        unsigned long long*, BigItem*, unsigned long long*,
+                                        uint64_t, hipStream_t);
 
 }  // namespace svo

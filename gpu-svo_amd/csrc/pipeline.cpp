@@ -400,7 +400,7 @@ uint64_t estimate_bytes(uint64_t n_points, uint64_t n_tris, const svo_params* p)
   const double per_node = (p->flags & SVO_BUILD_NO_VERTEX_EDGE) ? 170.0
                           : (p->semantics == SVO_SEM_INTENDED ? 800.0 : 640.0);
   const double b = nodes * per_node + hits * 8.0 * 2.5 + (double)n_points * 12.0 +
-                   (double)n_tris * 12.0 + (double)order_bytes(n_tris) + (1 << 20);
+                   (double)n_tris * 12.0 + (1 << 20);
   return (uint64_t)b;
 }
 
@@ -439,7 +439,7 @@ double pass_bytes_bound(const svo_params* p, int kb, uint64_t P, uint64_t T, int
     lv += K * cap + (l >= 2 ? 9.0 * cap : 0.0) + 4 * 256.0;
   }
   const double n_big = (double)T + rows / 512.0;
-  const double ws_common = 12.0 * P + 12.0 * T + (double)order_bytes(T) + 2 * 256.0 + lv +
+  const double ws_common = 12.0 * P + 12.0 * T + 2 * 256.0 + lv +
                            (double)level_tmp_bytes(kc) +
                            sizeof(BigItem) * std::max(n_big, 1.0) + 4.1 * N + 4096.0 +
                            (1 << 20);  // keep masks; control buffers of one mesh
@@ -915,12 +915,6 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
   }
   const uint64_t T = tri_base[n];
   if (T >= (1ull << 32)) return SVO_E_RES_LIMIT;  // triangle indices are 32-bit on the device
-  // per-class limits shrink with the pass's triangle count as the global one
-  // does (below)
-  for (MeshDev& d : md)
-    if (d.small_max)
-      d.small_max = (uint32_t)std::min<uint64_t>(d.small_max, std::max<uint64_t>(32, T / 128));
-
   // occupancy-bitmap words per mesh: one bit per Morton code below
   // morton(res - 1) + 1 (the reference's dense array size, SVO.cu:342-345),
   // each mesh's region rounded up to whole tiles of the level-1 pass
@@ -939,7 +933,7 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
   // params, counters
   const size_t sz_md = align256(sizeof(MeshDev) * n), sz_tb = align256(8 * (n + 1)),
                sz_bo = align256(8 * (n + 1)), sz_acc = align256(32 * n),
-               sz_par = align256(sizeof(MeshParams) * n), sz_cnt = align256(8 * 8);
+               sz_par = align256(sizeof(MeshParams) * n), sz_cnt = align256(8 * (8 + HIT_SLOTS * HIT_STRIDE));
   char* ctl = nullptr;
   SVO_TRY(W.get("ctl", sz_md + sz_tb + sz_bo + sz_acc + sz_par + sz_cnt, (void**)&ctl));
   MeshDev* d_md = (MeshDev*)ctl;
@@ -950,7 +944,7 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
   unsigned long long* d_cnt =
       (unsigned long long*)(ctl + sz_md + sz_tb + sz_bo + sz_acc + sz_par);
   // d_cnt: [0] box cells, [1] big chunks, [2] keys emitted, [3] big queued,
-  // [4] bitmap bytes zeroed by the level-1 pass
+  // [4] bitmap bytes zeroed by the level-1 pass, [8] on the hit counters
   if (!capture) {
     SVO_TRY(L.ensure_pinned(sz_md + sz_tb + sz_bo + 64 + sizeof(MeshParams) * n));
     // stage the mesh descriptors, triangle bases and bitmap offsets through
@@ -961,24 +955,13 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     std::memcpy((char*)L.pinned + sz_md + sz_tb, bm_off.data(), 8 * (n + 1));
     HIP_TRY(hipMemcpyAsync(d_md, L.pinned, sz_md + sz_tb + sz_bo, hipMemcpyHostToDevice, s));
   }
-  launch_fill_u32((uint32_t*)d_cnt, 0u, 16, s);
+  launch_fill_u32((uint32_t*)d_cnt, 0u, 2 * (8 + HIT_SLOTS * HIT_STRIDE), s);
   timer.mark("start");
 
   // ---- A0: bbox, params, classification
   launch_bbox(d_md, n, max_points, d_acc, s);
   launch_params(d_md, n, d_acc, d_par, s);
-  // Triangles with at most small_max_cells box cells are voxelized one lane
-  // each, larger ones by whole waves over 512-row items.  A pass with few
-  // triangles has too few lanes to hide a long per-lane loop, so its limit
-  // shrinks with the triangle count: T / 128 cells (32 below 4K triangles,
-  // 512 at 64K, the default 1024 from 128K).
-  Tuning tn = plan.tuning;
-  tn.small_max_cells = (uint32_t)std::min<uint64_t>(tn.small_max_cells,
-                                                    std::max<uint64_t>(32, T / 128));
-  uint32_t* order = nullptr;
-  SVO_TRY(W.get("order", order_bytes(T), (void**)&order));
-  launch_classify(d_md, d_par, d_tb, n, T, tn, d_cnt, order,
-                  (uint8_t*)order + align256(4 * T), s);
+  launch_classify(d_md, d_par, d_tb, n, T, plan.tuning, d_cnt, s);
   timer.mark("classify");
   uint64_t cells = 0, n_big = 0;
   if (capture) {
@@ -1102,12 +1085,12 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     bm_clean_after = std::max(clean, (size_t)bm_bytes);
     clean = 0;
   }
-  launch_voxelize<K>(d_md, d_par, d_tb, n, T, plan.cb, tn, keys_a, bitmap, d_bo,
-                     d_cnt + 2, order, big, d_cnt + 3, n_big, s);
+  launch_voxelize<K>(d_md, d_par, d_tb, n, T, plan.cb, plan.tuning, keys_a, bitmap, d_bo,
+                     d_cnt + 2, d_cnt + 8, big, d_cnt + 3, n_big, s);
   timer.mark("voxelize");
   if (use_bm) {
     launch_level_first_bitmap<K>(bitmap, bm_words, d_bo, n, kl, lv[1], lv[2], d_counts, d_spans,
-                                 NL, d_state, bm_tmp, lvl_tmp, d_cnt + 4, s);
+                                 NL, d_state, bm_tmp, lvl_tmp, d_cnt + 4, d_cnt + 8, d_cnt + 2, s);
     W.clean_bytes("bitmap") = bm_clean_after;
   } else {
     K* sorted = nullptr;

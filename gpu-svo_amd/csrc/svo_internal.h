@@ -13,7 +13,7 @@ namespace svo {
 constexpr int SIZE_CLASSES = 15;
 
 struct Tuning {
-  uint32_t small_max_cells = 1024;  // bbox cells handled by one lane
+  uint32_t small_max_cells = 1024;  // largest box (cells) whose triangle shares a wave
   uint32_t sort_blocks = 65536;     // grid bound of the radix sort passes (tiles stride)
   uint32_t scan_blocks = 1024;      // fixed grid of the level / attribute scans
   // Occupancy bitmap instead of the sort (level 1 straight from the bitmap)
@@ -26,8 +26,7 @@ struct Tuning {
   // up to batch_lanes concurrent passes
   uint32_t batch_lanes = 2;
   uint32_t batch_min_meshes = 16;
-  // Per size class (size_class_of) box-cell limit of the one-lane
-  // voxelization; 0 = small_max_cells.  Set by the tuning search.
+  // The same per size class (size_class_of); 0 = small_max_cells.  Set by the tuning search.
   uint32_t class_small_max[SIZE_CLASSES] = {};
 };
 
@@ -51,25 +50,23 @@ void launch_bbox(const MeshDev* meshes, uint32_t n_meshes, uint64_t max_points, 
                  hipStream_t s);
 void launch_params(const MeshDev* meshes, uint32_t n_meshes, const uint32_t* acc,
                    MeshParams* params, hipStream_t s);
-// Candidate cells and big-triangle chunk counts (2 x uint64 added to
-// `totals`), and the order launch_voxelize takes the triangles in
-// (`order`: n_tris uint32, a permutation of the triangle indices that
-// groups triangles of about one box size).  `order` heads a buffer of
-// order_bytes(n_tris) bytes whose tail `bins` (at byte 4 * n_tris rounded up
-// to 256) holds the triangles' size classes.
-size_t order_bytes(uint64_t n_tris);
+// Candidate cells and big-triangle chunk counts (2 x uint64 added to `totals`).
 void launch_classify(const MeshDev* meshes, const MeshParams* params, const uint64_t* tri_base,
                      uint32_t n_meshes, uint64_t n_tris, const Tuning& tn,
-                     unsigned long long* totals, uint32_t* order, uint8_t* bins, hipStream_t s);
+                     unsigned long long* totals, hipStream_t s);
+// Raw hits of the bitmap path are counted in HIT_SLOTS counters of a cache
+// line each (atomics on one address serialize); launch_level_first_bitmap
+// adds them up.
+constexpr uint32_t HIT_SLOTS = 64, HIT_STRIDE = 8;
 // Surface voxelization (SVO.cu:37-188): emits composite keys.
+// Hits go to `keys` (raw, for the sort; *key_count receives their number) when
+// `bitmap` is null, else into the occupancy bitmap (word bm_off[mesh] + code /
+// 32, bit code % 32, which the caller has zeroed; counted in `hits`).
 template <typename K>
-// Hits go to `keys` (raw, for the sort) when `bitmap` is null, else into the
-// occupancy bitmap (word bm_off[mesh] + code / 32, bit code % 32, which the
-// caller has zeroed); *key_count receives the number of raw hits.
 void launch_voxelize(const MeshDev* meshes, const MeshParams* params, const uint64_t* tri_base,
                      uint32_t n_meshes, uint64_t n_tris, int cb, const Tuning& tn, K* keys,
                      uint32_t* bitmap, const uint64_t* bm_off, unsigned long long* key_count,
-                     const uint32_t* order, BigItem* big, unsigned long long* big_count,
+                     unsigned long long* hits, BigItem* big, unsigned long long* big_count,
                      uint64_t big_cap, hipStream_t s);
 
 // ------------------------------------------------------------ k_sort.hip
@@ -105,7 +102,8 @@ void launch_level_first(const K* sorted, const unsigned long long* n_sorted, uin
 // [bm_off[m], bm_off[m+1]), and every bm_off[m] is a multiple of
 // BITMAP_TILE_WORDS): the same outputs as launch_level_first followed
 // by launch_level_first_finalize, and the bitmap is left all zero (the bytes
-// that takes are added to *reset_bytes).  `tmp` needs
+// that takes are added to *reset_bytes); *n_hits receives the sum of the
+// voxelization's hit counters `hits`.  `tmp` needs
 // bitmap_level_tmp_bytes(n_words); `lvl_tmp` (level_tmp_bytes of l1.cap) is
 // prepared for the later levels.
 size_t bitmap_level_tmp_bytes(uint64_t n_words);
@@ -120,7 +118,9 @@ void launch_level_first_bitmap(uint32_t* bits, uint64_t n_words, const uint64_t*
                                uint32_t n_meshes, KeyLayout<K> kl, LevelArrays l1,
                                LevelArrays l2, unsigned long long* counts, LevelSpan* spans1,
                                uint32_t n_levels, MeshTreeState* state, void* tmp,
-                               void* lvl_tmp, unsigned long long* reset_bytes, hipStream_t s);
+                               void* lvl_tmp, unsigned long long* reset_bytes,
+                               const unsigned long long* hits, unsigned long long* n_hits,
+                               hipStream_t s);
 // Marks meshes whose level-1 set holds a single voxel as depth-1 trees (the
 // sort path; launch_level_first_bitmap does it itself).
 void launch_level_first_finalize(const LevelSpan* spans, uint32_t n_meshes, uint32_t n_levels,

@@ -58,6 +58,18 @@ __device__ inline uint32_t wave_incl_scan_dpp(uint32_t v) {
   return (uint32_t)x;
 }
 
+// Inclusive maximum over the lanes up to each, the same way.
+__device__ inline uint32_t wave_incl_max_dpp(uint32_t v) {
+  auto up = [](uint32_t a, int b) { return a > (uint32_t)b ? a : (uint32_t)b; };
+  v = up(v, __builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, true));
+  v = up(v, __builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, true));
+  v = up(v, __builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, true));
+  v = up(v, __builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, true));
+  v = up(v, __builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false));
+  v = up(v, __builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false));
+  return v;
+}
+
 // Exclusive scan of two 32-bit values over a 256-thread block, in place;
 // ta / tb receive the block sums.  `tmp` holds 8 values.  One barrier: a
 // caller that scans again with the same `tmp` must put a barrier between the

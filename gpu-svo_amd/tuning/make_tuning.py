@@ -1,8 +1,8 @@
 """Writes a tuning file for this device: the library's tuning search
-(svo_ctx_autotune: global one-lane box limit and concurrent passes, then the
-one-lane box limit per size class) on the 256-mesh mixed batch (icospheres
+(svo_ctx_autotune: global box limit and concurrent passes, then the
+box limit per size class) on the 256-mesh mixed batch (icospheres
 and tori, 320-81,920 triangles, res 64-256, seed 3), device-resident; then
-the one-lane box limit of the size classes of two single large meshes the
+the box limit of the size classes of two single large meshes the
 batch does not hold, by timing their builds: the 2,000,000-triangle soup at
 res 1024 and icosphere-7 with value noise at res 512.
 
@@ -32,7 +32,7 @@ def size_class(res, n_tris):
 
 
 def tune_single(ctx, name, P, T, res, reps):
-    """Times builds of one mesh for each one-lane box limit of its size class
+    """Times builds of one mesh for each box limit of its size class
     and keeps the fastest if it beats the current limit by 3%."""
     cls = size_class(res, T.shape[0])
     opt = f"class_small_max_{cls}"
@@ -76,10 +76,10 @@ def main():
         d.free()
     singles = []
     P, T = meshgen.soup(2_000_000, seed=2)
-    print("one-lane limit of the soup's size class", file=sys.stderr, flush=True)
+    print("box limit of the soup's size class", file=sys.stderr, flush=True)
     singles.append(tune_single(ctx, "soup 2M res 1024", P, T, 1024, args.reps))
     P, T = meshgen.noisy_icosphere(7, seed=1)
-    print("one-lane limit of the icosphere's size class", file=sys.stderr, flush=True)
+    print("box limit of the icosphere's size class", file=sys.stderr, flush=True)
     singles.append(tune_single(ctx, "icosphere-7 + noise res 512", P, T, 512, args.reps))
     r["single_meshes"] = singles
     ctx.save_tuning(args.out)

@@ -176,7 +176,8 @@ int svo_plan_destroy(svo_plan* plan);
 
 /* Tuning options of the context (no counterpart in the reference), set
  * between builds:
- *   "small_max_cells"        box cells up to which one lane voxelizes a triangle (1024)
+ *   "small_max_cells"        box cells up to which a triangle shares a wave's lanes with
+ *                            others when it is voxelized (1024)
  *   "sort_blocks"            grid bound of the radix sort passes (65536)
  *   "scan_blocks"            persistent grid bound of the level passes (1024)
  *   "bitmap_max_bytes"       largest occupancy bitmap used instead of the sort (32 GiB)
@@ -194,7 +195,7 @@ int svo_ctx_get_option(svo_ctx* ctx, const char* name, int64_t* value);
  *     the fastest;
  *  2. then, per size class present in the sample (5 resolution bands x 3
  *     bands of res^2 / triangles; the option names class_small_max_<k>),
- *     builds that class's meshes alone with the one-lane box limit of the
+ *     builds that class's meshes alone with the box limit of the
  *     class in {64, 128, 256, 512, 1024, 2048, 4096} and keeps the limit
  *     whose voxelization (classify + voxelize stages, HIP events) is
  *     fastest, when it beats the global limit by more than 3 %.
