@@ -18,12 +18,13 @@
 // records are written later from these arrays (k_attrs.hip), once the node
 // counts are known.
 //
-// Each pass is a single-pass scan: persistent workgroups claim 4096-element
-// tiles by ticket, each thread loads 16 consecutive keys with vector loads,
-// the tile's counts are scanned in the workgroup and its offset found by
-// decoupled look-back (svo_scan.h); compacted outputs are staged in LDS and
-// written contiguously.  The element count is read from device memory, so no
-// launch shape depends on it.
+// Each pass is a single-pass scan: workgroups claim tiles by ticket, each
+// thread loads consecutive keys with vector loads, the tile's counts are
+// scanned in the workgroup and its offset found by decoupled look-back
+// (svo_scan.h); compacted outputs are staged in LDS and written contiguously.
+// The element count is read from device memory, so no launch shape depends on
+// it.  The coarse levels, a few thousand elements at most, run in one
+// workgroup and one launch together.
 #include <algorithm>
 
 #include "svo_internal.h"
@@ -36,6 +37,18 @@ constexpr int BLOCK = 256;
 constexpr int EPT = 16;             // consecutive elements per thread
 constexpr int TILE = BLOCK * EPT;   // 4096
 constexpr int MAX_TICKETS = 64;     // one per pass: level 1 .. level 63
+// Level passes over fewer elements than fill the chip with 4096-element tiles
+// take 1024-element tiles (4 per thread).
+constexpr int EPT_SMALL = 4, TILE_SMALL = BLOCK * EPT_SMALL;
+constexpr uint64_t SMALL_ELEMS = 256 * TILE;
+
+// Tiles, at most, of a level pass over up to n elements.
+__host__ __device__ inline uint64_t level_tiles(uint64_t n) {
+  const uint64_t big = (n + TILE - 1) / TILE;
+  const uint64_t m = n < SMALL_ELEMS ? n : SMALL_ELEMS;
+  const uint64_t small = (m + TILE_SMALL - 1) / TILE_SMALL;
+  return big > small ? big : small;
+}
 
 // flags of sorted hit key `cur`: bit0 = first copy of its key, bit1 = head of
 // its parent group
@@ -61,7 +74,7 @@ __device__ inline uint32_t level_flags_v(K prev, K cur, K next, bool has_prev, b
 
 __global__ __launch_bounds__(BLOCK) void k_level_clear(uint64_t* status, uint32_t* tickets,
                                                        const unsigned long long* n_ptr) {
-  const uint64_t words = 2 * ((*n_ptr + TILE - 1) / TILE);
+  const uint64_t words = 2 * level_tiles(*n_ptr);
   const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
   for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < words; i += stride)
     status[i] = 0;
@@ -453,7 +466,7 @@ __global__ __launch_bounds__(BLOCK) void k_bm_emit(uint32_t* bits, uint64_t n_wo
   {
     // the later levels' look-back words and tickets start at zero (as
     // k_level_clear leaves them), a slice per workgroup
-    const uint64_t words = 2 * ((counts[0] + TILE - 1) / TILE);
+    const uint64_t words = 2 * level_tiles(counts[0]);
     const uint64_t per = (words + gridDim.x - 1) / gridDim.x;
     const uint64_t i1 = std::min<uint64_t>(words, (uint64_t)(blockIdx.x + 1) * per);
     for (uint64_t i = (uint64_t)blockIdx.x * per + threadIdx.x; i < i1; i += BLOCK) status[i] = 0;
@@ -610,144 +623,278 @@ __global__ void k_first_finalize(const LevelSpan* spans, uint32_t n_meshes, uint
 
 // ---------------------------------------------------------------- level l >= 2
 // Level elements -> their group (group_l, NONE for roots and finished
-// meshes), the next level's keys with their first child, the spans of this
-// level, roots into state, and counts[level] (elements of the next level).
+// meshes), the next level's keys with their first child and child mask, the
+// spans of this level, roots into state, and counts[level] (elements of the
+// next level).
 template <typename K>
-__global__ __launch_bounds__(BLOCK) void k_level_pass(
-    int level, const K* elem, const unsigned long long* n_ptr, KeyLayout<K> kl,
-    MeshTreeState* state, uint32_t* group_l, K* elem_next, uint32_t* first_child_next,
-    uint8_t* kids_next, LevelSpan* spans, uint32_t n_levels, uint64_t* status, uint32_t* ticket,
-    uint32_t epoch, unsigned long long* count_next) {
-  __shared__ K s_edge[2][BLOCK];
-  __shared__ K s_key[TILE];
-  __shared__ uint32_t s_val[TILE];
-  __shared__ uint8_t s_kid[TILE];
-  __shared__ uint32_t tmp[4];
-  __shared__ uint32_t s_tile;
-  __shared__ uint32_t s_base;
-  const uint64_t n = *n_ptr;
-  const uint32_t li = (uint32_t)(level - 1);
-  const bool vec_out = ((uintptr_t)group_l & 15) == 0;
-  TileRun<K> r;
-  while (claim_tile(elem, n, ticket, &s_tile, s_edge, r)) {
-    // 4 flag bits per element: bit0 live (its mesh is still being built),
-    // bit1 group head, bit2 root
-    uint64_t f = 0;
-    uint32_t ng = 0;
-    {
-      uint32_t last_m = 0xFFFFFFFFu, done = 0;
-      K pk = r.prev;
-      bool hp = r.has_prev;
+struct LevelIo {
+  int level;
+  KeyLayout<K> kl;
+  MeshTreeState* state;
+  const K* elem;
+  uint32_t* group;
+  K* elem_next;
+  uint32_t* first_child_next;
+  uint8_t* kids_next;
+  LevelSpan* spans;
+  uint32_t n_levels;
+};
+
+// The keys before and after a tile, as far as its first and last threads
+// look: a group has at most eight members.
+constexpr int AHEAD = 8;
+// The workgroup's barrier for what it shares in LDS alone: __syncthreads()
+// also waits for the global stores in flight, which beside another stream's
+// emission take 10 us and more (a tail of five levels 184 us in place of 18).
+__device__ inline void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+template <typename K, int T, int E>
+struct LevelLds {
+  K key[T * E];  // the tile's keys, then its groups' keys
+  K before, after[AHEAD];
+  uint32_t val[T * E];
+  uint8_t kid[T * E];
+  uint32_t wave[T / 64];
+  uint32_t base;
+};
+
+// One tile of up to T * E elements from element tb on, T threads; base_of
+// (called by the first wave, all lanes) turns the tile's group count into its
+// first group.  Returns the group count; S.key then holds the groups' keys.
+// `resident`: S.key already holds the tile's keys, the whole level (the keys
+// that a tile left there).  Ends behind a barrier.
+template <typename K, int T, int E, typename F>
+__device__ inline uint32_t level_tile(const LevelIo<K>& A, uint64_t n, uint64_t tb,
+                                      LevelLds<K, T, E>& S, bool resident, F base_of) {
+  const uint32_t tn = (uint32_t)(n - tb < T * E ? n - tb : T * E), l0 = threadIdx.x * E;
+  const uint32_t cnt = l0 < tn ? (tn - l0 < E ? tn - l0 : E) : 0u;
+  const uint64_t i0 = tb + l0;
+  const KeyLayout<K> kl = A.kl;
+  K kk[E];
+  if (resident) {
 #pragma unroll
-      for (int e = 0; e < EPT; ++e) {
-        if ((uint32_t)e < r.cnt) {
-          const K cur = r.kk[e];
+    for (int e = 0; e < E; ++e) kk[e] = S.key[l0 + e];
+  } else {
+    load_consecutive(A.elem + (cnt ? i0 : 0), ((uintptr_t)A.elem & 15) == 0 && cnt, cnt, kk);
+    if (threadIdx.x < AHEAD && tb + tn + threadIdx.x < n)
+      S.after[threadIdx.x] = A.elem[tb + tn + threadIdx.x];
+    if (threadIdx.x == T - 1 && tb > 0) S.before = A.elem[tb - 1];
+#pragma unroll
+    for (int e = 0; e < E; ++e) S.key[l0 + e] = kk[e];
+    lds_barrier();
+  }
+  const bool has_prev = cnt && i0 > 0, has_next = cnt && i0 + cnt < n;
+  // the key after the thread's run and beyond (inside the level)
+  auto ahead = [&](uint32_t j) -> K {
+    const uint32_t i = l0 + cnt + j;
+    return i < tn ? S.key[i] : S.after[i - tn];
+  };
+  const K prev = !has_prev ? (K)0 : l0 > 0 ? S.key[l0 - 1] : S.before;
+  const K next = !has_next ? (K)0 : ahead(0);
+  // 4 flag bits per element: bit0 live (its mesh is still being built),
+  // bit1 group head, bit2 root
+  uint64_t f = 0;
+  uint32_t ng = 0, mask_ahead = 0;
+  {
+    uint32_t last_m = 0xFFFFFFFFu, done = 0;
+    K pk = prev;
+    bool hp = has_prev;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      if ((uint32_t)e < cnt) {
+        const K cur = kk[e];
+        // only level 2 holds an element of a finished mesh: the group of a
+        // single voxel (a later level's root is no group)
+        if (A.level == 2) {
           const uint32_t m = kl.mesh(cur);
           if (m != last_m) {
-            done = state[m].depth;
+            done = A.state[m].depth;
             last_m = m;
           }
-          if (done == 0) {
-            const bool more = e + 1 < EPT && (uint32_t)(e + 1) < r.cnt;
-            const bool hn = more || r.has_next;
-            const K nk = more ? r.kk[(e + 1) % EPT] : r.next;
-            const uint32_t fl = level_flags_v(pk, cur, nk, hp, hn, kl) | 1u;
-            f |= (uint64_t)fl << (4 * e);
-            ng += (fl >> 1) & 1u;
-          }
-          pk = cur;
-          hp = true;
         }
+        if (done == 0) {
+          const bool more = e + 1 < E && (uint32_t)(e + 1) < cnt;
+          const uint32_t fl = level_flags_v(pk, cur, more ? kk[(e + 1) % E] : next, hp,
+                                            more || has_next, kl) | 1u;
+          f |= (uint64_t)fl << (4 * e);
+          ng += (fl >> 1) & 1u;
+        }
+        pk = cur;
+        hp = true;
       }
     }
-    uint32_t tg;
-    const uint32_t exg = block_excl_scan256(ng, tmp, tg);
-    if (threadIdx.x < 64) {
-      const uint32_t pre = lookback_exclusive_wave(status + 1, 2, r.tile, tg, epoch);
-      if (threadIdx.x == 0) {
-        s_base = pre;
-        if (r.tb + r.tn == n) *count_next = (unsigned long long)pre + tg;
+    // the thread's last group may go on past its run: at most seven more keys
+    if (ng) {
+      const K P = kl.parent(pk);
+      for (uint32_t j = 0; j < AHEAD - 1 && i0 + cnt + j < n; ++j) {
+        const K key = ahead(j);
+        if (kl.parent(key) != P) break;
+        mask_ahead |= 1u << (uint32_t)(key & 7);
       }
     }
-    __syncthreads();
-    const uint32_t bg = s_base;
-    uint32_t gv[EPT];
-    {
-      uint32_t rg = exg;
-      K pk = r.prev;
-      bool hp = r.has_prev;
-      uint32_t mask = 0;  // children of the thread's current group so far
+  }
+  const uint32_t inc = wave_incl_scan_dpp(ng);
+  if ((threadIdx.x & 63) == 63) S.wave[threadIdx.x >> 6] = inc;
+  lds_barrier();
+  uint32_t exg = inc - ng, tg = 0;
 #pragma unroll
-      for (int e = 0; e < EPT; ++e) {
-        gv[e] = NONE;
-        if ((uint32_t)e < r.cnt) {
-          const K key = r.kk[e];
-          const uint64_t i = r.i0 + e;
-          const uint32_t fl = (uint32_t)(f >> (4 * e)) & 15u;
-          const uint32_t m = kl.mesh(key);
-          if (fl & 4u) {  // the only key of its mesh at this level: the root
-            state[m].depth = (uint32_t)level;
-            state[m].root_elem = (uint32_t)i;
-            LevelSpan& sp = spans[(uint64_t)m * n_levels + li];
-            sp.elem_first = (uint32_t)i;
-            sp.elem_end = (uint32_t)i + 1;
-            sp.group_first = sp.group_end = 0;
-          } else if (fl & 1u) {
-            if (fl & 2u) {
-              if (rg > exg) s_kid[rg - 1] = (uint8_t)mask;
-              s_key[rg] = kl.parent(key);
-              s_val[rg] = (uint32_t)i;
-              ++rg;
-              mask = 0;
-            }
-            mask |= 1u << (uint32_t)(key & 7);
-            gv[e] = bg + rg - 1;
-            const bool more = e + 1 < EPT && (uint32_t)(e + 1) < r.cnt;
-            const bool hn = more || r.has_next;
-            const K nk = more ? r.kk[(e + 1) % EPT] : r.next;
-            LevelSpan& sp = spans[(uint64_t)m * n_levels + li];
-            if (!hp || kl.mesh(pk) != m) {
-              sp.elem_first = (uint32_t)i;
-              sp.group_first = bg + rg - 1;
-            }
-            if (!hn || kl.mesh(nk) != m) {
-              sp.elem_end = (uint32_t)i + 1;
-              sp.group_end = bg + rg;
-            }
+  for (uint32_t w = 0; w < T / 64; ++w) {
+    const uint32_t x = S.wave[w];
+    if (w < threadIdx.x >> 6) exg += x;
+    tg += x;
+  }
+  if (threadIdx.x < 64) {
+    const uint32_t b = base_of(tg);
+    if (threadIdx.x == 0) S.base = b;
+  }
+  lds_barrier();
+  const uint32_t bg = S.base;
+  uint32_t gv[E];
+  {
+    uint32_t rg = exg;
+    K pk = prev;
+    bool hp = has_prev;
+    uint32_t mask = 0;  // children of the thread's current group so far
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      gv[e] = NONE;
+      if ((uint32_t)e < cnt) {
+        const K key = kk[e];
+        const uint64_t i = i0 + e;
+        const uint32_t fl = (uint32_t)(f >> (4 * e)) & 15u;
+        const uint32_t m = kl.mesh(key);
+        LevelSpan& sp = A.spans[(uint64_t)m * A.n_levels + (uint32_t)(A.level - 1)];
+        if (fl & 4u) {  // the only key of its mesh at this level: the root
+          A.state[m].depth = (uint32_t)A.level;
+          A.state[m].root_elem = (uint32_t)i;
+          sp.elem_first = (uint32_t)i;
+          sp.elem_end = (uint32_t)i + 1;
+          sp.group_first = sp.group_end = 0;
+        } else if (fl & 1u) {
+          if (fl & 2u) {
+            if (rg > exg) S.kid[rg - 1] = (uint8_t)mask;
+            S.key[rg] = kl.parent(key);
+            S.val[rg] = (uint32_t)i;
+            ++rg;
+            mask = 0;
           }
-          pk = key;
-          hp = true;
-        }
-      }
-      if (rg > exg) {
-        // the thread's last group may go on past its run: at most seven more
-        // keys, which the next thread or tile holds too
-        const K P = s_key[rg - 1];
-        for (uint64_t i = r.i0 + r.cnt; i < n; ++i) {
-          const K key = elem[i];
-          if (kl.parent(key) != P) break;
           mask |= 1u << (uint32_t)(key & 7);
+          gv[e] = bg + rg - 1;
+          const bool more = e + 1 < E && (uint32_t)(e + 1) < cnt;
+          if (!hp || kl.mesh(pk) != m) {
+            sp.elem_first = (uint32_t)i;
+            sp.group_first = bg + rg - 1;
+          }
+          if (!(more || has_next) || kl.mesh(more ? kk[(e + 1) % E] : next) != m) {
+            sp.elem_end = (uint32_t)i + 1;
+            sp.group_end = bg + rg;
+          }
         }
-        s_kid[rg - 1] = (uint8_t)mask;
+        pk = key;
+        hp = true;
       }
     }
-    if (vec_out && r.cnt == EPT) {
-      uint4* q = (uint4*)(group_l + r.i0);
+    if (rg > exg) S.kid[rg - 1] = (uint8_t)(mask | mask_ahead);
+  }
+  if (((uintptr_t)A.group & 15) == 0 && cnt == E) {
+    uint4* q = (uint4*)(A.group + i0);
 #pragma unroll
-      for (int v = 0; v < EPT / 4; ++v)
-        q[v] = make_uint4(gv[4 * v], gv[4 * v + 1], gv[4 * v + 2], gv[4 * v + 3]);
-    } else {
+    for (int v = 0; v < E / 4; ++v)
+      q[v] = make_uint4(gv[4 * v], gv[4 * v + 1], gv[4 * v + 2], gv[4 * v + 3]);
+  } else {
 #pragma unroll
-      for (int e = 0; e < EPT; ++e)
-        if ((uint32_t)e < r.cnt) group_l[r.i0 + e] = gv[e];
-    }
+    for (int e = 0; e < E; ++e)
+      if ((uint32_t)e < cnt) A.group[i0 + e] = gv[e];
+  }
+  lds_barrier();
+  for (uint32_t i = threadIdx.x; i < tg; i += T) {
+    A.elem_next[(uint64_t)bg + i] = S.key[i];
+    A.first_child_next[(uint64_t)bg + i] = S.val[i];
+    A.kids_next[(uint64_t)bg + i] = S.kid[i];
+  }
+  lds_barrier();
+  return tg;
+}
+
+// A level's tiles, claimed in order by ticket.  Workgroups past the tiles
+// leave without a ticket and, when every tile has a workgroup, each takes one
+// only: tickets on one address follow each other at about 6 ns, and a grid
+// sized for the level's capacity holds mostly workgroups without a tile.
+template <typename K, int E>
+__device__ inline void level_pass(const LevelIo<K>& A, uint64_t n, LevelLds<K, BLOCK, E>& S,
+                                  uint32_t* s_tile, uint64_t* status, uint32_t* ticket,
+                                  uint32_t epoch, unsigned long long* count_next) {
+  constexpr uint64_t T = BLOCK * E;
+  const uint64_t tiles = (n + T - 1) / T;
+  if (blockIdx.x >= tiles) return;
+  const bool once = tiles <= gridDim.x;
+  do {
+    if (threadIdx.x == 0) *s_tile = atomicAdd(ticket, 1u);
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < tg; i += BLOCK) {
-      elem_next[(uint64_t)bg + i] = s_key[i];
-      first_child_next[(uint64_t)bg + i] = s_val[i];
-      kids_next[(uint64_t)bg + i] = s_kid[i];
-    }
-    __syncthreads();
+    const uint64_t tile = *s_tile;
+    if (tile >= tiles) return;  // uniform over the workgroup
+    level_tile<K, BLOCK, E>(A, n, tile * T, S, false, [&](uint32_t tg) {
+      const uint32_t pre = lookback_exclusive_wave(status + 1, 2, tile, tg, epoch);
+      if (threadIdx.x == 0 && tile + 1 == tiles) *count_next = (unsigned long long)pre + tg;
+      return pre;
+    });
+  } while (!once);
+}
+
+template <typename K>
+__global__ __launch_bounds__(BLOCK) void k_level_pass(LevelIo<K> A,
+                                                      const unsigned long long* n_ptr,
+                                                      uint64_t* status, uint32_t* ticket,
+                                                      uint32_t epoch,
+                                                      unsigned long long* count_next) {
+  __shared__ union {
+    LevelLds<K, BLOCK, EPT> big;
+    LevelLds<K, BLOCK, EPT_SMALL> small;
+  } S;
+  __shared__ uint32_t s_tile;
+  const uint64_t n = *n_ptr;
+  if (n <= SMALL_ELEMS)
+    level_pass<K, EPT_SMALL>(A, n, S.small, &s_tile, status, ticket, epoch, count_next);
+  else
+    level_pass<K, EPT>(A, n, S.big, &s_tile, status, ticket, epoch, count_next);
+}
+
+// Levels `first` .. n_levels in one workgroup, a tile per level: at these sizes
+// (TAIL_TILE elements at most, by the grid) a launch and its look-back cost
+// more than the work.  With several tiles in turn (levels to 32768 elements)
+// it was slower than the launches: 63 us against 43 where the level is full.
+constexpr int TAIL_THREADS = 1024, TAIL_EPT = 4, TAIL_TILE = TAIL_THREADS * TAIL_EPT;
+template <typename K>
+struct TailArgs {
+  LevelIo<K> io;  // what the levels share
+  int first, last;
+  struct Level {
+    K* elem;
+    uint32_t* group;
+    uint32_t* first_child;
+    uint8_t* kids;
+  } lv[24];  // level l at [l - 1], up to last + 1
+};
+template <typename K>
+__global__ __launch_bounds__(TAIL_THREADS) void k_level_tail(TailArgs<K> A,
+                                                             unsigned long long* counts) {
+  __shared__ LevelLds<K, TAIL_THREADS, TAIL_EPT> S;
+  uint64_t n = counts[A.first - 1];
+  for (int l = A.first; l <= A.last && n; ++l) {
+    LevelIo<K> io = A.io;
+    io.level = l;
+    io.elem = A.lv[l - 1].elem;
+    io.group = A.lv[l - 1].group;
+    io.elem_next = A.lv[l].elem;
+    io.first_child_next = A.lv[l].first_child;
+    io.kids_next = A.lv[l].kids;
+    // a level leaves the next level's keys in LDS
+    n = level_tile<K, TAIL_THREADS, TAIL_EPT>(io, n, 0, S, l > A.first,
+                                              [](uint32_t) { return 0u; });
+    if (threadIdx.x == 0) counts[l] = n;
   }
 }
 
@@ -759,8 +906,7 @@ uint32_t grid_tiles(uint64_t cap, uint32_t blocks) {
 }  // namespace
 
 size_t level_tmp_bytes(uint64_t cap) {
-  const uint64_t tiles = (std::max<uint64_t>(cap, 1) + TILE - 1) / TILE;
-  return 256 + 2 * tiles * sizeof(uint64_t);
+  return 256 + 2 * level_tiles(std::max<uint64_t>(cap, 1)) * sizeof(uint64_t);
 }
 
 template <typename K>
@@ -770,7 +916,7 @@ void launch_level_first(const K* sorted, const unsigned long long* n_sorted, uin
                         uint32_t blocks, void* tmp, hipStream_t s) {
   uint32_t* tickets = (uint32_t*)tmp;
   uint64_t* status = (uint64_t*)((char*)tmp + 256);
-  const uint64_t tiles = (std::max<uint64_t>(cap, 1) + TILE - 1) / TILE;
+  const uint64_t tiles = level_tiles(std::max<uint64_t>(cap, 1));
   const uint32_t cg = (uint32_t)std::min<uint64_t>(2048, (2 * tiles + BLOCK - 1) / BLOCK);
   hipLaunchKernelGGL(k_level_clear, dim3(std::max<uint32_t>(cg, 1)), dim3(BLOCK), 0, s, status,
                      tickets, n_sorted);
@@ -814,7 +960,7 @@ void launch_level_first_bitmap(uint32_t* bits, uint64_t n_words, const uint64_t*
                      (const uint32_t*)tile_r, (uint32_t)tiles, scan_status, counts, reset_bytes, hits,
                      n_hits);
   // the emission also writes the level-1 spans and depth-1 roots, and clears
-  // the later levels' look-back words and tickets (launch_level)
+  // the later levels' look-back words and tickets (launch_levels)
   uint32_t* tickets = (uint32_t*)lvl_tmp;
   uint64_t* status = (uint64_t*)((char*)lvl_tmp + 256);
   hipLaunchKernelGGL(k_bm_emit<K>, dim3((uint32_t)tiles), dim3(BLOCK), 0, s, bits, n_words,
@@ -831,16 +977,35 @@ void launch_level_first_finalize(const LevelSpan* spans, uint32_t n_meshes, uint
 }
 
 template <typename K>
-void launch_level(int level, KeyLayout<K> kl, LevelArrays cur, LevelArrays next,
-                  unsigned long long* counts, LevelSpan* spans, uint32_t n_levels,
-                  MeshTreeState* state, uint32_t blocks, void* tmp, hipStream_t s) {
+void launch_levels(KeyLayout<K> kl, const LevelArrays* lv, uint32_t n_levels,
+                   unsigned long long* counts, LevelSpan* spans, MeshTreeState* state,
+                   uint32_t blocks, void* tmp, hipStream_t s) {
   uint32_t* tickets = (uint32_t*)tmp;
   uint64_t* status = (uint64_t*)((char*)tmp + 256);
-  // counts[level-1] = elements of this level; counts[level] = elements of the next
-  hipLaunchKernelGGL(k_level_pass<K>, dim3(grid_tiles(cur.cap, blocks)), dim3(BLOCK), 0, s,
-                     level, (const K*)cur.elem, counts + (level - 1), kl, state,
-                     cur.elem_group, (K*)next.elem, next.first_child, next.kids, spans, n_levels,
-                     status, tickets + (level - 1), (uint32_t)level, counts + level);
+  LevelIo<K> io{2, kl, state, nullptr, nullptr, nullptr, nullptr, nullptr, spans, n_levels};
+  uint32_t l = 2;
+  for (; l <= n_levels && lv[l].cap > TAIL_TILE; ++l) {
+    io.level = (int)l;
+    io.elem = (const K*)lv[l].elem;
+    io.group = lv[l].elem_group;
+    io.elem_next = (K*)lv[l + 1].elem;
+    io.first_child_next = lv[l + 1].first_child;
+    io.kids_next = lv[l + 1].kids;
+    // counts[l - 1] = elements of this level; counts[l] = elements of the next
+    const uint32_t grid =
+        (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(level_tiles(lv[l].cap), blocks));
+    hipLaunchKernelGGL(k_level_pass<K>, dim3(grid), dim3(BLOCK), 0, s, io,
+                       (const unsigned long long*)counts + (l - 1), status, tickets + (l - 1), l,
+                       counts + l);
+  }
+  if (l > n_levels) return;
+  TailArgs<K> t{};
+  t.io = io;
+  t.first = (int)l;
+  t.last = (int)n_levels;
+  for (uint32_t k = l; k <= n_levels + 1; ++k)
+    t.lv[k - 1] = {(K*)lv[k].elem, lv[k].elem_group, lv[k].first_child, lv[k].kids};
+  hipLaunchKernelGGL(k_level_tail<K>, dim3(1), dim3(TAIL_THREADS), 0, s, t, counts);
 }
 
 template void launch_level_first<uint32_t>(const uint32_t*, const unsigned long long*, uint64_t,
@@ -863,11 +1028,11 @@ template void launch_level_first_bitmap<uint64_t>(uint32_t*, uint64_t, const uin
                                                   uint32_t, MeshTreeState*, void*, void*,
                                                   unsigned long long*, const unsigned long long*,
                                                   unsigned long long*, hipStream_t);
-template void launch_level<uint32_t>(int, KeyLayout<uint32_t>, LevelArrays, LevelArrays,
-                                     unsigned long long*, LevelSpan*, uint32_t, MeshTreeState*,
-                                     uint32_t, void*, hipStream_t);
-template void launch_level<uint64_t>(int, KeyLayout<uint64_t>, LevelArrays, LevelArrays,
-                                     unsigned long long*, LevelSpan*, uint32_t, MeshTreeState*,
-                                     uint32_t, void*, hipStream_t);
+template void launch_levels<uint32_t>(KeyLayout<uint32_t>, const LevelArrays*, uint32_t,
+                                      unsigned long long*, LevelSpan*, MeshTreeState*, uint32_t,
+                                      void*, hipStream_t);
+template void launch_levels<uint64_t>(KeyLayout<uint64_t>, const LevelArrays*, uint32_t,
+                                      unsigned long long*, LevelSpan*, MeshTreeState*, uint32_t,
+                                      void*, hipStream_t);
 
 }  // namespace svo

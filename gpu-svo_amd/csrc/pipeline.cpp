@@ -1102,9 +1102,8 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     launch_level_first_finalize(d_spans, n, NL, d_state, s);
   }
   timer.mark("unique_level1");
-  for (uint32_t l = 2; l <= NL; ++l)
-    launch_level<K>((int)l, kl, lv[l], lv[l + 1], d_counts, d_spans, NL, d_state,
-                    plan.tuning.scan_blocks, lvl_tmp, s);
+  launch_levels<K>(kl, lv.data(), NL, d_counts, d_spans, d_state, plan.tuning.scan_blocks, lvl_tmp,
+                   s);
   timer.mark("levels");
 
   // ---- readback of the level phase

@@ -125,12 +125,13 @@ void launch_level_first_bitmap(uint32_t* bits, uint64_t n_words, const uint64_t*
 // sort path; launch_level_first_bitmap does it itself).
 void launch_level_first_finalize(const LevelSpan* spans, uint32_t n_meshes, uint32_t n_levels,
                                  MeshTreeState* state, hipStream_t s);
-// One level l >= 2: roots of meshes whose level holds one element; groups of
-// the others feed level l+1.
+// Levels 2 .. n_levels (at most 23; level l's arrays at lv[l], up to n_levels +
+// 1): roots of meshes whose level holds one element; groups of the others feed
+// the next level.
 template <typename K>
-void launch_level(int level, KeyLayout<K> kl, LevelArrays cur, LevelArrays next,
-                  unsigned long long* counts, LevelSpan* spans, uint32_t n_levels,
-                  MeshTreeState* state, uint32_t blocks, void* tmp, hipStream_t s);
+void launch_levels(KeyLayout<K> kl, const LevelArrays* lv, uint32_t n_levels,
+                   unsigned long long* counts, LevelSpan* spans, MeshTreeState* state,
+                   uint32_t blocks, void* tmp, hipStream_t s);
 size_t level_tmp_bytes(uint64_t cap);
 
 // ------------------------------------------------------------ k_attrs.hip
