@@ -844,6 +844,12 @@ void launch_emit(const EmitArgs<K>& a, hipStream_t s) {
                        a.out);
 }
 
+__global__ void k_copy_u32(uint32_t* dst, const uint32_t* src, uint64_t n) {
+  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n;
+       i += (uint64_t)gridDim.x * blockDim.x)
+    dst[i] = src[i];
+}
+
 // Sets *flag when any of the n words differs from its expected value.
 __global__ void k_check_equal(const uint32_t* got, const uint32_t* want, uint64_t n,
                               uint32_t* flag) {
@@ -861,6 +867,12 @@ void launch_check_equal(const void* got, const void* want, uint64_t bytes, uint3
   const uint64_t blocks = std::min<uint64_t>((n + BLOCK - 1) / BLOCK, 256);
   hipLaunchKernelGGL(k_check_equal, dim3((uint32_t)blocks), dim3(BLOCK), 0, s,
                      (const uint32_t*)got, (const uint32_t*)want, n, flag);
+}
+
+void launch_copy_u32(uint32_t* dst, const uint32_t* src, uint64_t n, hipStream_t s) {
+  if (n == 0) return;
+  const uint64_t blocks = std::min<uint64_t>((n + BLOCK - 1) / BLOCK, 256);
+  hipLaunchKernelGGL(k_copy_u32, dim3((uint32_t)blocks), dim3(BLOCK), 0, s, dst, src, n);
 }
 
 void launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s) {

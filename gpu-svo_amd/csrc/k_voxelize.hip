@@ -26,7 +26,6 @@ namespace {
 constexpr int BLOCK = 256;
 constexpr int WAVES = BLOCK / 64;
 constexpr int STAGE = 1024;        // keys staged per wave
-constexpr int BBOX_CHUNK = 4096;   // points per bbox block
 
 __device__ inline void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -80,47 +79,101 @@ __device__ inline K dilated_inc(K code, K mask) {
 }
 
 // ------------------------------------------------------------------ bbox
-__global__ void k_bbox_init(uint32_t* acc, uint32_t n_meshes) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n_meshes * 8) return;
-  const uint32_t f = i & 7;
-  acc[i] = f < 3 ? 0xFFFFFFFFu : 0u;  // ordered min starts at +max, max at 0
+// Everything a pass sets up before its first kernel: the control tables from
+// pinned host memory, the boxes at their start values, zeros.
+__global__ __launch_bounds__(BLOCK) void k_begin(PassBegin B) {
+  const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
+  const uint64_t i0 = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
+  for (uint64_t i = i0; i < B.n_table; i += stride) B.table[i] = B.host_table[i];
+  for (uint64_t i = i0; i < 8ull * B.n_meshes; i += stride)
+    B.acc[i] = (i & 7) < 3 ? 0xFFFFFFFFu : 0u;  // ordered min starts at +max, max at 0
+  for (uint64_t i = i0; i < B.n_zero; i += stride) B.zero[i] = 0u;
 }
 
-__global__ __launch_bounds__(BLOCK) void k_bbox(const MeshDev* meshes, uint32_t* acc) {
-  const MeshDev md = meshes[blockIdx.y];
-  const uint64_t start = (uint64_t)blockIdx.x * BBOX_CHUNK;
-  if (start >= md.n_points) return;
-  const uint64_t end = start + BBOX_CHUNK < md.n_points ? start + BBOX_CHUNK : md.n_points;
+// Bounding boxes of the points (workgroups x < point_blocks) and a check of
+// the triangles' indices (the others); acc[8 m ..]: ordered minima, maxima, a
+// flag for a non-finite coordinate and one for an index out of range.  A
+// workgroup takes its points and indices as dwords, twelve loads a thread in
+// flight: 6.5 us for 163,842 points and 327,680 triangles (points taken one
+// after the other in 41 workgroups and the indices in a launch of their own:
+// 10.6 and 3).
+constexpr int FLAT = 12;
+constexpr uint32_t FLAT_CHUNK = BLOCK * FLAT;
+constexpr uint32_t BBOX_BLOCKS = 256;  // per mesh: its six atomics follow each other
+__global__ __launch_bounds__(BLOCK) void k_bbox(const MeshDev* meshes, uint32_t point_blocks,
+                                                uint32_t* acc) {
+  const MeshDev& md = meshes[blockIdx.y];
+  uint32_t* a = acc + 8 * blockIdx.y;
+  if (blockIdx.x >= point_blocks) {
+    const uint64_t n = 3 * md.n_tris;
+    const uint64_t n_points = md.n_points;
+    uint32_t bad = 0;
+    for (uint64_t start = (uint64_t)(blockIdx.x - point_blocks) * FLAT_CHUNK; start < n;
+         start += (uint64_t)(gridDim.x - point_blocks) * FLAT_CHUNK) {
+      int32_t v[FLAT];
+#pragma unroll
+      for (int j = 0; j < FLAT; ++j) {
+        const uint64_t i = start + (uint64_t)j * BLOCK + threadIdx.x;
+        v[j] = i < n ? md.tri[i] : 0;
+      }
+#pragma unroll
+      for (int j = 0; j < FLAT; ++j) bad |= v[j] < 0 || (uint64_t)v[j] >= n_points;
+    }
+    if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(a + 7, 1u);
+    return;
+  }
+  const uint64_t n = 3 * md.n_points;
+  if ((uint64_t)blockIdx.x * FLAT_CHUNK >= n) return;
+  // a thread's dword j is of axis (threadIdx.x + j) mod 3: FLAT_CHUNK and
+  // BLOCK - 1 are multiples of 3
+  static_assert(FLAT_CHUNK % 3 == 0 && BLOCK % 3 == 1 && FLAT % 3 == 0, "axes by position");
   uint32_t mn[3] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu}, mx[3] = {0, 0, 0};
   uint32_t bad = 0;
-  for (uint64_t i = start + threadIdx.x; i < end; i += BLOCK) {
-    for (int a = 0; a < 3; ++a) {
-      const float v = md.pts[3 * i + a];
-      if (!isfinite(v)) {
+  for (uint64_t start = (uint64_t)blockIdx.x * FLAT_CHUNK; start < n;
+       start += (uint64_t)point_blocks * FLAT_CHUNK) {
+    float v[FLAT];
+#pragma unroll
+    for (int j = 0; j < FLAT; ++j) {
+      const uint64_t i = start + (uint64_t)j * BLOCK + threadIdx.x;
+      v[j] = i < n ? md.pts[i] : md.pts[(threadIdx.x + j) % 3];  // the first point again
+    }
+#pragma unroll
+    for (int j = 0; j < FLAT; ++j) {
+      if (!isfinite(v[j])) {
         bad = 1;
         continue;
       }
-      const uint32_t k = float_to_ordered(v);
-      mn[a] = k < mn[a] ? k : mn[a];
-      mx[a] = k > mx[a] ? k : mx[a];
+      const uint32_t k = float_to_ordered(v[j]);
+      mn[j % 3] = k < mn[j % 3] ? k : mn[j % 3];
+      mx[j % 3] = k > mx[j % 3] ? k : mx[j % 3];
     }
   }
+  // by axis: axis x is at (x - threadIdx.x) mod 3
+  {
+    const uint32_t r = threadIdx.x % 3;
+    const uint32_t n0 = mn[0], n1 = mn[1], n2 = mn[2], x0 = mx[0], x1 = mx[1], x2 = mx[2];
+    mn[0] = r == 0 ? n0 : r == 1 ? n2 : n1;
+    mn[1] = r == 0 ? n1 : r == 1 ? n0 : n2;
+    mn[2] = r == 0 ? n2 : r == 1 ? n1 : n0;
+    mx[0] = r == 0 ? x0 : r == 1 ? x2 : x1;
+    mx[1] = r == 0 ? x1 : r == 1 ? x0 : x2;
+    mx[2] = r == 0 ? x2 : r == 1 ? x1 : x0;
+  }
   for (int off = 32; off > 0; off >>= 1) {
-    for (int a = 0; a < 3; ++a) {
-      const uint32_t omn = __shfl_xor(mn[a], off);
-      const uint32_t omx = __shfl_xor(mx[a], off);
-      mn[a] = omn < mn[a] ? omn : mn[a];
-      mx[a] = omx > mx[a] ? omx : mx[a];
+    for (int x = 0; x < 3; ++x) {
+      const uint32_t omn = __shfl_xor(mn[x], off);
+      const uint32_t omx = __shfl_xor(mx[x], off);
+      mn[x] = omn < mn[x] ? omn : mn[x];
+      mx[x] = omx > mx[x] ? omx : mx[x];
     }
     bad |= __shfl_xor(bad, off);
   }
   __shared__ uint32_t red[WAVES][7];
   const uint32_t w = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) {
-    for (int a = 0; a < 3; ++a) {
-      red[w][a] = mn[a];
-      red[w][3 + a] = mx[a];
+    for (int x = 0; x < 3; ++x) {
+      red[w][x] = mn[x];
+      red[w][3 + x] = mx[x];
     }
     red[w][6] = bad;
   }
@@ -133,7 +186,6 @@ __global__ __launch_bounds__(BLOCK) void k_bbox(const MeshDev* meshes, uint32_t*
       else if (threadIdx.x < 6) v = o > v ? o : v;
       else v |= o;
     }
-    uint32_t* a = acc + 8 * blockIdx.y;
     if (threadIdx.x < 3) atomicMin(a + threadIdx.x, v);
     else if (threadIdx.x < 6) atomicMax(a + threadIdx.x, v);
     else if (v) atomicOr(a + 6, 1u);
@@ -141,13 +193,9 @@ __global__ __launch_bounds__(BLOCK) void k_bbox(const MeshDev* meshes, uint32_t*
 }
 
 // createMeshBBCube (BaseModel.h:24-49) and the voxel size (SVO.cu:348-350).
-__global__ void k_params(const MeshDev* meshes, uint32_t n_meshes, const uint32_t* acc,
-                         MeshParams* params) {
-  const uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= n_meshes) return;
-  const uint32_t* a = acc + 8 * m;
+__device__ inline MeshParams mesh_params(const MeshDev& md, const uint32_t* a) {
   MeshParams P;
-  P.status = a[6] ? ERR_NONFINITE : 0u;
+  P.status = (a[6] ? ERR_NONFINITE : 0u) | (a[7] ? ERR_INDEX : 0u);
   float mn[3], mx[3], len[3], amin[3], amax[3];
   for (int k = 0; k < 3; ++k) {
     mn[k] = ordered_to_float(a[k]);
@@ -155,7 +203,7 @@ __global__ void k_params(const MeshDev* meshes, uint32_t n_meshes, const uint32_
     len[k] = mx[k] - mn[k];
     amin[k] = mn[k];
     amax[k] = mx[k];
-    P.res[k] = meshes[m].res[k];
+    P.res[k] = md.res[k];
   }
   const float max_length = fmax_r(len[0], fmax_r(len[1], len[2]));
   if (!(max_length > 0.0f)) P.status |= ERR_DEGENERATE;
@@ -177,7 +225,7 @@ __global__ void k_params(const MeshDev* meshes, uint32_t n_meshes, const uint32_
     P.origin[k] = amin[k];
     P.unit[k] = P.width[k] / (float)P.res[k];
   }
-  params[m] = P;
+  return P;
 }
 
 // ------------------------------------------------------------------ triangle setup
@@ -430,22 +478,32 @@ struct VoxOut {
 
 // Big-triangle work item: 512 rows (y, z) of the box.
 constexpr uint64_t BIG_ROWS = 512;
+constexpr uint64_t BIG_BLOCKS = 8192;
 
-// Candidate cells and big-triangle chunk counts (added to totals[0],
-// totals[1]).  A grid-stride loop over a bounded grid: the two totals take one atomic per
-// workgroup, and atomics on one address serialize.
+// The meshes' parameters from their boxes, and the candidate cells and
+// big-triangle chunk counts (added to totals[0], totals[1]).  A grid-stride
+// loop over a bounded grid: the two totals take one atomic per workgroup, and
+// atomics on one address serialize.
 constexpr uint32_t CLASSIFY_BLOCKS = 1024;
-__global__ __launch_bounds__(BLOCK) void k_classify(const MeshDev* meshes,
-                                                    const MeshParams* params,
-                                                    const uint64_t* tri_base, uint32_t n_meshes,
-                                                    uint64_t n_tris, uint32_t small_max,
+__global__ __launch_bounds__(BLOCK) void k_classify(const MeshDev* meshes, const uint32_t* acc,
+                                                    MeshParams* params, const uint64_t* tri_base,
+                                                    uint32_t n_meshes, uint64_t n_tris,
+                                                    uint32_t small_max,
                                                     unsigned long long* totals) {
   uint64_t cells = 0, chunks = 0;
-  for (uint64_t gid = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; gid < n_tris;
-       gid += (uint64_t)gridDim.x * BLOCK) {
+  const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
+  const uint64_t gid0 = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
+  for (uint64_t m = gid0; m < n_meshes; m += stride)
+    params[m] = mesh_params(meshes[m], acc + 8 * m);
+  uint32_t last_m = 0xFFFFFFFFu;
+  MeshParams P;
+  for (uint64_t gid = gid0; gid < n_tris; gid += stride) {
     const uint32_t m = find_mesh(tri_base, n_meshes, gid);
     const MeshDev& md = meshes[m];
-    const MeshParams& P = params[m];
+    if (m != last_m) {
+      P = mesh_params(md, acc + 8ull * m);
+      last_m = m;
+    }
     float v[3][3];
     if (P.status == 0 && load_tri(md, P, gid - md.tri_base, v)) {
       int g0[3], g1[3];
@@ -472,17 +530,6 @@ __global__ __launch_bounds__(BLOCK) void k_classify(const MeshDev* meshes,
     for (int w = 0; w < WAVES; ++w) t += red[w][threadIdx.x];
     if (t) atomicAdd(totals + threadIdx.x, (unsigned long long)t);
   }
-}
-
-__global__ void k_flag_bad_index(const MeshDev* meshes, MeshParams* params,
-                                 const uint64_t* tri_base, uint32_t n_meshes, uint64_t n_tris) {
-  const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= n_tris) return;
-  const uint32_t m = find_mesh(tri_base, n_meshes, gid);
-  const MeshDev& md = meshes[m];
-  const int32_t* t = md.tri + 3 * (gid - md.tri_base);
-  for (int k = 0; k < 3; ++k)
-    if (t[k] < 0 || (uint64_t)t[k] >= md.n_points) atomicOr(&params[m].status, ERR_INDEX);
 }
 
 // Voxelizes runs of `per_wave` triangles, a wave each (ITEMS: the queued items
@@ -534,7 +581,12 @@ __global__ __launch_bounds__(BLOCK) void k_vox_rows(
   __shared__ K s_key[BITMAP ? 1 : WAVES][BITMAP ? 1 : STAGE];
   __shared__ WordTable s_words[1];  // (bitmap path only: the key path leaves it out)
   const uint32_t w = threadIdx.x >> 6, lane = __lane_id();
-  const uint64_t wave = (uint64_t)blockIdx.x * WAVES + w;
+  uint64_t wave = (uint64_t)blockIdx.x * WAVES + w, n_items = 0;
+  if (ITEMS) {
+    const uint64_t queued = *big_count;
+    n_items = queued < big_cap ? queued : big_cap;
+    if ((uint64_t)blockIdx.x * WAVES >= n_items) return;
+  }
   if (BITMAP) {
     for (uint32_t i = threadIdx.x; i < WORD_SLOTS; i += BLOCK) {
       s_words[0].word[i] = NO_WORD;
@@ -542,73 +594,8 @@ __global__ __launch_bounds__(BLOCK) void k_vox_rows(
     }
     __syncthreads();
   }
-  // ---- set-up: a lane per triangle
-  uint64_t gid = n_tris, first = 0;
-  uint32_t row0 = 0;
-  bool mine;
-  if (ITEMS) {
-    const uint64_t queued = *big_count, n_items = queued < big_cap ? queued : big_cap;
-    mine = lane == 0 && wave < n_items;
-    if (mine) {
-      gid = big[wave].tri;
-      row0 = big[wave].row0;
-    }
-    mine = mine && gid < n_tris;
-    first = bcast_first(gid);
-  } else {
-    first = wave * per_wave;
-    gid = first + lane;
-    mine = lane < per_wave && gid < n_tris;
-  }
-  uint32_t rows = 0;
-  const uint32_t m =
-      first < n_tris ? find_mesh_wave(tri_base, n_meshes, first, mine ? gid : first) : 0u;
-  {
-    uint32_t chunks = 0;
-    TriSetup S;
-    if (mine) {
-      const MeshDev& md = meshes[m];
-      const MeshParams P = params[m];
-      float v[3][3];
-      if (P.status == 0 && load_tri(md, P, gid - md.tri_base, v)) {
-        tri_setup(v, P, S);
-        const uint64_t nx = S.g1[0] - S.g0[0] + 1, ny = S.g1[1] - S.g0[1] + 1,
-                       nz = S.g1[2] - S.g0[2] + 1;
-        if (ITEMS) {
-          rows = (uint32_t)std::min<uint64_t>(BIG_ROWS, ny * nz - row0);
-        } else if (nx * ny * nz <= (md.small_max ? md.small_max : small_max)) {
-          rows = (uint32_t)(ny * nz);
-        } else {
-          chunks = (uint32_t)((ny * nz + BIG_ROWS - 1) / BIG_ROWS);
-        }
-      }
-    }
-    if (!ITEMS && __any(chunks != 0)) {
-      // one atomic per wave for its triangles' items
-      const uint32_t inc = wave_incl_scan_dpp(chunks);
-      uint64_t at = 0;
-      if (lane == 63) at = atomicAdd(big_count, (unsigned long long)inc);
-      at = (uint64_t)__shfl((uint32_t)at, 63) | ((uint64_t)__shfl((uint32_t)(at >> 32), 63) << 32);
-      at += inc - chunks;
-      for (uint32_t j = 0; j < chunks; ++j)
-        if (at + j < big_cap) big[at + j] = BigItem{(uint32_t)gid, j * (uint32_t)BIG_ROWS};
-    }
-    if (rows) {
-      RowTri& T = s_tri[w][ITEMS ? 0 : lane];
-      row_setup(S, T);
-      const uint64_t k = BITMAP ? out.bm_off[m] / 2 : (uint64_t)m << cb;  // (whole tiles)
-      T.key_lo = (uint32_t)k;
-      T.key_hi = (uint32_t)(k >> 32);
-    }
-  }
-  const uint32_t inc_rows = wave_incl_scan_dpp(rows), start = inc_rows - rows;
-  const uint32_t total = __builtin_amdgcn_readlane(inc_rows, 63);
-  if (rows) s_tri[w][ITEMS ? 0 : lane].row0 = start - row0;
-  wave_sync();
-  // ---- rows: a lane each
   uint64_t n_hits = 0;      // bitmap path: this lane's
   uint32_t staged = 0;      // key path: keys in s_key (the same in every lane)
-  uint32_t owner = 0;       // 1 + the triangle of the last item taken
   constexpr K MX = (K)(sizeof(K) == 4 ? 0x09249249u : 0x1249249249249249ull);
   auto flush = [&]() {
     wave_sync();
@@ -619,84 +606,153 @@ __global__ __launch_bounds__(BLOCK) void k_vox_rows(
     wave_sync();
     staged = 0;
   };
-  for (uint32_t base = 0; base < total; base += 64) {
-    const uint32_t item = base + lane;
-    // the triangle of an item: triangles mark where their rows begin, and the
-    // last mark at or before the item counts
-    uint32_t tr = 0;
-    if (!ITEMS) {
-      s_mark[w][lane] = 0;
-      wave_sync();
-      if (rows && start >= base && start - base < 64) s_mark[w][start - base] = lane + 1;
-      wave_sync();
-      const uint32_t mark = s_mark[w][lane];
-      owner = wave_incl_max_dpp(lane == 0 && mark == 0 ? owner : mark);
-      tr = owner - 1;
-      owner = __builtin_amdgcn_readlane(owner, 63);
-    }
-    const RowTri& T = s_tri[w][tr];
-    const uint32_t r = item - T.row0;
-    int y, z;
+  for (;;) {
+    // ---- set-up: a lane per triangle
+    uint64_t gid = n_tris, first = 0;
+    uint32_t row0 = 0;
+    bool mine;
     if (ITEMS) {
-      z = (int)(r / (uint32_t)T.ny);
-      y = (int)(r - (uint32_t)z * (uint32_t)T.ny);
+      mine = lane == 0 && wave < n_items;
+      if (mine) {
+        gid = big[wave].tri;
+        row0 = big[wave].row0;
+      }
+      mine = mine && gid < n_tris;
+      first = bcast_first(gid);
     } else {
-      // r < 2^20 (the limit on box cells), so that the quotient of
-      // r + 1/2 lies at least 2^-21 of itself from a whole number: exact
-      z = (int)(((float)r + 0.5f) * T.inv_ny);
-      y = (int)r - z * T.ny;
+      first = wave * per_wave;
+      gid = first + lane;
+      mine = lane < per_wave && gid < n_tris;
     }
-    y += T.y0;
-    z += T.z0;
-    int xa = 0, xb = -1, ia = 0, ib = -1;
-    RowTerms R;
-    if (item < total && row_terms(T, y, z, R)) row_range(T, R, xa, xb, ia, ib);
-    // four cells at a time: they share a bitmap word
-    const uint64_t kbase = (uint64_t)T.key_lo | ((uint64_t)T.key_hi << 32);
-    int x = xa & ~3;
-    K code = morton3<K>((uint32_t)x, (uint32_t)y, (uint32_t)z);
-    while (__any(x <= xb)) {
-      uint32_t hit = 0, test = 0;
-      if (x <= xb) {
-        // bits [a, b] of four
-        auto span = [&](int a, int b) -> uint32_t {
-          a = a > x ? a - x : 0;
-          b = b < x + 3 ? b - x : 3;
-          return a <= b ? (2u << b) - (1u << a) : 0u;
-        };
-        test = span(xa, xb);
-        hit = span(ia, ib) & test;
-        test &= ~hit;
-      }
-      while (__any(test != 0)) {  // cells that rounding could decide either way
-        if (test) {
-          const uint32_t j = __builtin_ctz(test);
-          if (cell_hit(T, R, x + (int)j)) hit |= 1u << j;
-          test &= test - 1u;
+    uint32_t rows = 0;
+    const uint32_t m =
+        first < n_tris ? find_mesh_wave(tri_base, n_meshes, first, mine ? gid : first) : 0u;
+    {
+      uint32_t chunks = 0;
+      TriSetup S;
+      if (mine) {
+        const MeshDev& md = meshes[m];
+        const MeshParams P = params[m];
+        float v[3][3];
+        if (P.status == 0 && load_tri(md, P, gid - md.tri_base, v)) {
+          tri_setup(v, P, S);
+          const uint64_t nx = S.g1[0] - S.g0[0] + 1, ny = S.g1[1] - S.g0[1] + 1,
+                         nz = S.g1[2] - S.g0[2] + 1;
+          if (ITEMS) {
+            rows = (uint32_t)std::min<uint64_t>(BIG_ROWS, ny * nz - row0);
+          } else if (nx * ny * nz <= (md.small_max ? md.small_max : small_max)) {
+            rows = (uint32_t)(ny * nz);
+          } else {
+            chunks = (uint32_t)((ny * nz + BIG_ROWS - 1) / BIG_ROWS);
+          }
         }
       }
-      if (BITMAP) {
-        if (hit) {
-          n_hits += __popc(hit);
-          // cells 0-3 of the group are bits 0, 1, 8, 9 from its place
-          set_bits(s_words[0], out.bits, kbase + (uint64_t)(code >> 6),
-                   (unsigned long long)((hit & 3u) | ((hit & 12u) << 6)) << (code & 63));
-        }
+      if (!ITEMS && __any(chunks != 0)) {
+        // one atomic per wave for its triangles' items
+        const uint32_t inc = wave_incl_scan_dpp(chunks);
+        uint64_t at = 0;
+        if (lane == 63) at = atomicAdd(big_count, (unsigned long long)inc);
+        at = (uint64_t)__shfl((uint32_t)at, 63) | ((uint64_t)__shfl((uint32_t)(at >> 32), 63) << 32);
+        at += inc - chunks;
+        for (uint32_t j = 0; j < chunks; ++j)
+          if (at + j < big_cap) big[at + j] = BigItem{(uint32_t)gid, j * (uint32_t)BIG_ROWS};
+      }
+      if (rows) {
+        RowTri& T = s_tri[w][ITEMS ? 0 : lane];
+        row_setup(S, T);
+        const uint64_t k = BITMAP ? out.bm_off[m] / 2 : (uint64_t)m << cb;  // (whole tiles)
+        T.key_lo = (uint32_t)k;
+        T.key_hi = (uint32_t)(k >> 32);
+      }
+    }
+    const uint32_t inc_rows = wave_incl_scan_dpp(rows), start = inc_rows - rows;
+    const uint32_t total = __builtin_amdgcn_readlane(inc_rows, 63);
+    if (rows) s_tri[w][ITEMS ? 0 : lane].row0 = start - row0;
+    wave_sync();
+    // ---- rows: a lane each
+    uint32_t owner = 0;       // 1 + the triangle of the last item taken
+    for (uint32_t base = 0; base < total; base += 64) {
+      const uint32_t item = base + lane;
+      // the triangle of an item: triangles mark where their rows begin, and the
+      // last mark at or before the item counts
+      uint32_t tr = 0;
+      if (!ITEMS) {
+        s_mark[w][lane] = 0;
+        wave_sync();
+        if (rows && start >= base && start - base < 64) s_mark[w][start - base] = lane + 1;
+        wave_sync();
+        const uint32_t mark = s_mark[w][lane];
+        owner = wave_incl_max_dpp(lane == 0 && mark == 0 ? owner : mark);
+        tr = owner - 1;
+        owner = __builtin_amdgcn_readlane(owner, 63);
+      }
+      const RowTri& T = s_tri[w][tr];
+      const uint32_t r = item - T.row0;
+      int y, z;
+      if (ITEMS) {
+        z = (int)(r / (uint32_t)T.ny);
+        y = (int)(r - (uint32_t)z * (uint32_t)T.ny);
       } else {
-        const uint32_t cnt = __popc(hit), inc = wave_incl_scan_dpp(cnt);
-        uint32_t at = staged + inc - cnt;
-        for (uint32_t h = hit; h; h &= h - 1u) {
-          const uint32_t j = __builtin_ctz(h);
-          s_key[BITMAP ? 0 : w][at++] = (K)kbase | code | (K)((j & 1u) | ((j & 2u) << 2));
-        }
-        staged += __builtin_amdgcn_readlane(inc, 63);
-        if (staged > STAGE - 256) flush();
+        // r < 2^20 (the limit on box cells), so that the quotient of
+        // r + 1/2 lies at least 2^-21 of itself from a whole number: exact
+        z = (int)(((float)r + 0.5f) * T.inv_ny);
+        y = (int)r - z * T.ny;
       }
-      x += 4;
-      // x + 4 in the code: the bits of x from bit 2 on (bits 0 and 1 are zero)
-      constexpr K M4 = MX & ~(K)9;
-      code = (((code | ~M4) + 1) & M4) | (code & ~M4);
+      y += T.y0;
+      z += T.z0;
+      int xa = 0, xb = -1, ia = 0, ib = -1;
+      RowTerms R;
+      if (item < total && row_terms(T, y, z, R)) row_range(T, R, xa, xb, ia, ib);
+      // four cells at a time: they share a bitmap word
+      const uint64_t kbase = (uint64_t)T.key_lo | ((uint64_t)T.key_hi << 32);
+      int x = xa & ~3;
+      K code = morton3<K>((uint32_t)x, (uint32_t)y, (uint32_t)z);
+      while (__any(x <= xb)) {
+        uint32_t hit = 0, test = 0;
+        if (x <= xb) {
+          // bits [a, b] of four
+          auto span = [&](int a, int b) -> uint32_t {
+            a = a > x ? a - x : 0;
+            b = b < x + 3 ? b - x : 3;
+            return a <= b ? (2u << b) - (1u << a) : 0u;
+          };
+          test = span(xa, xb);
+          hit = span(ia, ib) & test;
+          test &= ~hit;
+        }
+        while (__any(test != 0)) {  // cells that rounding could decide either way
+          if (test) {
+            const uint32_t j = __builtin_ctz(test);
+            if (cell_hit(T, R, x + (int)j)) hit |= 1u << j;
+            test &= test - 1u;
+          }
+        }
+        if (BITMAP) {
+          if (hit) {
+            n_hits += __popc(hit);
+            // cells 0-3 of the group are bits 0, 1, 8, 9 from its place
+            set_bits(s_words[0], out.bits, kbase + (uint64_t)(code >> 6),
+                     (unsigned long long)((hit & 3u) | ((hit & 12u) << 6)) << (code & 63));
+          }
+        } else {
+          const uint32_t cnt = __popc(hit), inc = wave_incl_scan_dpp(cnt);
+          uint32_t at = staged + inc - cnt;
+          for (uint32_t h = hit; h; h &= h - 1u) {
+            const uint32_t j = __builtin_ctz(h);
+            s_key[BITMAP ? 0 : w][at++] = (K)kbase | code | (K)((j & 1u) | ((j & 2u) << 2));
+          }
+          staged += __builtin_amdgcn_readlane(inc, 63);
+          if (staged > STAGE - 256) flush();
+        }
+        x += 4;
+        // x + 4 in the code: the bits of x from bit 2 on (bits 0 and 1 are zero)
+        constexpr K M4 = MX & ~(K)9;
+        code = (((code | ~M4) + 1) & M4) | (code & ~M4);
+      }
     }
+    wave += (uint64_t)gridDim.x * WAVES;
+    if (!ITEMS || wave >= n_items) break;
+    wave_sync();  // s_tri is written again
   }
   if (BITMAP) {
     uint32_t h = (uint32_t)n_hits;  // a lane's rows hold fewer than 2^32 cells
@@ -714,30 +770,29 @@ __global__ __launch_bounds__(BLOCK) void k_vox_rows(
 
 }  // namespace
 
-void launch_bbox(const MeshDev* meshes, uint32_t n_meshes, uint64_t max_points, uint32_t* acc,
-                 hipStream_t s) {
-  hipLaunchKernelGGL(k_bbox_init, dim3((n_meshes * 8 + 255) / 256), dim3(256), 0, s, acc,
-                     n_meshes);
-  if (max_points == 0) return;
-  const uint32_t gx = (uint32_t)((max_points + BBOX_CHUNK - 1) / BBOX_CHUNK);
-  hipLaunchKernelGGL(k_bbox, dim3(gx, n_meshes), dim3(BLOCK), 0, s, meshes, acc);
+void launch_begin(const PassBegin& B, hipStream_t s) {
+  const uint64_t n = std::max({B.n_table, B.n_zero, (uint64_t)B.n_meshes * 8});
+  const uint64_t blocks = std::min<uint64_t>((n + BLOCK - 1) / BLOCK, 1024);
+  hipLaunchKernelGGL(k_begin, dim3((uint32_t)std::max<uint64_t>(blocks, 1)), dim3(BLOCK), 0, s, B);
 }
 
-void launch_params(const MeshDev* meshes, uint32_t n_meshes, const uint32_t* acc,
-                   MeshParams* params, hipStream_t s) {
-  hipLaunchKernelGGL(k_params, dim3((n_meshes + 63) / 64), dim3(64), 0, s, meshes, n_meshes, acc,
-                     params);
+void launch_bbox(const MeshDev* meshes, uint32_t n_meshes, uint64_t max_points, uint64_t max_tris,
+                 uint32_t* acc, hipStream_t s) {
+  const auto blocks = [](uint64_t n) {
+    return (uint32_t)std::min<uint64_t>((3 * n + FLAT_CHUNK - 1) / FLAT_CHUNK, BBOX_BLOCKS);
+  };
+  const uint32_t pb = blocks(max_points), tb = blocks(max_tris);
+  if (pb + tb == 0) return;
+  hipLaunchKernelGGL(k_bbox, dim3(pb + tb, n_meshes), dim3(BLOCK), 0, s, meshes, pb, acc);
 }
 
-void launch_classify(const MeshDev* meshes, const MeshParams* params, const uint64_t* tri_base,
-                     uint32_t n_meshes, uint64_t n_tris, const Tuning& tn,
-                     unsigned long long* totals, hipStream_t s) {
-  if (n_tris == 0) return;
-  const uint32_t blocks = (uint32_t)((n_tris + BLOCK - 1) / BLOCK);
-  hipLaunchKernelGGL(k_flag_bad_index, dim3(blocks), dim3(BLOCK), 0, s, meshes,
-                     const_cast<MeshParams*>(params), tri_base, n_meshes, n_tris);
-  hipLaunchKernelGGL(k_classify, dim3(std::min<uint32_t>(blocks, CLASSIFY_BLOCKS)), dim3(BLOCK), 0,
-                     s, meshes, params, tri_base, n_meshes, n_tris, tn.small_max_cells, totals);
+void launch_classify(const MeshDev* meshes, const uint32_t* acc, MeshParams* params,
+                     const uint64_t* tri_base, uint32_t n_meshes, uint64_t n_tris,
+                     const Tuning& tn, unsigned long long* totals, hipStream_t s) {
+  const uint64_t blocks = (std::max<uint64_t>(n_tris, n_meshes) + BLOCK - 1) / BLOCK;
+  hipLaunchKernelGGL(k_classify, dim3((uint32_t)std::min<uint64_t>(blocks, CLASSIFY_BLOCKS)),
+                     dim3(BLOCK), 0, s, meshes, acc, params, tri_base, n_meshes, n_tris,
+                     tn.small_max_cells, totals);
 }
 
 template <typename K, bool BITMAP>
@@ -758,7 +813,8 @@ static void launch_rows(const MeshDev* meshes, const MeshParams* params, const u
                      tn.small_max_cells, per, out, big, big_count, big_cap);
   if (big_cap)
     hipLaunchKernelGGL((k_vox_rows<K, BITMAP, true>),
-                       dim3((uint32_t)((big_cap + WAVES - 1) / WAVES)), dim3(BLOCK), 0, s, meshes,
+                       dim3((uint32_t)std::min<uint64_t>((big_cap + WAVES - 1) / WAVES, BIG_BLOCKS)),
+                       dim3(BLOCK), 0, s, meshes,
                        params, tri_base, n_meshes, n_tris, cb, tn.small_max_cells, 1u, out, big,
                        big_count, big_cap);
 }

@@ -282,9 +282,9 @@ int svo_k_voxelize(int device, const float* xyz, uint64_t n_points, const int32_
       hipMemcpyAsync(md, &h, sizeof h, hipMemcpyHostToDevice, s) == hipSuccess &&
       hipMemcpyAsync(tb, htb, 16, hipMemcpyHostToDevice, s) == hipSuccess &&
       hipMemcpyAsync(cnt, zero, 64, hipMemcpyHostToDevice, s) == hipSuccess) {
-    launch_bbox(md, 1, n_points, acc, s);
-    launch_params(md, 1, acc, par, s);
-    launch_classify(md, par, tb, 1, n_tris, tn, cnt, s);
+    launch_begin(PassBegin{nullptr, nullptr, 0, acc, 1, nullptr, 0}, s);
+    launch_bbox(md, 1, n_points, n_tris, acc, s);
+    launch_classify(md, acc, par, tb, 1, n_tris, tn, cnt, s);
     if (hipMemcpyAsync(tot, cnt, 32, hipMemcpyDeviceToHost, s) == hipSuccess &&
         hipStreamSynchronize(s) == hipSuccess)
       st = SVO_OK;

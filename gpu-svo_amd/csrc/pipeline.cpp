@@ -879,7 +879,7 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
   // ---- inputs on the device
   std::vector<MeshDev> md(n);
   std::vector<uint64_t> tri_base(n + 1, 0);
-  uint64_t host_bytes = 0, max_points = 0;
+  uint64_t host_bytes = 0, max_points = 0, max_tris = 0;
   for (uint32_t i = 0; i < n; ++i) {
     const MeshInput& mi = in[plan.idx[i]];
     if (!mi.on_device) host_bytes += align256(12 * mi.desc.n_points) + align256(12 * mi.desc.n_tris);
@@ -912,6 +912,7 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     d.pt_base = 0;
     tri_base[i + 1] = tri_base[i] + d.n_tris;
     max_points = std::max<uint64_t>(max_points, d.n_points);
+    max_tris = std::max<uint64_t>(max_tris, d.n_tris);
   }
   const uint64_t T = tri_base[n];
   if (T >= (1ull << 32)) return SVO_E_RES_LIMIT;  // triangle indices are 32-bit on the device
@@ -929,54 +930,64 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
   }
   const uint64_t bm_words = bm_off[n];
 
-  // small control buffers: mesh descriptors, tri bases, bitmap offsets, bbox,
-  // params, counters
+  // small control buffers: the tables (mesh descriptors, tri bases, bitmap
+  // offsets), boxes, hit counters, and what is read back after the levels as
+  // one run of words: counters, level counts, spans, states, parameters
   const size_t sz_md = align256(sizeof(MeshDev) * n), sz_tb = align256(8 * (n + 1)),
                sz_bo = align256(8 * (n + 1)), sz_acc = align256(32 * n),
-               sz_par = align256(sizeof(MeshParams) * n), sz_cnt = align256(8 * (8 + HIT_SLOTS * HIT_STRIDE));
+               sz_hit = 8 * HIT_SLOTS * HIT_STRIDE;
+  const size_t rb_counts = 8 * 8, rb_spans = rb_counts + 8 * (NL + 2),
+               rb_state = rb_spans + sizeof(LevelSpan) * n * NL,
+               rb_par = rb_state + sizeof(MeshTreeState) * n,
+               rb_bytes = rb_par + sizeof(MeshParams) * n;
+  const size_t sz_tables = sz_md + sz_tb + sz_bo;
   char* ctl = nullptr;
-  SVO_TRY(W.get("ctl", sz_md + sz_tb + sz_bo + sz_acc + sz_par + sz_cnt, (void**)&ctl));
+  SVO_TRY(W.get("ctl", sz_tables + sz_acc + sz_hit + rb_bytes, (void**)&ctl));
   MeshDev* d_md = (MeshDev*)ctl;
   uint64_t* d_tb = (uint64_t*)(ctl + sz_md);
   uint64_t* d_bo = (uint64_t*)(ctl + sz_md + sz_tb);
-  uint32_t* d_acc = (uint32_t*)(ctl + sz_md + sz_tb + sz_bo);
-  MeshParams* d_par = (MeshParams*)(ctl + sz_md + sz_tb + sz_bo + sz_acc);
-  unsigned long long* d_cnt =
-      (unsigned long long*)(ctl + sz_md + sz_tb + sz_bo + sz_acc + sz_par);
+  uint32_t* d_acc = (uint32_t*)(ctl + sz_tables);
+  unsigned long long* d_hits = (unsigned long long*)(ctl + sz_tables + sz_acc);
+  char* rb = ctl + sz_tables + sz_acc + sz_hit;
   // d_cnt: [0] box cells, [1] big chunks, [2] keys emitted, [3] big queued,
-  // [4] bitmap bytes zeroed by the level-1 pass, [8] on the hit counters
+  // [4] bitmap bytes zeroed by the level-1 pass
+  unsigned long long* d_cnt = (unsigned long long*)rb;
+  unsigned long long* d_counts = (unsigned long long*)(rb + rb_counts);
+  LevelSpan* d_spans = (LevelSpan*)(rb + rb_spans);
+  MeshTreeState* d_state = (MeshTreeState*)(rb + rb_state);
+  MeshParams* d_par = (MeshParams*)(rb + rb_par);
+  PassBegin pb{};
   if (!capture) {
-    SVO_TRY(L.ensure_pinned(sz_md + sz_tb + sz_bo + 64 + sizeof(MeshParams) * n));
-    // stage the mesh descriptors, triangle bases and bitmap offsets through
-    // the pinned buffer in one copy; the host does not touch the buffer again
-    // before the next stream synchronization
+    // the tables and the readbacks go through the pinned buffer, which the
+    // host writes again only after the stream's next synchronization
+    SVO_TRY(L.ensure_pinned(std::max(sz_tables, rb_bytes)));
     std::memcpy(L.pinned, md.data(), sizeof(MeshDev) * n);
     std::memcpy((char*)L.pinned + sz_md, tri_base.data(), 8 * (n + 1));
     std::memcpy((char*)L.pinned + sz_md + sz_tb, bm_off.data(), 8 * (n + 1));
-    HIP_TRY(hipMemcpyAsync(d_md, L.pinned, sz_md + sz_tb + sz_bo, hipMemcpyHostToDevice, s));
+    pb.host_table = (const uint32_t*)L.pinned;
+    pb.table = (uint32_t*)ctl;
+    pb.n_table = sz_tables / 4;
   }
-  launch_fill_u32((uint32_t*)d_cnt, 0u, 2 * (8 + HIT_SLOTS * HIT_STRIDE), s);
+  pb.acc = d_acc;
+  pb.n_meshes = n;
+  pb.zero = (uint32_t*)d_hits;
+  pb.n_zero = (sz_hit + rb_par) / 4;
+  launch_begin(pb, s);
   timer.mark("start");
 
   // ---- A0: bbox, params, classification
-  launch_bbox(d_md, n, max_points, d_acc, s);
-  launch_params(d_md, n, d_acc, d_par, s);
-  launch_classify(d_md, d_par, d_tb, n, T, plan.tuning, d_cnt, s);
+  launch_bbox(d_md, n, max_points, max_tris, d_acc, s);
+  launch_classify(d_md, d_acc, d_par, d_tb, n, T, plan.tuning, d_cnt, s);
   timer.mark("classify");
   uint64_t cells = 0, n_big = 0;
   if (capture) {
-    cells = rec->a0[0];
-    n_big = rec->a0[1];
-    launch_check_equal(d_cnt, rec->d_expect, 16, rec->d_flag, s);
+    cells = ((const uint64_t*)rec->a1.data())[0];
+    n_big = ((const uint64_t*)rec->a1.data())[1];
   } else {
-    HIP_TRY(hipMemcpyAsync(L.pinned, d_cnt, 16, hipMemcpyDeviceToHost, s));
+    launch_copy_u32((uint32_t*)L.pinned, (const uint32_t*)d_cnt, 4, s);
     HIP_TRY(hipStreamSynchronize(s));
     cells = ((uint64_t*)L.pinned)[0];
     n_big = ((uint64_t*)L.pinned)[1];
-    if (rec) {
-      rec->a0[0] = cells;
-      rec->a0[1] = n_big;
-    }
   }
   if (cells >= (1ull << 32) - 1) return SVO_E_OOM;  // key counts are 32-bit in the sort
   const uint64_t key_cap = std::max<uint64_t>(cells, 1);
@@ -1059,15 +1070,6 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
       }
     }
   }
-  const size_t sz_counts = align256(8 * (NL + 2)), sz_spans = align256(sizeof(LevelSpan) * n * NL),
-               sz_state = align256(sizeof(MeshTreeState) * n);
-  char* lctl = nullptr;
-  SVO_TRY(W.get("lctl", sz_counts + sz_spans + sz_state, (void**)&lctl));
-  unsigned long long* d_counts = (unsigned long long*)lctl;
-  LevelSpan* d_spans = (LevelSpan*)(lctl + sz_counts);
-  MeshTreeState* d_state = (MeshTreeState*)(lctl + sz_counts + sz_spans);
-  launch_fill_u32((uint32_t*)lctl, 0u, (sz_counts + sz_spans + sz_state) / 4, s);
-
   // ---- A1: voxelize, sort, levels
   timer.mark("setup_a1");
   // The level-1 pass zeroes the bitmap words it reads, so the lane's bitmap
@@ -1086,11 +1088,11 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     clean = 0;
   }
   launch_voxelize<K>(d_md, d_par, d_tb, n, T, plan.cb, plan.tuning, keys_a, bitmap, d_bo,
-                     d_cnt + 2, d_cnt + 8, big, d_cnt + 3, n_big, s);
+                     d_cnt + 2, d_hits, big, d_cnt + 3, n_big, s);
   timer.mark("voxelize");
   if (use_bm) {
     launch_level_first_bitmap<K>(bitmap, bm_words, d_bo, n, kl, lv[1], lv[2], d_counts, d_spans,
-                                 NL, d_state, bm_tmp, lvl_tmp, d_cnt + 4, d_cnt + 8, d_cnt + 2, s);
+                                 NL, d_state, bm_tmp, lvl_tmp, d_cnt + 4, d_hits, d_cnt + 2, s);
     W.clean_bytes("bitmap") = bm_clean_after;
   } else {
     K* sorted = nullptr;
@@ -1107,40 +1109,22 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
   timer.mark("levels");
 
   // ---- readback of the level phase
-  // counts, spans, states, params, then the three 8-byte hit counters on an
-  // 8-byte boundary (76-byte MeshParams leave an odd count 4-byte aligned)
-  const size_t off_spans = 8 * (NL + 2), off_state = off_spans + sizeof(LevelSpan) * n * NL,
-               off_par = off_state + sizeof(MeshTreeState) * n,
-               off_hits = (off_par + sizeof(MeshParams) * n + 7) & ~(size_t)7;
   char* hp = nullptr;
   if (capture) {
-    if (rec->a1.size() != off_hits + 24) return SVO_E_INVALID;
+    if (rec->a1.size() != rb_bytes) return SVO_E_INVALID;
     hp = rec->a1.data();
-    const char* e1 = rec->d_expect + 16;
-    launch_check_equal(d_counts, e1, 8 * (NL + 2), rec->d_flag, s);
-    launch_check_equal(d_spans, e1 + off_spans, sizeof(LevelSpan) * n * NL, rec->d_flag, s);
-    launch_check_equal(d_state, e1 + off_state, sizeof(MeshTreeState) * n, rec->d_flag, s);
-    launch_check_equal(d_par, e1 + off_par, sizeof(MeshParams) * n, rec->d_flag, s);
-    launch_check_equal(d_cnt + 2, e1 + off_hits, 24, rec->d_flag, s);
+    launch_check_equal(rb, rec->d_expect, rb_bytes, rec->d_flag, s);
   } else {
-    SVO_TRY(L.ensure_pinned(off_hits + 24));
     hp = (char*)L.pinned;
-  }
-  uint64_t* h_counts = (uint64_t*)hp;
-  LevelSpan* h_spans = (LevelSpan*)(hp + off_spans);
-  MeshTreeState* h_state = (MeshTreeState*)(hp + off_state);
-  MeshParams* h_par = (MeshParams*)(hp + off_par);
-  uint64_t* h_hits = (uint64_t*)(hp + off_hits);
-  if (!capture) {
-    HIP_TRY(hipMemcpyAsync(h_counts, d_counts, 8 * (NL + 2), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(h_spans, d_spans, sizeof(LevelSpan) * n * NL, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(h_state, d_state, sizeof(MeshTreeState) * n, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(h_par, d_par, sizeof(MeshParams) * n, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(h_hits, d_cnt + 2, 24, hipMemcpyDeviceToHost, s));
+    launch_copy_u32((uint32_t*)hp, (const uint32_t*)rb, rb_bytes / 4, s);
     HIP_TRY(hipStreamSynchronize(s));
-    if (rec) rec->a1.assign(hp, hp + off_hits + 24);
+    if (rec) rec->a1.assign(hp, hp + rb_bytes);
   }
-  const uint64_t n_hits = h_hits[0], bm_reset = h_hits[2];
+  uint64_t* h_counts = (uint64_t*)(hp + rb_counts);
+  LevelSpan* h_spans = (LevelSpan*)(hp + rb_spans);
+  MeshTreeState* h_state = (MeshTreeState*)(hp + rb_state);
+  MeshParams* h_par = (MeshParams*)(hp + rb_par);
+  const uint64_t n_hits = ((uint64_t*)hp)[2], bm_reset = ((uint64_t*)hp)[4];
   if (n_hits > key_cap) return SVO_E_HIP;  // cannot happen: hits <= box cells
   // the pinned area is reused below: keep host copies of the readback
   const std::vector<uint64_t> v_counts(h_counts, h_counts + NL + 2);
@@ -1322,7 +1306,7 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     std::memcpy(up + sz_segs, seg_first.data(), 4 * n_segs);
     std::memcpy(up + sz_segs + sz_sf, level_segs.data(), 4 * level_segs.size());
     std::memcpy(up + sz_segs + 2 * sz_sf, level_blocks.data(), 4 * level_blocks.size());
-    HIP_TRY(hipMemcpyAsync(bctl, up, sz_up, hipMemcpyHostToDevice, s));
+    launch_copy_u32((uint32_t*)bctl, (const uint32_t*)up, sz_up / 4, s);
   }
   timer.mark("setup_b");
   // Reference records stand at the identity offsets when no record can equal
@@ -1375,12 +1359,12 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     if (rec->tot.size() != tot.size()) return SVO_E_INVALID;
     if (counted) {
       tot = rec->tot;
-      launch_check_equal(d_tot, rec->d_expect + 16 + rec->a1.size(), 8 * tot.size(), rec->d_flag,
+      launch_check_equal(d_tot, rec->d_expect + rec->a1.size(), 8 * tot.size(), rec->d_flag,
                          s);
     }
   } else {
     uint64_t* h_tot = (uint64_t*)L.pinned;
-    if (counted) HIP_TRY(hipMemcpyAsync(h_tot, d_tot, 8 * tot.size(), hipMemcpyDeviceToHost, s));
+    if (counted) launch_copy_u32((uint32_t*)h_tot, (const uint32_t*)d_tot, 2 * tot.size(), s);
     HIP_TRY(hipStreamSynchronize(s));
     HIP_TRY(hipGetLastError());
     if (counted) tot.assign(h_tot, h_tot + tot.size());
@@ -1684,12 +1668,11 @@ int plan_create(Context& C, const std::vector<MeshInput>& user, std::unique_ptr<
     bp->plans.push_back(pl);
     bp->recs.push_back(std::move(rec));
   }
-  // expected readbacks on the device, [a0 | a1 | tot] per pass
+  // expected readbacks on the device, [a1 | tot] per pass
   for (auto& rec : bp->recs) {
-    std::vector<char> img(16 + rec->a1.size() + 8 * rec->tot.size());
-    std::memcpy(img.data(), rec->a0, 16);
-    std::memcpy(img.data() + 16, rec->a1.data(), rec->a1.size());
-    std::memcpy(img.data() + 16 + rec->a1.size(), rec->tot.data(), 8 * rec->tot.size());
+    std::vector<char> img(rec->a1.size() + 8 * rec->tot.size());
+    std::memcpy(img.data(), rec->a1.data(), rec->a1.size());
+    std::memcpy(img.data() + rec->a1.size(), rec->tot.data(), 8 * rec->tot.size());
     void* d = nullptr;
     SVO_TRY(C.dev_malloc(&d, img.size()));
     bp->expect.push_back({d, img.size()});

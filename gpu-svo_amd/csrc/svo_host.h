@@ -138,18 +138,17 @@ struct svo_tree {
 };
 
 namespace svo {
-// The host values one pass reads back at its three synchronization points,
+// The host values one pass reads back at its synchronization points,
 // kept by a batch plan (api: svo_plan_*): recorded from an eager run, they
 // let the same pass be captured into a HIP graph with no readback at all;
 // the captured pass compares what it computes with them on the device and
 // sets a flag when anything differs.
 struct PassRecord {
   enum Mode { RECORD, CAPTURE } mode = RECORD;
-  uint64_t a0[2] = {0, 0};  // candidate cells, big-triangle work items
-  std::vector<char> a1;     // level readback: counts, spans, states, params, hits
+  std::vector<char> a1;       // level readback: counters, counts, spans, states, params
   std::vector<uint64_t> tot;  // record totals and per-mesh record offsets
   std::shared_ptr<BatchOutput> out;  // output block, written by every replay
-  // CAPTURE: expected readbacks on the device ([a0 | a1 | tot]) and the flag
+  // CAPTURE: expected readbacks on the device ([a1 | tot]) and the flag
   const char* d_expect = nullptr;
   uint32_t* d_flag = nullptr;
   // CAPTURE: the trees a replay hands out (copied per replay), by input index

@@ -44,16 +44,28 @@ inline int size_class_of(const int32_t res[3], uint64_t n_tris) {
 }
 
 // ------------------------------------------------------------ k_voxelize.hip
-// Per-mesh ordered-float min/max of all points (6 x uint32 per mesh) and the
-// grid parameters derived from it (BaseModel.h:24-73, SVO.cu:342-351).
-void launch_bbox(const MeshDev* meshes, uint32_t n_meshes, uint64_t max_points, uint32_t* acc,
-                 hipStream_t s);
-void launch_params(const MeshDev* meshes, uint32_t n_meshes, const uint32_t* acc,
-                   MeshParams* params, hipStream_t s);
-// Candidate cells and big-triangle chunk counts (2 x uint64 added to `totals`).
-void launch_classify(const MeshDev* meshes, const MeshParams* params, const uint64_t* tri_base,
-                     uint32_t n_meshes, uint64_t n_tris, const Tuning& tn,
-                     unsigned long long* totals, hipStream_t s);
+// What a pass sets up before its first kernel, in one launch: `n_table` words
+// copied from pinned host memory (0: they are in place), the boxes `acc` (8
+// words a mesh) at their start values, `n_zero` words cleared.
+struct PassBegin {
+  const uint32_t* host_table;
+  uint32_t* table;
+  uint64_t n_table;
+  uint32_t* acc;
+  uint32_t n_meshes;
+  uint32_t* zero;
+  uint64_t n_zero;
+};
+void launch_begin(const PassBegin& B, hipStream_t s);
+// Per-mesh ordered-float min/max of all points, and whether a coordinate is
+// not finite or an index out of range (8 x uint32 per mesh, launch_begin's acc).
+void launch_bbox(const MeshDev* meshes, uint32_t n_meshes, uint64_t max_points, uint64_t max_tris,
+                 uint32_t* acc, hipStream_t s);
+// Grid parameters from the boxes (BaseModel.h:24-73, SVO.cu:342-351); candidate
+// cells and big-triangle chunk counts (2 x uint64 added to `totals`).
+void launch_classify(const MeshDev* meshes, const uint32_t* acc, MeshParams* params,
+                     const uint64_t* tri_base, uint32_t n_meshes, uint64_t n_tris,
+                     const Tuning& tn, unsigned long long* totals, hipStream_t s);
 // Raw hits of the bitmap path are counted in HIT_SLOTS counters of a cache
 // line each (atomics on one address serialize); launch_level_first_bitmap
 // adds them up.
@@ -210,6 +222,10 @@ struct EmitArgs {
 template <typename K>
 void launch_emit(const EmitArgs<K>& a, hipStream_t s);
 void launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s);
+// Copies n words; either side may be pinned host memory.  For a pass's tables
+// and readbacks of a few KB: 2 to 4 us, and less host time than asynchronous
+// copies (five of them read the levels back in 25 to 40 us).
+void launch_copy_u32(uint32_t* dst, const uint32_t* src, uint64_t n, hipStream_t s);
 // Sets *flag (atomic OR of 1) when the `bytes` bytes (a multiple of 4, both
 // 4-byte aligned) at `got` differ from those at `want`.
 void launch_check_equal(const void* got, const void* want, uint64_t bytes, uint32_t* flag,
