@@ -261,6 +261,93 @@ __device__ inline void load_words(const uint32_t* bits, uint64_t n_words, uint64
   }
 }
 
+// A bitmap past the caches (one mesh's, LINES) is not read whole: the
+// voxelization flags the 64-byte lines (512 cells) that it sets bits of, a byte
+// a line, and the tiles are made of 128 flagged lines each, in order.  100,000
+// triangles at 2048^3: 72 us in all and 22 more for the flags' stores, where
+// counting and emitting over the 1.07 GB took 180 and 284 us.
+constexpr int LINE_WORDS = BITMAP_LINE_BYTES / 4;
+constexpr int TILE_LINES = BM_TILE / LINE_WORDS;
+struct LineList {
+  const uint32_t* line;  // flagged lines in order
+  const uint32_t* n;     // their number
+};
+__device__ inline uint64_t line_tiles(const LineList& L) {
+  return ((uint64_t)*L.n + TILE_LINES - 1) / TILE_LINES;
+}
+// The first bitmap word of this thread's eight in a tile (past n_words: none).
+template <bool LINES>
+__device__ inline uint64_t tile_words(const LineList& L, uint64_t tile, uint64_t n_words,
+                                      uint32_t* s_line) {
+  if (!LINES) return tile * BM_TILE + threadIdx.x * BM_WPT;
+  static_assert(2 * BM_WPT == LINE_WORDS, "two threads a line");
+  const uint64_t i = tile * TILE_LINES + (threadIdx.x >> 1);
+  if (i >= *L.n) return n_words;
+  const uint32_t line = L.line[i];
+  if (s_line) s_line[threadIdx.x >> 1] = line;
+  return (uint64_t)line * LINE_WORDS + (threadIdx.x & 1) * BM_WPT;
+}
+
+// Number of flagged lines per run of `per` pieces of LINE_PIECE flags.
+constexpr int LINE_PIECE = BLOCK * 64;
+constexpr uint32_t LINE_RUNS = 2048;
+constexpr uint64_t LINE_GRID = 8192;
+__device__ inline uint32_t load_flags(const uint8_t* flags, uint64_t n_lines, uint64_t i0,
+                                      uint4 (&f)[4]) {
+  uint32_t c = 0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    f[q] = make_uint4(0u, 0u, 0u, 0u);
+    if (i0 + 16 * q < n_lines) f[q] = ((const uint4*)(flags + i0))[q];  // (n_lines: whole tiles)
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) c += __popc(f[q].x) + __popc(f[q].y) + __popc(f[q].z) + __popc(f[q].w);
+  return c;
+}
+__global__ __launch_bounds__(BLOCK) void k_line_count(const uint8_t* flags, uint64_t n_lines,
+                                                      uint32_t per, uint32_t* run_count) {
+  __shared__ uint32_t tmp[8];
+  uint32_t c = 0;
+  for (uint32_t k = 0; k < per; ++k) {
+    uint4 f[4];
+    c += load_flags(flags, n_lines, ((uint64_t)blockIdx.x * per + k) * LINE_PIECE + threadIdx.x * 64,
+                    f);
+  }
+  uint32_t none = 0, t, u;
+  block_excl_scan256_2(c, none, tmp, t, u);
+  if (threadIdx.x == 0) run_count[blockIdx.x] = t;
+}
+__global__ __launch_bounds__(BLOCK) void k_line_list(const uint8_t* flags, uint64_t n_lines,
+                                                     uint32_t per, const uint32_t* run_count,
+                                                     uint32_t* line, uint32_t* n) {
+  __shared__ uint32_t tmp[8];
+  uint32_t before = 0, none = 0, t, u;
+  for (uint32_t i = threadIdx.x; i < blockIdx.x; i += BLOCK) before += run_count[i];
+  block_excl_scan256_2(before, none, tmp, t, u);
+  uint64_t base = t;
+  for (uint32_t k = 0; k < per; ++k) {
+    const uint64_t i0 = ((uint64_t)blockIdx.x * per + k) * LINE_PIECE + threadIdx.x * 64;
+    uint4 f[4];
+    const uint32_t c = load_flags(flags, n_lines, i0, f);
+    __syncthreads();  // tmp is read above
+    uint32_t a = c, b = 0;
+    block_excl_scan256_2(a, b, tmp, t, u);
+    uint64_t o = base + a;
+    if (c) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t w[4] = {f[q].x, f[q].y, f[q].z, f[q].w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          for (uint32_t r = w[j]; r; r &= r - 1u)
+            line[o++] = (uint32_t)(i0 + 16 * q + 4 * j + (__builtin_ctz(r) >> 3));
+      }
+    }
+    base += t;
+  }
+  if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) *n = (uint32_t)base;
+}
+
 // Zeroes the 16-byte pieces of the words loaded by load_words that are not
 // already zero.
 __device__ inline void clear_words(uint32_t* bits, uint64_t n_words, uint64_t w0,
@@ -285,39 +372,44 @@ constexpr int SC_CHUNK = BLOCK * SC_PER;     // 1024 tiles per scan workgroup
 
 // Per tile: set bits, nonzero bytes, and the 4-byte units k_bm_emit will
 // zero.
+template <bool LINES>
 __global__ __launch_bounds__(BLOCK) void k_bm_count(const uint32_t* bits, uint64_t n_words,
-                                                    uint32_t* tile_u, uint32_t* tile_g,
+                                                    LineList L, uint32_t* tile_u, uint32_t* tile_g,
                                                     uint32_t* tile_r, uint64_t* scan_status,
                                                     uint32_t n_status) {
   __shared__ uint32_t tmp[8];
   // the tile-count scan's look-back words and ticket start at zero
   if (blockIdx.x == 0)
     for (uint32_t i = threadIdx.x; i < n_status; i += BLOCK) scan_status[i] = 0;
-  const uint64_t w0 = (uint64_t)blockIdx.x * BM_TILE + threadIdx.x * BM_WPT;
-  uint32_t w[BM_WPT];
-  load_words(bits, n_words, w0, w);
-  // a: set bits (0-16) and the 4-byte units clear_words will zero (17-28);
-  // b: nonzero bytes
-  uint32_t a = 0, b = 0;
+  const uint64_t tiles = LINES ? line_tiles(L) : gridDim.x;
+  for (uint64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    const uint64_t w0 = tile_words<LINES>(L, tile, n_words, nullptr);
+    uint32_t w[BM_WPT];
+    load_words(bits, n_words, w0, w);
+    // a: set bits (0-16) and the 4-byte units clear_words will zero (17-28);
+    // b: nonzero bytes
+    uint32_t a = 0, b = 0;
 #pragma unroll
-  for (int j = 0; j < BM_WPT; ++j) {
-    a += __popc(w[j]);
-    b += nonzero_bytes(w[j]);
-  }
-  if (w0 + BM_WPT <= n_words) {
+    for (int j = 0; j < BM_WPT; ++j) {
+      a += __popc(w[j]);
+      b += nonzero_bytes(w[j]);
+    }
+    if (w0 + BM_WPT <= n_words) {
 #pragma unroll
-    for (int q = 0; q < BM_WPT / 4; ++q)
-      a += (w[4 * q] | w[4 * q + 1] | w[4 * q + 2] | w[4 * q + 3]) ? (4u << 17) : 0u;
-  } else {
+      for (int q = 0; q < BM_WPT / 4; ++q)
+        a += (w[4 * q] | w[4 * q + 1] | w[4 * q + 2] | w[4 * q + 3]) ? (4u << 17) : 0u;
+    } else {
 #pragma unroll
-    for (int j = 0; j < BM_WPT; ++j) a += (uint32_t)(w[j] != 0) << 17;
-  }
-  uint32_t ta, tb;
-  block_excl_scan256_2(a, b, tmp, ta, tb);  // only the totals are used
-  if (threadIdx.x == 0) {
-    tile_u[blockIdx.x] = ta & 0x1FFFFu;
-    tile_g[blockIdx.x] = tb;
-    tile_r[blockIdx.x] = ta >> 17;
+      for (int j = 0; j < BM_WPT; ++j) a += (uint32_t)(w[j] != 0) << 17;
+    }
+    uint32_t ta, tb;
+    block_excl_scan256_2(a, b, tmp, ta, tb);  // only the totals are used
+    if (threadIdx.x == 0) {
+      tile_u[tile] = ta & 0x1FFFFu;
+      tile_g[tile] = tb;
+      tile_r[tile] = ta >> 17;
+    }
+    if (LINES) __syncthreads();
   }
 }
 
@@ -327,7 +419,7 @@ __global__ __launch_bounds__(BLOCK) void k_bm_count(const uint32_t* bits, uint64
 // elements); the bytes k_bm_emit will zero are added to *reset_bytes.
 __global__ __launch_bounds__(BLOCK) void k_bm_scan(uint32_t* tile_u, uint32_t* tile_g,
                                                    const uint32_t* tile_r, uint32_t tiles,
-                                                   uint64_t* scan_status,
+                                                   LineList L, uint64_t* scan_status,
                                                    unsigned long long* counts,
                                                    unsigned long long* reset_bytes,
                                                    const unsigned long long* hits,
@@ -338,6 +430,10 @@ __global__ __launch_bounds__(BLOCK) void k_bm_scan(uint32_t* tile_u, uint32_t* t
   if (blockIdx.x == 0 && threadIdx.x < 64) {
     const uint64_t h = wave_sum((uint64_t)hits[threadIdx.x * HIT_STRIDE]);
     if (threadIdx.x == 0) *n_hits = h;
+  }
+  if (L.line) {  // flagged lines only: the later workgroups have no chunk
+    tiles = (uint32_t)line_tiles(L);
+    if ((uint64_t)blockIdx.x * SC_CHUNK >= tiles) return;
   }
   uint32_t* ticket = (uint32_t*)scan_status;  // word 0; chunk c uses words 2 + 2c, 3 + 2c
   if (threadIdx.x == 0) s_chunk = atomicAdd(ticket, 1u);
@@ -419,8 +515,8 @@ static_assert((EMIT_CAP & (EMIT_CAP - 1)) == 0, "the copy-out masks slot indices
 static_assert(BM_TILE % BLOCK == 0, "a round's words lie inside the tile's LDS arrays");
 static_assert(BM_TILE == BITMAP_TILE_WORDS, "mesh regions start on tile boundaries");
 
-template <typename K>
-__global__ __launch_bounds__(BLOCK) void k_bm_emit(uint32_t* bits, uint64_t n_words,
+template <typename K, bool LINES>
+__global__ __launch_bounds__(BLOCK) void k_bm_emit(uint32_t* bits, uint64_t n_words, LineList L,
                                                    const uint64_t* bm_off, uint32_t n_meshes,
                                                    KeyLayout<K> kl, const uint32_t* tile_u,
                                                    const uint32_t* tile_g, K* elem1, K* elem2,
@@ -433,36 +529,8 @@ __global__ __launch_bounds__(BLOCK) void k_bm_emit(uint32_t* bits, uint64_t n_wo
   __shared__ uint32_t s_word[BM_TILE], s_pre[BM_TILE];
   __shared__ uint16_t s_idx[BM_TILE], s_key[EMIT_CAP], s_grp[BLOCK * 4];
   __shared__ K s_kbase;  // key of the tile's bit 0
-  const uint64_t tw0 = (uint64_t)blockIdx.x * BM_TILE;
+  __shared__ uint32_t s_line[LINES ? TILE_LINES : 1];
   const uint32_t l0 = threadIdx.x * BM_WPT;
-  // the bitmap words and the tile's output offsets are loaded first, so that
-  // the mesh lookup's dependent loads run while they are in flight
-  uint32_t w[BM_WPT];
-  load_words(bits, n_words, tw0 + l0, w);
-  const uint32_t bu = tile_u[blockIdx.x], bg = tile_g[blockIdx.x];
-  if (threadIdx.x == 0) {
-    const uint32_t m = mesh_of_word(bm_off, n_meshes, tw0);
-    const uint64_t off = bm_off[m];
-    s_kbase = ((K)m << kl.cb) | ((K)(tw0 - off) << 5);
-    if (tw0 == off) {
-      // the mesh's first tile: its level-1 span ends where the next mesh's
-      // first tile starts (every region is whole tiles) and, for a mesh whose
-      // level 1 holds a single voxel, its depth-1 root (what
-      // k_first_finalize does on the sort path)
-      const uint64_t tn = bm_off[m + 1] / BM_TILE;
-      const uint32_t ue = tn < gridDim.x ? tile_u[tn] : (uint32_t)counts[0];
-      const uint32_t ge = tn < gridDim.x ? tile_g[tn] : (uint32_t)counts[1];
-      LevelSpan& sp = spans[(uint64_t)m * n_levels];
-      sp.elem_first = bu;
-      sp.elem_end = ue;
-      sp.group_first = bg;
-      sp.group_end = ge;
-      if (ue - bu == 1) {
-        state[m].depth = 1;
-        state[m].root_elem = bu;
-      }
-    }
-  }
   {
     // the later levels' look-back words and tickets start at zero (as
     // k_level_clear leaves them), a slice per workgroup
@@ -472,119 +540,166 @@ __global__ __launch_bounds__(BLOCK) void k_bm_emit(uint32_t* bits, uint64_t n_wo
     for (uint64_t i = (uint64_t)blockIdx.x * per + threadIdx.x; i < i1; i += BLOCK) status[i] = 0;
     if (blockIdx.x == 0 && threadIdx.x < MAX_TICKETS) tickets[threadIdx.x] = 0;
   }
-  clear_words(bits, n_words, tw0 + l0, w);  // the bitmap is left clear for the next pass
-  // a: set bits (0-16) and nonzero words (17-28); b: nonzero bytes
-  uint32_t a = 0, b = 0;
-#pragma unroll
-  for (int j = 0; j < BM_WPT; ++j) {
-    a += __popc(w[j]) + ((uint32_t)(w[j] != 0) << 17);
-    b += nonzero_bytes(w[j]);
-  }
-  uint32_t ta, tb;
-  block_excl_scan256_2(a, b, tmp, ta, tb);  // tmp is not used again
-  {
-    uint32_t pu = a & 0x1FFFFu, pg = b, pz = a >> 17;
-#pragma unroll
-    for (int j = 0; j < BM_WPT; ++j) {
-      if (w[j]) {
-        s_word[pz] = w[j];
-        s_pre[pz] = pu | (pg << 17);  // pu <= 65535, pg <= 8191 for a nonzero word
-        s_idx[pz] = (uint16_t)(l0 + j);
-        ++pz;
-      }
-      pu += __popc(w[j]);
-      pg += nonzero_bytes(w[j]);
+  if (LINES && blockIdx.x == 0 && threadIdx.x == 0) {
+    // the one mesh's level-1 span, and its depth-1 root if that is one voxel
+    spans[0].elem_first = spans[0].group_first = 0;
+    spans[0].elem_end = (uint32_t)counts[0];
+    spans[0].group_end = (uint32_t)counts[1];
+    if (counts[0] == 1) {
+      state[0].depth = 1;
+      state[0].root_elem = 0;
     }
   }
-  __syncthreads();
-  const uint32_t nz = ta >> 17;
-  const uint32_t pre_end = (ta & 0x1FFFFu) | (tb << 17);
-  const K kbase = s_kbase;
-  for (uint32_t r0 = 0; r0 < nz; r0 += BLOCK) {
-    const uint32_t r1 = r0 + BLOCK < nz ? r0 + BLOCK : nz;
-    const uint32_t pre0 = s_pre[r0], pre1 = r1 < nz ? s_pre[r1] : pre_end;
-    const uint32_t u0 = pre0 & 0x1FFFFu, nu = (pre1 & 0x1FFFFu) - u0;
-    const uint32_t g0 = pre0 >> 17, ng = (pre1 >> 17) - g0;
-    const bool stage = nu <= EMIT_CAP;  // the same for the whole block
-    const uint32_t it = r0 + threadIdx.x;
-    if (it < r1) {
-      const uint32_t word = s_word[it], pre = s_pre[it];
-      const uint32_t wb = (uint32_t)s_idx[it] << 5;  // tile bit index of the word's bit 0
-      const uint32_t lu = (pre & 0x1FFFFu) - u0;
-      // unique keys: the set bits in order
-      if (stage) {
-        uint32_t o = lu;
-        for (uint32_t r = word; r; r &= r - 1u) s_key[o++] = (uint16_t)(wb | __builtin_ctz(r));
-      } else {
-        K* out = elem1 + (uint64_t)bu + u0 + lu;
-        const K hi = kbase + (K)wb;
-        for (uint32_t r = word; r; r &= r - 1u) *out++ = hi | (K)__builtin_ctz(r);
-      }
-      // groups: the nonzero bytes in order, tested in turn (a loop over the
-      // nonzero bytes runs as often as the wave's fullest word has them,
-      // nearly always four).  A group's first child is the unique key of
-      // the byte's lowest set bit (the set bits below it are those of the
-      // lower bytes); its parent is parent(word's key 0) + byte index, its
-      // child mask the byte itself.
-      uint32_t lg = (pre >> 17) - g0;
-      if (stage) {
-#pragma unroll
-        for (uint32_t b = 0; b < 4; ++b) {
-          if ((word >> (8 * b)) & 0xFFu) s_grp[lg++] = (uint16_t)((threadIdx.x << 2) | b);
+  const uint64_t tiles = LINES ? line_tiles(L) : gridDim.x;
+  for (uint64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    // the bitmap words and the tile's output offsets are loaded first, so that
+    // the mesh lookup's dependent loads run while they are in flight
+    uint32_t w[BM_WPT];
+    const uint64_t w0 = tile_words<LINES>(L, tile, n_words, s_line);
+    load_words(bits, n_words, w0, w);
+    const uint32_t bu = tile_u[tile], bg = tile_g[tile];
+    if (!LINES && threadIdx.x == 0) {
+      const uint64_t tw0 = tile * BM_TILE;
+      const uint32_t m = mesh_of_word(bm_off, n_meshes, tw0);
+      const uint64_t off = bm_off[m];
+      s_kbase = ((K)m << kl.cb) | ((K)(tw0 - off) << 5);
+      if (tw0 == off) {
+        // the mesh's first tile: its level-1 span ends where the next mesh's
+        // first tile starts (every region is whole tiles) and, for a mesh whose
+        // level 1 holds a single voxel, its depth-1 root (what
+        // k_first_finalize does on the sort path)
+        const uint64_t tn = bm_off[m + 1] / BM_TILE;
+        const uint32_t ue = tn < gridDim.x ? tile_u[tn] : (uint32_t)counts[0];
+        const uint32_t ge = tn < gridDim.x ? tile_g[tn] : (uint32_t)counts[1];
+        LevelSpan& sp = spans[(uint64_t)m * n_levels];
+        sp.elem_first = bu;
+        sp.elem_end = ue;
+        sp.group_first = bg;
+        sp.group_end = ge;
+        if (ue - bu == 1) {
+          state[m].depth = 1;
+          state[m].root_elem = bu;
         }
-      } else {
-        const uint32_t pu_w = pre & 0x1FFFFu;
-        const K phi = kl.parent(kbase + (K)wb);
-        const uint64_t d0 = (uint64_t)bg + g0;
+      }
+    }
+    clear_words(bits, n_words, w0, w);  // the bitmap is left clear for the next pass
+    // a: set bits (0-16) and nonzero words (17-28); b: nonzero bytes
+    uint32_t a = 0, b = 0;
 #pragma unroll
-        for (uint32_t b = 0; b < 4; ++b) {
-          if ((word >> (8 * b)) & 0xFFu) {
-            elem2[d0 + lg] = phi | (K)b;
-            first_child2[d0 + lg] = bu + pu_w + (b ? __popc(word & ((1u << (8 * b)) - 1u)) : 0u);
-            kids2[d0 + lg] = (uint8_t)(word >> (8 * b));
-            ++lg;
+    for (int j = 0; j < BM_WPT; ++j) {
+      a += __popc(w[j]) + ((uint32_t)(w[j] != 0) << 17);
+      b += nonzero_bytes(w[j]);
+    }
+    uint32_t ta, tb;
+    block_excl_scan256_2(a, b, tmp, ta, tb);  // tmp is not used again
+    {
+      uint32_t pu = a & 0x1FFFFu, pg = b, pz = a >> 17;
+#pragma unroll
+      for (int j = 0; j < BM_WPT; ++j) {
+        if (w[j]) {
+          s_word[pz] = w[j];
+          s_pre[pz] = pu | (pg << 17);  // pu <= 65535, pg <= 8191 for a nonzero word
+          s_idx[pz] = (uint16_t)(l0 + j);
+          ++pz;
+        }
+        pu += __popc(w[j]);
+        pg += nonzero_bytes(w[j]);
+      }
+    }
+    __syncthreads();
+    const uint32_t nz = ta >> 17;
+    const uint32_t pre_end = (ta & 0x1FFFFu) | (tb << 17);
+    // key of a tile bit
+    const K kbase = LINES ? (K)0 : s_kbase;
+    auto key_of = [&](uint32_t b) -> K {
+      return LINES ? ((K)s_line[b >> 9] << 9) | (K)(b & 511u) : kbase + (K)b;
+    };
+    for (uint32_t r0 = 0; r0 < nz; r0 += BLOCK) {
+      const uint32_t r1 = r0 + BLOCK < nz ? r0 + BLOCK : nz;
+      const uint32_t pre0 = s_pre[r0], pre1 = r1 < nz ? s_pre[r1] : pre_end;
+      const uint32_t u0 = pre0 & 0x1FFFFu, nu = (pre1 & 0x1FFFFu) - u0;
+      const uint32_t g0 = pre0 >> 17, ng = (pre1 >> 17) - g0;
+      const bool stage = nu <= EMIT_CAP;  // the same for the whole block
+      const uint32_t it = r0 + threadIdx.x;
+      if (it < r1) {
+        const uint32_t word = s_word[it], pre = s_pre[it];
+        const uint32_t wb = (uint32_t)s_idx[it] << 5;  // tile bit index of the word's bit 0
+        const uint32_t lu = (pre & 0x1FFFFu) - u0;
+        // unique keys: the set bits in order
+        if (stage) {
+          uint32_t o = lu;
+          for (uint32_t r = word; r; r &= r - 1u) s_key[o++] = (uint16_t)(wb | __builtin_ctz(r));
+        } else {
+          K* out = elem1 + (uint64_t)bu + u0 + lu;
+          const K hi = key_of(wb);
+          for (uint32_t r = word; r; r &= r - 1u) *out++ = hi | (K)__builtin_ctz(r);
+        }
+        // groups: the nonzero bytes in order, tested in turn (a loop over the
+        // nonzero bytes runs as often as the wave's fullest word has them,
+        // nearly always four).  A group's first child is the unique key of
+        // the byte's lowest set bit (the set bits below it are those of the
+        // lower bytes); its parent is parent(word's key 0) + byte index, its
+        // child mask the byte itself.
+        uint32_t lg = (pre >> 17) - g0;
+        if (stage) {
+#pragma unroll
+          for (uint32_t b = 0; b < 4; ++b) {
+            if ((word >> (8 * b)) & 0xFFu) s_grp[lg++] = (uint16_t)((threadIdx.x << 2) | b);
+          }
+        } else {
+          const uint32_t pu_w = pre & 0x1FFFFu;
+          const K phi = kl.parent(key_of(wb));
+          const uint64_t d0 = (uint64_t)bg + g0;
+#pragma unroll
+          for (uint32_t b = 0; b < 4; ++b) {
+            if ((word >> (8 * b)) & 0xFFu) {
+              elem2[d0 + lg] = phi | (K)b;
+              first_child2[d0 + lg] = bu + pu_w + (b ? __popc(word & ((1u << (8 * b)) - 1u)) : 0u);
+              kids2[d0 + lg] = (uint8_t)(word >> (8 * b));
+              ++lg;
+            }
           }
         }
       }
-    }
-    __syncthreads();
-    // copy-out, four elements per thread per step: the LDS reads are issued
-    // together (slots past the round's count read stale entries inside the
-    // buffers and store nothing)
-    if (stage) {
-      K* dst = elem1 + (uint64_t)bu + u0;
-      for (uint32_t i0 = threadIdx.x; i0 < nu; i0 += 4 * BLOCK) {
-        uint32_t v[4];
+      __syncthreads();
+      // copy-out, four elements per thread per step: the LDS reads are issued
+      // together (slots past the round's count read stale entries inside the
+      // buffers and store nothing)
+      if (stage) {
+        K* dst = elem1 + (uint64_t)bu + u0;
+        for (uint32_t i0 = threadIdx.x; i0 < nu; i0 += 4 * BLOCK) {
+          uint32_t v[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = s_key[(i0 + j * BLOCK) & (EMIT_CAP - 1)];
+          for (int j = 0; j < 4; ++j) v[j] = s_key[(i0 + j * BLOCK) & (EMIT_CAP - 1)];
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (i0 + j * BLOCK < nu) dst[i0 + j * BLOCK] = key_of(v[j]);
+        }
+        // groups, ng <= 4 * BLOCK: one step
+        const uint32_t i0 = threadIdx.x;
+        uint32_t c[4], word[4], pre[4], idx[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) c[j] = s_grp[i0 + j * BLOCK] & (4 * BLOCK - 1);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t wi = r0 + (c[j] >> 2);  // r0 <= BM_TILE - BLOCK
+          word[j] = s_word[wi];
+          pre[j] = s_pre[wi];
+          idx[j] = s_idx[wi];
+        }
+        const uint64_t d0 = (uint64_t)bg + g0;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (i0 + j * BLOCK < nu) dst[i0 + j * BLOCK] = kbase + (K)v[j];
+          if (i0 + j * BLOCK < ng) {
+            const uint32_t sh = 8 * (c[j] & 3u);
+            const uint64_t d = d0 + i0 + j * BLOCK;
+            elem2[d] = kl.parent(key_of((idx[j] << 5) | sh));
+            first_child2[d] = bu + (pre[j] & 0x1FFFFu) + __popc(word[j] & ((1u << sh) - 1u));
+            kids2[d] = (uint8_t)(word[j] >> sh);
+          }
       }
-      // groups, ng <= 4 * BLOCK: one step
-      const uint32_t i0 = threadIdx.x;
-      uint32_t c[4], word[4], pre[4], idx[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) c[j] = s_grp[i0 + j * BLOCK] & (4 * BLOCK - 1);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t wi = r0 + (c[j] >> 2);  // r0 <= BM_TILE - BLOCK
-        word[j] = s_word[wi];
-        pre[j] = s_pre[wi];
-        idx[j] = s_idx[wi];
-      }
-      const uint64_t d0 = (uint64_t)bg + g0;
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (i0 + j * BLOCK < ng) {
-          const uint32_t sh = 8 * (c[j] & 3u);
-          const uint64_t d = d0 + i0 + j * BLOCK;
-          elem2[d] = kl.parent(kbase + (K)((idx[j] << 5) | sh));
-          first_child2[d] = bu + (pre[j] & 0x1FFFFu) + __popc(word[j] & ((1u << sh) - 1u));
-          kids2[d] = (uint8_t)(word[j] >> sh);
-        }
+      __syncthreads();
     }
-    __syncthreads();
   }
 }
 
@@ -935,7 +1050,7 @@ void launch_level_first(const K* sorted, const unsigned long long* n_sorted, uin
 size_t bitmap_level_tmp_bytes(uint64_t n_words) {
   const uint64_t tiles = (std::max<uint64_t>(n_words, 1) + BM_TILE - 1) / BM_TILE;
   const uint64_t chunks = (tiles + SC_CHUNK - 1) / SC_CHUNK;
-  return 3 * tiles * sizeof(uint32_t) + 256 + (2 + 2 * chunks) * sizeof(uint64_t);
+  return 3 * tiles * sizeof(uint32_t) + 256 + (2 + 2 * chunks) * sizeof(uint64_t) + 64;
 }
 
 template <typename K>
@@ -945,7 +1060,7 @@ void launch_level_first_bitmap(uint32_t* bits, uint64_t n_words, const uint64_t*
                                uint32_t n_levels, MeshTreeState* state, void* tmp,
                                void* lvl_tmp, unsigned long long* reset_bytes,
                                const unsigned long long* hits, unsigned long long* n_hits,
-                               hipStream_t s) {
+                               const uint8_t* line_flags, uint32_t* line_list, hipStream_t s) {
   const uint64_t tiles = (std::max<uint64_t>(n_words, 1) + BM_TILE - 1) / BM_TILE;
   const uint64_t chunks = (tiles + SC_CHUNK - 1) / SC_CHUNK;
   uint32_t* tile_u = (uint32_t*)tmp;
@@ -954,20 +1069,36 @@ void launch_level_first_bitmap(uint32_t* bits, uint64_t n_words, const uint64_t*
   uint64_t* scan_status =
       (uint64_t*)((char*)tmp + ((3 * tiles * sizeof(uint32_t) + 255) / 256) * 256);
   const uint32_t n_status = (uint32_t)(2 + 2 * chunks);
-  hipLaunchKernelGGL(k_bm_count, dim3((uint32_t)tiles), dim3(BLOCK), 0, s, bits, n_words, tile_u,
-                     tile_g, tile_r, scan_status, n_status);
-  hipLaunchKernelGGL(k_bm_scan, dim3((uint32_t)chunks), dim3(BLOCK), 0, s, tile_u, tile_g,
-                     (const uint32_t*)tile_r, (uint32_t)tiles, scan_status, counts, reset_bytes, hits,
-                     n_hits);
-  // the emission also writes the level-1 spans and depth-1 roots, and clears
-  // the later levels' look-back words and tickets (launch_levels)
   uint32_t* tickets = (uint32_t*)lvl_tmp;
   uint64_t* status = (uint64_t*)((char*)lvl_tmp + 256);
-  hipLaunchKernelGGL(k_bm_emit<K>, dim3((uint32_t)tiles), dim3(BLOCK), 0, s, bits, n_words,
-                     bm_off, n_meshes, kl, (const uint32_t*)tile_u, (const uint32_t*)tile_g,
-                     (K*)l1.elem, (K*)l2.elem, l2.first_child, l2.kids,
-                     (const unsigned long long*)counts, spans1, n_levels, state, status,
-                     tickets);
+  auto run = [&](auto lines, const LineList& L, uint32_t grid) {
+    constexpr bool LINES = decltype(lines)::value;
+    hipLaunchKernelGGL(k_bm_count<LINES>, dim3(grid), dim3(BLOCK), 0, s, bits, n_words, L, tile_u,
+                       tile_g, tile_r, scan_status, n_status);
+    hipLaunchKernelGGL(k_bm_scan, dim3((uint32_t)chunks), dim3(BLOCK), 0, s, tile_u, tile_g,
+                       (const uint32_t*)tile_r, (uint32_t)tiles, L, scan_status, counts,
+                       reset_bytes, hits, n_hits);
+    // the emission also writes the level-1 spans and depth-1 roots, and clears
+    // the later levels' look-back words and tickets (launch_levels)
+    hipLaunchKernelGGL((k_bm_emit<K, LINES>), dim3(grid), dim3(BLOCK), 0, s, bits, n_words, L,
+                       bm_off, n_meshes, kl, (const uint32_t*)tile_u, (const uint32_t*)tile_g,
+                       (K*)l1.elem, (K*)l2.elem, l2.first_child, l2.kids,
+                       (const unsigned long long*)counts, spans1, n_levels, state, status,
+                       tickets);
+  };
+  if (!line_flags) {
+    run(std::false_type{}, LineList{}, (uint32_t)tiles);
+    return;
+  }
+  // runs of flags: at least a piece each (tile_g holds their counts for now)
+  const uint64_t n_lines = n_words / LINE_WORDS, pieces = (n_lines + LINE_PIECE - 1) / LINE_PIECE;
+  const uint32_t per = (uint32_t)((pieces + LINE_RUNS - 1) / LINE_RUNS);
+  const uint32_t runs = (uint32_t)((pieces + per - 1) / per);
+  uint32_t* n = (uint32_t*)(scan_status + n_status);
+  hipLaunchKernelGGL(k_line_count, dim3(runs), dim3(BLOCK), 0, s, line_flags, n_lines, per, tile_g);
+  hipLaunchKernelGGL(k_line_list, dim3(runs), dim3(BLOCK), 0, s, line_flags, n_lines, per,
+                     (const uint32_t*)tile_g, line_list, n);
+  run(std::true_type{}, LineList{line_list, n}, (uint32_t)std::min<uint64_t>(tiles, LINE_GRID));
 }
 
 void launch_level_first_finalize(const LevelSpan* spans, uint32_t n_meshes, uint32_t n_levels,
@@ -1021,13 +1152,15 @@ template void launch_level_first_bitmap<uint32_t>(uint32_t*, uint64_t, const uin
                                                   LevelArrays, unsigned long long*, LevelSpan*,
                                                   uint32_t, MeshTreeState*, void*, void*,
                                                   unsigned long long*, const unsigned long long*,
-                                                  unsigned long long*, hipStream_t);
+                                                  unsigned long long*, const uint8_t*, uint32_t*,
+                                                  hipStream_t);
 template void launch_level_first_bitmap<uint64_t>(uint32_t*, uint64_t, const uint64_t*,
                                                   uint32_t, KeyLayout<uint64_t>, LevelArrays,
                                                   LevelArrays, unsigned long long*, LevelSpan*,
                                                   uint32_t, MeshTreeState*, void*, void*,
                                                   unsigned long long*, const unsigned long long*,
-                                                  unsigned long long*, hipStream_t);
+                                                  unsigned long long*, const uint8_t*, uint32_t*,
+                                                  hipStream_t);
 template void launch_levels<uint32_t>(KeyLayout<uint32_t>, const LevelArrays*, uint32_t,
                                       unsigned long long*, LevelSpan*, MeshTreeState*, uint32_t,
                                       void*, hipStream_t);

@@ -472,6 +472,7 @@ struct VoxOut {
   K* keys;                // key path
   uint32_t* bits;         // bitmap path
   const uint64_t* bm_off; // bitmap words before each mesh
+  uint8_t* line_flags;    // bitmap path: a byte per 64-byte line, or null
   unsigned long long* count;  // key path: keys stored
   unsigned long long* hits;   // bitmap path: HIT_SLOTS counters HIT_STRIDE apart
 };
@@ -554,12 +555,15 @@ struct WordTable {
   unsigned long long bits[WORD_SLOTS];
   uint32_t word[WORD_SLOTS];
 };
-__device__ inline void or_memory(uint32_t* bitmap, uint64_t word, unsigned long long bits) {
+__device__ inline void or_memory(uint32_t* bitmap, uint8_t* line_flags, uint64_t word,
+                                 unsigned long long bits) {
+  // (every writer of a flag stores the same value)
+  if (line_flags) line_flags[word / (BITMAP_LINE_BYTES / 8)] = 1;
   __hip_atomic_fetch_or((unsigned long long*)bitmap + word, bits, __ATOMIC_RELAXED,
                         __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ inline void set_bits(WordTable& t, uint32_t* bitmap, uint64_t word,
-                                unsigned long long bits) {
+__device__ inline void set_bits(WordTable& t, uint32_t* bitmap, uint8_t* line_flags,
+                                uint64_t word, unsigned long long bits) {
   if (word < NO_WORD) {
     const uint32_t slot = ((uint32_t)word * 0x9E3779B1u) >> (32 - WORD_SLOT_BITS);
     const uint32_t old = atomicCAS(&t.word[slot], NO_WORD, (uint32_t)word);
@@ -568,7 +572,7 @@ __device__ inline void set_bits(WordTable& t, uint32_t* bitmap, uint64_t word,
       return;
     }
   }
-  or_memory(bitmap, word, bits);
+  or_memory(bitmap, line_flags, word, bits);
 }
 
 template <typename K, bool BITMAP, bool ITEMS>
@@ -731,7 +735,7 @@ __global__ __launch_bounds__(BLOCK) void k_vox_rows(
           if (hit) {
             n_hits += __popc(hit);
             // cells 0-3 of the group are bits 0, 1, 8, 9 from its place
-            set_bits(s_words[0], out.bits, kbase + (uint64_t)(code >> 6),
+            set_bits(s_words[0], out.bits, out.line_flags, kbase + (uint64_t)(code >> 6),
                      (unsigned long long)((hit & 3u) | ((hit & 12u) << 6)) << (code & 63));
           }
         } else {
@@ -762,7 +766,7 @@ __global__ __launch_bounds__(BLOCK) void k_vox_rows(
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < WORD_SLOTS; i += BLOCK)
       if (s_words[0].word[i] != NO_WORD)
-        or_memory(out.bits, s_words[0].word[i], s_words[0].bits[i]);
+        or_memory(out.bits, out.line_flags, s_words[0].word[i], s_words[0].bits[i]);
   } else if (staged) {
     flush();
   }
@@ -822,11 +826,11 @@ static void launch_rows(const MeshDev* meshes, const MeshParams* params, const u
 template <typename K>
 void launch_voxelize(const MeshDev* meshes, const MeshParams* params, const uint64_t* tri_base,
                      uint32_t n_meshes, uint64_t n_tris, int cb, const Tuning& tn, K* keys,
-                     uint32_t* bitmap, const uint64_t* bm_off, unsigned long long* key_count,
-                     unsigned long long* hits, BigItem* big, unsigned long long* big_count,
-                     uint64_t big_cap, hipStream_t s) {
+                     uint32_t* bitmap, const uint64_t* bm_off, uint8_t* line_flags,
+                     unsigned long long* key_count, unsigned long long* hits, BigItem* big,
+                     unsigned long long* big_count, uint64_t big_cap, hipStream_t s) {
   if (n_tris == 0) return;
-  const VoxOut<K> out{keys, bitmap, bm_off, key_count, hits};
+  const VoxOut<K> out{keys, bitmap, bm_off, line_flags, key_count, hits};
   if (bitmap)
     launch_rows<K, true>(meshes, params, tri_base, n_meshes, n_tris, cb, tn, out, big, big_count,
                          big_cap, s);
@@ -837,12 +841,14 @@ void launch_voxelize(const MeshDev* meshes, const MeshParams* params, const uint
 
 template void launch_voxelize<uint32_t>(const MeshDev*, const MeshParams*, const uint64_t*,
                                         uint32_t, uint64_t, int, const Tuning&, uint32_t*,
-                                        uint32_t*, const uint64_t*, unsigned long long*,
+                                        uint32_t*, const uint64_t*, uint8_t*,
+                                        unsigned long long*,
                                         unsigned long long*, BigItem*, unsigned long long*,
                                         uint64_t, hipStream_t);
 template void launch_voxelize<uint64_t>(const MeshDev*, const MeshParams*, const uint64_t*,
                                         uint32_t, uint64_t, int, const Tuning&, uint64_t*,
-                                        uint32_t*, const uint64_t*, unsigned long long*,
+                                        uint32_t*, const uint64_t*, uint8_t*,
+                                        unsigned long long*,
                                         unsigned long long*, BigItem*, unsigned long long*,
                                         uint64_t, hipStream_t);
 

@@ -306,10 +306,10 @@ int svo_k_voxelize(int device, const float* xyz, uint64_t n_points, const int32_
     } else {
       if (kb == 64)
         launch_voxelize<uint64_t>(md, par, tb, 1, n_tris, 3 * bits, tn, (uint64_t*)keys, nullptr,
-                                  nullptr, cnt + 2, nullptr, big, cnt + 3, n_big, s);
+                                  nullptr, nullptr, cnt + 2, nullptr, big, cnt + 3, n_big, s);
       else
         launch_voxelize<uint32_t>(md, par, tb, 1, n_tris, 3 * bits, tn, (uint32_t*)keys, nullptr,
-                                  nullptr, cnt + 2, nullptr, big, cnt + 3, n_big, s);
+                                  nullptr, nullptr, cnt + 2, nullptr, big, cnt + 3, n_big, s);
       st = SVO_E_HIP;
       if (hipMemcpyAsync(tot, cnt, 32, hipMemcpyDeviceToHost, s) == hipSuccess &&
           hipStreamSynchronize(s) == hipSuccess) {

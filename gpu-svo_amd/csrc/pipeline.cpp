@@ -830,6 +830,8 @@ struct StageTimer {
 // ------------------------------------------------------------------ the pass
 namespace {
 
+constexpr uint64_t LINE_FLAGS_MIN = 256ull << 20;  // bitmap bytes (run_typed)
+
 // True when the reference's consecutive unique (uniqueVert / uniqueEdge,
 // SVO.cu:679-720) provably removes nothing: every node width w is positive,
 // finite and at least 2^-22 times the largest coordinate magnitude a node
@@ -1087,12 +1089,23 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     bm_clean_after = std::max(clean, (size_t)bm_bytes);
     clean = 0;
   }
-  launch_voxelize<K>(d_md, d_par, d_tb, n, T, plan.cb, plan.tuning, keys_a, bitmap, d_bo,
+  // A bitmap past the 256 MB of cache is read by its flagged lines (k_levels):
+  // at 134 MB, 1024^3, reading it whole costs 66 us and the flags would save
+  // none of it.  The flags stand where level 1's keys go afterwards, the list
+  // of lines, which are level 4's elements, where its groups do.
+  uint8_t* line_flags = nullptr;
+  if (use_bm && n == 1 && NL >= 4 && bm_bytes >= LINE_FLAGS_MIN &&
+      bm_bytes / BITMAP_LINE_BYTES <= sizeof(K) * cap[1]) {
+    line_flags = (uint8_t*)lv[1].elem;
+    launch_fill_u32((uint32_t*)line_flags, 0u, bm_bytes / BITMAP_LINE_BYTES / 4, s);
+  }
+  launch_voxelize<K>(d_md, d_par, d_tb, n, T, plan.cb, plan.tuning, keys_a, bitmap, d_bo, line_flags,
                      d_cnt + 2, d_hits, big, d_cnt + 3, n_big, s);
   timer.mark("voxelize");
   if (use_bm) {
     launch_level_first_bitmap<K>(bitmap, bm_words, d_bo, n, kl, lv[1], lv[2], d_counts, d_spans,
-                                 NL, d_state, bm_tmp, lvl_tmp, d_cnt + 4, d_hits, d_cnt + 2, s);
+                                 NL, d_state, bm_tmp, lvl_tmp, d_cnt + 4, d_hits, d_cnt + 2, line_flags,
+                                 line_flags ? lv[4].elem_group : nullptr, s);
     W.clean_bytes("bitmap") = bm_clean_after;
   } else {
     K* sorted = nullptr;

@@ -73,13 +73,16 @@ constexpr uint32_t HIT_SLOTS = 64, HIT_STRIDE = 8;
 // Surface voxelization (SVO.cu:37-188): emits composite keys.
 // Hits go to `keys` (raw, for the sort; *key_count receives their number) when
 // `bitmap` is null, else into the occupancy bitmap (word bm_off[mesh] + code /
-// 32, bit code % 32, which the caller has zeroed; counted in `hits`).
+// 32, bit code % 32, which the caller has zeroed; counted in `hits`).  With
+// `line_flags`, byte k of it (zeroed as well) is set for each line of
+// BITMAP_LINE_BYTES bitmap bytes that receives a bit.
+constexpr uint64_t BITMAP_LINE_BYTES = 64;
 template <typename K>
 void launch_voxelize(const MeshDev* meshes, const MeshParams* params, const uint64_t* tri_base,
                      uint32_t n_meshes, uint64_t n_tris, int cb, const Tuning& tn, K* keys,
-                     uint32_t* bitmap, const uint64_t* bm_off, unsigned long long* key_count,
-                     unsigned long long* hits, BigItem* big, unsigned long long* big_count,
-                     uint64_t big_cap, hipStream_t s);
+                     uint32_t* bitmap, const uint64_t* bm_off, uint8_t* line_flags,
+                     unsigned long long* key_count, unsigned long long* hits, BigItem* big,
+                     unsigned long long* big_count, uint64_t big_cap, hipStream_t s);
 
 // ------------------------------------------------------------ k_sort.hip
 // LSD radix sort of n (device-resident count) keys on bits [0, bits).
@@ -115,7 +118,9 @@ void launch_level_first(const K* sorted, const unsigned long long* n_sorted, uin
 // BITMAP_TILE_WORDS): the same outputs as launch_level_first followed
 // by launch_level_first_finalize, and the bitmap is left all zero (the bytes
 // that takes are added to *reset_bytes); *n_hits receives the sum of the
-// voxelization's hit counters `hits`.  `tmp` needs
+// voxelization's hit counters `hits`.  With the flags of launch_voxelize (one
+// mesh, bm_off[0] = 0) only the flagged lines are read; `line_list` receives
+// their numbers.  `tmp` needs
 // bitmap_level_tmp_bytes(n_words); `lvl_tmp` (level_tmp_bytes of l1.cap) is
 // prepared for the later levels.
 size_t bitmap_level_tmp_bytes(uint64_t n_words);
@@ -132,7 +137,7 @@ void launch_level_first_bitmap(uint32_t* bits, uint64_t n_words, const uint64_t*
                                uint32_t n_levels, MeshTreeState* state, void* tmp,
                                void* lvl_tmp, unsigned long long* reset_bytes,
                                const unsigned long long* hits, unsigned long long* n_hits,
-                               hipStream_t s);
+                               const uint8_t* line_flags, uint32_t* line_list, hipStream_t s);
 // Marks meshes whose level-1 set holds a single voxel as depth-1 trees (the
 // sort path; launch_level_first_bitmap does it itself).
 void launch_level_first_finalize(const LevelSpan* spans, uint32_t n_meshes, uint32_t n_levels,
