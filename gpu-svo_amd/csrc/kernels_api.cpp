@@ -204,7 +204,7 @@ int svo_k_radix_sort_noalloc(int device, void* keys, uint64_t n, int key_bytes, 
   if (n == 0) return SVO_OK;
   // layout: [count | ping-pong keys | digit counts], each on a 256-byte boundary
   const size_t o_keys = 256, o_tmp = o_keys + 8 * NOALLOC_SORT_MAX_KEYS;
-  if (o_tmp + radix_sort_tmp_bytes(NOALLOC_SORT_MAX_KEYS) > NOALLOC_SCRATCH_BYTES)
+  if (o_tmp + radix_sort_tmp_bound(NOALLOC_SORT_MAX_KEYS) > NOALLOC_SCRATCH_BYTES)
     return SVO_E_TOO_LARGE;
   int prev = -1;
   if (hipGetDevice(&prev) != hipSuccess || hipSetDevice(device) != hipSuccess) return SVO_E_HIP;
@@ -218,23 +218,13 @@ int svo_k_radix_sort_noalloc(int device, void* keys, uint64_t n, int key_bytes, 
     void* tmp = (char*)base + o_tmp;
     const uint32_t blocks = Tuning{}.sort_blocks;
     hipLaunchKernelGGL(k_set_count, dim3(1), dim3(64), 0, s, cnt, (unsigned long long)n);
-    void* out = nullptr;
-    if (key_bytes == 4) {
-      uint32_t* r = nullptr;
+    if (key_bytes == 4)
       launch_radix_sort<uint32_t>((uint32_t*)keys, (uint32_t*)pong, cnt, n, bits, blocks, tmp,
-                                  &r, s);
-      out = r;
-    } else {
-      uint64_t* r = nullptr;
+                                  nullptr, s);
+    else
       launch_radix_sort<uint64_t>((uint64_t*)keys, (uint64_t*)pong, cnt, n, bits, blocks, tmp,
-                                  &r, s);
-      out = r;
-    }
+                                  nullptr, s);
     if (hipGetLastError() != hipSuccess) st = SVO_E_HIP;
-    // an odd number of passes leaves the keys in the scratch buffer
-    if (st == SVO_OK && out != keys &&
-        hipMemcpyAsync(keys, out, (size_t)key_bytes * n, hipMemcpyDeviceToDevice, s) != hipSuccess)
-      st = SVO_E_HIP;
     if (st == SVO_OK && !stream && hipStreamSynchronize(s) != hipSuccess) st = SVO_E_HIP;
   }
   (void)hipSetDevice(prev);

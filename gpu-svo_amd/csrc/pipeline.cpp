@@ -444,7 +444,7 @@ double pass_bytes_bound(const svo_params* p, int kb, uint64_t P, uint64_t T, int
                            sizeof(BigItem) * std::max(n_big, 1.0) + 4.1 * N + 4096.0 +
                            (1 << 20);  // keep masks; control buffers of one mesh
   const double ws_bitmap = 4.0 * bm_words + (double)bitmap_level_tmp_bytes(bm_words);
-  const double ws_sort = 2.0 * K * key_cap + (double)radix_sort_tmp_bytes(kc);
+  const double ws_sort = 2.0 * K * key_cap + (double)radix_sort_tmp_bound(kc);
   const double ws = ws_common + std::max(ws_bitmap, ws_sort);
   // allocator: 1/8 growth headroom on workspace buffers, size classes <= 1.25x
   return 1.25 * out + 1.25 * 1.125 * ws + (2 << 20);

@@ -86,10 +86,11 @@ void launch_voxelize(const MeshDev* meshes, const MeshParams* params, const uint
 
 // ------------------------------------------------------------ k_sort.hip
 // LSD radix sort of n (device-resident count) keys on bits [0, bits).
-// Returns in *result which of (a, b) holds the sorted keys.  n must not exceed
-// cap; `tmp` needs radix_sort_tmp_bytes(cap) bytes.  `blocks` bounds the
-// persistent grid of the digit passes.
+// Returns in *result which of (a, b) holds the sorted keys; a null result asks
+// for them in a.  n must not exceed cap; `tmp` needs radix_sort_tmp_bytes(cap)
+// bytes.  `blocks` bounds the persistent grid of the digit passes.
 size_t radix_sort_tmp_bytes(uint64_t cap);
+size_t radix_sort_tmp_bound(uint64_t cap);  // over all capacities up to cap
 template <typename K>
 void launch_radix_sort(K* a, K* b, const unsigned long long* n, uint64_t cap, int bits,
                        uint32_t blocks, void* tmp, K** result, hipStream_t s);
