@@ -422,14 +422,21 @@ __global__ __launch_bounds__(BLOCK) void k_bm_scan(uint32_t* tile_u, uint32_t* t
                                                    LineList L, uint64_t* scan_status,
                                                    unsigned long long* counts,
                                                    unsigned long long* reset_bytes,
-                                                   const unsigned long long* hits,
-                                                   unsigned long long* n_hits) {
+                                                   const unsigned long long* slots,
+                                                   unsigned long long* totals) {
   __shared__ uint64_t tmp[4];
   __shared__ uint32_t s_chunk, s_base[2], s_reset[BLOCK / 64];
-  static_assert(HIT_SLOTS == 64, "a wave adds up the hit counters");
+  static_assert(COUNT_SLOTS == 64, "a wave adds up the counters");
   if (blockIdx.x == 0 && threadIdx.x < 64) {
-    const uint64_t h = wave_sum((uint64_t)hits[threadIdx.x * HIT_STRIDE]);
-    if (threadIdx.x == 0) *n_hits = h;
+    const unsigned long long* slot = slots + threadIdx.x * COUNT_STRIDE;
+    const uint64_t c = wave_sum((uint64_t)slot[COUNT_CELLS]);
+    const uint64_t k = wave_sum((uint64_t)slot[COUNT_CHUNKS]);
+    const uint64_t h = wave_sum((uint64_t)slot[COUNT_HITS]);
+    if (threadIdx.x == 0) {
+      totals[0] = c;
+      totals[1] = k;
+      totals[2] = h;
+    }
   }
   if (L.line) {  // flagged lines only: the later workgroups have no chunk
     tiles = (uint32_t)line_tiles(L);
@@ -1059,7 +1066,7 @@ void launch_level_first_bitmap(uint32_t* bits, uint64_t n_words, const uint64_t*
                                LevelArrays l2, unsigned long long* counts, LevelSpan* spans1,
                                uint32_t n_levels, MeshTreeState* state, void* tmp,
                                void* lvl_tmp, unsigned long long* reset_bytes,
-                               const unsigned long long* hits, unsigned long long* n_hits,
+                               const unsigned long long* slots, unsigned long long* totals,
                                const uint8_t* line_flags, uint32_t* line_list, hipStream_t s) {
   const uint64_t tiles = (std::max<uint64_t>(n_words, 1) + BM_TILE - 1) / BM_TILE;
   const uint64_t chunks = (tiles + SC_CHUNK - 1) / SC_CHUNK;
@@ -1077,7 +1084,7 @@ void launch_level_first_bitmap(uint32_t* bits, uint64_t n_words, const uint64_t*
                        tile_g, tile_r, scan_status, n_status);
     hipLaunchKernelGGL(k_bm_scan, dim3((uint32_t)chunks), dim3(BLOCK), 0, s, tile_u, tile_g,
                        (const uint32_t*)tile_r, (uint32_t)tiles, L, scan_status, counts,
-                       reset_bytes, hits, n_hits);
+                       reset_bytes, slots, totals);
     // the emission also writes the level-1 spans and depth-1 roots, and clears
     // the later levels' look-back words and tickets (launch_levels)
     hipLaunchKernelGGL((k_bm_emit<K, LINES>), dim3(grid), dim3(BLOCK), 0, s, bits, n_words, L,

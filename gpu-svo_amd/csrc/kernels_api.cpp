@@ -252,8 +252,10 @@ int svo_k_voxelize(int device, const float* xyz, uint64_t n_points, const int32_
   uint64_t* tb = (uint64_t*)B.get(16);
   uint32_t* acc = (uint32_t*)B.get(32);
   MeshParams* par = (MeshParams*)B.get(sizeof(MeshParams));
-  unsigned long long* cnt = (unsigned long long*)B.get(64);
-  if (!dp || !dt || !md || !tb || !acc || !par || !cnt) return SVO_E_OOM;
+  const uint64_t slot_words = COUNT_SLOTS * COUNT_STRIDE;
+  unsigned long long* slots = (unsigned long long*)B.get(8 * slot_words + 64);
+  if (!dp || !dt || !md || !tb || !acc || !par || !slots) return SVO_E_OOM;
+  unsigned long long* cnt = slots + slot_words;
   MeshDev h{};
   h.pts = dp;
   h.tri = dt;
@@ -261,7 +263,6 @@ int svo_k_voxelize(int device, const float* xyz, uint64_t n_points, const int32_
   h.n_tris = n_tris;
   for (int a = 0; a < 3; ++a) h.res[a] = res[a];
   const uint64_t htb[2] = {0, n_tris};
-  const unsigned long long zero[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   hipStream_t s;
   if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) return SVO_E_HIP;
   Tuning tn;
@@ -270,11 +271,11 @@ int svo_k_voxelize(int device, const float* xyz, uint64_t n_points, const int32_
   if (hipMemcpyAsync(dp, xyz, 12 * n_points, hipMemcpyHostToDevice, s) == hipSuccess &&
       hipMemcpyAsync(dt, tri, 12 * n_tris, hipMemcpyHostToDevice, s) == hipSuccess &&
       hipMemcpyAsync(md, &h, sizeof h, hipMemcpyHostToDevice, s) == hipSuccess &&
-      hipMemcpyAsync(tb, htb, 16, hipMemcpyHostToDevice, s) == hipSuccess &&
-      hipMemcpyAsync(cnt, zero, 64, hipMemcpyHostToDevice, s) == hipSuccess) {
-    launch_begin(PassBegin{nullptr, nullptr, 0, acc, 1, nullptr, 0}, s);
+      hipMemcpyAsync(tb, htb, 16, hipMemcpyHostToDevice, s) == hipSuccess) {
+    launch_begin(PassBegin{nullptr, nullptr, 0, acc, 1, (uint32_t*)slots, 2 * slot_words + 16}, s);
     launch_bbox(md, 1, n_points, n_tris, acc, s);
-    launch_classify(md, acc, par, tb, 1, n_tris, tn, cnt, s);
+    launch_classify(md, acc, par, tb, 1, n_tris, tn, slots, s);
+    launch_read_totals(slots, cnt, s);
     if (hipMemcpyAsync(tot, cnt, 32, hipMemcpyDeviceToHost, s) == hipSuccess &&
         hipStreamSynchronize(s) == hipSuccess)
       st = SVO_OK;

@@ -933,24 +933,24 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
   const uint64_t bm_words = bm_off[n];
 
   // small control buffers: the tables (mesh descriptors, tri bases, bitmap
-  // offsets), boxes, hit counters, and what is read back after the levels as
+  // offsets), boxes, counter slots, and what is read back after the levels as
   // one run of words: counters, level counts, spans, states, parameters
   const size_t sz_md = align256(sizeof(MeshDev) * n), sz_tb = align256(8 * (n + 1)),
                sz_bo = align256(8 * (n + 1)), sz_acc = align256(32 * n),
-               sz_hit = 8 * HIT_SLOTS * HIT_STRIDE;
+               sz_slots = 8 * COUNT_SLOTS * COUNT_STRIDE;
   const size_t rb_counts = 8 * 8, rb_spans = rb_counts + 8 * (NL + 2),
                rb_state = rb_spans + sizeof(LevelSpan) * n * NL,
                rb_par = rb_state + sizeof(MeshTreeState) * n,
                rb_bytes = rb_par + sizeof(MeshParams) * n;
   const size_t sz_tables = sz_md + sz_tb + sz_bo;
   char* ctl = nullptr;
-  SVO_TRY(W.get("ctl", sz_tables + sz_acc + sz_hit + rb_bytes, (void**)&ctl));
+  SVO_TRY(W.get("ctl", sz_tables + sz_acc + sz_slots + rb_bytes, (void**)&ctl));
   MeshDev* d_md = (MeshDev*)ctl;
   uint64_t* d_tb = (uint64_t*)(ctl + sz_md);
   uint64_t* d_bo = (uint64_t*)(ctl + sz_md + sz_tb);
   uint32_t* d_acc = (uint32_t*)(ctl + sz_tables);
-  unsigned long long* d_hits = (unsigned long long*)(ctl + sz_tables + sz_acc);
-  char* rb = ctl + sz_tables + sz_acc + sz_hit;
+  unsigned long long* d_slots = (unsigned long long*)(ctl + sz_tables + sz_acc);
+  char* rb = ctl + sz_tables + sz_acc + sz_slots;
   // d_cnt: [0] box cells, [1] big chunks, [2] keys emitted, [3] big queued,
   // [4] bitmap bytes zeroed by the level-1 pass
   unsigned long long* d_cnt = (unsigned long long*)rb;
@@ -972,21 +972,21 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
   }
   pb.acc = d_acc;
   pb.n_meshes = n;
-  pb.zero = (uint32_t*)d_hits;
-  pb.n_zero = (sz_hit + rb_par) / 4;
+  pb.zero = (uint32_t*)d_slots;
+  pb.n_zero = (sz_slots + rb_par) / 4;
   launch_begin(pb, s);
   timer.mark("start");
 
   // ---- A0: bbox, params, classification
   launch_bbox(d_md, n, max_points, max_tris, d_acc, s);
-  launch_classify(d_md, d_acc, d_par, d_tb, n, T, plan.tuning, d_cnt, s);
+  launch_classify(d_md, d_acc, d_par, d_tb, n, T, plan.tuning, d_slots, s);
   timer.mark("classify");
   uint64_t cells = 0, n_big = 0;
   if (capture) {
     cells = ((const uint64_t*)rec->a1.data())[0];
     n_big = ((const uint64_t*)rec->a1.data())[1];
   } else {
-    launch_copy_u32((uint32_t*)L.pinned, (const uint32_t*)d_cnt, 4, s);
+    launch_read_totals(d_slots, (unsigned long long*)L.pinned, s);
     HIP_TRY(hipStreamSynchronize(s));
     cells = ((uint64_t*)L.pinned)[0];
     n_big = ((uint64_t*)L.pinned)[1];
@@ -1100,11 +1100,11 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     launch_fill_u32((uint32_t*)line_flags, 0u, bm_bytes / BITMAP_LINE_BYTES / 4, s);
   }
   launch_voxelize<K>(d_md, d_par, d_tb, n, T, plan.cb, plan.tuning, keys_a, bitmap, d_bo, line_flags,
-                     d_cnt + 2, d_hits, big, d_cnt + 3, n_big, s);
+                     d_cnt + 2, d_slots, big, d_cnt + 3, n_big, s);
   timer.mark("voxelize");
   if (use_bm) {
     launch_level_first_bitmap<K>(bitmap, bm_words, d_bo, n, kl, lv[1], lv[2], d_counts, d_spans,
-                                 NL, d_state, bm_tmp, lvl_tmp, d_cnt + 4, d_hits, d_cnt + 2, line_flags,
+                                 NL, d_state, bm_tmp, lvl_tmp, d_cnt + 4, d_slots, d_cnt, line_flags,
                                  line_flags ? lv[4].elem_group : nullptr, s);
     W.clean_bytes("bitmap") = bm_clean_after;
   } else {

@@ -61,19 +61,21 @@ void launch_begin(const PassBegin& B, hipStream_t s);
 // not finite or an index out of range (8 x uint32 per mesh, launch_begin's acc).
 void launch_bbox(const MeshDev* meshes, uint32_t n_meshes, uint64_t max_points, uint64_t max_tris,
                  uint32_t* acc, hipStream_t s);
+// A pass's counters: COUNT_SLOTS slots of a cache line each, since atomics on
+// one address serialize; a total is the sum over the slots.
+constexpr uint32_t COUNT_SLOTS = 64, COUNT_STRIDE = 8;
+constexpr uint32_t COUNT_HITS = 0, COUNT_CELLS = 1, COUNT_CHUNKS = 2;
 // Grid parameters from the boxes (BaseModel.h:24-73, SVO.cu:342-351); candidate
-// cells and big-triangle chunk counts (2 x uint64 added to `totals`).
+// cells and big-triangle chunk counts, added to `slots`.
 void launch_classify(const MeshDev* meshes, const uint32_t* acc, MeshParams* params,
                      const uint64_t* tri_base, uint32_t n_meshes, uint64_t n_tris,
-                     const Tuning& tn, unsigned long long* totals, hipStream_t s);
-// Raw hits of the bitmap path are counted in HIT_SLOTS counters of a cache
-// line each (atomics on one address serialize); launch_level_first_bitmap
-// adds them up.
-constexpr uint32_t HIT_SLOTS = 64, HIT_STRIDE = 8;
+                     const Tuning& tn, unsigned long long* slots, hipStream_t s);
+// Candidate cells and chunks to out[0], out[1] (device or pinned host memory).
+void launch_read_totals(const unsigned long long* slots, unsigned long long* out, hipStream_t s);
 // Surface voxelization (SVO.cu:37-188): emits composite keys.
 // Hits go to `keys` (raw, for the sort; *key_count receives their number) when
 // `bitmap` is null, else into the occupancy bitmap (word bm_off[mesh] + code /
-// 32, bit code % 32, which the caller has zeroed; counted in `hits`).  With
+// 32, bit code % 32, which the caller has zeroed; counted in `slots`).  With
 // `line_flags`, byte k of it (zeroed as well) is set for each line of
 // BITMAP_LINE_BYTES bitmap bytes that receives a bit.
 constexpr uint64_t BITMAP_LINE_BYTES = 64;
@@ -81,7 +83,7 @@ template <typename K>
 void launch_voxelize(const MeshDev* meshes, const MeshParams* params, const uint64_t* tri_base,
                      uint32_t n_meshes, uint64_t n_tris, int cb, const Tuning& tn, K* keys,
                      uint32_t* bitmap, const uint64_t* bm_off, uint8_t* line_flags,
-                     unsigned long long* key_count, unsigned long long* hits, BigItem* big,
+                     unsigned long long* key_count, unsigned long long* slots, BigItem* big,
                      unsigned long long* big_count, uint64_t big_cap, hipStream_t s);
 
 // ------------------------------------------------------------ k_sort.hip
@@ -118,8 +120,8 @@ void launch_level_first(const K* sorted, const unsigned long long* n_sorted, uin
 // [bm_off[m], bm_off[m+1]), and every bm_off[m] is a multiple of
 // BITMAP_TILE_WORDS): the same outputs as launch_level_first followed
 // by launch_level_first_finalize, and the bitmap is left all zero (the bytes
-// that takes are added to *reset_bytes); *n_hits receives the sum of the
-// voxelization's hit counters `hits`.  With the flags of launch_voxelize (one
+// that takes are added to *reset_bytes); totals[0..2] receive the counters'
+// sums (candidate cells, chunks, raw hits).  With the flags of launch_voxelize (one
 // mesh, bm_off[0] = 0) only the flagged lines are read; `line_list` receives
 // their numbers.  `tmp` needs
 // bitmap_level_tmp_bytes(n_words); `lvl_tmp` (level_tmp_bytes of l1.cap) is
@@ -137,7 +139,7 @@ void launch_level_first_bitmap(uint32_t* bits, uint64_t n_words, const uint64_t*
                                LevelArrays l2, unsigned long long* counts, LevelSpan* spans1,
                                uint32_t n_levels, MeshTreeState* state, void* tmp,
                                void* lvl_tmp, unsigned long long* reset_bytes,
-                               const unsigned long long* hits, unsigned long long* n_hits,
+                               const unsigned long long* slots, unsigned long long* totals,
                                const uint8_t* line_flags, uint32_t* line_list, hipStream_t s);
 // Marks meshes whose level-1 set holds a single voxel as depth-1 trees (the
 // sort path; launch_level_first_bitmap does it itself).
