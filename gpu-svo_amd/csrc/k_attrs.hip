@@ -844,6 +844,43 @@ void launch_emit(const EmitArgs<K>& a, hipStream_t s) {
                        a.out);
 }
 
+// RING_BLOCKS workgroups take a part of each piece, in the pieces' order, so
+// that the first pieces arrive while the later ones are on their way.  Bound
+// by the link to the host.
+template <typename W>
+__device__ inline void copy_part(const char* src, char* dst, uint64_t bytes) {
+  constexpr int AHEAD = 4;
+  const uint64_t n = bytes / sizeof(W), step = (uint64_t)RING_BLOCKS * BLOCK;
+  for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < n; i += AHEAD * step) {
+    W w[AHEAD];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+      if (i + j * step < n) w[j] = ((const W*)src)[i + j * step];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+      if (i + j * step < n) ((W*)dst)[i + j * step] = w[j];
+  }
+  // the bytes behind the last whole word
+  if (blockIdx.x == 0 && threadIdx.x < bytes - n * sizeof(W))
+    dst[n * sizeof(W) + threadIdx.x] = src[n * sizeof(W) + threadIdx.x];
+}
+__global__ __launch_bounds__(BLOCK) void k_ring_copy(const char* src, uint64_t bytes, char* ring,
+                                                     uint32_t* flags, uint64_t slot,
+                                                     uint32_t number) {
+  for (uint64_t at = 0; at < bytes; at += RING_PIECE, slot = (slot + 1) % RING_SLOTS) {
+    const uint64_t k = bytes - at < RING_PIECE ? bytes - at : RING_PIECE;
+    char* dst = ring + slot * RING_PIECE;
+    if (((uintptr_t)src & 15) == 0) copy_part<uint4>(src + at, dst, k);
+    else if (((uintptr_t)src & 3) == 0) copy_part<uint32_t>(src + at, dst, k);
+    else copy_part<uint8_t>(src + at, dst, k);
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0)
+      __hip_atomic_store(flags + slot * RING_BLOCKS + blockIdx.x, number, __ATOMIC_RELEASE,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 __global__ void k_copy_u32(uint32_t* dst, const uint32_t* src, uint64_t n) {
   for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * blockDim.x)
@@ -867,6 +904,12 @@ void launch_check_equal(const void* got, const void* want, uint64_t bytes, uint3
   const uint64_t blocks = std::min<uint64_t>((n + BLOCK - 1) / BLOCK, 256);
   hipLaunchKernelGGL(k_check_equal, dim3((uint32_t)blocks), dim3(BLOCK), 0, s,
                      (const uint32_t*)got, (const uint32_t*)want, n, flag);
+}
+
+void launch_ring_copy(const void* src, uint64_t bytes, void* ring, uint32_t* flags, uint64_t slot,
+                      uint32_t number, hipStream_t s) {
+  hipLaunchKernelGGL(k_ring_copy, dim3(RING_BLOCKS), dim3(BLOCK), 0, s, (const char*)src, bytes,
+                     (char*)ring, flags, slot, number);
 }
 
 void launch_copy_u32(uint32_t* dst, const uint32_t* src, uint64_t n, hipStream_t s) {

@@ -162,6 +162,7 @@ Context::~Context() {
   hipSetDevice(device);
   if (aux_stream) hipStreamDestroy(aux_stream);
   aux_stream = nullptr;
+  if (ring.pinned) hipHostFree(ring.pinned);
 }
 
 // A batch's sub-batch pass g asks for lane g: the sub-batches of a batch

@@ -67,6 +67,16 @@ struct BatchOutput {
   int code_bytes = 4;
 };
 
+// Pinned ring that a read-out's pieces pass through (their flags behind it),
+// made by the context's first large read-out and freed with the context
+// (guarded by aux_mu).
+struct CopyRing {
+  static constexpr size_t PIECE = RING_PIECE, SLOTS = RING_SLOTS, THREADS = 3;
+  static constexpr size_t BYTES = SLOTS * (PIECE + 4 * RING_BLOCKS);
+  void* pinned = nullptr;
+  uint32_t launches = 0;
+};
+
 // The device state behind an svo_ctx.  Shared: the caller's handle, every
 // tree (through its output block) and every server hold a reference, so
 // trees stay readable after svo_ctx_destroy, which only gives the lanes
@@ -84,6 +94,7 @@ struct Context : std::enable_shared_from_this<Context> {
   std::vector<Lane*> free_lanes;
   hipStream_t aux_stream = nullptr;  // copies for read-out
   std::mutex aux_mu;
+  CopyRing ring;
   std::atomic<bool> timing{false};
   std::mutex stage_mu;
   std::vector<std::string> stage_names;

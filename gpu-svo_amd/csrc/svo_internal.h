@@ -230,6 +230,13 @@ struct EmitArgs {
 template <typename K>
 void launch_emit(const EmitArgs<K>& a, hipStream_t s);
 void launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s);
+// Copies `bytes` device bytes into a pinned ring of RING_SLOTS pieces from
+// slot `slot` on (at most the whole ring), piece after piece; the RING_BLOCKS
+// flags of a piece's slot become `number` when it has arrived.
+constexpr size_t RING_PIECE = 512 << 10, RING_SLOTS = 16;
+constexpr uint32_t RING_BLOCKS = 32;
+void launch_ring_copy(const void* src, uint64_t bytes, void* ring, uint32_t* flags, uint64_t slot,
+                      uint32_t number, hipStream_t s);
 // Copies n words; either side may be pinned host memory.  For a pass's tables
 // and readbacks of a few KB: 2 to 4 us, and less host time than asynchronous
 // copies (five of them read the levels back in 25 to 40 us).
