@@ -74,16 +74,28 @@ bool ensure_ring(Context& C) {
     R.pinned = nullptr;
     return false;
   }
-  std::memset((char*)R.pinned + CopyRing::SLOTS * CopyRing::PIECE, 0,
-              CopyRing::BYTES - CopyRing::SLOTS * CopyRing::PIECE);
+  std::memset(R.flags(), 0, CopyRing::BYTES - CopyRing::SLOTS * CopyRing::PIECE);
   return true;
+}
+
+// Waits until the kernel of launch `number` has set the flags of a slot.
+int wait_slot(Context& C, const uint32_t* flags, uint32_t number, uint32_t blocks = RING_BLOCKS) {
+  for (uint32_t b = 0, polls = 0; b < blocks;) {
+    if (__atomic_load_n(flags + b, __ATOMIC_ACQUIRE) == number) {
+      ++b;
+    } else if (++polls % 4096 == 0 && hipStreamQuery(C.aux_stream) != hipErrorNotReady &&
+               __atomic_load_n(flags + b, __ATOMIC_ACQUIRE) != number) {
+      return SVO_E_HIP;  // the stream has ended without it: a device error
+    }
+  }
+  return SVO_OK;
 }
 
 // Under C.aux_mu.
 int copy_staged(Context& C, char* dst, const char* src, size_t bytes) {
   CopyRing& R = C.ring;
   constexpr size_t PIECE = CopyRing::PIECE, SLOTS = CopyRing::SLOTS;
-  uint32_t* const flags = (uint32_t*)((char*)R.pinned + SLOTS * PIECE);
+  uint32_t* const flags = R.flags();
   const size_t n = (bytes + PIECE - 1) / PIECE;
   auto size_of = [&](size_t i) { return std::min(PIECE, bytes - i * PIECE); };
   std::atomic<size_t> arrived{0}, claimed{0};
@@ -133,17 +145,7 @@ int copy_staged(Context& C, char* dst, const char* src, size_t bytes) {
         for (; sent < end; ++sent) number[sent % SLOTS] = k;
       }
     }
-    const uint32_t* f = flags + i % SLOTS * RING_BLOCKS;
-    for (uint32_t b = 0, polls = 0; b < RING_BLOCKS && st == SVO_OK;) {
-      if (__atomic_load_n(f + b, __ATOMIC_ACQUIRE) == number[i % SLOTS]) {
-        ++b;
-      } else if (++polls % 4096 == 0) {
-        // the stream has ended without the piece: a device error
-        const hipError_t e = hipStreamQuery(C.aux_stream);
-        if (e != hipErrorNotReady && __atomic_load_n(f + b, __ATOMIC_ACQUIRE) != number[i % SLOTS])
-          st = SVO_E_HIP;
-      }
-    }
+    st = wait_slot(C, flags + i % SLOTS * RING_BLOCKS, number[i % SLOTS]);
     if (st != SVO_OK) break;
     arrived.store(i + 1, std::memory_order_release);
     if (helpers.empty()) take(i);
@@ -815,6 +817,31 @@ int svo_query_neighbors(const svo_tree* tree, const uint32_t* node, const uint8_
   if (!tree || (n && (!node || !slot || !out))) return SVO_E_INVALID;
   if (!n) return SVO_OK;
   Context& C = *tree->ctx;
+  // In the pinned ring: the kernel reads the lookups there and puts the answers
+  // there, with no copy and no synchronization (1000 lookups: 33 us with three
+  // copies, 19 so; 50,000: 54 and 45; 200,000: the same, 103 us).
+  constexpr uint64_t RING_LOOKUPS = 1 << 17;
+  static_assert(9 * RING_LOOKUPS <= CopyRing::SLOTS * CopyRing::PIECE, "they fit the ring");
+  if (n <= RING_LOOKUPS) {
+    std::lock_guard<std::mutex> lk(C.aux_mu);
+    hipSetDevice(C.device);
+    if (ensure_ring(C)) {
+      CopyRing& R = C.ring;
+      uint32_t* r_node = (uint32_t*)R.pinned;
+      uint32_t* r_out = r_node + n;
+      uint8_t* r_slot = (uint8_t*)(r_out + n);
+      std::memcpy(r_node, node, 4 * n);
+      std::memcpy(r_slot, slot, n);
+      const uint32_t number = ++R.launches;
+      const uint32_t blocks =
+          launch_query_ring(tree->out->nodes.neighbors + 27 * tree->node_base, tree->info.n_nodes,
+                            r_node, r_slot, n, r_out, R.flags(), number, C.aux_stream);
+      if (hipGetLastError() != hipSuccess) return SVO_E_HIP;
+      const int st = wait_slot(C, R.flags(), number, blocks);
+      if (st == SVO_OK) std::memcpy(out, r_out, 4 * n);
+      return st;
+    }
+  }
   const size_t bytes = 4 * n + 4 * n + n + 512;
   void* tmp = nullptr;
   int st = C.dev_malloc(&tmp, bytes);

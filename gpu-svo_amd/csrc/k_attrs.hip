@@ -823,6 +823,37 @@ __global__ void k_query(const uint32_t* nb, uint64_t n_nodes, const uint32_t* no
   out[i] = (t < n_nodes && s < 27) ? nb[27 * (uint64_t)t + s] : NONE;
 }
 
+// At most RING_BLOCKS workgroups; bound by the two trips over the link to the host.
+constexpr int QUERY_THREADS = 1024;
+__global__ __launch_bounds__(QUERY_THREADS) void k_query_ring(const uint32_t* nb, uint64_t n_nodes,
+                                                              const uint32_t* node,
+                                                              const uint8_t* slot, uint64_t n,
+                                                              uint32_t* out, uint32_t* flags,
+                                                              uint32_t number) {
+  constexpr int AHEAD = 4;
+  const uint64_t step = (uint64_t)gridDim.x * QUERY_THREADS;
+  for (uint64_t i = (uint64_t)blockIdx.x * QUERY_THREADS + threadIdx.x; i < n; i += AHEAD * step) {
+    uint32_t t[AHEAD], v[AHEAD];
+    uint8_t s[AHEAD];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) {
+      const bool in = i + j * step < n;
+      t[j] = in ? node[i + j * step] : NONE;
+      s[j] = in ? slot[i + j * step] : 27;
+    }
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+      v[j] = t[j] < n_nodes && s[j] < 27 ? nb[27 * (uint64_t)t[j] + s[j]] : NONE;
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+      if (i + j * step < n) out[i + j * step] = v[j];
+  }
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(flags + blockIdx.x, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 inline uint32_t grid_for(uint64_t threads) { return (uint32_t)((threads + BLOCK - 1) / BLOCK); }
 
 }  // namespace
@@ -984,6 +1015,16 @@ void launch_query_neighbors(const uint32_t* neighbors, uint64_t n_nodes, const u
   if (n == 0) return;
   hipLaunchKernelGGL(k_query, dim3(grid_for(n)), dim3(BLOCK), 0, s, neighbors, n_nodes, node,
                      slot, n, out);
+}
+
+uint32_t launch_query_ring(const uint32_t* neighbors, uint64_t n_nodes, const uint32_t* node,
+                           const uint8_t* slot, uint64_t n, uint32_t* out, uint32_t* flags,
+                           uint32_t number, hipStream_t s) {
+  const uint32_t blocks =
+      (uint32_t)std::min<uint64_t>((n + QUERY_THREADS - 1) / QUERY_THREADS, RING_BLOCKS);
+  hipLaunchKernelGGL(k_query_ring, dim3(blocks), dim3(QUERY_THREADS), 0, s, neighbors, n_nodes,
+                     node, slot, n, out, flags, number);
+  return blocks;
 }
 
 template void launch_emit<uint32_t>(const EmitArgs<uint32_t>&, hipStream_t);

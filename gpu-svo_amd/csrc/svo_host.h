@@ -67,14 +67,15 @@ struct BatchOutput {
   int code_bytes = 4;
 };
 
-// Pinned ring that a read-out's pieces pass through (their flags behind it),
-// made by the context's first large read-out and freed with the context
-// (guarded by aux_mu).
+// Pinned ring that a read-out's pieces and the lookups' arrays pass through
+// (their flags behind it), made by the context's first large read-out or
+// lookup and freed with the context (guarded by aux_mu).
 struct CopyRing {
   static constexpr size_t PIECE = RING_PIECE, SLOTS = RING_SLOTS, THREADS = 3;
   static constexpr size_t BYTES = SLOTS * (PIECE + 4 * RING_BLOCKS);
   void* pinned = nullptr;
   uint32_t launches = 0;
+  uint32_t* flags() const { return (uint32_t*)((char*)pinned + SLOTS * PIECE); }
 };
 
 // The device state behind an svo_ctx.  Shared: the caller's handle, every

@@ -274,6 +274,11 @@ void launch_ref_records(const float* origin, const float* width, uint64_t n_node
 // 168-byte SVONode records for nodes [first, first + n) (32-bit codes).
 void launch_pack_aos(const NodeArrays& nodes, uint64_t first, uint64_t n, void* dst,
                      hipStream_t s);
+// The same with node, slot and out in pinned host memory; the first flags, as
+// many as returned, become `number` when the answers are there.
+uint32_t launch_query_ring(const uint32_t* neighbors, uint64_t n_nodes, const uint32_t* node,
+                           const uint8_t* slot, uint64_t n, uint32_t* out, uint32_t* flags,
+                           uint32_t number, hipStream_t s);
 void launch_query_neighbors(const uint32_t* neighbors, uint64_t n_nodes, const uint32_t* node,
                             const uint8_t* slot, uint64_t n, uint32_t* out, hipStream_t s);
 
