@@ -26,6 +26,7 @@
 // index.  A word per node says which it keeps; count -> scan -> write,
 // node-major.
 #include <algorithm>
+#include <type_traits>
 
 #include "svo_internal.h"
 #include "svo_scan.h"
@@ -103,21 +104,29 @@ __device__ inline bool edge_eq(const float* a0, const float* b0, const float* a1
 }
 
 // Writes words [w0, w0 + n) of dst, value(i) the word w0 + i: 16-byte pieces,
-// single words where a piece lies across either end.  dst is 16-byte aligned.
-template <typename F>
+// single words where a piece lies across either end; four(i) gives the words
+// i .. i + 3 at once.  dst is 16-byte aligned.
+template <typename F, typename F4>
 __device__ inline void write_words(uint32_t* dst, uint64_t w0, uint32_t n, uint32_t tid,
-                                   uint32_t threads, F value) {
+                                   uint32_t threads, F value, F4 four) {
   const uint32_t head = (uint32_t)w0 & 3u;  // words of the first piece before w0
   uint32_t* p = dst + (w0 - head);
   for (uint32_t q = tid; 4 * q < head + n; q += threads) {
     const uint32_t i = 4 * q - head;  // wraps for words before w0
     if (4 * q >= head && i + 4 <= n) {
-      store_stream((uint4*)p + q, make_uint4(value(i), value(i + 1), value(i + 2), value(i + 3)));
+      store_stream((uint4*)p + q, four(i));
     } else {
       for (uint32_t j = 0; j < 4; ++j)
         if (i + j < n) p[4 * (uint64_t)q + j] = value(i + j);
     }
   }
+}
+template <typename F>
+__device__ inline void write_words(uint32_t* dst, uint64_t w0, uint32_t n, uint32_t tid,
+                                   uint32_t threads, F value) {
+  write_words(dst, w0, n, tid, threads, value, [&](uint32_t i) {
+    return make_uint4(value(i), value(i + 1), value(i + 2), value(i + 3));
+  });
 }
 
 // ---------------------------------------------------------------- emission
@@ -691,52 +700,55 @@ __global__ __launch_bounds__(KEEP_SCAN) void k_keep_scan(const uint32_t* counts,
   if (threadIdx.x < 3) totals[threadIdx.x] = carry[threadIdx.x];
 }
 
-// Words of the records in the LDS slots of a node's values (REC_VALS per node;
-// slots 10 and 11 hold width and width * 0).
+// The LDS slot (of a node's REC_VALS values; 10 and 11 hold width and width *
+// 0) of each word of a record, four bits a word.
 struct WordTable {
-  uint8_t edge[84], face[42], vert[32], ref_vert[32];
+  uint32_t edge[12], face[6], vert[8], ref_vert[8];
 };
 constexpr WordTable make_word_table() {
   WordTable t{};
   auto slot = [](const uint8_t(&e)[3], int a) {
-    return (uint8_t)(!e[0] && !e[1] && !e[2] ? a : e[a] ? 6 + a : 3 + a);
+    return (uint32_t)(!e[0] && !e[1] && !e[2] ? a : e[a] ? 6 + a : 3 + a);
   };
   for (int w = 0; w < 84; ++w)
-    t.edge[w] = w % 7 == 6 ? 9 : slot(EDGE_ENDS[w / 7][w % 7 / 3], w % 7 % 3);
+    t.edge[w / 7] |= (w % 7 == 6 ? 9u : slot(EDGE_ENDS[w / 7][w % 7 / 3], w % 7 % 3)) << 4 * (w % 7);
   for (int w = 0; w < 42; ++w)
-    t.face[w] = w % 7 == 6 ? 9 : slot(FACE_ENDS[w / 7][w % 7 / 3], w % 7 % 3);
+    t.face[w / 7] |= (w % 7 == 6 ? 9u : slot(FACE_ENDS[w / 7][w % 7 / 3], w % 7 % 3)) << 4 * (w % 7);
   for (int j = 0; j < 8; ++j) {
     const uint8_t corner[3] = {(uint8_t)(j & 1), (uint8_t)(j >> 1 & 1), (uint8_t)(j >> 2 & 1)};
     for (int a = 0; a < 3; ++a) {
-      t.vert[4 * j + a] = slot(corner, a);
-      t.ref_vert[4 * j + a] = corner[a] ? 10 : 11;
+      t.vert[j] |= slot(corner, a) << 4 * a;
+      t.ref_vert[j] |= (corner[a] ? 10u : 11u) << 4 * a;
     }
-    t.vert[4 * j + 3] = t.ref_vert[4 * j + 3] = 9;
+    t.vert[j] |= 9u << 12;
+    t.ref_vert[j] |= 9u << 12;
   }
   return t;
 }
 __constant__ WordTable WORDS = make_word_table();
 
-// Writes the kept records of a block of nodes: the nodes' values and the list
-// of kept records (node and record, in order) are staged in LDS, then every
-// record array's run of words is written in 16-byte pieces, each word looked
-// up from its record.  (A thread per node that wrote its own records scattered
+// Writes the kept records of a block of nodes: the nodes' values (from the
+// level's keys, as in the emission) and the list of kept records (node and
+// record, in order) are staged in LDS; then a thread looks up a record's
+// words, and the array's run of words is written in 16-byte pieces from LDS.  (A thread per node that wrote its own records scattered
 // 16- and 28-byte stores, after deciding twice from its neighbor row which they
-// are: 1,240 us on 3.3 M nodes and 300 for the count; 188 and 5 now.)
+// are: 1,240 us on 3.3 M nodes and 300 for the count.  Now 173 and 5, 792 MB; a word at a time from the list it
+// was 190, bound by its instructions.)
+template <typename K>
 __global__ __launch_bounds__(KEEP_BLOCK) void k_keep_write(
-    bool reference, NodeArrays nodes, uint64_t n_nodes, const NodeSeg* segs,
+    bool reference, KeyLayout<K> kl, NodeArrays nodes, uint64_t n_nodes, const NodeSeg* segs,
     const uint32_t* seg_first, uint32_t n_segs, const uint32_t* keep, const uint64_t* offsets,
     AttrOut out) {
   if (nodes.skip && *nodes.skip) return;  // graph replay over changed sizes
   __shared__ uint32_t s_val[KEEP_BLOCK * REC_VALS];
+  __shared__ __align__(16) uint32_t s_stage[7 * KEEP_BLOCK + 4];
   __shared__ uint16_t s_list[KEEP_BLOCK * 12];
-  __shared__ uint8_t s_word[84 + 42 + 32];
+  __shared__ uint32_t s_word[12 + 6 + 8];
   __shared__ uint32_t s_sum[2][KEEP_BLOCK / 64];
   const uint32_t tid = threadIdx.x, t = blockIdx.x * KEEP_BLOCK + tid;
-  if (tid < 84) s_word[tid] = WORDS.edge[tid];
-  else if (tid < 84 + 42) s_word[tid] = WORDS.face[tid - 84];
-  else if (tid < 84 + 42 + 32)
-    s_word[tid] = reference ? WORDS.ref_vert[tid - 126] : WORDS.vert[tid - 126];
+  if (tid < 12) s_word[tid] = WORDS.edge[tid];
+  else if (tid < 18) s_word[tid] = WORDS.face[tid - 12];
+  else if (tid < 26) s_word[tid] = reference ? WORDS.ref_vert[tid - 18] : WORDS.vert[tid - 18];
   const uint32_t k = t < n_nodes ? keep[t] : 0u;
   uint32_t nv, ne, nf;
   keep_counts(k, nv, ne, nf);
@@ -764,14 +776,19 @@ __global__ __launch_bounds__(KEEP_BLOCK) void k_keep_write(
                  of = offsets[3 * (uint64_t)blockIdx.x + 2];
   if ((t & ~63u) < n_nodes)
     for_segments(segs, seg_first, n_segs, t & ~63u, t, t < n_nodes, [&](auto* sg, uint32_t d) {
+      // origin and width from the level's keys, as emit_nodes has them
       const uint32_t local = sg->local0 + d;
-      const NodeGeom g = load_geom(nodes, t);
+      const float w = sg->width;
+      const K* elem = (const K*)sg->elem;
+      const K code = sg->level_kind & SEG_ROOT ? kl.code(elem[0])
+                                               : (K)((kl.code(elem[d >> 3]) << 3) | (K)(d & 7));
       uint32_t* v = s_val + REC_VALS * tid;
 #pragma unroll
-      for (uint32_t x = 0; x < 3; ++x) stage_axis(v, x, g.o[x], g.w);
+      for (uint32_t x = 0; x < 3; ++x)
+        stage_axis(v, x, sg->origin[x] + w * (float)axis_of(code, x), w);
       v[9] = local;
-      v[10] = __float_as_uint(g.w * 1.0f);
-      v[11] = __float_as_uint(g.w * 0.0f);
+      v[10] = __float_as_uint(w * 1.0f);
+      v[11] = __float_as_uint(w * 0.0f);
       if (local == 0) {
         unsigned long long* first = out.totals + 4 + 3 * sg->mesh;
         first[0] = ov + (a & 0xFFFFu);
@@ -780,19 +797,40 @@ __global__ __launch_bounds__(KEEP_BLOCK) void k_keep_write(
       }
     });
   // kind by kind through one list: `bits` the node's records, `at` its place
-  auto records = [&](uint32_t bits, uint32_t at, uint32_t count, uint32_t words,
-                     const uint8_t* word, uint32_t* dst, uint64_t first) {
+  auto list = [&](uint32_t bits, uint32_t at) {
     for (; bits; bits &= bits - 1u) s_list[at++] = (uint16_t)((tid << 4) | __builtin_ctz(bits));
     __syncthreads();
-    write_words(dst, first * words, count * words, tid, KEEP_BLOCK, [&](uint32_t i) {
-      const uint32_t r = i / words, e = s_list[r];
-      return s_val[REC_VALS * (e >> 4) + word[words * (e & 15u) + (i - r * words)]];
-    });
-    __syncthreads();
   };
-  records(k & 0xFFu, a & 0xFFFFu, ta & 0xFFFFu, 4u, s_word + 126, (uint32_t*)out.verts, ov);
-  records((k >> KEEP_EDGES) & 0xFFFu, a >> 16, ta >> 16, 7u, s_word, (uint32_t*)out.edges, oe);
-  if (!reference) records(k >> KEEP_FACES, b, tb, 7u, s_word + 84, (uint32_t*)out.faces, of);
+  // a vertex is a piece
+  list(k & 0xFFu, a & 0xFFFFu);
+  for (uint32_t r = tid; r < (ta & 0xFFFFu); r += KEEP_BLOCK) {
+    const uint32_t e = s_list[r], w = s_word[18 + (e & 15u)], *v = s_val + REC_VALS * (e >> 4);
+    store_stream((uint4*)out.verts + ov + r,
+                 make_uint4(v[w & 15u], v[w >> 4 & 15u], v[w >> 8 & 15u], v[w >> 12]));
+  }
+  __syncthreads();
+  // edges and faces, KEEP_BLOCK at a time
+  auto records = [&](uint32_t bits, uint32_t at, uint32_t count, const uint32_t* word,
+                     uint32_t* dst, uint64_t first) {
+    list(bits, at);
+    for (uint32_t c = 0; c < count; c += KEEP_BLOCK) {
+      const uint32_t n = count - c < KEEP_BLOCK ? count - c : KEEP_BLOCK;
+      const uint64_t w0 = 7 * (first + c);
+      uint32_t* stage = s_stage + (w0 & 3u);
+      if (tid < n) {
+        const uint32_t e = s_list[c + tid], w = word[e & 15u], *v = s_val + REC_VALS * (e >> 4);
+#pragma unroll
+        for (uint32_t j = 0; j < 7; ++j) stage[7 * tid + j] = v[w >> 4 * j & 15u];
+      }
+      __syncthreads();
+      write_words(
+          dst, w0, 7 * n, tid, KEEP_BLOCK, [&](uint32_t i) { return stage[i]; },
+          [&](uint32_t i) { return *(const uint4*)(stage + i); });
+      __syncthreads();
+    }
+  };
+  records((k >> KEEP_EDGES) & 0xFFFu, a >> 16, ta >> 16, s_word, (uint32_t*)out.edges, oe);
+  if (!reference) records(k >> KEEP_FACES, b, tb, s_word + 12, (uint32_t*)out.faces, of);
 }
 
 // 168-byte SVONode records (SVO.h:20-35), one thread per 32-bit word.
@@ -973,7 +1011,8 @@ size_t keep_bytes(uint64_t n_nodes) {
   return (size_t)(4 * KEEP_BLOCK + 16 + 24) * keep_blocks(n_nodes);
 }
 
-void launch_kept_records(int semantics, const NodeArrays& nodes, uint64_t n_nodes,
+template <typename K>
+void launch_kept_records(int semantics, KeyLayout<K> kl, const NodeArrays& nodes, uint64_t n_nodes,
                          const NodeSeg* segs, const uint32_t* seg_first, uint32_t n_segs,
                          void* tmp, AttrOut out, hipStream_t s) {
   const uint32_t nb = (uint32_t)keep_blocks(n_nodes);
@@ -988,7 +1027,7 @@ void launch_kept_records(int semantics, const NodeArrays& nodes, uint64_t n_node
                      n_nodes, counts, nodes.skip);
   hipLaunchKernelGGL(k_keep_scan, dim3(1), dim3(KEEP_SCAN), 0, s, (const uint32_t*)counts, nb,
                      offsets, out.totals, nodes.skip);
-  hipLaunchKernelGGL(k_keep_write, dim3(nb), dim3(KEEP_BLOCK), 0, s, reference, nodes, n_nodes,
+  hipLaunchKernelGGL(k_keep_write<K>, dim3(nb), dim3(KEEP_BLOCK), 0, s, reference, kl, nodes, n_nodes,
                      segs, seg_first, n_segs, (const uint32_t*)keep, (const uint64_t*)offsets,
                      out);
 }
@@ -1027,6 +1066,12 @@ uint32_t launch_query_ring(const uint32_t* neighbors, uint64_t n_nodes, const ui
   return blocks;
 }
 
+template void launch_kept_records<uint32_t>(int, KeyLayout<uint32_t>, const NodeArrays&, uint64_t,
+                                            const NodeSeg*, const uint32_t*, uint32_t, void*,
+                                            AttrOut, hipStream_t);
+template void launch_kept_records<uint64_t>(int, KeyLayout<uint64_t>, const NodeArrays&, uint64_t,
+                                            const NodeSeg*, const uint32_t*, uint32_t, void*,
+                                            AttrOut, hipStream_t);
 template void launch_emit<uint32_t>(const EmitArgs<uint32_t>&, hipStream_t);
 template void launch_emit<uint64_t>(const EmitArgs<uint64_t>&, hipStream_t);
 

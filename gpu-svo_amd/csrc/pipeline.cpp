@@ -1320,7 +1320,8 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
     std::memcpy(up + sz_segs, seg_first.data(), 4 * n_segs);
     std::memcpy(up + sz_segs + sz_sf, level_segs.data(), 4 * level_segs.size());
     std::memcpy(up + sz_segs + 2 * sz_sf, level_blocks.data(), 4 * level_blocks.size());
-    launch_copy_u32((uint32_t*)bctl, (const uint32_t*)up, sz_up / 4, s);
+    std::memset(up + sz_up, 0, sz_tot);
+    launch_copy_u32((uint32_t*)bctl, (const uint32_t*)up, (sz_up + sz_tot) / 4, s);
   }
   timer.mark("setup_b");
   // Reference records stand at the identity offsets when no record can equal
@@ -1357,9 +1358,9 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
   }
   std::vector<uint64_t> tot(4 + 3 * (size_t)n, 0);
   if (counted) {
-    launch_fill_u32((uint32_t*)d_tot, 0u, sz_tot / 4, s);
+    if (capture) launch_fill_u32((uint32_t*)d_tot, 0u, sz_tot / 4, s);  // (uploaded otherwise)
     AttrOut ao{out->verts, out->edges, out->faces, d_tot};
-    launch_kept_records(sem, na, N, d_segs, d_seg_first, n_segs, keep, ao, s);
+    launch_kept_records<K>(sem, kl, na, N, d_segs, d_seg_first, n_segs, keep, ao, s);
     timer.mark("attr_write");
   } else if (identity) {
     tot[0] = 8 * N;

@@ -264,7 +264,8 @@ struct AttrOut {
 // `tmp` holds keep_bytes(n_nodes) bytes and begins with the nodes' keep masks
 // (written by launch_neighbors_level; by this call, reference semantics).
 size_t keep_bytes(uint64_t n_nodes);
-void launch_kept_records(int semantics, const NodeArrays& nodes, uint64_t n_nodes,
+template <typename K>
+void launch_kept_records(int semantics, KeyLayout<K> kl, const NodeArrays& nodes, uint64_t n_nodes,
                          const NodeSeg* segs, const uint32_t* seg_first, uint32_t n_segs,
                          void* tmp, AttrOut out, hipStream_t s);
 // The reference's vertex and edge records of given nodes (origin 3 floats and
