@@ -730,10 +730,11 @@ __constant__ WordTable WORDS = make_word_table();
 // Writes the kept records of a block of nodes: the nodes' values (from the
 // level's keys, as in the emission) and the list of kept records (node and
 // record, in order) are staged in LDS; then a thread looks up a record's
-// words, and the array's run of words is written in 16-byte pieces from LDS.  (A thread per node that wrote its own records scattered
-// 16- and 28-byte stores, after deciding twice from its neighbor row which they
-// are: 1,240 us on 3.3 M nodes and 300 for the count.  Now 173 and 5, 792 MB; a word at a time from the list it
-// was 190, bound by its instructions.)
+// words, and the array's run of words is written in 16-byte pieces from LDS.
+// 173 us on 3.3 M nodes, 792 MB, and 5 for the count.  (A word at a time from
+// the list: 190, bound by its instructions.  A thread per node that wrote its
+// own records scattered 16- and 28-byte stores, after deciding twice from its
+// neighbor row which they are: 1,240 and 300 for the count.)
 template <typename K>
 __global__ __launch_bounds__(KEEP_BLOCK) void k_keep_write(
     bool reference, KeyLayout<K> kl, NodeArrays nodes, uint64_t n_nodes, const NodeSeg* segs,

@@ -413,6 +413,20 @@ __global__ __launch_bounds__(BLOCK) void k_bm_count(const uint32_t* bits, uint64
   }
 }
 
+// The counter slots' sums, by one wave.
+__device__ inline void sum_counters(const unsigned long long* slots, unsigned long long* totals) {
+  static_assert(COUNT_SLOTS == 64, "a lane per slot");
+  const unsigned long long* slot = slots + threadIdx.x * COUNT_STRIDE;
+  const uint64_t c = wave_sum((uint64_t)slot[COUNT_CELLS]);
+  const uint64_t k = wave_sum((uint64_t)slot[COUNT_CHUNKS]);
+  const uint64_t h = wave_sum((uint64_t)slot[COUNT_HITS]);
+  if (threadIdx.x == 0) {
+    totals[0] = c;
+    totals[1] = k;
+    totals[2] = h;
+  }
+}
+
 // Exclusive scan of the tile counts in place, SC_CHUNK tiles per workgroup, chunk
 // offsets by decoupled look-back (chunks claimed by ticket); totals to
 // counts[0] (unique keys = level-1 elements) and counts[1] (groups = level-2
@@ -426,18 +440,7 @@ __global__ __launch_bounds__(BLOCK) void k_bm_scan(uint32_t* tile_u, uint32_t* t
                                                    unsigned long long* totals) {
   __shared__ uint64_t tmp[4];
   __shared__ uint32_t s_chunk, s_base[2], s_reset[BLOCK / 64];
-  static_assert(COUNT_SLOTS == 64, "a wave adds up the counters");
-  if (blockIdx.x == 0 && threadIdx.x < 64) {
-    const unsigned long long* slot = slots + threadIdx.x * COUNT_STRIDE;
-    const uint64_t c = wave_sum((uint64_t)slot[COUNT_CELLS]);
-    const uint64_t k = wave_sum((uint64_t)slot[COUNT_CHUNKS]);
-    const uint64_t h = wave_sum((uint64_t)slot[COUNT_HITS]);
-    if (threadIdx.x == 0) {
-      totals[0] = c;
-      totals[1] = k;
-      totals[2] = h;
-    }
-  }
+  if (blockIdx.x == 0 && threadIdx.x < 64) sum_counters(slots, totals);
   if (L.line) {  // flagged lines only: the later workgroups have no chunk
     tiles = (uint32_t)line_tiles(L);
     if ((uint64_t)blockIdx.x * SC_CHUNK >= tiles) return;
@@ -522,9 +525,17 @@ static_assert((EMIT_CAP & (EMIT_CAP - 1)) == 0, "the copy-out masks slot indices
 static_assert(BM_TILE % BLOCK == 0, "a round's words lie inside the tile's LDS arrays");
 static_assert(BM_TILE == BITMAP_TILE_WORDS, "mesh regions start on tile boundaries");
 
-template <typename K, bool LINES>
+struct BmSums {  // SUMS: what k_bm_scan does otherwise
+  const uint32_t* tile_r;
+  unsigned long long *counts, *reset_bytes, *totals;
+  const unsigned long long* slots;
+};
+// SUMS: up to SUM_TILES tiles a workgroup adds up the tile counts before its
+// own itself, 8 loads a thread, which saves the scan's launch (5 us).
+constexpr uint64_t SUM_TILES = 2048;
+template <typename K, bool LINES, bool SUMS>
 __global__ __launch_bounds__(BLOCK) void k_bm_emit(uint32_t* bits, uint64_t n_words, LineList L,
-                                                   const uint64_t* bm_off, uint32_t n_meshes,
+                                                   BmSums sums, const uint64_t* bm_off, uint32_t n_meshes,
                                                    KeyLayout<K> kl, const uint32_t* tile_u,
                                                    const uint32_t* tile_g, K* elem1, K* elem2,
                                                    uint32_t* first_child2, uint8_t* kids2,
@@ -538,10 +549,79 @@ __global__ __launch_bounds__(BLOCK) void k_bm_emit(uint32_t* bits, uint64_t n_wo
   __shared__ K s_kbase;  // key of the tile's bit 0
   __shared__ uint32_t s_line[LINES ? TILE_LINES : 1];
   const uint32_t l0 = threadIdx.x * BM_WPT;
+  // the bitmap words and the tile's output offsets are loaded first, so that
+  // the mesh lookup's dependent loads run while they are in flight
+  uint32_t w[BM_WPT];
+  uint64_t w0 = 0;
+  if (!LINES) {
+    w0 = tile_words<LINES>(L, blockIdx.x, n_words, s_line);
+    load_words(bits, n_words, w0, w);
+  }
+  // SUMS: set bits and nonzero bytes before this tile, before the tile that
+  // follows its mesh, and in all
+  enum { BEFORE, MESH_END, ALL };
+  __shared__ uint32_t s_sum[3][2][BLOCK / 64], s_reset[BLOCK / 64];
+  uint32_t sum_u[3], sum_g[3], first_mesh = 0;
+  uint64_t mesh_off = 0;
+  if (SUMS) {
+    const uint64_t tw0 = (uint64_t)blockIdx.x * BM_TILE;
+    first_mesh = mesh_of_word(bm_off, n_meshes, tw0);
+    mesh_off = bm_off[first_mesh];
+    const uint64_t limit[3] = {blockIdx.x, bm_off[first_mesh + 1] / BM_TILE, gridDim.x};
+    uint32_t u[SUM_TILES / BLOCK], g[SUM_TILES / BLOCK], r = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < SUM_TILES / BLOCK; ++j) {
+      const uint32_t i = j * BLOCK + threadIdx.x;
+      u[j] = i < gridDim.x ? tile_u[i] : 0u;
+      g[j] = i < gridDim.x ? tile_g[i] : 0u;
+      if (blockIdx.x == 0 && i < gridDim.x) r += sums.tile_r[i];
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      uint32_t a = 0, b = 0;
+#pragma unroll
+      for (uint32_t j = 0; j < SUM_TILES / BLOCK; ++j) {
+        const bool in = j * BLOCK + threadIdx.x < limit[k];
+        a += in ? u[j] : 0u;
+        b += in ? g[j] : 0u;
+      }
+      a = wave_sum_u32(a);
+      b = wave_sum_u32(b);
+      if (__lane_id() == 0) {
+        s_sum[k][0][threadIdx.x >> 6] = a;
+        s_sum[k][1][threadIdx.x >> 6] = b;
+      }
+    }
+    if (blockIdx.x == 0) {
+      r = wave_sum_u32(r);
+      if (__lane_id() == 0) s_reset[threadIdx.x >> 6] = r;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      sum_u[k] = sum_g[k] = 0;
+#pragma unroll
+      for (int w = 0; w < BLOCK / 64; ++w) {
+        sum_u[k] += s_sum[k][0][w];
+        sum_g[k] += s_sum[k][1][w];
+      }
+    }
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+      sum_counters(sums.slots, sums.totals);
+      if (threadIdx.x == 0) {
+        sums.counts[0] = sum_u[ALL];
+        sums.counts[1] = sum_g[ALL];
+        uint64_t t = 0;
+        for (int w = 0; w < BLOCK / 64; ++w) t += s_reset[w];
+        *sums.reset_bytes += 4 * t;
+      }
+    }
+  }
+  const uint64_t n_unique = SUMS ? sum_u[ALL] : counts[0];
   {
     // the later levels' look-back words and tickets start at zero (as
     // k_level_clear leaves them), a slice per workgroup
-    const uint64_t words = 2 * level_tiles(counts[0]);
+    const uint64_t words = 2 * level_tiles(n_unique);
     const uint64_t per = (words + gridDim.x - 1) / gridDim.x;
     const uint64_t i1 = std::min<uint64_t>(words, (uint64_t)(blockIdx.x + 1) * per);
     for (uint64_t i = (uint64_t)blockIdx.x * per + threadIdx.x; i < i1; i += BLOCK) status[i] = 0;
@@ -559,16 +639,16 @@ __global__ __launch_bounds__(BLOCK) void k_bm_emit(uint32_t* bits, uint64_t n_wo
   }
   const uint64_t tiles = LINES ? line_tiles(L) : gridDim.x;
   for (uint64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-    // the bitmap words and the tile's output offsets are loaded first, so that
-    // the mesh lookup's dependent loads run while they are in flight
-    uint32_t w[BM_WPT];
-    const uint64_t w0 = tile_words<LINES>(L, tile, n_words, s_line);
-    load_words(bits, n_words, w0, w);
-    const uint32_t bu = tile_u[tile], bg = tile_g[tile];
+    if (LINES) {
+      w0 = tile_words<LINES>(L, tile, n_words, s_line);
+      load_words(bits, n_words, w0, w);
+    }
+    const uint32_t bu = SUMS ? sum_u[BEFORE] : tile_u[tile],
+                   bg = SUMS ? sum_g[BEFORE] : tile_g[tile];
     if (!LINES && threadIdx.x == 0) {
       const uint64_t tw0 = tile * BM_TILE;
-      const uint32_t m = mesh_of_word(bm_off, n_meshes, tw0);
-      const uint64_t off = bm_off[m];
+      const uint32_t m = SUMS ? first_mesh : mesh_of_word(bm_off, n_meshes, tw0);
+      const uint64_t off = SUMS ? mesh_off : bm_off[m];
       s_kbase = ((K)m << kl.cb) | ((K)(tw0 - off) << 5);
       if (tw0 == off) {
         // the mesh's first tile: its level-1 span ends where the next mesh's
@@ -576,8 +656,12 @@ __global__ __launch_bounds__(BLOCK) void k_bm_emit(uint32_t* bits, uint64_t n_wo
         // level 1 holds a single voxel, its depth-1 root (what
         // k_first_finalize does on the sort path)
         const uint64_t tn = bm_off[m + 1] / BM_TILE;
-        const uint32_t ue = tn < gridDim.x ? tile_u[tn] : (uint32_t)counts[0];
-        const uint32_t ge = tn < gridDim.x ? tile_g[tn] : (uint32_t)counts[1];
+        const uint32_t ue = SUMS                ? sum_u[MESH_END]
+                            : tn < gridDim.x ? tile_u[tn]
+                                             : (uint32_t)counts[0];
+        const uint32_t ge = SUMS                ? sum_g[MESH_END]
+                            : tn < gridDim.x ? tile_g[tn]
+                                             : (uint32_t)counts[1];
         LevelSpan& sp = spans[(uint64_t)m * n_levels];
         sp.elem_first = bu;
         sp.elem_end = ue;
@@ -1078,23 +1162,26 @@ void launch_level_first_bitmap(uint32_t* bits, uint64_t n_words, const uint64_t*
   const uint32_t n_status = (uint32_t)(2 + 2 * chunks);
   uint32_t* tickets = (uint32_t*)lvl_tmp;
   uint64_t* status = (uint64_t*)((char*)lvl_tmp + 256);
-  auto run = [&](auto lines, const LineList& L, uint32_t grid) {
-    constexpr bool LINES = decltype(lines)::value;
+  auto run = [&](auto lines, auto sums, const LineList& L, uint32_t grid) {
+    constexpr bool LINES = decltype(lines)::value, SUMS = decltype(sums)::value;
     hipLaunchKernelGGL(k_bm_count<LINES>, dim3(grid), dim3(BLOCK), 0, s, bits, n_words, L, tile_u,
                        tile_g, tile_r, scan_status, n_status);
-    hipLaunchKernelGGL(k_bm_scan, dim3((uint32_t)chunks), dim3(BLOCK), 0, s, tile_u, tile_g,
+    if (!SUMS)
+      hipLaunchKernelGGL(k_bm_scan, dim3((uint32_t)chunks), dim3(BLOCK), 0, s, tile_u, tile_g,
                        (const uint32_t*)tile_r, (uint32_t)tiles, L, scan_status, counts,
                        reset_bytes, slots, totals);
     // the emission also writes the level-1 spans and depth-1 roots, and clears
     // the later levels' look-back words and tickets (launch_levels)
-    hipLaunchKernelGGL((k_bm_emit<K, LINES>), dim3(grid), dim3(BLOCK), 0, s, bits, n_words, L,
-                       bm_off, n_meshes, kl, (const uint32_t*)tile_u, (const uint32_t*)tile_g,
+    const BmSums bs{tile_r, counts, reset_bytes, totals, slots};
+    hipLaunchKernelGGL((k_bm_emit<K, LINES, SUMS>), dim3(grid), dim3(BLOCK), 0, s, bits, n_words,
+                       L, bs, bm_off, n_meshes, kl, (const uint32_t*)tile_u, (const uint32_t*)tile_g,
                        (K*)l1.elem, (K*)l2.elem, l2.first_child, l2.kids,
                        (const unsigned long long*)counts, spans1, n_levels, state, status,
                        tickets);
   };
   if (!line_flags) {
-    run(std::false_type{}, LineList{}, (uint32_t)tiles);
+    if (tiles <= SUM_TILES) run(std::false_type{}, std::true_type{}, LineList{}, (uint32_t)tiles);
+    else run(std::false_type{}, std::false_type{}, LineList{}, (uint32_t)tiles);
     return;
   }
   // runs of flags: at least a piece each (tile_g holds their counts for now)
@@ -1105,7 +1192,8 @@ void launch_level_first_bitmap(uint32_t* bits, uint64_t n_words, const uint64_t*
   hipLaunchKernelGGL(k_line_count, dim3(runs), dim3(BLOCK), 0, s, line_flags, n_lines, per, tile_g);
   hipLaunchKernelGGL(k_line_list, dim3(runs), dim3(BLOCK), 0, s, line_flags, n_lines, per,
                      (const uint32_t*)tile_g, line_list, n);
-  run(std::true_type{}, LineList{line_list, n}, (uint32_t)std::min<uint64_t>(tiles, LINE_GRID));
+  run(std::true_type{}, std::false_type{}, LineList{line_list, n},
+      (uint32_t)std::min<uint64_t>(tiles, LINE_GRID));
 }
 
 void launch_level_first_finalize(const LevelSpan* spans, uint32_t n_meshes, uint32_t n_levels,

@@ -92,3 +92,20 @@ def test_tile_size_changes(gpu_ctx, n, path):
     assert np.array_equal(tree.field("code"), code)
     assert np.array_equal(tree.field("parent"), parent)
     assert np.array_equal(tree.field("childs").reshape(-1, 8), childs)
+
+
+def test_tile_sums(gpu_ctx):
+    """Bitmaps of 2048 tiles, whose emission adds the tile counts up itself, and
+    of one tile more, which a scan of their own adds up; each mesh's span ends
+    at the next mesh's first tile, a single voxel's as well."""
+    from svo_amd import meshgen
+    p, t = meshgen.icosphere(3)
+    big, small = (p, t, 512), (p, t, 9)
+    one = (p[:3], np.array([[0, 1, 2]], np.int32), 1)
+    want = {id(m): po.build(*m) for m in (big, small, one)}
+    for batch in ([big], [big, one], [small, big], [one, small, one, one, small]):
+        trees, st = gpu_ctx.build_batch(batch)
+        assert not any(st)
+        for m, tree in zip(batch, trees):
+            compare(tree, want[id(m)], fields=FIELDS, check_aos=False)
+            tree.free()
