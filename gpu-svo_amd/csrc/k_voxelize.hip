@@ -560,6 +560,7 @@ __global__ void k_read_totals(const unsigned long long* slots, unsigned long lon
 // neighboring rows and triangles set bits of the same words.  A word whose
 // slot holds another goes to memory at once.
 constexpr uint32_t MAX_PER_WAVE = 32;
+constexpr uint64_t SMALL_MAX = 1 << 20;  // cells of a triangle that shares a wave, at most
 constexpr int WORD_SLOT_BITS = 9;
 constexpr uint32_t WORD_SLOTS = 1u << WORD_SLOT_BITS, NO_WORD = 0xFFFFFFFFu;
 struct WordTable {
@@ -589,8 +590,8 @@ __device__ inline void set_bits(WordTable& t, uint32_t* bitmap, uint8_t* line_fl
 template <typename K, bool BITMAP, bool ITEMS>
 __global__ __launch_bounds__(BLOCK) void k_vox_rows(
     const MeshDev* meshes, const MeshParams* params, const uint64_t* tri_base, uint32_t n_meshes,
-    uint64_t n_tris, int cb, uint32_t small_max, uint32_t per_wave, VoxOut<K> out, BigItem* big,
-    unsigned long long* big_count, uint64_t big_cap) {
+    uint64_t n_tris, int cb, uint32_t small_max, uint32_t per_wave, uint32_t scale, VoxOut<K> out,
+    BigItem* big, unsigned long long* big_count, uint64_t big_cap) {
   __shared__ RowTri s_tri[WAVES][ITEMS ? 1 : MAX_PER_WAVE];
   __shared__ uint32_t s_mark[WAVES][64];
   __shared__ K s_key[BITMAP ? 1 : WAVES][BITMAP ? 1 : STAGE];
@@ -655,7 +656,8 @@ __global__ __launch_bounds__(BLOCK) void k_vox_rows(
                          nz = S.g1[2] - S.g0[2] + 1;
           if (ITEMS) {
             rows = (uint32_t)std::min<uint64_t>(BIG_ROWS, ny * nz - row0);
-          } else if (nx * ny * nz <= (md.small_max ? md.small_max : small_max)) {
+          } else if (nx * ny * nz <= std::min<uint64_t>((uint64_t)(md.small_max ? md.small_max : small_max) * scale,
+                                                    SMALL_MAX)) {
             rows = (uint32_t)(ny * nz);
           } else {
             chunks = (uint32_t)((ny * nz + BIG_ROWS - 1) / BIG_ROWS);
@@ -708,7 +710,7 @@ __global__ __launch_bounds__(BLOCK) void k_vox_rows(
         z = (int)(r / (uint32_t)T.ny);
         y = (int)(r - (uint32_t)z * (uint32_t)T.ny);
       } else {
-        // r < 2^20 (the limit on box cells), so that the quotient of
+        // r < 2^20 (SMALL_MAX), so that the quotient of
         // r + 1/2 lies at least 2^-21 of itself from a whole number: exact
         z = (int)(((float)r + 0.5f) * T.inv_ny);
         y = (int)r - z * T.ny;
@@ -826,15 +828,23 @@ static void launch_rows(const MeshDev* meshes, const MeshParams* params, const u
   // atomics on the one key count follow each other at about 6 ns.
   uint32_t per = MAX_PER_WAVE;
   while (per > 4 && n_tris / per < (BITMAP ? 8192 : 2048)) per /= 2;
+  // The size limit is that of triangles that share a wave by 16 or 32; where
+  // fewer do, as many times larger ones may (100,000 triangles, 8 to a wave,
+  // limits of 1024 / 2048 / 4096 cells: 269 / 214 / 189 us at 2048^3, 83 / 85 /
+  // 94 at 1024^3; the batch's coarse meshes, 32 to a wave: 306 / 354 / 528).  A
+  // queued item costs a wave that stages keys its own place in the output, so
+  // that these take twice the limit (sparse hits at 4096^3: 255 / 199 / 203).
+  // The classification counts the items with the limit itself: a bound.
+  const uint32_t scale = std::max(1u, MAX_PER_WAVE / 2 / per) * (BITMAP ? 1 : 2);
   const uint64_t waves = (n_tris + per - 1) / per;
   hipLaunchKernelGGL((k_vox_rows<K, BITMAP, false>), dim3((uint32_t)((waves + WAVES - 1) / WAVES)),
                      dim3(BLOCK), 0, s, meshes, params, tri_base, n_meshes, n_tris, cb,
-                     tn.small_max_cells, per, out, big, big_count, big_cap);
+                     tn.small_max_cells, per, scale, out, big, big_count, big_cap);
   if (big_cap)
     hipLaunchKernelGGL((k_vox_rows<K, BITMAP, true>),
                        dim3((uint32_t)std::min<uint64_t>((big_cap + WAVES - 1) / WAVES, BIG_BLOCKS)),
                        dim3(BLOCK), 0, s, meshes,
-                       params, tri_base, n_meshes, n_tris, cb, tn.small_max_cells, 1u, out, big,
+                       params, tri_base, n_meshes, n_tris, cb, tn.small_max_cells, 1u, 1u, out, big,
                        big_count, big_cap);
 }
 
