@@ -105,16 +105,17 @@ __device__ inline bool edge_eq(const float* a0, const float* b0, const float* a1
 
 // Writes words [w0, w0 + n) of dst, value(i) the word w0 + i: 16-byte pieces,
 // single words where a piece lies across either end; four(i) gives the words
-// i .. i + 3 at once.  dst is 16-byte aligned.
+// i .. i + 3 at once.  dst is 16-byte aligned.  `stream`: past the caches.
 template <typename F, typename F4>
 __device__ inline void write_words(uint32_t* dst, uint64_t w0, uint32_t n, uint32_t tid,
-                                   uint32_t threads, F value, F4 four) {
+                                   uint32_t threads, F value, F4 four, bool stream = true) {
   const uint32_t head = (uint32_t)w0 & 3u;  // words of the first piece before w0
   uint32_t* p = dst + (w0 - head);
   for (uint32_t q = tid; 4 * q < head + n; q += threads) {
     const uint32_t i = 4 * q - head;  // wraps for words before w0
     if (4 * q >= head && i + 4 <= n) {
-      store_stream((uint4*)p + q, four(i));
+      if (stream) store_stream((uint4*)p + q, four(i));
+      else ((uint4*)p)[q] = four(i);
     } else {
       for (uint32_t j = 0; j < 4; ++j)
         if (i + j < n) p[4 * (uint64_t)q + j] = value(i + j);
@@ -123,10 +124,13 @@ __device__ inline void write_words(uint32_t* dst, uint64_t w0, uint32_t n, uint3
 }
 template <typename F>
 __device__ inline void write_words(uint32_t* dst, uint64_t w0, uint32_t n, uint32_t tid,
-                                   uint32_t threads, F value) {
-  write_words(dst, w0, n, tid, threads, value, [&](uint32_t i) {
-    return make_uint4(value(i), value(i + 1), value(i + 2), value(i + 3));
-  });
+                                   uint32_t threads, F value, bool stream = true) {
+  write_words(
+      dst, w0, n, tid, threads, value,
+      [&](uint32_t i) {
+        return make_uint4(value(i), value(i + 1), value(i + 2), value(i + 3));
+      },
+      stream);
 }
 
 // ---------------------------------------------------------------- emission
@@ -590,9 +594,13 @@ __global__ __launch_bounds__(8 * NB_GROUPS) void k_neighbors_level(
     }
   }
   __syncthreads();
-  // the rows, 216 * ng words from a 4-byte boundary
+  // the rows, 216 * ng words from a 4-byte boundary; the finest level's go past
+  // the caches, the others the next level reads (96 -> 86 us for the finest of
+  // 2.4 M nodes; 104 when its own rows stay in the caches as well)
   const uint64_t w0 = 27 * ((uint64_t)sg->t0 + 8 * g0);
-  write_words(nodes.neighbors, w0, 216 * ng, tid, THREADS, [&](uint32_t i) { return s_row[i]; });
+  write_words(
+      nodes.neighbors, w0, 216 * ng, tid, THREADS, [&](uint32_t i) { return s_row[i]; },
+      (kind & 255u) == 1);
 }
 
 // ---------------------------------------------------------------- kept records
@@ -637,10 +645,11 @@ __device__ inline void keep_counts(uint32_t k, uint32_t& v, uint32_t& e, uint32_
   f = __popc(k >> KEEP_FACES);
 }
 
-// One wave per block of KEEP_BLOCK nodes: counts[3 * block + {v, e, f}].
+// One wave per block of KEEP_BLOCK nodes: counts[{v, e, f} * n_blocks + block].
 constexpr uint32_t KEEP_BLOCK = 512;
 __global__ __launch_bounds__(BLOCK) void k_keep_count(const uint32_t* keep, uint64_t n_nodes,
-                                                      uint32_t* counts, const uint32_t* skip) {
+                                                      uint32_t n_blocks, uint32_t* counts,
+                                                      const uint32_t* skip) {
   if (skip && *skip) return;  // graph replay over changed sizes
   const uint64_t block = (uint64_t)blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6);
   if (block * KEEP_BLOCK >= n_nodes) return;
@@ -658,46 +667,54 @@ __global__ __launch_bounds__(BLOCK) void k_keep_count(const uint32_t* keep, uint
   se = wave_sum_u32(se);
   sf = wave_sum_u32(sf);
   if (__lane_id() == 0) {
-    counts[3 * block] = sv;
-    counts[3 * block + 1] = se;
-    counts[3 * block + 2] = sf;
+    counts[block] = sv;
+    counts[n_blocks + block] = se;
+    counts[2 * (uint64_t)n_blocks + block] = sf;
   }
 }
 
-// Exclusive sums of the block counts (one workgroup) and the totals.
-constexpr uint32_t KEEP_SCAN = 1024;
+// Exclusive sums of the block counts and the totals: a workgroup per kind, four
+// rounds' loads in flight (one workgroup for all kinds, a round at a time: 12
+// us for 6382 blocks, 5 so).
+constexpr uint32_t KEEP_SCAN = 1024, KEEP_AHEAD = 4;
 __global__ __launch_bounds__(KEEP_SCAN) void k_keep_scan(const uint32_t* counts, uint32_t n_blocks,
                                                          uint64_t* offsets,
                                                          unsigned long long* totals,
                                                          const uint32_t* skip) {
   if (skip && *skip) return;  // graph replay over changed sizes
-  __shared__ uint32_t s_wave[3][KEEP_SCAN / 64];
-  uint64_t carry[3] = {0, 0, 0};
+  __shared__ uint32_t s_wave[KEEP_AHEAD][KEEP_SCAN / 64];
+  const uint32_t* in = counts + (uint64_t)blockIdx.x * n_blocks;
+  uint64_t* out = offsets + (uint64_t)blockIdx.x * n_blocks;
+  uint64_t carry = 0;
   const uint32_t wave = threadIdx.x >> 6;
-  for (uint32_t b0 = 0; b0 < n_blocks; b0 += KEEP_SCAN) {
-    const uint32_t b = b0 + threadIdx.x;
-    uint32_t c[3], inc[3];
+  for (uint32_t b0 = 0; b0 < n_blocks; b0 += KEEP_SCAN * KEEP_AHEAD) {
+    uint32_t c[KEEP_AHEAD], inc[KEEP_AHEAD];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      c[k] = b < n_blocks ? counts[3 * (uint64_t)b + k] : 0u;
-      inc[k] = wave_incl_scan_dpp(c[k]);  // at most 1024 * 6144 over the workgroup
-      if ((threadIdx.x & 63) == 63) s_wave[k][wave] = inc[k];
+    for (uint32_t j = 0; j < KEEP_AHEAD; ++j) {
+      const uint32_t b = b0 + j * KEEP_SCAN + threadIdx.x;
+      c[j] = b < n_blocks ? in[b] : 0u;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < KEEP_AHEAD; ++j) {
+      inc[j] = wave_incl_scan_dpp(c[j]);  // at most 1024 * 6144 over the workgroup
+      if ((threadIdx.x & 63) == 63) s_wave[j][wave] = inc[j];
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
+    for (uint32_t j = 0; j < KEEP_AHEAD; ++j) {
       uint32_t pre = 0, all = 0;
       for (uint32_t w = 0; w < KEEP_SCAN / 64; ++w) {
-        const uint32_t x = s_wave[k][w];
+        const uint32_t x = s_wave[j][w];
         if (w < wave) pre += x;
         all += x;
       }
-      if (b < n_blocks) offsets[3 * (uint64_t)b + k] = carry[k] + pre + inc[k] - c[k];
-      carry[k] += all;
+      const uint32_t b = b0 + j * KEEP_SCAN + threadIdx.x;
+      if (b < n_blocks) out[b] = carry + pre + inc[j] - c[j];
+      carry += all;
     }
     __syncthreads();
   }
-  if (threadIdx.x < 3) totals[threadIdx.x] = carry[threadIdx.x];
+  if (threadIdx.x == 0) totals[blockIdx.x] = carry;
 }
 
 // The LDS slot (of a node's REC_VALS values; 10 and 11 hold width and width *
@@ -773,8 +790,8 @@ __global__ __launch_bounds__(KEEP_BLOCK) void k_keep_write(
   }
   a = pa + ia - a;
   b = pb + ib - b;
-  const uint64_t ov = offsets[3 * (uint64_t)blockIdx.x], oe = offsets[3 * (uint64_t)blockIdx.x + 1],
-                 of = offsets[3 * (uint64_t)blockIdx.x + 2];
+  const uint64_t ov = offsets[blockIdx.x], oe = offsets[gridDim.x + blockIdx.x],
+                 of = offsets[2 * (uint64_t)gridDim.x + blockIdx.x];
   if ((t & ~63u) < n_nodes)
     for_segments(segs, seg_first, n_segs, t & ~63u, t, t < n_nodes, [&](auto* sg, uint32_t d) {
       // origin and width from the level's keys, as emit_nodes has them
@@ -1025,8 +1042,8 @@ void launch_kept_records(int semantics, KeyLayout<K> kl, const NodeArrays& nodes
     hipLaunchKernelGGL(k_ref_keep, dim3((uint32_t)((n_nodes + ROW - 1) / ROW)), dim3(ROW), 0, s,
                        nodes, n_nodes, segs, seg_first, n_segs, keep);
   hipLaunchKernelGGL(k_keep_count, dim3((nb + 3) / 4), dim3(BLOCK), 0, s, (const uint32_t*)keep,
-                     n_nodes, counts, nodes.skip);
-  hipLaunchKernelGGL(k_keep_scan, dim3(1), dim3(KEEP_SCAN), 0, s, (const uint32_t*)counts, nb,
+                     n_nodes, nb, counts, nodes.skip);
+  hipLaunchKernelGGL(k_keep_scan, dim3(3), dim3(KEEP_SCAN), 0, s, (const uint32_t*)counts, nb,
                      offsets, out.totals, nodes.skip);
   hipLaunchKernelGGL(k_keep_write<K>, dim3(nb), dim3(KEEP_BLOCK), 0, s, reference, kl, nodes, n_nodes,
                      segs, seg_first, n_segs, (const uint32_t*)keep, (const uint64_t*)offsets,
