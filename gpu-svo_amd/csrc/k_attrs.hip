@@ -103,16 +103,20 @@ __device__ inline bool edge_eq(const float* a0, const float* b0, const float* a1
   return (eq3(a0, a1) && eq3(b0, b1)) || (eq3(a0, b1) && eq3(b0, a1));
 }
 
+constexpr uint32_t LINE = 32;  // words of a cache line
+
 // Writes words [w0, w0 + n) of dst, value(i) the word w0 + i: 16-byte pieces,
 // single words where a piece lies across either end; four(i) gives the words
 // i .. i + 3 at once.  dst is 16-byte aligned.  `stream`: past the caches.
 template <typename F, typename F4>
 __device__ inline void write_words(uint32_t* dst, uint64_t w0, uint32_t n, uint32_t tid,
                                    uint32_t threads, F value, F4 four, bool stream = true) {
-  const uint32_t head = (uint32_t)w0 & 3u;  // words of the first piece before w0
+  // from the cache line that w0 lies in: a wave's 1024 bytes are whole lines
+  const uint32_t head = (uint32_t)w0 & (LINE - 1);
   uint32_t* p = dst + (w0 - head);
   for (uint32_t q = tid; 4 * q < head + n; q += threads) {
     const uint32_t i = 4 * q - head;  // wraps for words before w0
+    if (4 * q + 3 < head) continue;
     if (4 * q >= head && i + 4 <= n) {
       if (stream) store_stream((uint4*)p + q, four(i));
       else ((uint4*)p)[q] = four(i);
@@ -528,7 +532,7 @@ constexpr ShareTable SHARED = make_share_table();
 // writes them, one contiguous run, in 16-byte pieces.  On the way each node's
 // records are decided: one is kept by the sharing node of the smallest index
 // (`keep`, one word per node, when set), so that the records never read the
-// rows again.  2.4 M nodes of the finest level: 940 us before, 95 now.
+// rows again.  2.4 M nodes of the finest level: 940 us before, 86 now.
 constexpr uint32_t NB_GROUPS = 32;
 __global__ __launch_bounds__(8 * NB_GROUPS) void k_neighbors_level(
     const NodeSeg* segs, const uint32_t* level_segs, const uint32_t* level_blocks,
@@ -717,81 +721,70 @@ __global__ __launch_bounds__(KEEP_SCAN) void k_keep_scan(const uint32_t* counts,
   if (threadIdx.x == 0) totals[blockIdx.x] = carry;
 }
 
-// The LDS slot (of a node's REC_VALS values; 10 and 11 hold width and width *
-// 0) of each word of a record, four bits a word.
+// Coordinates of the records in order, two bits each: 0 the node's origin bare
+// (an end without offset), 1 origin + 0, 2 origin + width.
 struct WordTable {
-  uint32_t edge[12], face[6], vert[8], ref_vert[8];
+  uint16_t edge[12], face[6], vert[8];
 };
 constexpr WordTable make_word_table() {
   WordTable t{};
-  auto slot = [](const uint8_t(&e)[3], int a) {
-    return (uint32_t)(!e[0] && !e[1] && !e[2] ? a : e[a] ? 6 + a : 3 + a);
+  auto term = [](const uint8_t(&e)[3], int a) {
+    return !e[0] && !e[1] && !e[2] ? 0 : e[a] ? 2 : 1;
   };
-  for (int w = 0; w < 84; ++w)
-    t.edge[w / 7] |= (w % 7 == 6 ? 9u : slot(EDGE_ENDS[w / 7][w % 7 / 3], w % 7 % 3)) << 4 * (w % 7);
-  for (int w = 0; w < 42; ++w)
-    t.face[w / 7] |= (w % 7 == 6 ? 9u : slot(FACE_ENDS[w / 7][w % 7 / 3], w % 7 % 3)) << 4 * (w % 7);
+  for (int w = 0; w < 6; ++w) {
+    for (int i = 0; i < 12; ++i) t.edge[i] |= (uint16_t)(term(EDGE_ENDS[i][w / 3], w % 3) << 2 * w);
+    for (int f = 0; f < 6; ++f) t.face[f] |= (uint16_t)(term(FACE_ENDS[f][w / 3], w % 3) << 2 * w);
+  }
   for (int j = 0; j < 8; ++j) {
     const uint8_t corner[3] = {(uint8_t)(j & 1), (uint8_t)(j >> 1 & 1), (uint8_t)(j >> 2 & 1)};
-    for (int a = 0; a < 3; ++a) {
-      t.vert[j] |= slot(corner, a) << 4 * a;
-      t.ref_vert[j] |= (corner[a] ? 10u : 11u) << 4 * a;
-    }
-    t.vert[j] |= 9u << 12;
-    t.ref_vert[j] |= 9u << 12;
+    for (int a = 0; a < 3; ++a) t.vert[j] |= (uint16_t)(term(corner, a) << 2 * a);
   }
   return t;
 }
 __constant__ WordTable WORDS = make_word_table();
 
-// Writes the kept records of a block of nodes: the nodes' values (from the
-// level's keys, as in the emission) and the list of kept records (node and
-// record, in order) are staged in LDS; then a thread looks up a record's
-// words, and the array's run of words is written in 16-byte pieces from LDS.
-// 173 us on 3.3 M nodes, 792 MB, and 5 for the count.  (A word at a time from
-// the list: 190, bound by its instructions.  A thread per node that wrote its
-// own records scattered 16- and 28-byte stores, after deciding twice from its
-// neighbor row which they are: 1,240 and 300 for the count.)
+// Writes one kind of the kept records of a block of nodes (grid: the blocks'
+// vertices, then their edges, then their faces, so that the stores in flight
+// lie close together): the nodes' values, from the level's keys as in the
+// emission, and the list of kept records (node and record, in order) are
+// staged in LDS; then a thread looks up a record's words, and the array's run
+// of words is written in 16-byte pieces from LDS, a wave's 1024 bytes from the
+// start of a cache line.  3.3 M nodes, 792 MB: 160 us (172 with waves that
+// begin anywhere; 190 a word at a time from the list, bound by instructions),
+// and 5 for the count.  (A thread per node that wrote its own records
+// scattered 16- and 28-byte stores, after deciding twice from its neighbor row
+// which they are: 1,240 and 300 for the count.)
 template <typename K>
 __global__ __launch_bounds__(KEEP_BLOCK) void k_keep_write(
-    bool reference, KeyLayout<K> kl, NodeArrays nodes, uint64_t n_nodes, const NodeSeg* segs,
-    const uint32_t* seg_first, uint32_t n_segs, const uint32_t* keep, const uint64_t* offsets,
-    AttrOut out) {
+    bool reference, KeyLayout<K> kl, NodeArrays nodes, uint64_t n_nodes, uint32_t n_blocks,
+    const NodeSeg* segs, const uint32_t* seg_first, uint32_t n_segs, const uint32_t* keep,
+    const uint64_t* offsets, AttrOut out) {
   if (nodes.skip && *nodes.skip) return;  // graph replay over changed sizes
-  __shared__ uint32_t s_val[KEEP_BLOCK * REC_VALS];
+  constexpr uint32_t VALS = 5;  // origin, width, owner
+  __shared__ uint32_t s_val[KEEP_BLOCK * VALS];
   __shared__ __align__(16) uint32_t s_stage[7 * KEEP_BLOCK + 4];
   __shared__ uint16_t s_list[KEEP_BLOCK * 12];
-  __shared__ uint32_t s_word[12 + 6 + 8];
-  __shared__ uint32_t s_sum[2][KEEP_BLOCK / 64];
-  const uint32_t tid = threadIdx.x, t = blockIdx.x * KEEP_BLOCK + tid;
-  if (tid < 12) s_word[tid] = WORDS.edge[tid];
-  else if (tid < 18) s_word[tid] = WORDS.face[tid - 12];
-  else if (tid < 26) s_word[tid] = reference ? WORDS.ref_vert[tid - 18] : WORDS.vert[tid - 18];
-  const uint32_t k = t < n_nodes ? keep[t] : 0u;
-  uint32_t nv, ne, nf;
-  keep_counts(k, nv, ne, nf);
-  // exclusive sums over the block: vertices (low half) and edges, faces
-  uint32_t a = nv | (ne << 16), b = nf;
-  const uint32_t ia = wave_incl_scan_dpp(a), ib = wave_incl_scan_dpp(b);
-  if ((tid & 63) == 63) {
-    s_sum[0][tid >> 6] = ia;
-    s_sum[1][tid >> 6] = ib;
-  }
+  __shared__ uint32_t s_word[12];
+  __shared__ uint32_t s_sum[KEEP_BLOCK / 64];
+  const uint32_t what = blockIdx.x / n_blocks, block = blockIdx.x - what * n_blocks;
+  const uint32_t tid = threadIdx.x, t = block * KEEP_BLOCK + tid;
+  if (tid < 12)
+    s_word[tid] = what == 1 ? WORDS.edge[tid] : what == 2 ? WORDS.face[tid % 6] : WORDS.vert[tid & 7];
+  const uint32_t all = t < n_nodes ? keep[t] : 0u;
+  const uint32_t bits = what == 0   ? all & 0xFFu
+                        : what == 1 ? all >> KEEP_EDGES & 0xFFFu
+                                    : all >> KEEP_FACES;
+  // exclusive sums over the block
+  const uint32_t inc = wave_incl_scan_dpp(__popc(bits));
+  if ((tid & 63) == 63) s_sum[tid >> 6] = inc;
   __syncthreads();
-  uint32_t ta = 0, tb = 0, pa = 0, pb = 0;
+  uint32_t count = 0, at = inc - __popc(bits);
 #pragma unroll
   for (uint32_t w = 0; w < KEEP_BLOCK / 64; ++w) {
-    if (w < tid >> 6) {
-      pa += s_sum[0][w];
-      pb += s_sum[1][w];
-    }
-    ta += s_sum[0][w];
-    tb += s_sum[1][w];
+    if (w < tid >> 6) at += s_sum[w];
+    count += s_sum[w];
   }
-  a = pa + ia - a;
-  b = pb + ib - b;
-  const uint64_t ov = offsets[blockIdx.x], oe = offsets[gridDim.x + blockIdx.x],
-                 of = offsets[2 * (uint64_t)gridDim.x + blockIdx.x];
+  const uint64_t first = offsets[blockIdx.x];
   if ((t & ~63u) < n_nodes)
     for_segments(segs, seg_first, n_segs, t & ~63u, t, t < n_nodes, [&](auto* sg, uint32_t d) {
       // origin and width from the level's keys, as emit_nodes has them
@@ -800,55 +793,74 @@ __global__ __launch_bounds__(KEEP_BLOCK) void k_keep_write(
       const K* elem = (const K*)sg->elem;
       const K code = sg->level_kind & SEG_ROOT ? kl.code(elem[0])
                                                : (K)((kl.code(elem[d >> 3]) << 3) | (K)(d & 7));
-      uint32_t* v = s_val + REC_VALS * tid;
+      uint32_t* v = s_val + VALS * tid;
 #pragma unroll
       for (uint32_t x = 0; x < 3; ++x)
-        stage_axis(v, x, sg->origin[x] + w * (float)axis_of(code, x), w);
-      v[9] = local;
-      v[10] = __float_as_uint(w * 1.0f);
-      v[11] = __float_as_uint(w * 0.0f);
-      if (local == 0) {
-        unsigned long long* first = out.totals + 4 + 3 * sg->mesh;
-        first[0] = ov + (a & 0xFFFFu);
-        first[1] = oe + (a >> 16);
-        first[2] = of + b;
-      }
+        v[x] = __float_as_uint(sg->origin[x] + w * (float)axis_of(code, x));
+      v[3] = __float_as_uint(w);
+      v[4] = local;
+      if (local == 0) out.totals[4 + 3 * sg->mesh + what] = first + at;
     });
-  // kind by kind through one list: `bits` the node's records, `at` its place
-  auto list = [&](uint32_t bits, uint32_t at) {
-    for (; bits; bits &= bits - 1u) s_list[at++] = (uint16_t)((tid << 4) | __builtin_ctz(bits));
-    __syncthreads();
-  };
-  // a vertex is a piece
-  list(k & 0xFFu, a & 0xFFFFu);
-  for (uint32_t r = tid; r < (ta & 0xFFFFu); r += KEEP_BLOCK) {
-    const uint32_t e = s_list[r], w = s_word[18 + (e & 15u)], *v = s_val + REC_VALS * (e >> 4);
-    store_stream((uint4*)out.verts + ov + r,
-                 make_uint4(v[w & 15u], v[w >> 4 & 15u], v[w >> 8 & 15u], v[w >> 12]));
-  }
+  for (uint32_t r = bits, i = at; r; r &= r - 1u)
+    s_list[i++] = (uint16_t)((tid << 4) | __builtin_ctz(r));
   __syncthreads();
-  // edges and faces, KEEP_BLOCK at a time
-  auto records = [&](uint32_t bits, uint32_t at, uint32_t count, const uint32_t* word,
-                     uint32_t* dst, uint64_t first) {
-    list(bits, at);
-    for (uint32_t c = 0; c < count; c += KEEP_BLOCK) {
-      const uint32_t n = count - c < KEEP_BLOCK ? count - c : KEEP_BLOCK;
-      const uint64_t w0 = 7 * (first + c);
-      uint32_t* stage = s_stage + (w0 & 3u);
-      if (tid < n) {
-        const uint32_t e = s_list[c + tid], w = word[e & 15u], *v = s_val + REC_VALS * (e >> 4);
-#pragma unroll
-        for (uint32_t j = 0; j < 7; ++j) stage[7 * tid + j] = v[w >> 4 * j & 15u];
-      }
-      __syncthreads();
-      write_words(
-          dst, w0, 7 * n, tid, KEEP_BLOCK, [&](uint32_t i) { return stage[i]; },
-          [&](uint32_t i) { return *(const uint4*)(stage + i); });
-      __syncthreads();
-    }
+  // word j < 3 k of a record: its coordinate's term of that axis
+  struct Node {
+    float term[3][3];
+    uint32_t owner;
   };
-  records((k >> KEEP_EDGES) & 0xFFFu, a >> 16, ta >> 16, s_word, (uint32_t*)out.edges, oe);
-  if (!reference) records(k >> KEEP_FACES, b, tb, s_word + 12, (uint32_t*)out.faces, of);
+  auto node_of = [&](uint32_t e) {
+    const uint32_t* v = s_val + VALS * (e >> 4);
+    const float w = __uint_as_float(v[3]);
+    Node n;
+#pragma unroll
+    for (uint32_t x = 0; x < 3; ++x) {
+      const float o = __uint_as_float(v[x]);
+      n.term[0][x] = o;
+      n.term[1][x] = o + 0.0f;
+      n.term[2][x] = o + w;
+      if (what == 0 && reference) {  // the reference's vertices have no origin
+        n.term[0][x] = n.term[1][x] = w * 0.0f;
+        n.term[2][x] = w * 1.0f;
+      }
+    }
+    n.owner = v[4];
+    return n;
+  };
+  auto coord = [](const Node& n, uint32_t word, uint32_t j) {
+    const uint32_t k = word >> 2 * j & 3u, x = j % 3;
+    const uint32_t a = __float_as_uint(n.term[0][x]), b = __float_as_uint(n.term[1][x]),
+                   c = __float_as_uint(n.term[2][x]);
+    return k == 0 ? a : k == 1 ? b : c;
+  };
+  if (what == 0) {  // a vertex is a piece
+    for (uint32_t r = tid; r < count; r += KEEP_BLOCK) {
+      const uint32_t e = s_list[r], w = s_word[e & 15u];
+      const Node n = node_of(e);
+      store_stream((uint4*)out.verts + first + r,
+                   make_uint4(coord(n, w, 0), coord(n, w, 1), coord(n, w, 2), n.owner));
+    }
+    return;
+  }
+  // edges and faces, KEEP_BLOCK at a time
+  uint32_t* dst = (uint32_t*)(what == 1 ? out.edges : out.faces);
+  for (uint32_t c = 0; c < count; c += KEEP_BLOCK) {
+    const uint32_t k = count - c < KEEP_BLOCK ? count - c : KEEP_BLOCK;
+    const uint64_t w0 = 7 * (first + c);
+    uint32_t* stage = s_stage + (w0 & 3u);
+    if (tid < k) {
+      const uint32_t e = s_list[c + tid], w = s_word[e & 15u];
+      const Node n = node_of(e);
+#pragma unroll
+      for (uint32_t j = 0; j < 6; ++j) stage[7 * tid + j] = coord(n, w, j);
+      stage[7 * tid + 6] = n.owner;
+    }
+    __syncthreads();
+    write_words(
+        dst, w0, 7 * k, tid, KEEP_BLOCK, [&](uint32_t i) { return stage[i]; },
+        [&](uint32_t i) { return *(const uint4*)(stage + i); });
+    __syncthreads();
+  }
 }
 
 // 168-byte SVONode records (SVO.h:20-35), one thread per 32-bit word.
@@ -1045,9 +1057,9 @@ void launch_kept_records(int semantics, KeyLayout<K> kl, const NodeArrays& nodes
                      n_nodes, nb, counts, nodes.skip);
   hipLaunchKernelGGL(k_keep_scan, dim3(3), dim3(KEEP_SCAN), 0, s, (const uint32_t*)counts, nb,
                      offsets, out.totals, nodes.skip);
-  hipLaunchKernelGGL(k_keep_write<K>, dim3(nb), dim3(KEEP_BLOCK), 0, s, reference, kl, nodes, n_nodes,
-                     segs, seg_first, n_segs, (const uint32_t*)keep, (const uint64_t*)offsets,
-                     out);
+  hipLaunchKernelGGL(k_keep_write<K>, dim3(reference ? 2 * nb : 3 * nb), dim3(KEEP_BLOCK), 0, s,
+                     reference, kl, nodes, n_nodes, nb, segs, seg_first, n_segs,
+                     (const uint32_t*)keep, (const uint64_t*)offsets, out);
 }
 
 void launch_ref_records(const float* origin, const float* width, uint64_t n_nodes,
