@@ -66,8 +66,8 @@ def stage_bytes(stats, name):
         # the caller when the same launch writes them
         return (kb + 161) * N + (kb + 9) * N // 8 + 2 * kb * U
     if name == "attr_write":
-        # vertex / edge / face records written, node origin and width read
-        return 16 * stats["n_vertices"] + 28 * stats["n_edges"] + 28 * stats["n_faces"] + 16 * N
+        # vertex / edge / face records written, a keep mask per node read
+        return 16 * stats["n_vertices"] + 28 * stats["n_edges"] + 28 * stats["n_faces"] + 4 * N
     if name == "attr_count":
         return 32 * N
     return 0
@@ -78,7 +78,8 @@ def stage_bytes(stats, name):
 # scaled by the same counters on a device-to-device copy of 1 GiB: FETCH_SIZE
 # x 2, WRITE_SIZE x 1; profiles/batch256_hbm_traffic.md).  Used to fill
 # roofline.traffic for this run's launch.
-TRAFFIC_PER_ALG_BYTE = {"attr_write": 1.000, "unique_level1": 1.00, "voxelize": 4.2}
+TRAFFIC_PER_ALG_BYTE = {"emit": 1.003, "attr_write": 1.000, "unique_level1": 1.57,
+                        "voxelize": 1.7}
 
 
 def dedup_gbs(stats, stages):

@@ -530,7 +530,7 @@ uint64_t estimate_bytes_mesh(const svo_mesh_desc* m, const svo_params* p) {
     return m && p ? estimate_bytes(m->n_points, m->n_tris, p) : 0;
   const uint64_t P = m->n_points, T = m->n_tris;
   // grid: createMeshBBCube (BaseModel.h:24-49) and the voxel size
-  // (SVO.cu:348-350), in the same float operations as k_params
+  // (SVO.cu:348-350), in the same float operations as the device (mesh_params)
   float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
   for (uint64_t i = 0; i < P; ++i)
     for (int a = 0; a < 3; ++a) {
