@@ -69,7 +69,7 @@ constexpr size_t STAGED_MIN = 1 << 20;
 bool ensure_ring(Context& C) {
   CopyRing& R = C.ring;
   if (R.pinned) return true;
-  if (hipHostMalloc(&R.pinned, CopyRing::BYTES, hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc(&R.pinned, CopyRing::BYTES, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
     hipGetLastError();
     R.pinned = nullptr;
     return false;
