@@ -69,13 +69,29 @@ constexpr size_t STAGED_MIN = 1 << 20;
 bool ensure_ring(Context& C) {
   CopyRing& R = C.ring;
   if (R.pinned) return true;
-  if (hipHostMalloc(&R.pinned, CopyRing::BYTES, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+  if (hipHostMalloc(&R.pinned, CopyRing::BYTES, hipHostMallocMapped | hipHostMallocCoherent) !=
+      hipSuccess) {
     hipGetLastError();
     R.pinned = nullptr;
     return false;
   }
   std::memset(R.flags(), 0, CopyRing::BYTES - CopyRing::SLOTS * CopyRing::PIECE);
   return true;
+}
+
+// The number of the ring's next launch: never 0, which unused flags hold.
+uint32_t next_launch(CopyRing& R) {
+  if (++R.launches == 0) ++R.launches;
+  return R.launches;
+}
+
+// Memory that the runtime knows (pinned or on a device) takes its direct copy,
+// at the link's rate (57 GB/s to pinned memory).
+bool runtime_memory(const void* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+  hipGetLastError();
+  return false;
 }
 
 // Waits until the kernel of launch `number` has set the flags of a slot.
@@ -135,7 +151,7 @@ int copy_staged(Context& C, char* dst, const char* src, size_t bytes) {
           if (emptied[end % SLOTS].load(std::memory_order_acquire) >= end / SLOTS) ++end;
           else std::this_thread::yield();
         }
-        const uint32_t k = ++R.launches;
+        const uint32_t k = next_launch(R);
         launch_ring_copy(src + sent * PIECE, std::min(bytes, end * PIECE) - sent * PIECE, R.pinned,
                          flags, sent % SLOTS, k, C.aux_stream);
         if (hipGetLastError() != hipSuccess) {
@@ -162,7 +178,7 @@ int copy_d2h(Context& C, void* dst, const void* src, size_t bytes) {
   if (!bytes) return SVO_OK;
   std::lock_guard<std::mutex> lk(C.aux_mu);
   hipSetDevice(C.device);
-  if (bytes >= STAGED_MIN && ensure_ring(C))
+  if (bytes >= STAGED_MIN && !runtime_memory(dst) && ensure_ring(C))
     return copy_staged(C, (char*)dst, (const char*)src, bytes);
   if (hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, C.aux_stream) != hipSuccess)
     return SVO_E_HIP;
@@ -832,7 +848,7 @@ int svo_query_neighbors(const svo_tree* tree, const uint32_t* node, const uint8_
       uint8_t* r_slot = (uint8_t*)(r_out + n);
       std::memcpy(r_node, node, 4 * n);
       std::memcpy(r_slot, slot, n);
-      const uint32_t number = ++R.launches;
+      const uint32_t number = next_launch(R);
       const uint32_t blocks =
           launch_query_ring(tree->out->nodes.neighbors + 27 * tree->node_base, tree->info.n_nodes,
                             r_node, r_slot, n, r_out, R.flags(), number, C.aux_stream);

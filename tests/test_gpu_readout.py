@@ -2,6 +2,7 @@
 sizes around the least that does (1 MiB), around whole pieces and around the
 ring's 8 MiB, to destinations off every alignment, from several threads at
 once, against the same bytes read in small parts."""
+import ctypes
 import threading
 
 import numpy as np
@@ -98,3 +99,21 @@ def test_threads(gpu_ctx, tree):
     for x in th:
         x.join()
     assert not bad
+
+
+@pytest.mark.parametrize("at", [0, 4])
+def test_pinned_destination(tree, at):
+    """To pinned memory, which the runtime copies to directly."""
+    hip = svo_amd.lib()  # (finds the symbols of the runtime that it has loaded)
+    for field in ("neighbors", "nodes_aos"):
+        fid = svo_amd.FIELDS[field]
+        n = int(svo_amd.lib().svo_tree_field_bytes(tree._h, fid))
+        ptr = ctypes.c_void_p()
+        assert hip.hipHostMalloc(ctypes.byref(ptr), ctypes.c_size_t(n + 64), 0) == 0
+        buf = np.ctypeslib.as_array((ctypes.c_uint8 * (n + 64)).from_address(ptr.value))
+        buf[:] = 0xAB
+        svo_amd._check(svo_amd.lib().svo_tree_copy_field(tree._h, fid, ptr.value + at, n), field)
+        ok = np.array_equal(buf[at: at + n], _whole(tree, field))
+        ok = ok and (buf[:at] == 0xAB).all() and (buf[at + n:] == 0xAB).all()
+        assert hip.hipHostFree(ptr) == 0
+        assert ok, field
