@@ -11,13 +11,15 @@
 //   k_tile_hist   digit counts of each tile, stored digit-major
 //   k_tile_scan   per digit, exclusive scan over the tiles and the total
 //   k_scatter     the digits' offsets from the totals; ranks the tile's keys
-//                 stably with wave64 match masks (8 ballots per 64 keys) and writes them through an LDS reorder so the
-//                 stores are contiguous within each digit run
+//                 stably with wave64 match masks (8 ballots per 64 keys) and
+//                 writes them through an LDS reorder so the stores are
+//                 contiguous within each digit run
 // Stable, so the passes compose into a full LSD sort.  HBM traffic for n keys
-// of B bytes and P passes: P * 3*n*B, plus 2 KB of counts per tile and pass.  A single-pass scatter with decoupled look-back reads and
-// writes the keys once per pass, but over thousands of tiles its look-back
-// chain (and the digits' status words each tile walks) bounds the pass; here
-// no tile waits on another.
+// of B bytes and P passes: P * 3*n*B, plus 2 KB of counts per tile and pass.
+// A single-pass scatter with decoupled look-back reads and writes the keys
+// once per pass, but over thousands of tiles its look-back chain (and the
+// digits' status words each tile walks) bounds the pass; here no tile waits on
+// another.
 //
 // A pass of a million 4-byte keys costs 16 us, 10 of it the three launches
 // (83 -> 68 us for 30 bits since the digits' offsets come from the passes' own
