@@ -355,7 +355,8 @@ int Lane::ensure_pinned(size_t bytes) {
   pinned = nullptr;
   pinned_bytes = 0;
   const size_t want = std::max<size_t>(bytes, 1 << 16);
-  if (hipHostMalloc(&pinned, want, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) return SVO_E_HIP;
+  if (hipHostMalloc(&pinned, want, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
+    return SVO_E_HIP;
   pinned_bytes = want;
   return SVO_OK;
 }
