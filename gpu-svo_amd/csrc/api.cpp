@@ -1,6 +1,5 @@
 // api.cpp -- the C ABI declared in include/svo/svo.h.
 #include <algorithm>
-#include <atomic>
 #include <chrono>
 #include <cstdio>
 #include <cstring>
@@ -9,6 +8,7 @@
 #include <vector>
 
 #include "svo_host.h"
+#include "svo_ring.h"
 
 using namespace svo;
 
@@ -110,65 +110,21 @@ int wait_slot(Context& C, const uint32_t* flags, uint32_t number, uint32_t block
 // Under C.aux_mu.
 int copy_staged(Context& C, char* dst, const char* src, size_t bytes) {
   CopyRing& R = C.ring;
-  constexpr size_t PIECE = CopyRing::PIECE, SLOTS = CopyRing::SLOTS;
   uint32_t* const flags = R.flags();
-  const size_t n = (bytes + PIECE - 1) / PIECE;
-  auto size_of = [&](size_t i) { return std::min(PIECE, bytes - i * PIECE); };
-  std::atomic<size_t> arrived{0}, claimed{0};
-  std::atomic<bool> stop{false};
-  std::atomic<size_t> emptied[SLOTS] = {};  // pieces copied out of each slot
-  auto take = [&](size_t i) {
-    std::memcpy(dst + i * PIECE, (const char*)R.pinned + i % SLOTS * PIECE, size_of(i));
-    emptied[i % SLOTS].store(i / SLOTS + 1, std::memory_order_release);
+  uint32_t number[CopyRing::SLOTS];  // of each slot's last launch: its flags' value on arrival
+  auto launch = [&](size_t at, size_t n, size_t slot) -> int {
+    const uint32_t k = next_launch(R);
+    launch_ring_copy(src + at, n, R.pinned, flags, slot, k, C.aux_stream);
+    if (hipGetLastError() != hipSuccess) return SVO_E_HIP;
+    for (size_t i = 0; i * CopyRing::PIECE < n; ++i) number[(slot + i) % CopyRing::SLOTS] = k;
+    return SVO_OK;
   };
-  auto work = [&] {
-    for (size_t i; (i = claimed.fetch_add(1)) < n;) {
-      while (arrived.load(std::memory_order_acquire) <= i) {
-        if (stop.load()) return;
-        std::this_thread::yield();
-      }
-      take(i);
-    }
+  auto wait = [&](size_t slot) {
+    return wait_slot(C, flags + slot * RING_BLOCKS, number[slot]);
   };
-  std::vector<std::thread> helpers;
-  try {
-    const size_t want = std::min<size_t>(CopyRing::THREADS, n / 2);
-    helpers.reserve(want);
-    for (size_t k = 0; k < want; ++k) helpers.emplace_back(work);
-  } catch (...) {  // no more threads: those that started, or this one, do it
-  }
-  // A piece's flags hold its launch's number once it has arrived.
-  int st = SVO_OK;
-  size_t sent = 0;
-  uint32_t number[SLOTS];
-  for (size_t i = 0; i < n && st == SVO_OK; ++i) {
-    // as many pieces as have free slots, half a ring at a time
-    if (sent <= i || (sent < n && sent - i <= SLOTS / 2)) {
-      size_t end = sent;
-      while (end < n && emptied[end % SLOTS].load(std::memory_order_acquire) >= end / SLOTS) ++end;
-      if (end - sent >= std::min(SLOTS / 2, n - sent) || sent <= i) {
-        while (end <= i) {  // the slot of piece i is being emptied
-          if (emptied[end % SLOTS].load(std::memory_order_acquire) >= end / SLOTS) ++end;
-          else std::this_thread::yield();
-        }
-        const uint32_t k = next_launch(R);
-        launch_ring_copy(src + sent * PIECE, std::min(bytes, end * PIECE) - sent * PIECE, R.pinned,
-                         flags, sent % SLOTS, k, C.aux_stream);
-        if (hipGetLastError() != hipSuccess) {
-          st = SVO_E_HIP;
-          break;
-        }
-        for (; sent < end; ++sent) number[sent % SLOTS] = k;
-      }
-    }
-    st = wait_slot(C, flags + i % SLOTS * RING_BLOCKS, number[i % SLOTS]);
-    if (st != SVO_OK) break;
-    arrived.store(i + 1, std::memory_order_release);
-    if (helpers.empty()) take(i);
-  }
-  if (st != SVO_OK) stop.store(true);
-  else work();
-  for (auto& t : helpers) t.join();
+  int st = empty_ring(dst, bytes, (const char*)R.pinned, CopyRing::PIECE, CopyRing::SLOTS,
+                      CopyRing::THREADS, launch, wait,
+                      [](auto& work) { return std::thread(work); });
   // the ring is used again only after this launch's last stores
   if (hipStreamSynchronize(C.aux_stream) != hipSuccess) st = SVO_E_HIP;
   return st;
