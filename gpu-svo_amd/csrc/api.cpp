@@ -114,8 +114,8 @@ int copy_staged(Context& C, char* dst, const char* src, size_t bytes) {
   uint32_t number[CopyRing::SLOTS];  // of each slot's last launch: its flags' value on arrival
   auto launch = [&](size_t at, size_t n, size_t slot) -> int {
     const uint32_t k = next_launch(R);
-    launch_ring_copy(src + at, n, R.pinned, flags, slot, k, C.aux_stream);
-    if (hipGetLastError() != hipSuccess) return SVO_E_HIP;
+    if (launch_ring_copy(src + at, n, R.pinned, flags, slot, k, C.aux_stream) != hipSuccess)
+      return SVO_E_HIP;
     for (size_t i = 0; i * CopyRing::PIECE < n; ++i) number[(slot + i) % CopyRing::SLOTS] = k;
     return SVO_OK;
   };
@@ -805,11 +805,11 @@ int svo_query_neighbors(const svo_tree* tree, const uint32_t* node, const uint8_
       std::memcpy(r_node, node, 4 * n);
       std::memcpy(r_slot, slot, n);
       const uint32_t number = next_launch(R);
-      const uint32_t blocks =
-          launch_query_ring(tree->out->nodes.neighbors + 27 * tree->node_base, tree->info.n_nodes,
-                            r_node, r_slot, n, r_out, R.flags(), number, C.aux_stream);
-      if (hipGetLastError() != hipSuccess) return SVO_E_HIP;
-      const int st = wait_slot(C, R.flags(), number, blocks);
+      if (launch_query_ring(tree->out->nodes.neighbors + 27 * tree->node_base, tree->info.n_nodes,
+                            r_node, r_slot, n, r_out, R.flags(), number,
+                            C.aux_stream) != hipSuccess)
+        return SVO_E_HIP;
+      const int st = wait_slot(C, R.flags(), number, query_ring_blocks(n));
       if (st == SVO_OK) std::memcpy(out, r_out, 4 * n);
       return st;
     }

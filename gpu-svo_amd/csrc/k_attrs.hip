@@ -1005,10 +1005,10 @@ void launch_check_equal(const void* got, const void* want, uint64_t bytes, uint3
                      (const uint32_t*)got, (const uint32_t*)want, n, flag);
 }
 
-void launch_ring_copy(const void* src, uint64_t bytes, void* ring, uint32_t* flags, uint64_t slot,
-                      uint32_t number, hipStream_t s) {
-  hipLaunchKernelGGL(k_ring_copy, dim3(RING_BLOCKS), dim3(BLOCK), 0, s, (const char*)src, bytes,
-                     (char*)ring, flags, slot, number);
+hipError_t launch_ring_copy(const void* src, uint64_t bytes, void* ring, uint32_t* flags,
+                            uint64_t slot, uint32_t number, hipStream_t s) {
+  void* args[] = {&src, &bytes, &ring, &flags, &slot, &number};
+  return hipLaunchKernel((const void*)k_ring_copy, dim3(RING_BLOCKS), dim3(BLOCK), args, 0, s);
 }
 
 void launch_copy_u32(uint32_t* dst, const uint32_t* src, uint64_t n, hipStream_t s) {
@@ -1086,14 +1086,15 @@ void launch_query_neighbors(const uint32_t* neighbors, uint64_t n_nodes, const u
                      slot, n, out);
 }
 
-uint32_t launch_query_ring(const uint32_t* neighbors, uint64_t n_nodes, const uint32_t* node,
-                           const uint8_t* slot, uint64_t n, uint32_t* out, uint32_t* flags,
-                           uint32_t number, hipStream_t s) {
-  const uint32_t blocks =
-      (uint32_t)std::min<uint64_t>((n + QUERY_THREADS - 1) / QUERY_THREADS, RING_BLOCKS);
-  hipLaunchKernelGGL(k_query_ring, dim3(blocks), dim3(QUERY_THREADS), 0, s, neighbors, n_nodes,
-                     node, slot, n, out, flags, number);
-  return blocks;
+uint32_t query_ring_blocks(uint64_t n) {
+  return (uint32_t)std::min<uint64_t>((n + QUERY_THREADS - 1) / QUERY_THREADS, RING_BLOCKS);
+}
+hipError_t launch_query_ring(const uint32_t* neighbors, uint64_t n_nodes, const uint32_t* node,
+                             const uint8_t* slot, uint64_t n, uint32_t* out, uint32_t* flags,
+                             uint32_t number, hipStream_t s) {
+  void* args[] = {&neighbors, &n_nodes, &node, &slot, &n, &out, &flags, &number};
+  return hipLaunchKernel((const void*)k_query_ring, dim3(query_ring_blocks(n)),
+                         dim3(QUERY_THREADS), args, 0, s);
 }
 
 template void launch_kept_records<uint32_t>(int, KeyLayout<uint32_t>, const NodeArrays&, uint64_t,

@@ -232,11 +232,12 @@ void launch_emit(const EmitArgs<K>& a, hipStream_t s);
 void launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s);
 // Copies `bytes` device bytes into a pinned ring of RING_SLOTS pieces from
 // slot `slot` on (at most the whole ring), piece after piece; the RING_BLOCKS
-// flags of a piece's slot become `number` when it has arrived.
+// flags of a piece's slot become `number` when it has arrived.  Returns the
+// launch's own status (hipGetLastError could be an earlier error of the thread).
 constexpr size_t RING_PIECE = 512 << 10, RING_SLOTS = 16;
 constexpr uint32_t RING_BLOCKS = 32;
-void launch_ring_copy(const void* src, uint64_t bytes, void* ring, uint32_t* flags, uint64_t slot,
-                      uint32_t number, hipStream_t s);
+hipError_t launch_ring_copy(const void* src, uint64_t bytes, void* ring, uint32_t* flags,
+                            uint64_t slot, uint32_t number, hipStream_t s);
 // Copies n words; either side may be pinned host memory.  For a pass's tables
 // and readbacks of a few KB: 2 to 4 us, and less host time than asynchronous
 // copies (five of them read the levels back in 25 to 40 us).
@@ -275,11 +276,13 @@ void launch_ref_records(const float* origin, const float* width, uint64_t n_node
 // 168-byte SVONode records for nodes [first, first + n) (32-bit codes).
 void launch_pack_aos(const NodeArrays& nodes, uint64_t first, uint64_t n, void* dst,
                      hipStream_t s);
-// The same with node, slot and out in pinned host memory; the first flags, as
-// many as returned, become `number` when the answers are there.
-uint32_t launch_query_ring(const uint32_t* neighbors, uint64_t n_nodes, const uint32_t* node,
-                           const uint8_t* slot, uint64_t n, uint32_t* out, uint32_t* flags,
-                           uint32_t number, hipStream_t s);
+// The same with node, slot and out in pinned host memory; the first
+// query_ring_blocks(n) flags become `number` when the answers are there.
+// Returns the launch's own status.
+uint32_t query_ring_blocks(uint64_t n);
+hipError_t launch_query_ring(const uint32_t* neighbors, uint64_t n_nodes, const uint32_t* node,
+                             const uint8_t* slot, uint64_t n, uint32_t* out, uint32_t* flags,
+                             uint32_t number, hipStream_t s);
 void launch_query_neighbors(const uint32_t* neighbors, uint64_t n_nodes, const uint32_t* node,
                             const uint8_t* slot, uint64_t n, uint32_t* out, hipStream_t s);
 
