@@ -94,17 +94,11 @@ bool runtime_memory(const void* p) {
   return false;
 }
 
-// Waits until the kernel of launch `number` has set the flags of a slot.
+// Waits until the kernel of launch `number` has set the flags of a slot (an
+// error when the stream has ended without them).
 int wait_slot(Context& C, const uint32_t* flags, uint32_t number, uint32_t blocks = RING_BLOCKS) {
-  for (uint32_t b = 0, polls = 0; b < blocks;) {
-    if (__atomic_load_n(flags + b, __ATOMIC_ACQUIRE) == number) {
-      ++b;
-    } else if (++polls % 4096 == 0 && hipStreamQuery(C.aux_stream) != hipErrorNotReady &&
-               __atomic_load_n(flags + b, __ATOMIC_ACQUIRE) != number) {
-      return SVO_E_HIP;  // the stream has ended without it: a device error
-    }
-  }
-  return SVO_OK;
+  auto busy = [&] { return hipStreamQuery(C.aux_stream) == hipErrorNotReady; };
+  return wait_flags(flags, blocks, number, busy) ? SVO_OK : SVO_E_HIP;
 }
 
 // Under C.aux_mu.

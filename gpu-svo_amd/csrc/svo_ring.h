@@ -1,17 +1,61 @@
-// svo_ring.h -- the host's side of the pinned ring: how the pieces of a
-// read-out that the device puts there reach the caller's memory.  What is done
-// to the device comes in as callables.
+// svo_ring.h -- the host's side of the pinned ring: waits for what the device
+// puts there, and how the pieces of a read-out reach the caller's memory.  What
+// is done to the device comes in as callables.
 #pragma once
 #include <stddef.h>
 #include <stdint.h>
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstring>
 #include <thread>
 #include <vector>
 
 namespace svo {
+
+// The pauses of a thread that waits for the device or for another thread.  For
+// SPIN it only yields: a lookup is answered within 100 us and a piece of a
+// read-out arrives 10 us after the one before.  What takes longer stands behind
+// other work, a build's emission on the same hardware queue for instance, and
+// may take milliseconds: then it sleeps for an eighth of the time waited so far,
+// a millisecond at most.
+class Backoff {
+  using Clock = std::chrono::steady_clock;
+
+ public:
+  static constexpr Clock::duration SPIN = std::chrono::microseconds(200),
+                                   NAP_MAX = std::chrono::milliseconds(1);
+  bool sleeps() const { return sleeps_; }
+  void pause() {
+    const Clock::duration waited = Clock::now() - start_;
+    sleeps_ = waited > SPIN;
+    if (sleeps_) std::this_thread::sleep_for(std::min(waited / 8, NAP_MAX));
+    else std::this_thread::yield();
+  }
+
+ private:
+  Clock::time_point start_ = Clock::now();
+  bool sleeps_ = false;
+};
+
+// Waits until n flags hold `number`; false when busy() says that the device has
+// ended its work and one of them does not.
+template <class Busy>
+bool wait_flags(const uint32_t* flags, uint32_t n, uint32_t number, Busy busy) {
+  Backoff wait;
+  for (uint32_t b = 0, polls = 0; b < n;) {
+    if (__atomic_load_n(flags + b, __ATOMIC_ACQUIRE) == number) {
+      ++b;
+    } else if (wait.sleeps()) {
+      wait.pause();
+      if (!busy() && __atomic_load_n(flags + b, __ATOMIC_ACQUIRE) != number) return false;
+    } else if (++polls % 32 == 0) {
+      wait.pause();
+    }
+  }
+  return true;
+}
 
 // Copies `bytes` bytes to dst through the `slots` pieces of `piece` bytes at
 // `ring` (at most 64).  launch(at, n, slot) has the device put bytes
@@ -37,9 +81,10 @@ int empty_ring(char* dst, size_t bytes, const char* ring, size_t piece, size_t s
   };
   auto work = [&] {
     for (size_t i; (i = claimed.fetch_add(1)) < n;) {
+      Backoff wait;
       while (arrived.load(std::memory_order_acquire) <= i) {
         if (stop.load()) return;
-        std::this_thread::yield();
+        wait.pause();
       }
       take(i);
     }
@@ -59,9 +104,10 @@ int empty_ring(char* dst, size_t bytes, const char* ring, size_t piece, size_t s
       size_t end = sent;
       while (end < n && is_free(end)) ++end;
       if (end - sent >= std::min(slots / 2, n - sent) || sent <= i) {
+        Backoff wait;
         while (end <= i) {  // the slot of piece i is being emptied
           if (is_free(end)) ++end;
-          else std::this_thread::yield();
+          else wait.pause();
         }
         st = launch(sent * piece, std::min(bytes, end * piece) - sent * piece, sent % slots);
         if (st) break;
