@@ -1100,6 +1100,7 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
       bm_bytes / BITMAP_LINE_BYTES <= sizeof(K) * cap[1]) {
     line_flags = (uint8_t*)lv[1].elem;
     launch_fill_u32((uint32_t*)line_flags, 0u, bm_bytes / BITMAP_LINE_BYTES / 4, s);
+    timer.mark("line_flags");
   }
   launch_voxelize<K>(d_md, d_par, d_tb, n, T, plan.cb, plan.tuning, keys_a, bitmap, d_bo, line_flags,
                      d_cnt + 2, d_slots, big, d_cnt + 3, n_big, s);
