@@ -68,8 +68,6 @@ def stage_bytes(stats, name):
     if name == "attr_write":
         # vertex / edge / face records written, a keep mask per node read
         return 16 * stats["n_vertices"] + 28 * stats["n_edges"] + 28 * stats["n_faces"] + 4 * N
-    if name == "attr_count":
-        return 32 * N
     return 0
 
 

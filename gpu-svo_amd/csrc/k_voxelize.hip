@@ -65,19 +65,6 @@ __device__ inline uint32_t find_mesh_wave(const uint64_t* base, uint32_t n_meshe
   return lo;
 }
 
-// Morton code stepping: the bits of one axis are a dilated integer, so adding
-// one to that axis is an add through the other axes' bits (set to one so the
-// carry passes them) and a merge back.  x is bits 0, 3, 6, ...; y and z the
-// same shifted by one and two.
-template <typename K>
-__device__ inline K morton_x_mask() {
-  return sizeof(K) == 4 ? (K)0x09249249u : (K)0x1249249249249249ull;
-}
-template <typename K>
-__device__ inline K dilated_inc(K code, K mask) {
-  return (((code | ~mask) + (K)1) & mask) | (code & ~mask);
-}
-
 // ------------------------------------------------------------------ bbox
 // Everything a pass sets up before its first kernel: the control tables from
 // pinned host memory, the boxes at their start values, zeros.
@@ -613,6 +600,7 @@ __global__ __launch_bounds__(BLOCK) void k_vox_rows(
   }
   uint64_t n_hits = 0;      // bitmap path: this lane's
   uint32_t staged = 0;      // key path: keys in s_key (the same in every lane)
+  // the code's bits of x: 0, 3, 6, ...
   constexpr K MX = (K)(sizeof(K) == 4 ? 0x09249249u : 0x1249249249249249ull);
   auto flush = [&]() {
     wave_sync();
@@ -764,7 +752,8 @@ __global__ __launch_bounds__(BLOCK) void k_vox_rows(
           if (staged > STAGE - 256) flush();
         }
         x += 4;
-        // x + 4 in the code: the bits of x from bit 2 on (bits 0 and 1 are zero)
+        // x + 4 in the code: one added to the bits of x from bit 2 on (bits 0 and
+        // 1 are zero), the others set so that the carry passes them
         constexpr K M4 = MX & ~(K)9;
         code = (((code | ~M4) + 1) & M4) | (code & ~M4);
       }

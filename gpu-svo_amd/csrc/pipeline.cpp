@@ -2,17 +2,18 @@
 //
 // Host C++ drives the gfx950 kernels on one stream (a "lane"):
 //
-//   A0  bbox -> grid params -> triangle classification     (1 readback: box-cell
-//                                                            total, big chunks)
-//   A1  voxelize -> radix sort -> unique + level 1 -> levels 2..L
-//                                                         (1 readback: per-mesh
-//                                                          depth / level spans)
-//   B   node records -> roots -> voxels -> neighbors -> vertex/edge/face
-//                                                         (1 readback: totals)
+//   A0  boxes and index check -> grid params and triangle classification
+//                                  (readback: candidate cells, big-triangle items)
+//   A1  voxelize -> level 1 (occupancy bitmap, or radix sort) -> levels 2..L
+//                                  (readback: counters, level counts, spans,
+//                                   tree states, grid params)
+//   B   emission: node arrays, voxel codes, the reference's neighbor slots and
+//       records in one launch; intended neighbors level by level, and kept
+//       records, after it          (kept records only: their totals come back)
 //
-// The readbacks size the next phase's buffers exactly; inside a phase every
-// launch shape is fixed by host-known bounds and every data-dependent count
-// is read by the kernels from device memory.  A single mesh is a batch of one;
+// The readbacks size the next phase's buffers; inside a phase every launch
+// shape is fixed by host-known bounds and every data-dependent count is read by
+// the kernels from device memory.  A single mesh is a batch of one;
 // a batch sorts composite (mesh, Morton) keys, so all meshes share every
 // launch.  Reference correspondence: SparseVoxelOctree::create (SVO.cu:341-520)
 // and constructNodeAtrributes (SVO.cu:730-735).
@@ -1183,7 +1184,6 @@ int run_typed(Context& C, Lane& L, const std::vector<MeshInput>& in, const Plan&
       if (Lm.n_nodes >= (1ull << 32)) mstat[i] = SVO_E_RES_LIMIT;  // uint32 node links
     }
     if (mstat[i] != SVO_OK) Lm.n_nodes = 0;
-    Lm.key_out_bits = plan.code_bytes * 8;
     N += Lm.n_nodes;
     node_base[i + 1] = N;
   }
@@ -1593,15 +1593,15 @@ int run_set(Context& C, const std::vector<MeshInput>& in, const std::vector<uint
 // ------------------------------------------------------------------ batch plans
 // A batch recorded once and replayed as one HIP graph: an eager run of each
 // sub-batch pass on a lane of the plan's own records the host values of its
-// three readbacks (PassRecord) and sizes the lane's workspaces; the same
-// passes are then captured -- the sub-batches as parallel branches forked
-// from one stream -- with the readbacks replaced by device-side comparisons
-// against the recorded values.  A replay is one graph launch and one stream
-// synchronization; it recomputes every output from the (device-resident)
-// inputs into the recorded output blocks, and a set flag (a count, span or
-// total that differs from the recorded run) makes svo_plan_run fall back to
-// an eager build.  Replaces the per-level host synchronizations of the
-// reference's level loop (SVO.cu:383-495) by one per batch.
+// readbacks (PassRecord: levels and record totals) and sizes the lane's
+// workspaces; the same passes are then captured -- the sub-batches as parallel
+// branches forked from one stream -- with the readbacks replaced by device-side
+// comparisons against the recorded values.  A replay is one graph launch and
+// one stream synchronization; it recomputes every output from the
+// (device-resident) inputs into the recorded output blocks, and a set flag (a
+// count, span or total that differs from the recorded run) makes svo_plan_run
+// fall back to an eager build.  Replaces the per-level host synchronizations of
+// the reference's level loop (SVO.cu:383-495) by one per batch.
 BatchPlan::~BatchPlan() {
   Context& C = *ctx;
   hipSetDevice(C.device);

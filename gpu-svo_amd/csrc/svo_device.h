@@ -68,18 +68,6 @@ template <>
 __host__ __device__ inline uint64_t morton3<uint64_t>(uint32_t x, uint32_t y, uint32_t z) {
   return spread3_64(x) | (spread3_64(y) << 1) | (spread3_64(z) << 2);
 }
-template <typename K>
-__host__ __device__ inline void demorton3(K m, uint32_t& x, uint32_t& y, uint32_t& z) {
-  if (sizeof(K) == 4) {
-    x = compact3_32((uint32_t)m);
-    y = compact3_32((uint32_t)m >> 1);
-    z = compact3_32((uint32_t)m >> 2);
-  } else {
-    x = (uint32_t)compact3_64((uint64_t)m);
-    y = (uint32_t)compact3_64((uint64_t)m >> 1);
-    z = (uint32_t)compact3_64((uint64_t)m >> 2);
-  }
-}
 
 // Streaming 16-byte store for output written once and not read back by the
 // same kernel (non-temporal hint: no need to keep the lines in the caches).

@@ -160,7 +160,6 @@ struct MeshNodeLayout {
   uint64_t node_base;    // first node of the mesh in the batch arrays
   uint64_t n_nodes;
   uint32_t depth;
-  uint32_t key_out_bits; // 32 or 64
   uint64_t level_off[24];// node offset of each level within the mesh (level l at [l-1])
   float width[24];       // node width per level
 };

@@ -100,11 +100,6 @@ __device__ inline void block_excl_scan256_2(uint32_t& a, uint32_t& b, uint32_t* 
   b = pb + ib - b;
 }
 
-// Three-component exclusive scan (vertex, edge, face counts).
-struct U64x3 {
-  uint64_t a, b, c;
-};
-
 // Loads cnt <= N consecutive keys p[0 .. cnt) into kk (the rest zero); with
 // vec set (p 16-byte aligned) a full run is loaded as 16-byte vectors.
 template <typename K, int N>
