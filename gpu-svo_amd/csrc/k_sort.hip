@@ -43,7 +43,10 @@ static_assert(RADIX == BLOCK, "a thread per digit");
 // Keys per lane and tile: fewer for fewer keys, so that small sorts have
 // workgroups for the 256 CUs.  30-bit keys of 4 bytes, 4 / 8 / 16 keys a lane:
 // 100,000 keys 47 / 54 / 60 us, a million 78 / 68 / 71, four million
-// 193 / 146 / 125.
+// 193 / 146 / 125.  The size is chosen by `cap`, which is the number of keys at
+// the library's sort entry points; a build's pass knows its candidate cells
+// only, 5.5 times its keys where triangles are large (4.95 of 27.45 million on
+// 150,000 triangles at 4096^3), so that its tiles are those of a larger sort.
 constexpr uint64_t TINY_SORT = 1ull << 18, SMALL_SORT = 1ull << 21;
 constexpr int KPT_TINY = 4, KPT_SMALL = 8, KPT_LARGE = 16;
 
