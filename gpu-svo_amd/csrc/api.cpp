@@ -785,8 +785,8 @@ int svo_query_neighbors(const svo_tree* tree, const uint32_t* node, const uint8_
   Context& C = *tree->ctx;
   // In the pinned ring: the kernel reads the lookups there and puts the answers
   // there, with no copy and no synchronization (1000 lookups: 33.5 us with three
-  // copies, 22 so; 50,000: 59 and 42; 131,072: 82 and 65; above, copies:
-  // 200,000 in 101 us).
+  // copies, 20 so, 24 where the wait comes to ask for the stream's state;
+  // 50,000: 59 and 42; 131,072: 82 and 65; above, copies: 200,000 in 101 us).
   constexpr uint64_t RING_LOOKUPS = 1 << 17;
   static_assert(9 * RING_LOOKUPS <= CopyRing::SLOTS * CopyRing::PIECE, "they fit the ring");
   if (n <= RING_LOOKUPS) {
@@ -804,11 +804,6 @@ int svo_query_neighbors(const svo_tree* tree, const uint32_t* node, const uint8_
                             r_node, r_slot, n, r_out, R.flags(), number,
                             C.aux_stream) != hipSuccess)
         return SVO_E_HIP;
-      // The runtime puts the marker by which it will know the kernel's end
-      // behind it now and not into the next synchronization of the device:
-      // 22.7 us where lookups follow each other and 30 with a synchronization
-      // after each (18.2 and 35 without).
-      (void)hipStreamQuery(C.aux_stream);
       const int st = wait_slot(C, R.flags(), number, query_ring_blocks(n));
       if (st == SVO_OK) std::memcpy(out, r_out, 4 * n);
       return st;
